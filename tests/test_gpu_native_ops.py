@@ -1,0 +1,67 @@
+"""The autograd nodes behind the tprime operators: gradients of outputs that are not all used, graphs that are walked
+twice or differentiated, saved-tensor hooks, and traces through the dispatcher.  Reference: the same operator with the
+missing gradients passed as zeros, or run eagerly; the kernels are deterministic, so results are compared bit for bit."""
+
+import pytest
+import torch
+
+import torchprime_amd as tpa
+from tests.util import randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF = torch.bfloat16
+
+
+def _leaf(shape, seed, dtype=BF):
+  return randn(shape, seed, dtype).to(DEV).requires_grad_(True)
+
+
+@pytest.mark.parametrize("used", [0, 1])
+def test_one_of_two_outputs_used(used):
+  q, k = _leaf((1, 4, 9, 64), 1), _leaf((1, 2, 9, 64), 2)
+  cos, sin = randn((1, 9, 64), 3, BF).to(DEV), randn((1, 9, 64), 4, BF).to(DEV)
+  x, r, w = _leaf((5, 96), 5), _leaf((5, 96), 6), _leaf((96,), 7)
+  for make, leaves in ((lambda: tpa.ops.rope_apply(q, k, cos, sin), [q, k]), (lambda: tpa.ops.add_rmsnorm(x, r, w, 1e-5), [x, r, w])):
+    outs = make()
+    g = [torch.zeros_like(o) for o in outs]
+    g[used] = randn(outs[used].shape, 8, BF).to(DEV)
+    want = torch.autograd.grad(outs, leaves, g)
+    got = torch.autograd.grad(make()[used], leaves, g[used])
+    for a, b in zip(got, want):
+      assert torch.equal(a, b)
+
+
+def test_second_walk_and_second_derivative():
+  x, w = _leaf((5, 96), 1), _leaf((96,), 2)
+  y = tpa.ops.rmsnorm(x, w, 1e-5).float().sum()
+  a = torch.autograd.grad(y, [x, w], retain_graph=True)
+  b = torch.autograd.grad(y, [x, w])
+  assert all(torch.equal(s, t) for s, t in zip(a, b))
+  with pytest.raises(RuntimeError, match="second time"):
+    torch.autograd.grad(y, [x, w])
+  (g,) = torch.autograd.grad(tpa.ops.rmsnorm(x, w, 1e-5).float().pow(2).sum(), x, create_graph=True)
+  with pytest.raises(RuntimeError, match="not implemented"):
+    g.float().sum().backward()
+
+
+def test_saved_tensor_hooks_and_trace():
+  from functorch.compile import aot_function, nop
+
+  q = _leaf((1, 2, 70, 128), 1)
+  x, w = _leaf((5, 96), 2), _leaf((96,), 3)
+
+  def f(q, x, w):
+    return tpa.ops.attention(q, q, q), tpa.ops.rmsnorm(x, w, 1e-5), tpa.ops.swiglu(x, x)
+
+  def grads(outs):
+    return torch.autograd.grad([o.float().sum() for o in outs], [q, x, w])
+
+  want = f(q, x, w)
+  g_want = grads(want)
+  with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(DEV)):
+    hooked = f(q, x, w)
+  traced = aot_function(f, fw_compiler=nop, bw_compiler=nop)(q, x, w)
+  for outs in (hooked, traced):
+    assert all(torch.equal(a, b) for a, b in zip(outs, want))
+    assert all(torch.equal(a, b) for a, b in zip(grads(outs), g_want))

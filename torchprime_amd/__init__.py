@@ -13,8 +13,8 @@ functions in model/{llama,mixtral,
 deepseek_v3}/model.py
 =====================================  =============================================================
 
-Compute runs only in ``libtprime_hip.so`` (hand-written HIP kernels reached through ``torch.library``
-ops in :mod:`torchprime_amd.ops`); there is no CPU or torch-math fallback.
+Compute runs only in ``libtprime_hip.so`` (hand-written HIP kernels reached through the ``tprime`` operators of
+``_tprime_ops.so``, see :mod:`torchprime_amd.ops`); there is no CPU or torch-math fallback.
 """
 
 from . import kernel_utils, ops, parallelism_utils, rope  # noqa: F401

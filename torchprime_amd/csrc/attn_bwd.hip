@@ -1948,42 +1948,24 @@ static int dispatch_bwd(const BwdArgs& a, int causal, hipStream_t st, void* cons
   return launch_bwd<T, DQK, DV, false, false>(a, st, ev);
 }
 
-// One element type per translation unit: this file is compiled twice (TP_BWD_F16 = 0 and 1, side by side, which
-// halves the build time).  Either unit defines its own dispatcher over the head dims; the bf16 unit also holds
-// the C entry points.  A dispatcher returns TP_DIMS_NOT_BUILT for head dims it has no kernels for.
-#ifndef TP_BWD_F16
-#define TP_BWD_F16 0
-#endif
-constexpr int TP_DIMS_NOT_BUILT = -1000;
-int bwd_by_dims_bf16(const BwdArgs& a, int Dqk, int Dv, int causal, hipStream_t st, void* const* ev);
-int bwd_by_dims_f16(const BwdArgs& a, int Dqk, int Dv, int causal, hipStream_t st, void* const* ev);
-template <typename T>
-static int bwd_by_dims(const BwdArgs& a, int Dqk, int Dv, int causal, hipStream_t st, void* const* ev) {
-  // (TP_ONLY_HEAD_DIM_128 / TP_ONLY_HEAD_DIM_WIDE: build options for quick timing builds of one head-dim pair)
-#ifndef TP_ONLY_HEAD_DIM_WIDE
-  if (Dqk == 128 && Dv == 128) return dispatch_bwd<T, 128, 128>(a, causal, st, ev);
-#endif
-#if !defined(TP_ONLY_HEAD_DIM_128) && !defined(TP_ONLY_HEAD_DIM_WIDE)
-  if (Dqk == 64 && Dv == 64) return dispatch_bwd<T, 64, 64>(a, causal, st, ev);
-#endif
-#ifndef TP_ONLY_HEAD_DIM_128
-  if (Dqk == 192 && Dv == 128) return dispatch_bwd<T, 192, 128>(a, causal, st, ev);
-#endif
-  return TP_DIMS_NOT_BUILT;
-}
-#if TP_BWD_F16
-int bwd_by_dims_f16(const BwdArgs& a, int Dqk, int Dv, int causal, hipStream_t st, void* const* ev) {
-  return bwd_by_dims<f16_t>(a, Dqk, Dv, causal, st, ev);
-}
-#else
-int bwd_by_dims_bf16(const BwdArgs& a, int Dqk, int Dv, int causal, hipStream_t st, void* const* ev) {
-  return bwd_by_dims<bf16_t>(a, Dqk, Dv, causal, st, ev);
+// One element type and head-dim pair per translation unit: this file is compiled once per pair and type
+// (TP_BWD_UNIT(f) names the unit's dispatcher, TP_BWD_T / TP_BWD_DQK / TP_BWD_DV its kernels) and once more without
+// them for the C entry points, side by side: the kernels' tile bodies take minutes to compile one after the other.
+int bwd_bf16_64_64(const BwdArgs& a, int causal, hipStream_t st, void* const* ev);
+int bwd_bf16_128_128(const BwdArgs& a, int causal, hipStream_t st, void* const* ev);
+int bwd_bf16_192_128(const BwdArgs& a, int causal, hipStream_t st, void* const* ev);
+int bwd_f16_64_64(const BwdArgs& a, int causal, hipStream_t st, void* const* ev);
+int bwd_f16_128_128(const BwdArgs& a, int causal, hipStream_t st, void* const* ev);
+int bwd_f16_192_128(const BwdArgs& a, int causal, hipStream_t st, void* const* ev);
+#ifdef TP_BWD_UNIT
+int TP_BWD_UNIT(const BwdArgs& a, int causal, hipStream_t st, void* const* ev) {
+  return dispatch_bwd<TP_BWD_T, TP_BWD_DQK, TP_BWD_DV>(a, causal, st, ev);
 }
 #endif
 
 }  // namespace tp
 
-#if !TP_BWD_F16
+#ifndef TP_BWD_UNIT
 using namespace tp;
 
 extern "C" int tp_attn_bwd_dq_first(int Skv, int Dqk, int Dv, int causal, int has_seg, int masked, int dtype) {
@@ -2069,9 +2051,11 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   a.band_lo = BAND_INF;  // plain causality (used by the causal kernels only)
   a.band_hi = 0;
   hipStream_t st = (hipStream_t)stream;
-  const int rc = dtype == TP_BF16 ? bwd_by_dims_bf16(a, Dqk, Dv, causal, st, events) : bwd_by_dims_f16(a, Dqk, Dv, causal, st, events);
-  TP_REQUIRE(rc != TP_DIMS_NOT_BUILT, TP_ERR_UNSUPPORTED, "tp_attn_bwd: head dims (qk=%d, v=%d) not built", Dqk, Dv);
-  return rc;
+  const bool bf = dtype == TP_BF16;
+  if (Dqk == 128 && Dv == 128) return (bf ? bwd_bf16_128_128 : bwd_f16_128_128)(a, causal, st, events);
+  if (Dqk == 64 && Dv == 64) return (bf ? bwd_bf16_64_64 : bwd_f16_64_64)(a, causal, st, events);
+  if (Dqk == 192 && Dv == 128) return (bf ? bwd_bf16_192_128 : bwd_f16_192_128)(a, causal, st, events);
+  TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "tp_attn_bwd: head dims (qk=%d, v=%d) not built", Dqk, Dv);
 }
 
 extern "C" int tp_attn_bwd_ex(const void* dout, const void* q, const void* k, const void* v, const void* out,
@@ -2133,4 +2117,4 @@ extern "C" int tp_attn_bwd(const void* dout, const void* q, const void* k, const
                         k_strides, v_strides, o_strides, dq_strides, dk_strides, dv_strides, sm_scale, causal, dtype, stream,
                         nullptr);
 }
-#endif  // !TP_BWD_F16
+#endif  // !TP_BWD_UNIT

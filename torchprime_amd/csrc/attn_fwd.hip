@@ -623,6 +623,20 @@ static int dispatch_fwd(const FwdArgs& a, int B, int causal, hipStream_t st) {
   return launch_fwd<T, DQK, DV, true, false>(b, B, st);
 }
 
+// One element type and head-dim pair per translation unit, as in attn_bwd.hip; the unit without a pair holds the C
+// entry points.
+int fwd_bf16_64_64(const FwdArgs& a, int B, int causal, hipStream_t st);
+int fwd_bf16_128_128(const FwdArgs& a, int B, int causal, hipStream_t st);
+int fwd_bf16_192_128(const FwdArgs& a, int B, int causal, hipStream_t st);
+int fwd_f16_64_64(const FwdArgs& a, int B, int causal, hipStream_t st);
+int fwd_f16_128_128(const FwdArgs& a, int B, int causal, hipStream_t st);
+int fwd_f16_192_128(const FwdArgs& a, int B, int causal, hipStream_t st);
+#ifdef TP_FWD_UNIT
+int TP_FWD_UNIT(const FwdArgs& a, int B, int causal, hipStream_t st) {
+  return dispatch_fwd<TP_FWD_T, TP_FWD_DQK, TP_FWD_DV>(a, B, causal, st);
+}
+#endif
+
 // fp32 operands: attn_fwd_f32.hip
 int attn_fwd_f32(const void* q, const void* k, const void* v, const int32_t* seg, void* out, float* lse, int B, int Hq, int Hkv,
                  int Sq, int Skv, int Dqk, int Dv, const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
@@ -630,6 +644,7 @@ int attn_fwd_f32(const void* q, const void* k, const void* v, const int32_t* seg
 
 }  // namespace tp
 
+#ifndef TP_FWD_UNIT
 using namespace tp;
 
 static int attn_fwd_impl(const void* q, const void* k, const void* v, const int32_t* seg, void* out, float* lse,
@@ -665,17 +680,10 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, const int3
   a.band_lo = BAND_INF;  // plain causality (used by the causal kernels only)
   a.band_hi = 0;
   hipStream_t st = (hipStream_t)stream;
-#define TP_FWD(T, DQ, DVV) return dispatch_fwd<T, DQ, DVV>(a, B, causal, st)
-  if (dtype == TP_BF16) {
-    if (Dqk == 128 && Dv == 128) TP_FWD(bf16_t, 128, 128);
-    if (Dqk == 64 && Dv == 64) TP_FWD(bf16_t, 64, 64);
-    if (Dqk == 192 && Dv == 128) TP_FWD(bf16_t, 192, 128);
-  } else {
-    if (Dqk == 128 && Dv == 128) TP_FWD(f16_t, 128, 128);
-    if (Dqk == 64 && Dv == 64) TP_FWD(f16_t, 64, 64);
-    if (Dqk == 192 && Dv == 128) TP_FWD(f16_t, 192, 128);
-  }
-#undef TP_FWD
+  const bool bf = dtype == TP_BF16;
+  if (Dqk == 128 && Dv == 128) return (bf ? fwd_bf16_128_128 : fwd_f16_128_128)(a, B, causal, st);
+  if (Dqk == 64 && Dv == 64) return (bf ? fwd_bf16_64_64 : fwd_f16_64_64)(a, B, causal, st);
+  if (Dqk == 192 && Dv == 128) return (bf ? fwd_bf16_192_128 : fwd_f16_192_128)(a, B, causal, st);
   TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "tp_attn_fwd: head dims (qk=%d, v=%d) not built", Dqk, Dv);
 }
 
@@ -717,3 +725,4 @@ extern "C" int tp_attn_fwd_biased(const void* q, const void* k, const void* v, c
                        make_mask_ext(q_positions, causal, causal_offset, window_left, window_right, logits_soft_cap, sm_scale, bias,
                                      bias_strides));
 }
+#endif  // !TP_FWD_UNIT

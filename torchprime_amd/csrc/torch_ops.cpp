@@ -1,0 +1,867 @@
+// The ``tprime`` operators: registration with torch's dispatcher, autograd nodes and the Python entry points, over the
+// C ABI of libtprime_hip.so.
+//
+// Why this file is native: a pass over a small problem is nothing but host work.  With the operators defined in Python
+// (torch.library.custom_op around ctypes calls) one operator cost 25-45 us of host time forward and 50-80 us with its
+// backward, five to ten times what its kernel runs for at small sizes, and the gradients of outputs nobody uses (the
+// LSE, the 1 / rms) were zero-filled tensors, one more launch each.  Here an operator is one allocation per output, one
+// launch and one autograd node.
+//
+// What an operator is made of:
+//   *_cuda      checks, output allocation, the launch (registered for the CUDA key)
+//   *_autograd  saves what the backward needs in a node and redispatches below autograd (registered for the Autograd
+//               key).  The nodes call the backward operators through the dispatcher as well, so traces (fake tensors,
+//               AOT autograd) see tprime::*_bwd.
+// The backward operators have no derivative of their own: differentiating through one raises.
+#include <torch/extension.h>
+#include <torch/library.h>
+
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include <algorithm>
+#include <mutex>
+#include <tuple>
+#include <unordered_map>
+
+#include "../../include/tprime_hip.h"
+
+namespace {
+
+using at::Tensor;
+using c10::optional;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+typedef const std::optional<Tensor>& OptTensor;
+typedef std::array<int64_t, 3> Strides3;
+
+// ---- helpers ---------------------------------------------------------------------------------------------------
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kBFloat16: return TP_BF16;
+    case at::kHalf: return TP_F16;
+    case at::kFloat: return TP_F32;
+    default: TORCH_CHECK_TYPE(false, "unsupported dtype ", t, "; supported: bfloat16, float16, float32");
+  }
+}
+
+// status of a C ABI call -> the exception the Python binding (_lib.call) raises for it
+void check(int rc, const char* name) {
+  if (C10_LIKELY(rc == TP_OK)) return;
+  const char* msg = tp_last_error();
+  if (rc == TP_ERR_BAD_ARG) TORCH_CHECK_VALUE(false, name, " failed (status ", rc, "): ", msg);
+  if (rc == TP_ERR_UNSUPPORTED) TORCH_CHECK_NOT_IMPLEMENTED(false, name, " failed (status ", rc, "): ", msg);
+  TORCH_CHECK(false, name, " failed (status ", rc, "): ", msg);
+}
+
+// All tensors on one GPU; the kernels have no CPU implementation.
+struct OneGpu {
+  optional<c10::Device> dev;
+  void add(const Tensor& t) {
+    if (!t.defined()) return;
+    TORCH_CHECK(t.is_cuda(), "torchprime_amd ops run on MI355X only: got a tensor on '", t.device(),
+                "'. Move the inputs to the GPU (there is no CPU path).");
+    if (!dev) dev = t.device();
+    else TORCH_CHECK(t.device() == *dev, "tensors on different devices: ", *dev, " and ", t.device());
+  }
+  void add(OptTensor t) { if (t.has_value()) add(*t); }
+};
+template <typename... Ts>
+c10::Device require_gpu(const Ts&... ts) {
+  OneGpu g;
+  (g.add(ts), ...);
+  return *g.dev;
+}
+
+void* stream_of(c10::Device dev) { return (void*)c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+
+const Tensor& undef() { static const Tensor t; return t; }
+const Tensor& val(OptTensor t) { return t.has_value() ? *t : undef(); }
+void* opt_ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+Tensor empty_f32(at::IntArrayRef size, const Tensor& like) { return at::empty(size, like.options().dtype(at::kFloat)); }
+
+// (..., n) seen as rows of n elements: the tensor itself where its memory already is rows at one stride
+struct Rows {
+  Tensor t;  // keeps a copy alive
+  int64_t rows, cols, stride;
+  void* ptr() const { return t.data_ptr(); }
+};
+Rows rows_of(const Tensor& x, bool align16) {
+  const int64_t h = x.size(-1);
+  if (x.is_contiguous()) {
+    const int64_t rows = h > 0 ? x.numel() / h : 0;
+    if (!align16 || ((reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0) && (h * x.element_size()) % 16 == 0)) return {x, rows, h, h};
+  }
+  Tensor x2 = x.reshape({-1, h});
+  const bool bad = align16 ? (x2.stride(-1) != 1 || (x2.stride(0) * x2.element_size()) % 16 != 0 ||
+                              reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 != 0)
+                           : (x2.stride(-1) != 1 || (x2.size(0) > 1 && x2.stride(0) < h));
+  if (bad) x2 = x2.contiguous();
+  return {x2, x2.size(0), h, x2.size(0) > 1 ? x2.stride(0) : h};
+}
+
+// New (B,H,S,D') tensor.  Head-minor inputs (the (B,S,H,D)-memory views the attention modules build with
+// .view(B,S,H,D).transpose(1,2)) get the same head-minor memory order, so the caller's transpose(1,2).contiguous()
+// afterwards is free; anything else gets plain contiguous memory.
+Tensor empty_like_heads(const Tensor& x, int64_t D) {
+  const int64_t B = x.size(0), H = x.size(1), S = x.size(2);
+  if (x.stride(1) < x.stride(2)) return at::empty_strided({B, H, S, D}, {S * H * D, D, H * D, 1}, x.options());
+  return at::empty({B, H, S, D}, x.options());
+}
+// 16-byte rows with a unit inner stride, copied only if they are not
+Tensor prep_heads(const Tensor& t) {
+  const int64_t e = t.element_size();
+  const bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && (t.stride(0) * e) % 16 == 0 &&
+                  (t.stride(1) * e) % 16 == 0 && (t.stride(2) * e) % 16 == 0;
+  return ok ? t : t.contiguous();
+}
+Strides3 strides3(const Tensor& t) { return {t.stride(0), t.stride(1), t.stride(2)}; }
+
+template <typename F>
+struct Op;  // typed handle of one operator, looked up once
+template <typename R, typename... A>
+struct Op<R(A...)> {
+  c10::TypedOperatorHandle<R(A...)> h;
+  explicit Op(const char* name) : h(c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<R(A...)>()) {}
+  R operator()(A... a) const { return h.call(std::forward<A>(a)...); }
+};
+#define TP_OP(fn, ...)                                  \
+  static const auto& op_##fn() {                        \
+    static const Op<__VA_ARGS__> op("tprime::" #fn);    \
+    return op;                                          \
+  }
+
+typedef std::tuple<Tensor, Tensor> T2;
+typedef std::tuple<Tensor, Tensor, Tensor> T3;
+TP_OP(rmsnorm_fwd, T2(const Tensor&, const Tensor&, double))
+TP_OP(rmsnorm_bwd, T2(const Tensor&, const Tensor&, const Tensor&, const Tensor&))
+TP_OP(add_rmsnorm_fwd, T3(const Tensor&, const Tensor&, const Tensor&, double))
+TP_OP(add_rmsnorm_bwd, T2(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&))
+TP_OP(rope_table, T2(const Tensor&, const Tensor&, double, at::ScalarType))
+TP_OP(rope_apply, T2(const Tensor&, const Tensor&, const Tensor&, const Tensor&, OptTensor, int64_t, bool))
+TP_OP(attn_fwd, T2(const Tensor&, const Tensor&, const Tensor&, OptTensor, double, bool))
+TP_OP(attn_bwd, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, OptTensor, double, bool))
+TP_OP(attn_fwd_masked, T2(const Tensor&, const Tensor&, const Tensor&, OptTensor, OptTensor, double, bool, int64_t, int64_t, int64_t,
+                          double, OptTensor))
+TP_OP(attn_bwd_masked, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, OptTensor, OptTensor,
+                          double, bool, int64_t, int64_t, int64_t, double, OptTensor))
+TP_OP(l2norm_fwd, T2(const Tensor&, double))
+TP_OP(l2norm_bwd, Tensor(const Tensor&, const Tensor&, const Tensor&))
+TP_OP(scale_rows, Tensor(const Tensor&, const Tensor&))
+TP_OP(swiglu_fwd, Tensor(const Tensor&, const Tensor&))
+TP_OP(swiglu_bwd, T2(const Tensor&, const Tensor&, const Tensor&))
+TP_OP(cross_entropy_fwd, T3(const Tensor&, const Tensor&, int64_t))
+TP_OP(cross_entropy_bwd, Tensor(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, int64_t))
+
+// ---- autograd plumbing -----------------------------------------------------------------------------------------
+// A node with its saved tensors in one array.  ``bwd`` runs the backward operator: below autograd in an ordinary
+// backward, through it when a graph of the backward is being recorded (the operator then raises when that graph is
+// differentiated).
+struct OpNode : torch::autograd::Node {
+  std::vector<SavedVariable> saved;
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto& s : saved) s.reset_data();
+  }
+  Tensor get(size_t i) { return saved[i].unpack(shared_from_this()); }
+  void keep(const Tensor& t, bool is_output = false) { saved.emplace_back(t, is_output); }
+  virtual variable_list bwd(variable_list&& grads) = 0;
+  variable_list apply(variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (at::GradMode::is_enabled()) return bwd(std::move(grads));
+    at::AutoDispatchBelowADInplaceOrView below;
+    return bwd(std::move(grads));
+  }
+};
+template <typename N, typename... Ts>
+std::shared_ptr<N> make_node(const Ts&... inputs) {
+  const bool fw = (torch::autograd::isFwGradDefined(inputs) || ...);
+  TORCH_CHECK_NOT_IMPLEMENTED(!fw, "the tprime operators have no forward-mode derivative");
+  if (!torch::autograd::compute_requires_grad(inputs...)) return nullptr;
+  std::shared_ptr<N> n(new N(), torch::autograd::deleteNode);
+  n->set_next_edges(torch::autograd::collect_next_edges(inputs...));
+  return n;
+}
+variable_list list2(T2&& r) { return {std::move(std::get<0>(r)), std::move(std::get<1>(r))}; }
+
+// ---- RMSNorm ---------------------------------------------------------------------------------------------------
+void check_weight(const Tensor& weight, int64_t hidden) {
+  TORCH_CHECK_VALUE(weight.dim() == 1 && weight.size(0) == hidden, "weight shape (", weight.sizes(), ") does not match hidden size ", hidden);
+}
+
+T2 rmsnorm_fwd_cuda(const Tensor& x, const Tensor& weight, double eps) {
+  const c10::Device dev = require_gpu(x, weight);
+  check_weight(weight, x.size(-1));
+  c10::DeviceGuard guard(dev);
+  const Rows r = rows_of(x, false);
+  const Tensor w = weight.contiguous();
+  Tensor y = at::empty(x.sizes(), x.options().dtype(at::result_type(weight, x)));
+  Tensor rstd = empty_f32({r.rows}, x);
+  if (r.rows)
+    check(tp_rmsnorm_fwd(r.ptr(), w.data_ptr(), y.data_ptr(), (float*)rstd.data_ptr(), r.rows, (int)r.cols, r.stride, r.cols, (float)eps,
+                         dtype_code(x.scalar_type()), dtype_code(w.scalar_type()), stream_of(dev)), "tp_rmsnorm_fwd");
+  return {y, rstd};
+}
+
+T2 rmsnorm_bwd_cuda(const Tensor& dy, const Tensor& x, const Tensor& weight, const Tensor& rstd) {
+  const c10::Device dev = require_gpu(dy, x, weight, rstd);
+  c10::DeviceGuard guard(dev);
+  const Rows xr = rows_of(x, false), gr = rows_of(dy, false);
+  const Tensor w = weight.contiguous();
+  Tensor dx = at::empty(x.sizes(), x.options()), dw = at::empty({xr.cols}, w.options());
+  if (xr.rows == 0) return {dx, dw.zero_()};
+  Tensor ws = empty_f32({(int64_t)tp_rmsnorm_bwd_workspace_bytes(xr.rows, (int)xr.cols) / 4}, x);
+  check(tp_rmsnorm_bwd(gr.ptr(), xr.ptr(), w.data_ptr(), (const float*)rstd.data_ptr(), dx.data_ptr(), dw.data_ptr(), (float*)ws.data_ptr(),
+                       xr.rows, (int)xr.cols, gr.stride, xr.stride, xr.cols, dtype_code(x.scalar_type()), dtype_code(w.scalar_type()),
+                       stream_of(dev)), "tp_rmsnorm_bwd");
+  return {dx, dw};
+}
+
+struct RmsNormNode : OpNode {
+  std::string name() const override { return "TprimeRmsNormBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor()};
+    const Tensor x = get(0), w = get(1);
+    return list2(op_rmsnorm_bwd()(g[0].to(at::result_type(w, x)), x, w, get(2)));
+  }
+};
+T2 rmsnorm_fwd_autograd(const Tensor& x, const Tensor& weight, double eps) {
+  auto node = make_node<RmsNormNode>(x, weight);
+  T2 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_rmsnorm_fwd()(x, weight, eps); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    node->keep(x); node->keep(weight); node->keep(std::get<1>(r));
+  }
+  return r;
+}
+
+// (y, h, rstd): h = residual + x, y = RMSNorm(h) * weight, in one pass
+T3 add_rmsnorm_fwd_cuda(const Tensor& x, const Tensor& residual, const Tensor& weight, double eps) {
+  const c10::Device dev = require_gpu(x, residual, weight);
+  TORCH_CHECK_VALUE(residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type(), "residual (", residual.sizes(), ")/",
+                    residual.scalar_type(), " must match x (", x.sizes(), ")/", x.scalar_type());
+  check_weight(weight, x.size(-1));
+  c10::DeviceGuard guard(dev);
+  const Rows xr = rows_of(x, false), rr = rows_of(residual, false);
+  const Tensor w = weight.contiguous();
+  Tensor y = at::empty(x.sizes(), x.options().dtype(at::result_type(weight, x))), h = at::empty(x.sizes(), x.options());
+  Tensor rstd = empty_f32({xr.rows}, x);
+  if (xr.rows)
+    check(tp_add_rmsnorm_fwd(xr.ptr(), rr.ptr(), w.data_ptr(), h.data_ptr(), y.data_ptr(), (float*)rstd.data_ptr(), xr.rows, (int)xr.cols,
+                             xr.stride, rr.stride, xr.cols, xr.cols, (float)eps, dtype_code(x.scalar_type()), dtype_code(w.scalar_type()),
+                             stream_of(dev)), "tp_add_rmsnorm_fwd");
+  return {y, h, rstd};
+}
+
+T2 add_rmsnorm_bwd_cuda(const Tensor& dy, const Tensor& dh, const Tensor& h, const Tensor& weight, const Tensor& rstd) {
+  const c10::Device dev = require_gpu(dy, dh, h, weight, rstd);
+  c10::DeviceGuard guard(dev);
+  const Rows hr = rows_of(h, false), gr = rows_of(dy, false), dr = rows_of(dh, false);
+  const Tensor w = weight.contiguous();
+  Tensor dx = at::empty(h.sizes(), h.options()), dw = at::empty({hr.cols}, w.options());
+  if (hr.rows == 0) return {dx, dw.zero_()};
+  Tensor ws = empty_f32({(int64_t)tp_rmsnorm_bwd_workspace_bytes(hr.rows, (int)hr.cols) / 4}, h);
+  check(tp_add_rmsnorm_bwd(gr.ptr(), dr.ptr(), hr.ptr(), w.data_ptr(), (const float*)rstd.data_ptr(), dx.data_ptr(), dw.data_ptr(),
+                           (float*)ws.data_ptr(), hr.rows, (int)hr.cols, gr.stride, dr.stride, hr.stride, hr.cols,
+                           dtype_code(h.scalar_type()), dtype_code(w.scalar_type()), stream_of(dev)), "tp_add_rmsnorm_bwd");
+  return {dx, dw};
+}
+
+struct AddRmsNormNode : OpNode {
+  std::string name() const override { return "TprimeAddRmsNormBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined() && !g[1].defined()) return {Tensor(), Tensor(), Tensor()};
+    const Tensor h = get(0), w = get(1), rstd = get(2);
+    const auto out_dtype = at::result_type(w, h);
+    const Tensor dy = g[0].defined() ? g[0].to(out_dtype) : at::zeros_like(h, h.options().dtype(out_dtype));
+    T2 r = g[1].defined() ? op_add_rmsnorm_bwd()(dy, g[1].to(h.scalar_type()), h, w, rstd) : op_rmsnorm_bwd()(dy, h, w, rstd);
+    return {std::get<0>(r), std::get<0>(r), std::get<1>(r)};
+  }
+};
+T3 add_rmsnorm_fwd_autograd(const Tensor& x, const Tensor& residual, const Tensor& weight, double eps) {
+  auto node = make_node<AddRmsNormNode>(x, residual, weight);
+  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_add_rmsnorm_fwd()(x, residual, weight, eps); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    torch::autograd::set_history(std::get<1>(r), node);
+    node->keep(std::get<1>(r), true); node->keep(weight); node->keep(std::get<2>(r));
+  }
+  return r;
+}
+
+// ---- rotary ----------------------------------------------------------------------------------------------------
+// cos/sin tables (Bp, S, 2*half) from inv_freq (half) and position_ids (Bp, S)
+T2 rope_table_cuda(const Tensor& inv_freq, const Tensor& position_ids, double attention_scaling, at::ScalarType dtype) {
+  const c10::Device dev = require_gpu(inv_freq, position_ids);
+  TORCH_CHECK_VALUE(position_ids.dim() == 2 && inv_freq.dim() == 1, "expected inv_freq (half,) and position_ids (batch, seq)");
+  c10::DeviceGuard guard(dev);
+  const Tensor f = inv_freq.to(at::kFloat).contiguous(), p = position_ids.to(at::kFloat).contiguous();
+  const int64_t Bp = p.size(0), S = p.size(1), half = f.size(0);
+  Tensor cos = at::empty({Bp, S, 2 * half}, f.options().dtype(dtype)), sin = at::empty({Bp, S, 2 * half}, f.options().dtype(dtype));
+  check(tp_rope_table((const float*)f.data_ptr(), (const float*)p.data_ptr(), cos.data_ptr(), sin.data_ptr(), (int)Bp, (int)S, (int)half,
+                      (float)attention_scaling, dtype_code(dtype), stream_of(dev)), "tp_rope_table");
+  return {cos, sin};
+}
+
+// cos[position_ids] raises IndexError for ids outside the table (model/mixtral/model.py:136-137); so does this.  The
+// check is a device reduction and a host synchronisation, so its verdict is kept per tensor object (a weak reference
+// and the version counter, never the address alone): a model hands the same position_ids to every layer and to the
+// backward of each.
+void check_positions(const Tensor& pos, int64_t table_rows) {
+  struct Entry { c10::weak_intrusive_ptr<c10::TensorImpl> ref; uint32_t version; int64_t numel, rows; };
+  static std::mutex mu;
+  static std::unordered_map<c10::TensorImpl*, Entry> verdicts;
+  c10::TensorImpl* impl = pos.unsafeGetTensorImpl();
+  const bool tracked = !pos.is_inference();
+  const uint32_t version = tracked ? (uint32_t)pos._version() : 0;
+  if (tracked) {
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = verdicts.find(impl);
+    if (it != verdicts.end() && !it->second.ref.expired() && it->second.version == version && it->second.numel == pos.numel() &&
+        it->second.rows == table_rows) return;
+  }
+  int64_t lo = 0, hi = 0;
+  if (pos.numel()) {
+    const Tensor both = at::stack({pos.min(), pos.max()}).cpu();
+    lo = both.const_data_ptr<int64_t>()[0];
+    hi = both.const_data_ptr<int64_t>()[1];
+  }
+  TORCH_CHECK_INDEX(lo >= -table_rows && hi < table_rows, "position id ", hi >= table_rows ? hi : lo,
+                    " is out of bounds for a rotary table of ", table_rows, " rows");
+  TORCH_CHECK_NOT_IMPLEMENTED(lo >= 0, "negative position ids (indexing the table from its end) are not supported");
+  if (!tracked) return;
+  std::lock_guard<std::mutex> lock(mu);
+  if (verdicts.size() >= 64) {  // drop what died; if all live, start over
+    for (auto it = verdicts.begin(); it != verdicts.end();) it = it->second.ref.expired() ? verdicts.erase(it) : std::next(it);
+    if (verdicts.size() >= 64) verdicts.clear();
+  }
+  verdicts.insert_or_assign(impl, Entry{c10::weak_intrusive_ptr<c10::TensorImpl>(pos.getIntrusivePtr()), version, pos.numel(), table_rows});
+}
+
+// interleaved: 0 rotate-half, 1 DeepSeek ([evens | odds] output), 2 adjacent pairs in place (Llama-4)
+T2 rope_apply_cuda(const Tensor& q_, const Tensor& k_, const Tensor& cos_, const Tensor& sin_, OptTensor pos_, int64_t interleaved,
+                   bool backward) {
+  const c10::Device dev = require_gpu(q_, k_, cos_, sin_, pos_);
+  TORCH_CHECK_VALUE(q_.dim() == 4 && k_.dim() == 4, "rotary apply expects (batch, heads, seq, dim) tensors");
+  c10::DeviceGuard guard(dev);
+  const int64_t B = q_.size(0), Hq = q_.size(1), S = q_.size(2), D = q_.size(3);
+  TORCH_CHECK_VALUE(k_.size(0) == B && k_.size(2) == S && k_.size(3) == D && k_.scalar_type() == q_.scalar_type(), "q (", q_.sizes(),
+                    ") and k (", k_.sizes(), ") disagree on batch/seq/dim or dtype");
+  Tensor cos = cos_.to(q_.scalar_type()), sin = sin_.to(q_.scalar_type()), pos;
+  const Tensor q = prep_heads(q_), k = prep_heads(k_);
+  int64_t cs_b, cs_s, pos_b = 0, table_rows = 0;
+  if (pos_.has_value()) {
+    // table gather (Mixtral): cos/sin are (T, D), pos is (B or 1, S) integer
+    TORCH_CHECK_VALUE(cos.dim() == 2, "with position_ids the cos/sin tables must be (max_pos, dim)");
+    cos = cos.contiguous();
+    sin = sin.contiguous();
+    pos = pos_->to(at::kLong).contiguous();
+    if (pos.dim() == 1) pos = pos.unsqueeze(0);
+    TORCH_CHECK_VALUE(pos.size(-1) == S && (pos.size(0) == 1 || pos.size(0) == B), "position_ids shape (", pos.sizes(),
+                      ") does not match (batch, seq) = (", B, ", ", S, ")");
+    check_positions(pos, cos.size(0));
+    cs_b = 0; cs_s = cos.stride(0); pos_b = pos.size(0) == B && B > 1 ? pos.stride(0) : 0; table_rows = cos.size(0);
+  } else {
+    if (cos.dim() == 2) { cos = cos.unsqueeze(0); sin = sin.unsqueeze(0); }
+    TORCH_CHECK_VALUE(cos.dim() == 3 && cos.size(1) == S && cos.size(2) == D && (cos.size(0) == 1 || cos.size(0) == B), "cos/sin shape (",
+                      cos.sizes(), ") does not broadcast to (batch, seq, dim) = (", B, ", ", S, ", ", D, ")");
+    if (cos.stride(-1) != 1 || sin.strides() != cos.strides()) { cos = cos.contiguous(); sin = sin.contiguous(); }
+    cs_b = cos.size(0) == B && B > 1 ? cos.stride(0) : 0;
+    cs_s = cos.stride(1);
+  }
+  Tensor qo = empty_like_heads(q, D), ko = empty_like_heads(k, D);
+  const Strides3 qs = strides3(q), ks = strides3(k), qos = strides3(qo), kos = strides3(ko);
+  check(tp_rope_apply(q.data_ptr(), k.data_ptr(), cos.data_ptr(), sin.data_ptr(), (const int64_t*)opt_ptr(pos), qo.data_ptr(), ko.data_ptr(),
+                      (int)B, (int)Hq, (int)k.size(1), (int)S, (int)D, qs.data(), ks.data(), qos.data(), kos.data(), cs_b, cs_s, pos_b,
+                      table_rows, (int)interleaved, (int)backward, dtype_code(q.scalar_type()), stream_of(dev)), "tp_rope_apply");
+  return {qo, ko};
+}
+
+struct RopeNode : OpNode {
+  bool has_pos, backward;
+  int64_t interleaved;
+  // a gradient that did not arrive (only one of the two outputs is used) is zero
+  std::array<std::vector<int64_t>, 2> sizes;
+  at::TensorOptions opts;
+  std::string name() const override { return "TprimeRopeApplyBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined() && !g[1].defined()) return {Tensor(), Tensor()};
+    for (int i = 0; i < 2; i++)
+      if (!g[i].defined()) g[i] = at::zeros(sizes[i], opts);
+    const optional<Tensor> pos = has_pos ? optional<Tensor>(get(2)) : std::nullopt;
+    // the transpose of the transposed rotation is the rotation itself
+    return list2(op_rope_apply()(g[0], g[1], get(0), get(1), pos, interleaved, !backward));
+  }
+};
+T2 rope_apply_autograd(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, OptTensor pos, int64_t interleaved, bool backward) {
+  auto node = make_node<RopeNode>(q, k);
+  T2 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_rope_apply()(q, k, cos, sin, pos, interleaved, backward); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    torch::autograd::set_history(std::get<1>(r), node);
+    node->keep(cos); node->keep(sin);
+    if (pos.has_value()) node->keep(*pos);
+    node->has_pos = pos.has_value();
+    node->interleaved = interleaved;
+    node->backward = backward;
+    node->sizes = {q.sizes().vec(), k.sizes().vec()};
+    node->opts = q.options();
+  }
+  return r;
+}
+
+// ---- attention -------------------------------------------------------------------------------------------------
+struct AttnShape { int B, Hq, Hkv, Sq, Skv, Dqk, Dv; };
+AttnShape check_attn(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& seg) {
+  TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "attention expects (batch, heads, seq, dim) tensors");
+  const AttnShape s{(int)q.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2), (int)k.size(2), (int)q.size(3), (int)v.size(3)};
+  TORCH_CHECK_VALUE(k.size(0) == s.B && k.size(3) == s.Dqk && v.size(0) == s.B && v.size(1) == s.Hkv && v.size(2) == s.Skv, "q (", q.sizes(),
+                    "), k (", k.sizes(), "), v (", v.sizes(), ") are inconsistent");
+  TORCH_CHECK_VALUE(s.Hkv != 0 && s.Hq % s.Hkv == 0, "num query heads ", s.Hq, " must be a multiple of num kv heads ", s.Hkv);
+  const auto t = q.scalar_type();
+  TORCH_CHECK_TYPE((t == at::kBFloat16 || t == at::kHalf || t == at::kFloat) && k.scalar_type() == t && v.scalar_type() == t,
+                   "attention kernels take bfloat16, float16 or float32 q/k/v of one dtype, got ", t, "/", k.scalar_type(), "/", v.scalar_type());
+  const bool square = s.Dqk == s.Dv && (s.Dqk == 64 || s.Dqk == 128);
+  TORCH_CHECK_NOT_IMPLEMENTED(square || (t != at::kFloat && s.Dqk == 192 && s.Dv == 128), "head dims (qk=", s.Dqk, ", v=", s.Dv,
+                              ") not built for ", t, "; supported: (64, 64), (128, 128)", t == at::kFloat ? "" : ", (192, 128)");
+  // kernel_utils.py:238-241: segment ids must cover the whole (unsharded) sequence
+  if (seg.defined() && !(seg.dim() == 2 && seg.size(0) == s.B && seg.size(1) == s.Skv && s.Sq == s.Skv)) {
+    py::gil_scoped_acquire gil;
+    PyErr_SetString(PyExc_AssertionError, "Sharding along sequence dimension not allowed in tpu kernel attention");
+    throw py::error_already_set();
+  }
+  return s;
+}
+Tensor prep_ids(const Tensor& seg) { return seg.defined() ? seg.to(at::kInt).contiguous() : seg; }
+Tensor prep_qpos(const Tensor& qpos, int64_t Sq) {
+  if (!qpos.defined()) return qpos;
+  TORCH_CHECK_VALUE(qpos.dim() == 1 && qpos.size(0) == Sq, "q_positions must have shape (", Sq, ",), got (", qpos.sizes(), ")");
+  return qpos.to(at::kInt).contiguous();
+}
+// fp32 tensor with a contiguous key axis, its (batch, head, query) strides with 0 on broadcast axes
+Tensor prep_bias(const Tensor& bias, const AttnShape& s, Strides3& st) {
+  if (!bias.defined()) return bias;
+  TORCH_CHECK_VALUE(bias.dim() == 4 && (bias.size(0) == 1 || bias.size(0) == s.B) && (bias.size(1) == 1 || bias.size(1) == s.Hq) &&
+                    bias.size(2) == s.Sq && bias.size(3) == s.Skv, "mask must have shape (1|", s.B, ", 1|", s.Hq, ", ", s.Sq, ", ", s.Skv,
+                    "), got (", bias.sizes(), ")");
+  Tensor b = bias.to(at::kFloat);
+  if (b.stride(-1) != 1) b = b.contiguous();
+  st = {b.size(0) == 1 ? 0 : b.stride(0), b.size(1) == 1 ? 0 : b.stride(1), b.stride(2)};
+  return b;
+}
+
+T2 attn_fwd_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, OptTensor seg_, double sm_scale, bool causal) {
+  const c10::Device dev = require_gpu(q_, k_, v_, seg_);
+  const AttnShape s = check_attn(q_, k_, v_, val(seg_));
+  c10::DeviceGuard guard(dev);
+  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), seg = prep_ids(val(seg_));
+  Tensor out = empty_like_heads(q, s.Dv), lse = empty_f32({s.B, s.Hq, s.Sq}, q);
+  if (out.numel()) {
+    const Strides3 qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out);
+    check(tp_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const int32_t*)opt_ptr(seg), out.data_ptr(), (float*)lse.data_ptr(), s.B, s.Hq,
+                      s.Hkv, s.Sq, s.Skv, s.Dqk, s.Dv, qs.data(), ks.data(), vs.data(), os.data(), (float)sm_scale, (int)causal,
+                      dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_fwd");
+  }
+  return {out, lse};
+}
+
+T3 attn_bwd_cuda(const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
+                 OptTensor seg_, double sm_scale, bool causal) {
+  const c10::Device dev = require_gpu(dout_, q_, k_, v_, out_, lse_, seg_);
+  const AttnShape s = check_attn(q_, k_, v_, val(seg_));
+  c10::DeviceGuard guard(dev);
+  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), out = prep_heads(out_), dout = prep_heads(dout_);
+  const Tensor lse = lse_.contiguous(), seg = prep_ids(val(seg_));
+  Tensor dq = empty_like_heads(q, s.Dqk), dk = empty_like_heads(k, s.Dqk), dv = empty_like_heads(v, s.Dv);
+  if (dq.numel() == 0 || dk.numel() == 0) return {dq.zero_(), dk.zero_(), dv.zero_()};
+  Tensor ws = empty_f32({(int64_t)tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq) / 4}, q);
+  const Strides3 gs = strides3(dout), qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out), dqs = strides3(dq),
+                 dks = strides3(dk), dvs = strides3(dv);
+  check(tp_attn_bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (const float*)lse.data_ptr(),
+                    (const int32_t*)opt_ptr(seg), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)ws.data_ptr(), s.B, s.Hq, s.Hkv, s.Sq,
+                    s.Skv, s.Dqk, s.Dv, gs.data(), qs.data(), ks.data(), vs.data(), os.data(), dqs.data(), dks.data(), dvs.data(),
+                    (float)sm_scale, (int)causal, dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_bwd");
+  return {dq, dk, dv};
+}
+
+struct AttnNode : OpNode {
+  bool has_seg, causal;
+  double sm_scale;
+  std::string name() const override { return "TprimeAttnBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const optional<Tensor> seg = has_seg ? optional<Tensor>(get(5)) : std::nullopt;
+    T3 r = op_attn_bwd()(g[0], get(0), get(1), get(2), get(3), get(4), seg, sm_scale, causal);
+    return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
+  }
+};
+T2 attn_fwd_autograd(const Tensor& q, const Tensor& k, const Tensor& v, OptTensor seg, double sm_scale, bool causal) {
+  auto node = make_node<AttnNode>(q, k, v);
+  T2 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_attn_fwd()(q, k, v, seg, sm_scale, causal); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    node->keep(q); node->keep(k); node->keep(v); node->keep(std::get<0>(r), true); node->keep(std::get<1>(r));
+    if (seg.has_value()) node->keep(*seg);
+    node->has_seg = seg.has_value();
+    node->causal = causal;
+    node->sm_scale = sm_scale;
+  }
+  return r;
+}
+
+// mask extensions: sliding window, soft cap, query rows in another order than the keys, additive masks
+T2 attn_fwd_masked_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, OptTensor seg_, OptTensor qpos_, double sm_scale, bool causal,
+                        int64_t causal_offset, int64_t window_left, int64_t window_right, double soft_cap, OptTensor bias_) {
+  const c10::Device dev = require_gpu(q_, k_, v_, seg_, qpos_, bias_);
+  const AttnShape s = check_attn(q_, k_, v_, val(seg_));
+  c10::DeviceGuard guard(dev);
+  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), seg = prep_ids(val(seg_)), qpos = prep_qpos(val(qpos_), s.Sq);
+  Tensor out = empty_like_heads(q, s.Dv), lse = empty_f32({s.B, s.Hq, s.Sq}, q);
+  Strides3 bs{};
+  const Tensor bias = prep_bias(val(bias_), s, bs);
+  if (out.numel()) {
+    const Strides3 qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out);
+    const auto launch = [&](auto fn, const char* name, auto... bias_args) {
+      check(fn(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const int32_t*)opt_ptr(seg), (const int32_t*)opt_ptr(qpos), bias_args...,
+               out.data_ptr(), (float*)lse.data_ptr(), s.B, s.Hq, s.Hkv, s.Sq, s.Skv, s.Dqk, s.Dv, qs.data(), ks.data(), vs.data(), os.data(),
+               (float)sm_scale, (int)causal, (int)causal_offset, (int)window_left, (int)window_right, (float)soft_cap,
+               dtype_code(q.scalar_type()), stream_of(dev)), name);
+    };
+    if (bias.defined()) launch(tp_attn_fwd_biased, "tp_attn_fwd_biased", (const float*)bias.data_ptr(), (const int64_t*)bs.data());
+    else launch(tp_attn_fwd_masked, "tp_attn_fwd_masked");
+  }
+  return {out, lse};
+}
+
+T3 attn_bwd_masked_cuda(const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
+                        OptTensor seg_, OptTensor qpos_, double sm_scale, bool causal, int64_t causal_offset, int64_t window_left,
+                        int64_t window_right, double soft_cap, OptTensor bias_) {
+  const c10::Device dev = require_gpu(dout_, q_, k_, v_, out_, lse_, seg_, qpos_, bias_);
+  const AttnShape s = check_attn(q_, k_, v_, val(seg_));
+  c10::DeviceGuard guard(dev);
+  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), out = prep_heads(out_), dout = prep_heads(dout_);
+  const Tensor lse = lse_.contiguous(), seg = prep_ids(val(seg_)), qpos = prep_qpos(val(qpos_), s.Sq);
+  Tensor dq = empty_like_heads(q, s.Dqk), dk = empty_like_heads(k, s.Dqk), dv = empty_like_heads(v, s.Dv);
+  if (dq.numel() == 0 || dk.numel() == 0) return {dq.zero_(), dk.zero_(), dv.zero_()};
+  Tensor ws = empty_f32({(int64_t)tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq) / 4}, q);
+  Strides3 bs{};
+  const Tensor bias = prep_bias(val(bias_), s, bs);
+  const Strides3 gs = strides3(dout), qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out), dqs = strides3(dq),
+                 dks = strides3(dk), dvs = strides3(dv);
+  const auto launch = [&](auto fn, const char* name, auto... bias_args) {
+    check(fn(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (const float*)lse.data_ptr(),
+             (const int32_t*)opt_ptr(seg), (const int32_t*)opt_ptr(qpos), bias_args..., dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+             (float*)ws.data_ptr(), s.B, s.Hq, s.Hkv, s.Sq, s.Skv, s.Dqk, s.Dv, gs.data(), qs.data(), ks.data(), vs.data(), os.data(),
+             dqs.data(), dks.data(), dvs.data(), (float)sm_scale, (int)causal, (int)causal_offset, (int)window_left, (int)window_right,
+             (float)soft_cap, dtype_code(q.scalar_type()), stream_of(dev)), name);
+  };
+  if (bias.defined()) launch(tp_attn_bwd_biased, "tp_attn_bwd_biased", (const float*)bias.data_ptr(), (const int64_t*)bs.data());
+  else launch(tp_attn_bwd_masked, "tp_attn_bwd_masked");
+  return {dq, dk, dv};
+}
+
+struct AttnMaskedNode : OpNode {
+  int has_seg, has_qpos, has_bias;
+  bool causal;
+  double sm_scale, soft_cap;
+  int64_t causal_offset, window_left, window_right;
+  std::string name() const override { return "TprimeAttnMaskedBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const auto opt = [&](int has, int at) { return has ? optional<Tensor>(get(at)) : std::nullopt; };
+    const optional<Tensor> seg = opt(has_seg, 5), qpos = opt(has_qpos, 5 + has_seg), bias = opt(has_bias, 5 + has_seg + has_qpos);
+    T3 r = op_attn_bwd_masked()(g[0], get(0), get(1), get(2), get(3), get(4), seg, qpos, sm_scale, causal, causal_offset, window_left,
+                                window_right, soft_cap, bias);
+    return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
+  }
+};
+T2 attn_fwd_masked_autograd(const Tensor& q, const Tensor& k, const Tensor& v, OptTensor seg, OptTensor qpos, double sm_scale, bool causal,
+                            int64_t causal_offset, int64_t window_left, int64_t window_right, double soft_cap, OptTensor bias) {
+  auto node = make_node<AttnMaskedNode>(q, k, v);
+  T2 r = [&] {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return op_attn_fwd_masked()(q, k, v, seg, qpos, sm_scale, causal, causal_offset, window_left, window_right, soft_cap, bias);
+  }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    node->keep(q); node->keep(k); node->keep(v); node->keep(std::get<0>(r), true); node->keep(std::get<1>(r));
+    for (const auto* t : {&seg, &qpos, &bias})
+      if (t->has_value()) node->keep(**t);
+    node->has_seg = seg.has_value(); node->has_qpos = qpos.has_value(); node->has_bias = bias.has_value();
+    node->causal = causal; node->sm_scale = sm_scale; node->soft_cap = soft_cap;
+    node->causal_offset = causal_offset; node->window_left = window_left; node->window_right = window_right;
+  }
+  return r;
+}
+
+// ---- L2 norm, temperature scale ----------------------------------------------------------------------------------
+T2 l2norm_fwd_cuda(const Tensor& x, double eps) {
+  const c10::Device dev = require_gpu(x);
+  c10::DeviceGuard guard(dev);
+  const Rows r = rows_of(x, true);
+  Tensor y = at::empty(x.sizes(), x.options()), rstd = empty_f32({r.rows}, x);
+  if (r.rows)
+    check(tp_l2norm_fwd(r.ptr(), y.data_ptr(), (float*)rstd.data_ptr(), r.rows, (int)r.cols, r.stride, r.cols, (float)eps,
+                        dtype_code(x.scalar_type()), stream_of(dev)), "tp_l2norm_fwd");
+  return {y, rstd};
+}
+Tensor l2norm_bwd_cuda(const Tensor& dy, const Tensor& x, const Tensor& rstd) {
+  const c10::Device dev = require_gpu(dy, x, rstd);
+  c10::DeviceGuard guard(dev);
+  const Rows xr = rows_of(x, true), gr = rows_of(dy, true);
+  Tensor dx = at::empty(x.sizes(), x.options());
+  if (xr.rows)
+    check(tp_l2norm_bwd(gr.ptr(), xr.ptr(), (const float*)rstd.data_ptr(), dx.data_ptr(), xr.rows, (int)xr.cols, gr.stride, xr.stride, xr.cols,
+                        dtype_code(x.scalar_type()), stream_of(dev)), "tp_l2norm_bwd");
+  return dx;
+}
+struct L2NormNode : OpNode {
+  std::string name() const override { return "TprimeL2NormBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor()};
+    const Tensor x = get(0);
+    return {op_l2norm_bwd()(g[0].to(x.scalar_type()), x, get(1))};
+  }
+};
+T2 l2norm_fwd_autograd(const Tensor& x, double eps) {
+  auto node = make_node<L2NormNode>(x);
+  T2 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_l2norm_fwd()(x, eps); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    node->keep(x); node->keep(std::get<1>(r));
+  }
+  return r;
+}
+
+// x (B, S, N, D) times scale (S) fp32 per position, rounded to x's dtype
+Tensor scale_rows_cuda(const Tensor& x, const Tensor& scale) {
+  const c10::Device dev = require_gpu(x, scale);
+  TORCH_CHECK_VALUE(x.dim() == 4 && scale.dim() == 1 && scale.size(0) == x.size(1), "expected x (batch, seq, heads, dim) and scale (seq,), got (",
+                    x.sizes(), ") and (", scale.sizes(), ")");
+  c10::DeviceGuard guard(dev);
+  const Rows r = rows_of(x, true);
+  const Tensor s = scale.to(at::kFloat).contiguous();
+  Tensor y = at::empty(x.sizes(), x.options());
+  if (y.numel())
+    check(tp_scale_rows(r.ptr(), (const float*)s.data_ptr(), y.data_ptr(), r.rows, (int)r.cols, r.stride, r.cols, (int)x.size(2), (int)x.size(1),
+                        dtype_code(x.scalar_type()), stream_of(dev)), "tp_scale_rows");
+  return y;
+}
+struct ScaleRowsNode : OpNode {
+  std::string name() const override { return "TprimeScaleRowsBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor()};
+    return {op_scale_rows()(g[0], get(0))};
+  }
+};
+Tensor scale_rows_autograd(const Tensor& x, const Tensor& scale) {
+  auto node = make_node<ScaleRowsNode>(x);
+  Tensor r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_scale_rows()(x, scale); }();
+  if (node) {
+    torch::autograd::set_history(r, node);
+    node->keep(scale);
+  }
+  return r;
+}
+
+// ---- SwiGLU ------------------------------------------------------------------------------------------------------
+Tensor swiglu_fwd_cuda(const Tensor& gate, const Tensor& up) {
+  const c10::Device dev = require_gpu(gate, up);
+  TORCH_CHECK_VALUE(gate.sizes() == up.sizes() && gate.scalar_type() == up.scalar_type(), "gate (", gate.sizes(), ")/", gate.scalar_type(),
+                    " and up (", up.sizes(), ")/", up.scalar_type(), " must match");
+  c10::DeviceGuard guard(dev);
+  const Rows g = rows_of(gate, true), u = rows_of(up, true);
+  Tensor out = at::empty(gate.sizes(), gate.options());
+  if (out.numel())
+    check(tp_swiglu_fwd(g.ptr(), u.ptr(), out.data_ptr(), g.rows, (int)g.cols, g.stride, u.stride, g.cols, dtype_code(gate.scalar_type()),
+                        stream_of(dev)), "tp_swiglu_fwd");
+  return out;
+}
+T2 swiglu_bwd_cuda(const Tensor& dout, const Tensor& gate, const Tensor& up) {
+  const c10::Device dev = require_gpu(dout, gate, up);
+  c10::DeviceGuard guard(dev);
+  const Rows d = rows_of(dout, true), g = rows_of(gate, true), u = rows_of(up, true);
+  Tensor dg = at::empty(gate.sizes(), gate.options()), du = at::empty(up.sizes(), up.options());
+  if (dg.numel())
+    check(tp_swiglu_bwd(d.ptr(), g.ptr(), u.ptr(), dg.data_ptr(), du.data_ptr(), g.rows, (int)g.cols, d.stride, g.stride, u.stride, g.cols, g.cols,
+                        dtype_code(gate.scalar_type()), stream_of(dev)), "tp_swiglu_bwd");
+  return {dg, du};
+}
+struct SwigluNode : OpNode {
+  std::string name() const override { return "TprimeSwigluBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor()};
+    const Tensor gate = get(0);
+    return list2(op_swiglu_bwd()(g[0].to(gate.scalar_type()), gate, get(1)));
+  }
+};
+Tensor swiglu_fwd_autograd(const Tensor& gate, const Tensor& up) {
+  auto node = make_node<SwigluNode>(gate, up);
+  Tensor r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_swiglu_fwd()(gate, up); }();
+  if (node) {
+    torch::autograd::set_history(r, node);
+    node->keep(gate); node->keep(up);
+  }
+  return r;
+}
+
+// ---- cross entropy -----------------------------------------------------------------------------------------------
+Tensor prep_labels(const Tensor& labels) {
+  Tensor l = labels.to(at::kLong);
+  return l.stride(1) != 1 ? l.contiguous() : l;
+}
+// (loss (scalar fp32), lse (B*S), loss_and_count (2)) of the shifted next-token cross entropy
+T3 cross_entropy_fwd_cuda(const Tensor& logits_, const Tensor& labels_, int64_t ignore_index) {
+  const c10::Device dev = require_gpu(logits_, labels_);
+  TORCH_CHECK_VALUE(logits_.dim() == 3 && labels_.dim() == 2 && labels_.size(0) == logits_.size(0) && labels_.size(1) == logits_.size(1),
+                    "expected logits (batch, seq, vocab) and labels (batch, seq), got (", logits_.sizes(), ") and (", labels_.sizes(), ")");
+  TORCH_CHECK_TYPE(logits_.scalar_type() == at::kFloat || logits_.scalar_type() == at::kBFloat16,
+                   "cross entropy takes float32 or bfloat16 logits, got ", logits_.scalar_type());
+  c10::DeviceGuard guard(dev);
+  const int64_t B = logits_.size(0), S = logits_.size(1), V = logits_.size(2);
+  const Tensor logits = logits_.stride(2) != 1 ? logits_.contiguous() : logits_, labels = prep_labels(labels_);
+  Tensor lse = empty_f32({B * S}, logits), row_loss = empty_f32({B * S}, logits), lc = empty_f32({2}, logits);
+  check(tp_cross_entropy_fwd(logits.data_ptr(), (const int64_t*)labels.data_ptr(), (float*)lse.data_ptr(), (float*)row_loss.data_ptr(),
+                             (float*)lc.data_ptr(), (int)B, (int)S, (int)V, logits.stride(0), logits.stride(1), labels.stride(0),
+                             (int)ignore_index, dtype_code(logits.scalar_type()), stream_of(dev)), "tp_cross_entropy_fwd");
+  return {lc.select(0, 0).clone(), lse, lc};
+}
+Tensor cross_entropy_bwd_cuda(const Tensor& dloss, const Tensor& logits_, const Tensor& labels_, const Tensor& lse, const Tensor& lc,
+                              int64_t ignore_index) {
+  const c10::Device dev = require_gpu(dloss, logits_, labels_, lse, lc);
+  c10::DeviceGuard guard(dev);
+  const int64_t B = logits_.size(0), S = logits_.size(1), V = logits_.size(2);
+  const Tensor logits = logits_.stride(2) != 1 ? logits_.contiguous() : logits_, labels = prep_labels(labels_);
+  const Tensor dl = dloss.to(at::kFloat).contiguous();
+  Tensor dlogits = at::empty({B, S, V}, logits.options());
+  check(tp_cross_entropy_bwd(logits.data_ptr(), (const int64_t*)labels.data_ptr(), (const float*)lse.data_ptr(), (const float*)lc.data_ptr(),
+                             (const float*)dl.data_ptr(), dlogits.data_ptr(), (int)B, (int)S, (int)V, logits.stride(0), logits.stride(1),
+                             labels.stride(0), dlogits.stride(0), dlogits.stride(1), (int)ignore_index, dtype_code(logits.scalar_type()),
+                             stream_of(dev)), "tp_cross_entropy_bwd");
+  return dlogits;
+}
+struct CrossEntropyNode : OpNode {
+  int64_t ignore_index;
+  std::string name() const override { return "TprimeCrossEntropyBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor()};
+    return {op_cross_entropy_bwd()(g[0], get(0), get(1), get(2), get(3), ignore_index)};
+  }
+};
+T3 cross_entropy_fwd_autograd(const Tensor& logits, const Tensor& labels, int64_t ignore_index) {
+  auto node = make_node<CrossEntropyNode>(logits);
+  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_cross_entropy_fwd()(logits, labels, ignore_index); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    node->keep(logits); node->keep(labels); node->keep(std::get<1>(r)); node->keep(std::get<2>(r));
+    node->ignore_index = ignore_index;
+  }
+  return r;
+}
+
+// ---- Python entry points -----------------------------------------------------------------------------------------
+// What the Python functions of ops.py call: the GPU check with its own message, then the operator.
+Tensor py_rmsnorm(const Tensor& x, const Tensor& w, double eps) { require_gpu(x, w); return std::get<0>(op_rmsnorm_fwd()(x, w, eps)); }
+T2 py_add_rmsnorm(const Tensor& x, const Tensor& r, const Tensor& w, double eps) {
+  require_gpu(x, r, w);
+  T3 o = op_add_rmsnorm_fwd()(x, r, w, eps);
+  return {std::get<0>(o), std::get<1>(o)};
+}
+T2 py_rope_table(const Tensor& f, const Tensor& p, double scaling, const Tensor& like) {
+  require_gpu(f, p, like);
+  return op_rope_table()(f, p, scaling, like.scalar_type());
+}
+T2 py_rope_apply(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, OptTensor pos, int64_t interleaved) {
+  require_gpu(q, k, cos, sin, pos);
+  return op_rope_apply()(q, k, cos, sin, pos, interleaved, false);
+}
+Tensor py_attention(const Tensor& q, const Tensor& k, const Tensor& v, OptTensor seg, double sm_scale, bool causal) {
+  require_gpu(q, k, v, seg);
+  return std::get<0>(op_attn_fwd()(q, k, v, seg, sm_scale, causal));
+}
+Tensor py_attention_masked(const Tensor& q, const Tensor& k, const Tensor& v, OptTensor seg, OptTensor qpos, double sm_scale, bool causal,
+                           int64_t causal_offset, int64_t window_left, int64_t window_right, double soft_cap, OptTensor bias) {
+  require_gpu(q, k, v, seg, qpos, bias);
+  return std::get<0>(op_attn_fwd_masked()(q, k, v, seg, qpos, sm_scale, causal, causal_offset, window_left, window_right, soft_cap, bias));
+}
+Tensor py_l2norm(const Tensor& x, double eps) { return std::get<0>(op_l2norm_fwd()(x, eps)); }
+Tensor py_swiglu(const Tensor& g, const Tensor& u) { return op_swiglu_fwd()(g, u); }
+Tensor py_cross_entropy(const Tensor& l, const Tensor& y, int64_t ignore) { return std::get<0>(op_cross_entropy_fwd()(l, y, ignore)); }
+
+}  // namespace
+
+TORCH_LIBRARY(tprime, m) {
+  m.def("rmsnorm_fwd(Tensor x, Tensor weight, float eps) -> (Tensor, Tensor)");
+  m.def("rmsnorm_bwd(Tensor dy, Tensor x, Tensor weight, Tensor rstd) -> (Tensor, Tensor)");
+  m.def("add_rmsnorm_fwd(Tensor x, Tensor residual, Tensor weight, float eps) -> (Tensor, Tensor, Tensor)");
+  m.def("add_rmsnorm_bwd(Tensor dy, Tensor dh, Tensor h, Tensor weight, Tensor rstd) -> (Tensor, Tensor)");
+  m.def("rope_table(Tensor inv_freq, Tensor position_ids, float attention_scaling, ScalarType dtype) -> (Tensor, Tensor)");
+  m.def("rope_apply(Tensor q, Tensor k, Tensor cos, Tensor sin, Tensor? pos, int interleaved, bool backward) -> (Tensor, Tensor)");
+  m.def("attn_fwd(Tensor q, Tensor k, Tensor v, Tensor? seg, float sm_scale, bool causal) -> (Tensor, Tensor)");
+  m.def("attn_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor? seg, float sm_scale, bool causal) "
+        "-> (Tensor, Tensor, Tensor)");
+  m.def("attn_fwd_masked(Tensor q, Tensor k, Tensor v, Tensor? seg, Tensor? qpos, float sm_scale, bool causal, int causal_offset, "
+        "int window_left, int window_right, float soft_cap, Tensor? bias=None) -> (Tensor, Tensor)");
+  m.def("attn_bwd_masked(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor? seg, Tensor? qpos, float sm_scale, "
+        "bool causal, int causal_offset, int window_left, int window_right, float soft_cap, Tensor? bias=None) -> (Tensor, Tensor, Tensor)");
+  m.def("l2norm_fwd(Tensor x, float eps) -> (Tensor, Tensor)");
+  m.def("l2norm_bwd(Tensor dy, Tensor x, Tensor rstd) -> Tensor");
+  m.def("scale_rows(Tensor x, Tensor scale) -> Tensor");
+  m.def("swiglu_fwd(Tensor gate, Tensor up) -> Tensor");
+  m.def("swiglu_bwd(Tensor dout, Tensor gate, Tensor up) -> (Tensor, Tensor)");
+  m.def("cross_entropy_fwd(Tensor logits, Tensor labels, int ignore_index) -> (Tensor, Tensor, Tensor)");
+  m.def("cross_entropy_bwd(Tensor dloss, Tensor logits, Tensor labels, Tensor lse, Tensor loss_and_count, int ignore_index) -> Tensor");
+}
+
+TORCH_LIBRARY_IMPL(tprime, CUDA, m) {
+  m.impl("rmsnorm_fwd", rmsnorm_fwd_cuda);
+  m.impl("rmsnorm_bwd", rmsnorm_bwd_cuda);
+  m.impl("add_rmsnorm_fwd", add_rmsnorm_fwd_cuda);
+  m.impl("add_rmsnorm_bwd", add_rmsnorm_bwd_cuda);
+  m.impl("rope_table", rope_table_cuda);
+  m.impl("rope_apply", rope_apply_cuda);
+  m.impl("attn_fwd", attn_fwd_cuda);
+  m.impl("attn_bwd", attn_bwd_cuda);
+  m.impl("attn_fwd_masked", attn_fwd_masked_cuda);
+  m.impl("attn_bwd_masked", attn_bwd_masked_cuda);
+  m.impl("l2norm_fwd", l2norm_fwd_cuda);
+  m.impl("l2norm_bwd", l2norm_bwd_cuda);
+  m.impl("scale_rows", scale_rows_cuda);
+  m.impl("swiglu_fwd", swiglu_fwd_cuda);
+  m.impl("swiglu_bwd", swiglu_bwd_cuda);
+  m.impl("cross_entropy_fwd", cross_entropy_fwd_cuda);
+  m.impl("cross_entropy_bwd", cross_entropy_bwd_cuda);
+}
+
+TORCH_LIBRARY_IMPL(tprime, Autograd, m) {
+  m.impl("rmsnorm_fwd", rmsnorm_fwd_autograd);
+  m.impl("add_rmsnorm_fwd", add_rmsnorm_fwd_autograd);
+  m.impl("rope_apply", rope_apply_autograd);
+  m.impl("attn_fwd", attn_fwd_autograd);
+  m.impl("attn_fwd_masked", attn_fwd_masked_autograd);
+  m.impl("l2norm_fwd", l2norm_fwd_autograd);
+  m.impl("scale_rows", scale_rows_autograd);
+  m.impl("swiglu_fwd", swiglu_fwd_autograd);
+  m.impl("cross_entropy_fwd", cross_entropy_fwd_autograd);
+  for (const char* name : {"rope_table", "rmsnorm_bwd", "add_rmsnorm_bwd", "attn_bwd", "attn_bwd_masked", "l2norm_bwd", "swiglu_bwd",
+                           "cross_entropy_bwd"})
+    m.impl(name, torch::autograd::autogradNotImplementedFallback());
+}
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("rmsnorm", &py_rmsnorm);
+  m.def("add_rmsnorm", &py_add_rmsnorm);
+  m.def("rope_table", &py_rope_table);
+  m.def("rope_apply", &py_rope_apply);
+  m.def("attention", &py_attention);
+  m.def("attention_masked", &py_attention_masked);
+  m.def("l2norm", &py_l2norm);
+  m.def("swiglu", &py_swiglu);
+  m.def("cross_entropy", &py_cross_entropy);
+}

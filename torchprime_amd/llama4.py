@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from . import _lib, ops
+from . import ops
 from .rope import RopeScaling, llama3_rope_frequencies
 
 
@@ -38,8 +38,7 @@ class Llama4TextRotaryEmbedding(nn.Module):
 
   @torch.no_grad()
   def forward(self, x, position_ids):
-    _lib.require_gpu(x, position_ids)
-    return ops.rope_table(self.inv_freq, position_ids, 1.0, x.dtype)
+    return ops.rope_table_like(self.inv_freq, position_ids, 1.0, x)
 
 
 def apply_rotary_emb(q, k, freqs_cos_sin, unsqueeze_dim: int = 2):

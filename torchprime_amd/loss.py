@@ -19,4 +19,4 @@ def cross_entropy_loss(logits: torch.Tensor, labels: torch.Tensor, vocab_size: i
     logits = logits.reshape(-1, *logits.shape[-2:])
     labels = labels.reshape(-1, labels.shape[-1])
   labels = labels.to(logits.device)
-  return ops.cross_entropy_fwd(logits, labels, IGNORE_INDEX)[0]
+  return ops.cross_entropy(logits, labels, IGNORE_INDEX)

@@ -46,8 +46,7 @@ class LlamaRotaryEmbedding(_Fp32Frequencies):
   @torch.no_grad()
   def forward(self, x, position_ids):
     # x: [bs, num_attention_heads, seq_len, head_size]; position_ids: (bs or 1, seq_len), float in the models
-    _lib.require_gpu(x, position_ids)
-    return ops.rope_table(self.inv_freq, position_ids, 1.0, x.dtype)
+    return ops.rope_table_like(self.inv_freq, position_ids, 1.0, x)
 
 
 class DeepseekV3RotaryEmbedding(_Fp32Frequencies):
@@ -62,8 +61,7 @@ class DeepseekV3RotaryEmbedding(_Fp32Frequencies):
 
   @torch.no_grad()
   def forward(self, x: torch.Tensor, position_ids: torch.Tensor):
-    _lib.require_gpu(x, position_ids)
-    return ops.rope_table(self.inv_freq, position_ids, float(self.attention_scaling), x.dtype)
+    return ops.rope_table_like(self.inv_freq, position_ids, float(self.attention_scaling), x)
 
 
 class MixtralRotaryEmbedding(nn.Module):
