@@ -140,6 +140,33 @@ int tp_attn_fwd(const void* q, const void* k, const void* v, const int32_t* seg,
                 const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                 const int64_t o_strides[3], float sm_scale, int causal, int dtype, void* stream);
 
+/* ------------------------------------------------------------------------------------------------
+ * Additive masks that only drop pairs: every entry is 0 or lets its pair drop out (-inf, at most -1e30, or
+ * -65504 in a float16 mask; see csrc/attn_mask.hip for when that is exact).  Causality + padding, the masks
+ * the eager branch is given (torchprime/torch_xla_models/attention.py:151-158), are of this kind.
+ * tp_mask_pairs        turns such a mask into pair bits: one kernel, no synchronisation
+ *   mask          element (b, i, j) at mask[b*mask_strides[0] + i*mask_strides[1] + j], any of the three dtypes
+ *   pairs         tp_mask_pairs_bytes() bytes, 16-byte aligned
+ *   verdict       non-zero: also set the int32 flags at the start of `pairs`, which the caller has cleared:
+ *                 [0] some entry is neither 0 nor drops its pair, [1] the mask is not the exact causal mask
+ *                 (0 / -inf), [2] a row without a pair has entries other than -inf.  The attention entry
+ *                 points below give the eager formula's results if [0] and [2] are 0.
+ * tp_attn_fwd_pairs / tp_attn_bwd_pairs   tp_attn_fwd / tp_attn_bwd (no segment ids, no causality of their
+ *   own) over the pairs of `pairs`, made for mask_batches (1 or B) masks.  bf16 and fp16.
+ * ---------------------------------------------------------------------------------------------- */
+size_t tp_mask_pairs_bytes(int mask_batches, int Sq, int Skv);
+int tp_mask_pairs(const void* mask, const int64_t mask_strides[2], int mask_batches, int Sq, int Skv, int dtype, void* pairs,
+                  int verdict, void* stream);
+int tp_attn_fwd_pairs(const void* q, const void* k, const void* v, const void* pairs, int mask_batches, void* out, float* lse,
+                      int B, int Hq, int Hkv, int Sq, int Skv, int Dqk, int Dv, const int64_t q_strides[3],
+                      const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3], float sm_scale,
+                      int dtype, void* stream);
+int tp_attn_bwd_pairs(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
+                      const void* pairs, int mask_batches, void* dq, void* dk, void* dv, float* ws, int B, int Hq, int Hkv, int Sq,
+                      int Skv, int Dqk, int Dv, const int64_t do_strides[3], const int64_t q_strides[3], const int64_t k_strides[3],
+                      const int64_t v_strides[3], const int64_t o_strides[3], const int64_t dq_strides[3],
+                      const int64_t dk_strides[3], const int64_t dv_strides[3], float sm_scale, int dtype, void* stream);
+
 /* Bytes of fp32 workspace tp_attn_bwd needs (two floats per query row: rowsum(dO o O) and the LSE in
  * log2 units). */
 size_t tp_attn_bwd_workspace_bytes(int B, int Hq, int Sq);

@@ -1,0 +1,77 @@
+"""Additive masks that only drop pairs (causality + padding, block patterns), which the attention module turns into bits:
+kind of the mask, forward and backward against the oracle's eager attention at the edges of the 64-column tiles and the
+128-row blocks.  Bounds: the ones every 16-bit attention test here uses (tests/util.py)."""
+
+import pytest
+import torch
+
+import torchprime_amd as tpa
+from oracle import tprime_oracle as orc
+from tests.test_gpu_masks import _eager_grads, _padding_mask
+from tests.util import assert_close, heads_view
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LOWEST = {dt: torch.finfo(dt).min for dt in (torch.bfloat16, torch.float16, torch.float32)}
+
+
+def _blocks(B, Sq, Skv, seed, fill):
+  """A random 0 / fill pattern whose blocks of 48 x 80 are full, empty or mixed; key 0 is seen by every row."""
+  g = torch.Generator().manual_seed(seed)
+  up = lambda t: t.repeat_interleave(48, 1).repeat_interleave(80, 2)[:, :Sq, :Skv]  # noqa: E731
+  kind = up(torch.randint(0, 3, (B, (Sq + 47) // 48, (Skv + 79) // 80), generator=g))
+  keep = (kind == 1) | ((kind == 2) & (torch.rand((B, Sq, Skv), generator=g) < 0.5))
+  keep[:, :, 0] = True
+  return torch.zeros((B, 1, Sq, Skv)).masked_fill_(~keep[:, None], fill)
+
+
+def _check(B, Hq, Hkv, D, Dv, mask, dtype, seed=0):
+  Sq, Skv = mask.shape[-2:]
+  q, k, v, do = (heads_view(B, h, s, d, seed + i, dtype)
+                 for i, (h, s, d) in enumerate(((Hq, Sq, D), (Hkv, Skv, D), (Hkv, Skv, Dv), (Hq, Sq, Dv))))  # fmt: skip
+  qd, kd, vd = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
+  m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=Hq, num_key_value_heads=Hkv))
+  out = m(qd, kd, vd, mask.to(DEV))
+  assert out.grad_fn.name() == "TprimeAttnPairsBackward"
+  out.backward(do.to(DEV))
+  for got, ref, name in zip((out, qd.grad, kd.grad, vd.grad), _eager_grads(q, k, v, do, mask), ("out", "dq", "dk", "dv")):
+    assert_close(got, ref, name, scale_abs=name != "out")
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (64, 64), (192, 128)])
+# (The smallest is 16: in a row with a single key dS = P (dP - delta) is 0 up to the 16-bit rounding of the output in delta,
+# 2^-9 |dP|, against |dP| in other rows.  Where most rows are of that kind, as with 2 keys and padding, the relative bound
+# of dq, 1e-2, is not one the arithmetic can meet; with 16 keys they are under a tenth of the rows: 2^-9 * 0.3 < 1e-3.)
+@pytest.mark.parametrize("S", [16, 63, 64, 65, 128, 129, 333])
+def test_causal_and_padding(S, D, Dv):
+  lengths = [S, max(1, S // 2), max(1, S - 1)]
+  _check(3, 4, 2, D, Dv, _padding_mask(3, S, S, lengths, causal=True, dtype=torch.bfloat16, fill=LOWEST[torch.bfloat16]), torch.bfloat16, S)
+  _check(3, 4, 2, D, Dv, _padding_mask(3, S, S, lengths, causal=True, dtype=torch.float16, fill=LOWEST[torch.float16]), torch.float16, S)
+
+
+@pytest.mark.parametrize("Sq,Skv", [(70, 300), (300, 70), (257, 257)])
+@pytest.mark.parametrize("fill", [float("-inf"), LOWEST[torch.float32]])
+def test_block_patterns(Sq, Skv, fill):
+  _check(2, 4, 2, 128, 128, _blocks(2, Sq, Skv, Sq, fill), torch.bfloat16)
+  _check(2, 4, 4, 64, 64, _blocks(1, Sq, Skv, Skv, fill), torch.float16)  # one mask for all batches
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_kind(dtype):
+  kind = lambda m: tpa.ops.mask_kind(m.to(dtype).to(DEV))  # noqa: E731
+  K = tpa.ops
+  S, low = 130, LOWEST[dtype]
+  causal = orc.causal_additive_mask(S)
+  assert kind(causal) == K.MASK_CAUSAL
+  assert kind(causal.clamp(min=low)) == K.MASK_PAIRS  # the same pairs, written with the lowest value
+  one = causal.clone()
+  one[..., 100, 7] = float("-inf")
+  assert kind(one) == K.MASK_PAIRS
+  for value in (-1.0, 0.5, float("nan")):
+    one[..., 100, 7] = value
+    assert kind(one) == K.MASK_GENERAL
+  empty = causal.clone()
+  empty[..., 64, :] = float("-inf")  # a row without a pair: zeros, as in the general kernels
+  assert kind(empty) == K.MASK_PAIRS
+  empty[..., 64, :] = low  # ... of finite entries: uniform weights
+  assert kind(empty) == K.MASK_GENERAL

@@ -31,36 +31,30 @@ def repeat_kv(hidden_states: torch.Tensor, n_rep: int) -> torch.Tensor:
   return hidden_states.unsqueeze(2).expand(b, h, n_rep, s, d).reshape(b, h * n_rep, s, d)
 
 
-def _is_causal_additive_mask(mask: torch.Tensor, q_len: int, kv_len: int) -> bool:
-  """True when ``mask[..., :kv_len]`` is 0 on and below the diagonal and -inf above it, the mask the
-  models build at model/llama/model.py:347-355."""
-  if mask.dim() != 4 or mask.shape[1] != 1 or mask.shape[2] != q_len or mask.shape[3] < kv_len:
-    return False
-  m = mask[:, :, :, :kv_len]
-  keep = torch.ones((q_len, kv_len), dtype=torch.bool, device=mask.device).tril()
-  ok = ((m == 0) == keep) & ((m == float("-inf")) == ~keep)
-  return bool(ok.all())
-
-
-# Verdicts of the check above, kept per mask tensor object (a weak reference and the tensor's version counter).  A
-# model builds its mask once per forward and hands the same tensor to every layer, so the (S x S) compare and its
-# host sync run once per mask rather than once per layer.  The key is the object, never its address: a mask built
-# for the next forward is a new tensor that the caching allocator may well place where the last one was.
-# ``kernel_config={"assume_causal_mask": True}`` skips the check altogether.
+# Kinds of the masks handed to the eager branch (ops.mask_kind), kept per mask tensor object (a weak reference and the
+# tensor's version counter).  A model builds its mask once per forward and hands the same tensor to every layer, so the
+# pass over the mask and its host sync run once per mask rather than once per layer.  The key is the object, never its
+# address: a mask built for the next forward is a new tensor that the caching allocator may well place where the last
+# one was.  ``kernel_config={"assume_causal_mask": True}`` skips the check altogether.
 _MASK_VERDICTS: dict = {}
 
 
-def _causal_mask_verdict(mask: torch.Tensor, q_len: int, kv_len: int) -> bool:
+def _mask_verdict(mask: torch.Tensor, q_len: int, kv_len: int) -> int:
   ident = id(mask)
   key = (mask._version, tuple(mask.shape), q_len, kv_len)
   entry = _MASK_VERDICTS.get(ident)
   if entry is not None and entry[0]() is mask and entry[1] == key:
     return entry[2]
-  verdict = _is_causal_additive_mask(mask, q_len, kv_len)
+  kind = ops.MASK_GENERAL
+  # (per-head masks and other shapes are evaluated element by element)
+  if mask.dim() == 4 and mask.shape[1] == 1 and mask.shape[2] == q_len and mask.shape[3] >= kv_len and mask.dtype in (
+    torch.bfloat16, torch.float16, torch.float32,
+  ):  # fmt: skip
+    kind = ops.mask_kind(mask[:, :, :, :kv_len])
   # the entry leaves with the tensor (its id may be reused afterwards, hence also the identity check above)
   ref = weakref.ref(mask, lambda _r, ident=ident: _MASK_VERDICTS.pop(ident, None))
-  _MASK_VERDICTS[ident] = (ref, key, verdict)
-  return verdict
+  _MASK_VERDICTS[ident] = (ref, key, kind)
+  return kind
 
 
 class AttentionModule(nn.Module):
@@ -115,19 +109,26 @@ class AttentionModule(nn.Module):
         causal = False
       else:
         assume = bool(self.kernel_config and self.kernel_config.get("assume_causal_mask"))
-        causal = assume or _causal_mask_verdict(attention_mask, q_len, kv_seq_len)
+        kind = ops.MASK_CAUSAL if assume else _mask_verdict(attention_mask, q_len, kv_seq_len)
+        causal = kind == ops.MASK_CAUSAL
         if not causal:
-          # any other mask is added to the scaled logits as it is (attention.py:153-158); the causal one, which
-          # the models build, takes the kernels that skip the tiles above the diagonal instead
+          # any other mask is added to the scaled logits as it is (attention.py:153-158); the causal one takes the
+          # kernels that skip the tiles above the diagonal, one that only drops pairs (causal + padding) its bits
           if attention_mask.dim() != 4 or attention_mask.shape[-1] < kv_seq_len:
             raise ValueError(
               f"attention_mask must be 4-D with at least {kv_seq_len} keys, got {tuple(attention_mask.shape)}"
             )
           bias = attention_mask[:, :, :, :kv_seq_len]
       if bias is not None:
-        attn_output = ops.attention(
-          query_states, key_states, value_states, None, 1.0 / math.sqrt(head_dim), False, bias=bias
+        scale = 1.0 / math.sqrt(head_dim)
+        # (a float16 mask's lowest value drops a pair for float16 logits only; fp32 has no kernels for pair bits)
+        by_bits = kind == ops.MASK_PAIRS and bias.shape[0] in (1, bsz) and (
+          query_states.dtype == torch.bfloat16 and bias.dtype != torch.float16 or query_states.dtype == torch.float16
         )
+        if by_bits:
+          attn_output = ops.attention_pairs(query_states, key_states, value_states, bias.detach(), scale)
+        else:
+          attn_output = ops.attention(query_states, key_states, value_states, None, scale, False, bias=bias)
         if attn_output.size() != (bsz, num_heads, q_len, head_dim):
           raise ValueError(
             f"`attn_output` should be of size {(bsz, num_heads, q_len, head_dim)}, but is {attn_output.size()}"

@@ -69,6 +69,7 @@ struct BwdArgs {
   // Sliding windows and causal offsets without the other mask extensions run through these kernels.
   int band_lo, band_hi;
   MaskExt mx;
+  PairMask pm;
 };
 
 // ------------------------------------------------------------------------------------------------
@@ -190,21 +191,10 @@ struct Stage64 {
   }
 };
 
-// 4 bytes per lane straight into LDS at dst + 4 * lane (a 64-entry row vector per instruction)
-__device__ __forceinline__ void dma_dword(u32x4 rs, unsigned byte_offset, unsigned char* dst, int lane) {
-  const unsigned d = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
-  byte_offset = __builtin_amdgcn_readfirstlane(byte_offset);
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :: "s"(d), "v"((unsigned)lane * 4u), "s"(rs), "s"(byte_offset) : "memory", "m0");
-}
-__device__ __forceinline__ void dma_dword_at(u32x4 rs, unsigned byte_offset, unsigned dst, int lane) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :: "s"(dst), "v"((unsigned)lane * 4u), "s"(rs), "s"(byte_offset) : "memory", "m0");
-}
 // ------------------------------------------------------------------------------------------------
 // dK / dV
 // ------------------------------------------------------------------------------------------------
-template <typename T, int DQK, int DV, int NBUF, bool CAUSAL, bool SEG>
+template <typename T, int DQK, int DV, int NBUF, bool CAUSAL, int SEG>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   typedef typename MT<T>::v8 v8;
   constexpr int BMQ = 64;   // query rows per streamed tile
@@ -217,7 +207,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   typedef DmaTile<DQK, true> QT;
   typedef DmaTile<DV, true> OT;
   constexpr int Q_BYTES = QT::BYTES, DO_BYTES = OT::BYTES;
-  constexpr int ROW_BYTES = BMQ * 4 * 4;  // lse (log2 units), delta, segment id, position per query row
+  constexpr bool PAIRS = SEG == SEG_PAIRS;
+  static_assert(!PAIRS || CAUSAL, "pair masks run with the all-covering band of the causal kernels");
+  // lse (log2 units), delta, segment id, position per query row; the pair bits of the workgroup's kv rows
+  constexpr int VEC_BYTES = BMQ * 4 * 4, ROW_BYTES = VEC_BYTES + (PAIRS ? BNK * 8 : 0);
   constexpr int BUF_BYTES = Q_BYTES + DO_BYTES;
   // LDS layout: the NBUF copies of each kind of tile lie side by side (Q.. dO.., then the row vectors), so that with
   // the buffer index a constant every fragment address is a loop-invariant per-lane offset plus an immediate
@@ -233,8 +226,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   const int wkv0 = kv0 + wave * 32;
   const int Sq = a.Sq, Skv = a.Skv;
   // GEN: the instantiation that also evaluates the mask extensions (and then may run without segment ids)
-  constexpr bool GEN = !CAUSAL && SEG;
-  const bool has_seg = SEG && (!GEN || a.seg != nullptr);
+  constexpr bool GEN = !CAUSAL && SEG == SEG_IDS;
+  const bool has_seg = SEG == SEG_IDS && (!GEN || a.seg != nullptr);
   const bool ext = GEN && a.mx.on;
   const bool capped = GEN && a.mx.cap_in != 0.f;
   const bool biased = GEN && a.mx.bias != nullptr;
@@ -281,6 +274,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   int wkmin = 0, wkmax = 0;
   if (SEG) {
     wkmin = segk; wkmax = segk;
+    if (!PAIRS) {
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) {
       wkmin = min(wkmin, __shfl_xor(wkmin, o, 64));
@@ -289,8 +283,12 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     wkmin = __builtin_amdgcn_readfirstlane(wkmin);
     wkmax = __builtin_amdgcn_readfirstlane(wkmax);
     if (lane == 0) { bk[2 * wave] = wkmin; bk[2 * wave + 1] = wkmax; }
+    }
     if (has_seg) {
       seg_tile_ranges(segb, Sq, qt_first, nqt_all, qmin, qmax, tid, 256);
+    } else if (PAIRS) {  // (the tile's four classes take the place of the id range)
+      const int* cls = a.pm.kcls + ((int64_t)(a.pm.per_batch ? b : 0) * ((Skv + BNK - 1) / BNK) + tile) * nqt_tot;
+      for (int t = tid; t < nqt; t += 256) { qmin[t] = cls[t]; qmax[t] = 0; }
     } else {
       for (int t = tid; t < nqt; t += 256) { qmin[t] = 0; qmax[t] = 0; }
     }
@@ -307,7 +305,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     int cnt = 0;
     for (int base = 0; base < nqt; base += 64) {
       const int t = base + lane;
-      bool act = t < nqt && !(qmax[t] < bkmin || qmin[t] > bkmax);
+      bool act = t < nqt && (PAIRS ? qmin[t] != 0 : !(qmax[t] < bkmin || qmin[t] > bkmax));
       // (band: some row of the tile must reach into this workgroup's 128 kv rows)
       if (ext && act) act = kv0 <= pmax[t] + a.mx.hi_off && kv0 + BNK - 1 >= pmin[t] - a.mx.lo_off;
       const unsigned long long m = __ballot(act);
@@ -338,6 +336,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   // and all stream the same Q / dO tiles; each needs the tiles from its own kv rows on, so counting up they would start
   // at different tiles and never meet in the L2 (every tile fetched from memory once per workgroup); counting down
   // they start together at the last tile and stay within an L2's reach of each other.
+  // pair masks: this wave's 32 kv rows' words of a query tile, 256 bytes
+  const int skp = (Skv + BNK - 1) / BNK * BNK;
+  const u32x4 brw = make_rsrc_words(PAIRS ? (const void*)(a.pm.kbits + (int64_t)(a.pm.per_batch ? b : 0) * nqt_tot * skp) : a.k,
+                                    PAIRS ? (unsigned)nqt_tot * (unsigned)skp * 8u : 0u);
   auto qtile_of = [&](int idx) { return SEG ? ctl[4 * idx] : nqt_all - 1 - idx; };
   auto issue_tile = [&](int hl, int idx, int buf, int rslot) {
     const int hq = hk * a.n_rep + hl;
@@ -352,6 +354,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
                     : wave == 2 ? (const void*)segb : (const void*)a.mx.qpos;
     if (wave < 2 || (wave == 2 && has_seg) || (wave == 3 && has_pos))
       dma_dword(make_rsrc_words(src, (unsigned)Sq * 4u), (unsigned)(qt * BMQ) * 4u, rows_base + rslot * ROW_BYTES + wave * BMQ * 4, lane);
+    if constexpr (PAIRS)
+      dma_dword(brw, ((unsigned)qt * (unsigned)skp + (unsigned)wkv0) * 8u, rows_base + rslot * ROW_BYTES + VEC_BYTES + wave * 256, lane);
   };
 
   // per-lane byte offsets of the MFMA fragments inside a tile (the swizzles are resolved once, here)
@@ -390,8 +394,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     bool need_mask = (qi0 + BMQ > Sq) || (wkv0 + 32 > Skv) ||
                      (CAUSAL && (qi0 + band_hi < wkv0 + 31 || qi0 + BMQ - 1 - band_lo > wkv0));
     if (SEG) {
-      skip = skip || hi < wkmin || lo > wkmax;
-      need_mask = need_mask || !(lo == hi && wkmin == wkmax && lo == wkmin);
+      if (PAIRS) {
+        const int cls = (lo >> (8 * wave)) & 255;
+        skip = skip || cls == 0;
+        need_mask = need_mask || cls != 2;
+      } else {
+        skip = skip || hi < wkmin || lo > wkmax;
+        need_mask = need_mask || !(lo == hi && wkmin == wkmax && lo == wkmin);
+      }
     }
     if (ext) {
       const int plo = pmin[t], phi = pmax[t];
@@ -482,7 +492,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
       static_assert(AHEAD <= KS_QK, "the carried fragments all belong to S of the first query block");
       fr[i % NF] = ld16(aq[i] + Q_AT);
     });
-    struct { u32x4 rq, ro, rr; unsigned offq, offo, offr; } nx;
+    struct { u32x4 rq, ro, rr; unsigned offq, offo, offr, offb; } nx;
     const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
     const unsigned wave_q = __builtin_amdgcn_readfirstlane((unsigned)(wave * QT::PER_WAVE * 1024));
     const unsigned wave_o = __builtin_amdgcn_readfirstlane((unsigned)(wave * OT::PER_WAVE * 1024));
@@ -511,6 +521,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
       // LDS destinations of this wave's loads of tile t+2 (scalar byte addresses)
       const unsigned dma_q = lds_base + (unsigned)(Q_AT + buf2 * Q_BYTES) + wave_q;
       const unsigned dma_o = lds_base + (unsigned)(DO_AT + buf2 * DO_BYTES) + wave_o;
+      const unsigned dma_b = lds_base + (unsigned)(NBUF * BUF_BYTES + buf2 * ROW_BYTES + VEC_BYTES) + wave_r;  // (wave_r: 256 bytes a wave)
       const unsigned dma_r = lds_base + (unsigned)(NBUF * BUF_BYTES + buf2 * ROW_BYTES) + wave_r;
       // descriptors of tile t+2's loads (wave-uniform), issued piecewise in part 2.  The bases change with
       // the query head only; they are rebuilt when a new head starts (and when the tiles run out: size 0).
@@ -529,6 +540,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
         nx.offq = __builtin_amdgcn_readfirstlane((unsigned)qt * q_tile_bytes);
         nx.offo = __builtin_amdgcn_readfirstlane((unsigned)qt * do_tile_bytes);
         nx.offr = __builtin_amdgcn_readfirstlane((unsigned)(qt * BMQ) * 4u);
+        nx.offb = PAIRS ? __builtin_amdgcn_readfirstlane(((unsigned)qt * (unsigned)skp + (unsigned)wkv0) * 8u) : 0u;
       }
 
       // The tile body is laid out by hand as a sequence of slots, one MFMA each, with a scheduling barrier
@@ -554,7 +566,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
         constexpr int EPS = K2 >= 8 ? 1 : 2, VL = 16 / EPS;
         constexpr int VP0 = S1_AT, VP1 = D0_AT, VS0 = D1_AT, VS1 = C0;
         static_assert(VP0 + VL <= V0_AT && VS0 + VL <= K0_AT && VP1 + VL <= V1_AT && VS1 + VL <= K1_AT, "operands not ready");
-        constexpr int N_DMA = QT::PER_WAVE + OT::PER_WAVE + 1, DMA_EVERY = (NS - C0) / N_DMA;
+        constexpr int N_DMA = QT::PER_WAVE + OT::PER_WAVE + 1 + (PAIRS ? 1 : 0), DMA_EVERY = (NS - C0) / N_DMA;
         static_assert(DMA_EVERY >= 1, "second half too short for the loads");
         const int kvcol = wkv0 + ln;
         f32x16 s[2], dp[2];
@@ -571,13 +583,17 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
         // bit 8 (v / 4) + v % 4.
         unsigned rowbits[2] = {0u, 0u};
         const bool by_bits = MASKED && !(GEN && ext);
-        if (MASKED && by_bits) {
+        if (MASKED && PAIRS) {
+          const u32x2 w = *(const u32x2*)(rows_base + buf * ROW_BYTES + VEC_BYTES + wave * 256 + ln * 8);
+          rowbits[0] = w[0] >> (4 * g);
+          rowbits[1] = w[1] >> (4 * g);
+        } else if (MASKED && by_bits) {
           const int lo_r = CAUSAL ? max(kvcol - band_hi - qi0, 0) : 0;
           int hi_r = kvcol < Skv ? min(Sq - qi0, BMQ) : 0;
           if (CAUSAL) hi_r = min(hi_r, kvcol + band_lo - qi0 + 1);
           unsigned long long m = 0ull;
           if (hi_r > lo_r) m = (~0ull << lo_r) & (~0ull >> (64 - hi_r));
-          if (SEG && has_seg) {
+          if (SEG == SEG_IDS && has_seg) {
             const int rowseg = segl[lane];  // lane l: id of the tile's query row l
             unsigned long long ms = 0ull, todo = ~0ull;
             while (todo) {
@@ -727,7 +743,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
             // into buffers nobody reads any more)
             if constexpr (m < QT::PER_WAVE) qdma.template issue_one_at<m>(nx.rq, nx.offq, dma_q);
             else if constexpr (m < QT::PER_WAVE + OT::PER_WAVE) dodma.template issue_one_at<m - QT::PER_WAVE>(nx.ro, nx.offo, dma_o);
-            else dma_dword_at(nx.rr, nx.offr, dma_r, lane);
+            else if constexpr (m == QT::PER_WAVE + OT::PER_WAVE) dma_dword_at(nx.rr, nx.offr, dma_r, lane);
+            else dma_dword_at(brw, nx.offb, dma_b, lane);
           }
           if constexpr (COMPUTE) {
             // row vectors, a quad of rows at a time: -LSE of query block qb LEAD slots before the exponentials of that
@@ -818,7 +835,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
 // NW = waves per workgroup.  With 8 (head dims up to 128) two waves share a SIMD, 256 registers each: a wave
 // issues at most one instruction every four cycles, and at ~600 instructions for 48 MFMAs per tile a single
 // wave per SIMD leaves the matrix unit idle most of the time, whatever the order of its instructions.
-template <typename T, int DQK, int DV, int NW, bool CAUSAL, bool SEG>
+template <typename T, int DQK, int DV, int NW, bool CAUSAL, int SEG>
 __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
   typedef typename MT<T>::v8 v8;
   constexpr int BN = 64, BM = 32 * NW;
@@ -1423,7 +1440,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
 // a ballot over the tile's id vector, which wave 0 fetches with the tile (one more LDS-writing load).
 // Unequal head dims (192, 128): the same kernel with one workgroup per CU (its fragments and accumulators need more
 // than half a SIMD's registers) and the dQ accumulators pinned to the accumulation registers.
-template <typename T, int DQK, int DV, bool CAUSAL, bool SEG>
+template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
 __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kernel(const BwdArgs a) {
   typedef typename MT<T>::v8 v8;
   constexpr bool WIDE = DQK != DV;
@@ -1431,7 +1448,10 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   typedef DmaTile<DQK, true> KT;
   typedef DmaTile<DV, true> VT;
   constexpr int K_BYTES = KT::BYTES, V_BYTES = VT::BYTES, K_AT = 0, V_AT = 2 * K_BYTES;
-  constexpr int SEG_AT = 2 * (K_BYTES + V_BYTES), CTL_AT = SEG_AT + 2 * BN * 4;  // two id vectors; 16 bytes per visited tile
+  constexpr int SEG_AT = 2 * (K_BYTES + V_BYTES), VEC = SEG == SEG_PAIRS ? BM * 8 : BN * 4;  // id vectors or pair bits
+  constexpr int CTL_AT = SEG_AT + 2 * VEC;  // 16 bytes per visited tile
+  constexpr bool PAIRS = SEG == SEG_PAIRS;
+  static_assert(!PAIRS || CAUSAL, "pair masks run with the all-covering band of the causal kernels");
   constexpr int NLOAD_K = KT::PER_WAVE, NLOAD_V = VT::PER_WAVE, NLOAD2 = NLOAD_K + NLOAD_V;  // loads per wave and tile
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1496,11 +1516,25 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   }
 
   // ---- segment ids: the list of kv tiles to visit (tile, min id, max id), this wave's own id range
-  const int32_t* segb = SEG ? a.seg + (int64_t)b * Skv : nullptr;
-  const int segq = SEG ? segb[qrow_c] : 0;
+  const int32_t* segb = SEG == SEG_IDS ? a.seg + (int64_t)b * Skv : nullptr;
+  const int segq = SEG == SEG_IDS ? segb[qrow_c] : 0;
   const int* ctl = (const int*)(smem + CTL_AT);
   int nact = ntiles - t_first, wqmin = 0, wqmax = 0;
-  if (SEG) {
+  if constexpr (PAIRS) {
+    // the tiles with a pair of this block's 128 query rows in them, and their four classes
+    const int* cls = a.pm.qcls + ((int64_t)(a.pm.per_batch ? b : 0) * n_qt + qt) * ntiles;
+    int cnt = 0;
+    for (int base = 0; base < ntiles; base += 64) {
+      const int t = base + lane;
+      const int c4 = t < ntiles ? cls[t] : 0;
+      const unsigned long long m = __ballot(c4 != 0);
+      if (c4 != 0 && wave == 0) *(i32x4*)(smem + CTL_AT + 16 * (cnt + __popcll(m & ((1ull << lane) - 1ull)))) = i32x4{t, c4, 0, 0};
+      cnt += __popcll(m);
+    }
+    nact = cnt;
+    __syncthreads();
+  }
+  if (SEG == SEG_IDS) {
     wqmin = segq; wqmax = segq;
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) {
@@ -1540,7 +1574,9 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   VT vdma;
   kdma.init(a.ks[2], wave, lane);
   vdma.init(a.vs[2], wave, lane);
-  const u32x4 srw = make_rsrc_words(SEG ? (const void*)segb : (const void*)a.k, SEG ? (unsigned)Skv * 4u : 0u);
+  const int sqp = n_qt * BM;  // (rows of qbits are padded to the workgroup's 128)
+  const u32x4 srw = make_rsrc_words(PAIRS ? (const void*)(a.pm.qbits + (int64_t)(a.pm.per_batch ? b : 0) * ntiles * sqp) : SEG ? (const void*)segb : (const void*)a.k,
+                                    PAIRS ? (unsigned)ntiles * (unsigned)sqp * 8u : SEG ? (unsigned)Skv * 4u : 0u);
   const u32x4 krw = make_rsrc_words((const T*)a.k + b * a.ks[0] + hk * a.ks[1], span_bytes(Skv, a.ks[2], DQK));
   const u32x4 vrw = make_rsrc_words((const T*)a.v + b * a.vs[0] + hk * a.vs[1], span_bytes(Skv, a.vs[2], DV));
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
@@ -1554,8 +1590,10 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
     else
       vdma.template issue_one_at<p - NLOAD_K>(vrw, __builtin_amdgcn_readfirstlane((unsigned)t * v_tile_bytes), vdst0 + (unsigned)(buf * V_BYTES));
     // the tile's id vector rides with the first piece (rows past the end arrive as zeros and are masked by position)
-    if constexpr (SEG && p == 0) {
-      if (wave == 0) dma_dword_at(srw, __builtin_amdgcn_readfirstlane((unsigned)(t * BN) * 4u), lds_base + (unsigned)(SEG_AT + buf * BN * 4), lane);
+    if constexpr (PAIRS && p == 0)
+      dma_dword_at(srw, __builtin_amdgcn_readfirstlane(((unsigned)t * (unsigned)sqp + (unsigned)wq0_s) * 8u), lds_base + (unsigned)(SEG_AT + buf * VEC) + (unsigned)(wave_s * 256), lane);
+    if constexpr (SEG == SEG_IDS && p == 0) {
+      if (wave == 0) dma_dword_at(srw, __builtin_amdgcn_readfirstlane((unsigned)(t * BN) * 4u), lds_base + (unsigned)(SEG_AT + buf * VEC), lane);
     }
   };
 
@@ -1605,7 +1643,13 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
     // masked tiles: which of the tile's 64 kv rows this lane's query row may see, as bits (value v of a half: bit
     // 8 (v / 4) + v % 4 after the shift by 4 g)
     unsigned kbits[2] = {0u, 0u};
-    if (MASKED) {
+    if (MASKED && PAIRS) {
+      unsigned l4 = (unsigned)lane * 4u;  // (the load addresses keep it in a register; see below)
+      asm volatile("" : "+v"(l4));
+      const u32x2 w = *(const u32x2*)(smem + SEG_AT + buf * VEC + wave_s * 256 + ((l4 & 124u) << 1));
+      kbits[0] = w[0] >> (4 * g);
+      kbits[1] = w[1] >> (4 * g);
+    } else if (MASKED) {
       // (what only a masked tile needs is formed here from an opaque copy of lane * 4, which the loads of the
       // segment ids keep in a register anyway: the query row, the band offsets added to it and the address of the
       // lane's segment id, held across the loop as registers of their own, were spilled in the variant with
@@ -1622,8 +1666,8 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
       }
       if (qrow_m >= Sq) hi = 0;
       unsigned long long m = hi > lo ? ((~0ull << lo) & (~0ull >> (64 - hi))) : 0ull;
-      if (SEG) {
-        const int rowseg = *(const int*)(smem + SEG_AT + buf * BN * 4 + l4);  // lane l: id of the tile's kv row l
+      if (SEG == SEG_IDS) {
+        const int rowseg = *(const int*)(smem + SEG_AT + buf * VEC + l4);  // lane l: id of the tile's kv row l
         unsigned long long ms = 0ull, todo = ~0ull;
         while (todo) {
           const int x = __builtin_amdgcn_readlane(segq, (int)__builtin_ctzll(todo));
@@ -1750,7 +1794,13 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
     bool skip = CAUSAL && (kv0 > wq_last + band_hi || kv0 + BN - 1 < wq0 - band_lo);
     bool need_mask = (kv0 + BN > Skv) || (wq0 + 32 > Sq) ||
                      (CAUSAL && (kv0 + BN - 1 > wq0 + band_hi || kv0 < wq_last - band_lo));
-    if (SEG) {
+    if (PAIRS) {
+      const int cls = (cur[1] >> (8 * wave)) & 255;
+      // (added to the band's conditions, which never hold here: with decisions from the class alone the compiler keeps
+      // the two bodies' registers apart and spills)
+      skip = skip || cls == 0;
+      need_mask = need_mask || cls != 2;
+    } else if (SEG) {
       skip = skip || cur[2] < wqmin || cur[1] > wqmax;
       need_mask = need_mask || !(cur[1] == cur[2] && wqmin == wqmax && cur[1] == wqmin);
     }
@@ -1812,19 +1862,19 @@ static inline void mark(void* const* events, int i, hipStream_t st) {
 // The lean dQ kernel (attn_bwd_dq_plain_kernel) serves the plain and causal problems and segment ids with causality;
 // it computes delta itself and runs first.  Everything else (mask extensions, segment ids without causality, unequal
 // head dims without causality, a tile list too long for the LDS) takes the delta kernel and the general dQ kernel.
-template <int DQK, int DV, bool CAUSAL, bool SEG>
+template <int DQK, int DV, bool CAUSAL, int SEG>
 struct LeanDq {
   // (unequal head dims without causality stay with the general kernel: the compiler copies the pinned accumulators
   // between the branches of that variant's loop, right behind the MFMAs that write them)
   static constexpr bool BUILT = (!SEG || CAUSAL) && (DQK == DV || CAUSAL);
   static size_t lds_bytes(int Skv) {
     constexpr int BN = 64;
-    return 2 * (size_t)(DmaTile<DQK, true>::BYTES + DmaTile<DV, true>::BYTES) + (SEG ? 2 * BN * 4 + 16 * (size_t)((Skv + BN - 1) / BN) : 0);
+    return 2 * (size_t)(DmaTile<DQK, true>::BYTES + DmaTile<DV, true>::BYTES) + (SEG ? (SEG == SEG_PAIRS ? 2 * 128 * 8 : 2 * BN * 4) + 16 * (size_t)((Skv + BN - 1) / BN) : 0);
   }
   static bool taken(int Skv) { return BUILT && lds_bytes(Skv) <= 160 * 1024; }
 };
 
-template <typename T, int DQK, int DV, bool CAUSAL, bool SEG>
+template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
 static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
   typedef LeanDq<DQK, DV, CAUSAL, SEG> Lean;
   const bool lean = Lean::taken(a.Skv);
@@ -1833,7 +1883,7 @@ static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
   constexpr int DKDV_BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES;
   static_assert(DKDV_NBUF * DKDV_BUF <= 144 * 1024, "the three buffers must leave room for the row vectors and the tile list");
   const int nqt = (a.Sq + DKDV_BMQ - 1) / DKDV_BMQ;
-  const size_t dkdv_smem = (size_t)DKDV_NBUF * DKDV_BUF + 3 * DKDV_BMQ * 16 + (SEG ? (size_t)(6 * nqt + 8 + 4) * 4 : 0);
+  const size_t dkdv_smem = (size_t)DKDV_NBUF * DKDV_BUF + 3 * (DKDV_BMQ * 16 + (SEG == SEG_PAIRS ? DKDV_BNK * 8 : 0)) + (SEG ? (size_t)(6 * nqt + 8 + 4) * 4 : 0);
   TP_REQUIRE(dkdv_smem <= 160 * 1024 && (size_t)3 * nqt * 4 <= (size_t)DKDV_NBUF * DKDV_BUF, TP_ERR_UNSUPPORTED,
              "tp_attn_bwd: Sq=%d needs %zu bytes of LDS (max 163840)", a.Sq, dkdv_smem);
   mark(ev, 0, st);
@@ -1877,7 +1927,7 @@ static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
   }
   mark(ev, 2, st);
   // dQ, the general kernel
-  if constexpr (!Lean::BUILT || SEG) {
+  if constexpr (!Lean::BUILT || SEG == SEG_IDS) {
     if (!lean) {
     // eight waves (two per SIMD) where a wave's registers fit in half a SIMD's file
     // (the non-causal 128-wide variant does not fit 256 registers without spilling: it keeps four waves)
@@ -1906,46 +1956,50 @@ static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
 
 template <typename T, int DQK, int DV>
 static int dispatch_bwd(const BwdArgs& a, int causal, hipStream_t st, void* const* ev) {
+  if (a.pm.qbits) {
+    TP_REQUIRE((LeanDq<DQK, DV, true, SEG_PAIRS>::taken(a.Skv)), TP_ERR_UNSUPPORTED, "tp_attn_bwd_pairs: Skv=%d: the tile list does not fit the LDS", a.Skv);
+    return launch_bwd<T, DQK, DV, true, SEG_PAIRS>(a, st, ev);
+  }
   if (a.mx.on) {
     // a window and / or a causal offset and nothing else: the causal kernels, with that band instead of (-inf, 0]
     // (where the lean dQ kernel serves the problem; the general dQ kernel knows plain causality only)
-    const bool lean = a.seg ? LeanDq<DQK, DV, true, true>::taken(a.Skv) : LeanDq<DQK, DV, true, false>::taken(a.Skv);
+    const bool lean = a.seg ? LeanDq<DQK, DV, true, SEG_IDS>::taken(a.Skv) : LeanDq<DQK, DV, true, SEG_NONE>::taken(a.Skv);
     if (band_only(a.mx) && lean) {
       BwdArgs b = a;
       b.band_lo = a.mx.lo_off;
       b.band_hi = a.mx.hi_off;
       b.mx = no_mask_ext();
-      if (a.seg) return launch_bwd<T, DQK, DV, true, true>(b, st, ev);
-      return launch_bwd<T, DQK, DV, true, false>(b, st, ev);
+      if (a.seg) return launch_bwd<T, DQK, DV, true, SEG_IDS>(b, st, ev);
+      return launch_bwd<T, DQK, DV, true, SEG_NONE>(b, st, ev);
     }
     // the other mask extensions: the general instantiation (causality is part of the band then)
-    return launch_bwd<T, DQK, DV, false, true>(a, st, ev);
+    return launch_bwd<T, DQK, DV, false, SEG_IDS>(a, st, ev);
   }
   if (causal) {
-    if (a.seg) return launch_bwd<T, DQK, DV, true, true>(a, st, ev);
-    return launch_bwd<T, DQK, DV, true, false>(a, st, ev);
+    if (a.seg) return launch_bwd<T, DQK, DV, true, SEG_IDS>(a, st, ev);
+    return launch_bwd<T, DQK, DV, true, SEG_NONE>(a, st, ev);
   }
   if (a.seg) {
     // segment ids without causality: the causal kernels with a band that covers every key, where the lean dQ kernel
     // serves the problem (else the general instantiation)
-    if (LeanDq<DQK, DV, true, true>::taken(a.Skv)) {
+    if (LeanDq<DQK, DV, true, SEG_IDS>::taken(a.Skv)) {
       BwdArgs b = a;
       b.band_lo = BAND_INF;
       b.band_hi = BAND_INF;
-      return launch_bwd<T, DQK, DV, true, true>(b, st, ev);
+      return launch_bwd<T, DQK, DV, true, SEG_IDS>(b, st, ev);
     }
-    return launch_bwd<T, DQK, DV, false, true>(a, st, ev);
+    return launch_bwd<T, DQK, DV, false, SEG_IDS>(a, st, ev);
   }
-  if constexpr (!LeanDq<DQK, DV, false, false>::BUILT) {
+  if constexpr (!LeanDq<DQK, DV, false, SEG_NONE>::BUILT) {
     // (head dims for which the lean dQ kernel exists with causality only: the same band)
-    if (LeanDq<DQK, DV, true, false>::taken(a.Skv)) {
+    if (LeanDq<DQK, DV, true, SEG_NONE>::taken(a.Skv)) {
       BwdArgs b = a;
       b.band_lo = BAND_INF;
       b.band_hi = BAND_INF;
-      return launch_bwd<T, DQK, DV, true, false>(b, st, ev);
+      return launch_bwd<T, DQK, DV, true, SEG_NONE>(b, st, ev);
     }
   }
-  return launch_bwd<T, DQK, DV, false, false>(a, st, ev);
+  return launch_bwd<T, DQK, DV, false, SEG_NONE>(a, st, ev);
 }
 
 // One element type and head-dim pair per translation unit: this file is compiled once per pair and type
@@ -1972,10 +2026,10 @@ extern "C" int tp_attn_bwd_dq_first(int Skv, int Dqk, int Dv, int causal, int ha
   if (masked || (dtype != TP_BF16 && dtype != TP_F16)) return 0;
   auto pick = [&](auto dq, auto dv) -> int {
     constexpr int DQ = decltype(dq)::value, DVV = decltype(dv)::value;
-    if (causal) return has_seg ? LeanDq<DQ, DVV, true, true>::taken(Skv) : LeanDq<DQ, DVV, true, false>::taken(Skv);
+    if (causal) return has_seg ? LeanDq<DQ, DVV, true, SEG_IDS>::taken(Skv) : LeanDq<DQ, DVV, true, SEG_NONE>::taken(Skv);
     // (segment ids without causality run the causal kernels with an all-covering band where the lean kernel serves them)
-    if (has_seg || !LeanDq<DQ, DVV, false, false>::BUILT) return has_seg ? LeanDq<DQ, DVV, true, true>::taken(Skv) : LeanDq<DQ, DVV, true, false>::taken(Skv);
-    return LeanDq<DQ, DVV, false, false>::taken(Skv);
+    if (has_seg || !LeanDq<DQ, DVV, false, SEG_NONE>::BUILT) return has_seg ? LeanDq<DQ, DVV, true, SEG_IDS>::taken(Skv) : LeanDq<DQ, DVV, true, SEG_NONE>::taken(Skv);
+    return LeanDq<DQ, DVV, false, SEG_NONE>::taken(Skv);
   };
   typedef std::integral_constant<int, 64> I64;
   typedef std::integral_constant<int, 128> I128;
@@ -2006,7 +2060,7 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
                          const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                          const int64_t o_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
                          const int64_t dv_strides[3], float sm_scale, int causal, int dtype, void* stream,
-                         void* const* events, const MaskExt& mx) {
+                         void* const* events, const MaskExt& mx, const PairMask& pm = no_pair_mask()) {
   TP_REQUIRE(dout && q && k && v && out && lse && dq && dk && dv && ws, TP_ERR_BAD_ARG, "tp_attn_bwd: null pointer");
   TP_REQUIRE(do_strides && q_strides && k_strides && v_strides && o_strides && dq_strides && dk_strides && dv_strides,
              TP_ERR_BAD_ARG, "tp_attn_bwd: null stride array");
@@ -2048,8 +2102,9 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   a.scale_log2 = sm_scale * LOG2E;
   a.sm_scale = sm_scale;
   a.mx = mx;
-  a.band_lo = BAND_INF;  // plain causality (used by the causal kernels only)
-  a.band_hi = 0;
+  a.pm = pm;
+  a.band_lo = BAND_INF;  // plain causality (used by the causal kernels only); a pair mask's band covers every key
+  a.band_hi = pm.qbits ? BAND_INF : 0;
   hipStream_t st = (hipStream_t)stream;
   const bool bf = dtype == TP_BF16;
   if (Dqk == 128 && Dv == 128) return (bf ? bwd_bf16_128_128 : bwd_f16_128_128)(a, causal, st, events);
@@ -2116,5 +2171,21 @@ extern "C" int tp_attn_bwd(const void* dout, const void* q, const void* k, const
   return tp_attn_bwd_ex(dout, q, k, v, out, lse, seg, dq, dk, dv, ws, B, Hq, Hkv, Sq, Skv, Dqk, Dv, do_strides, q_strides,
                         k_strides, v_strides, o_strides, dq_strides, dk_strides, dv_strides, sm_scale, causal, dtype, stream,
                         nullptr);
+}
+
+extern "C" int tp_attn_bwd_pairs(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
+                                 const void* pairs, int mask_batches, void* dq, void* dk, void* dv, float* ws, int B, int Hq, int Hkv,
+                                 int Sq, int Skv, int Dqk, int Dv, const int64_t do_strides[3], const int64_t q_strides[3],
+                                 const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
+                                 const int64_t dq_strides[3], const int64_t dk_strides[3], const int64_t dv_strides[3], float sm_scale,
+                                 int dtype, void* stream) {
+  TP_REQUIRE(pairs && (mask_batches == 1 || mask_batches == B), TP_ERR_BAD_ARG, "tp_attn_bwd_pairs: null mask or %d masks for %d batches",
+             mask_batches, B);
+  TP_REQUIRE(Sq > 0 && Skv > 0, TP_ERR_BAD_ARG, "tp_attn_bwd_pairs: non-positive size");
+  TP_REQUIRE(dtype == TP_BF16 || dtype == TP_F16, TP_ERR_UNSUPPORTED, "tp_attn_bwd_pairs: dtype %d (bf16 and fp16 only)", dtype);
+  TP_REQUIRE((int64_t)((Sq + 127) / 128 + 1) * 128 * ((Skv + 127) / 128 + 1) * 16 < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_bwd_pairs: mask too large");
+  return attn_bwd_impl(dout, q, k, v, out, lse, nullptr, dq, dk, dv, ws, B, Hq, Hkv, Sq, Skv, Dqk, Dv, do_strides, q_strides, k_strides,
+                       v_strides, o_strides, dq_strides, dk_strides, dv_strides, sm_scale, 0, dtype, stream, nullptr, no_mask_ext(),
+                       pair_mask(pairs, mask_batches, Sq, Skv));
 }
 #endif  // !TP_BWD_UNIT

@@ -167,6 +167,47 @@ inline MaskExt no_mask_ext() {
   return m;
 }
 
+// ---- pair masks -----------------------------------------------------------------------------------
+// An additive mask whose entries are all either 0 or so negative that the pair drops out (padding, causal + padding,
+// block patterns: -inf or the lowest value of bfloat16 / float32) says only which (query, key) pairs take part.  It is
+// turned into bits once per forward (attn_mask.hip), in the two orders the kernels hold their scores in, with a class
+// per block of 32 rows and 64 columns:
+//   qbits[b][kv tile of 64][query row]   bit j: the row may see key 64 tile + j       (forward, dQ: a lane owns a row)
+//   kbits[b][query tile of 64][kv row]   bit i: query row 64 tile + i may see the key (dK/dV: a lane owns a key)
+//   qcls[b][128 query rows][kv tile], kcls[b][128 kv rows][query tile]: four bytes, one per 32 rows (one wave):
+//     0 no pair takes part (the tile is not visited), 2 every pair does (no masking), 1 anything else
+// Row counts are padded to 128 with zero bits.  All sections lie in one allocation, the flags first.
+struct PairMask {
+  const unsigned long long* qbits;
+  const unsigned long long* kbits;
+  const int* qcls;
+  const int* kcls;
+  int per_batch;  // 1: one mask per batch, 0: one for all
+};
+struct PairLayout {
+  int nqt, nkt, nqb, nkb;  // tiles of 64, blocks of 128
+  size_t qbits, kbits, qcls, kcls, bytes;  // byte offsets
+  PairLayout(int Bm, int Sq, int Skv) {
+    nqt = (Sq + 63) / 64; nkt = (Skv + 63) / 64; nqb = (Sq + 127) / 128; nkb = (Skv + 127) / 128;
+    size_t at = 64;  // flags: 16 ints
+    auto take = [&](size_t n) { const size_t o = at; at += (n + 63) / 64 * 64; return o; };
+    qbits = take((size_t)Bm * nkt * nqb * 128 * 8);
+    kbits = take((size_t)Bm * nqt * nkb * 128 * 8);
+    qcls = take((size_t)Bm * nqb * nkt * 4);
+    kcls = take((size_t)Bm * nkb * nqt * 4);
+    bytes = at;
+  }
+};
+inline PairMask no_pair_mask() { return PairMask{nullptr, nullptr, nullptr, nullptr, 0}; }
+inline PairMask pair_mask(const void* pairs, int Bm, int Sq, int Skv) {
+  const PairLayout l(Bm, Sq, Skv);
+  const unsigned char* p = (const unsigned char*)pairs;
+  return PairMask{(const unsigned long long*)(p + l.qbits), (const unsigned long long*)(p + l.kbits), (const int*)(p + l.qcls),
+                  (const int*)(p + l.kcls), Bm > 1 ? 1 : 0};
+}
+// SEG, the mask kind of an attention kernel: none, segment ids, a pair mask (with the all-covering band)
+constexpr int SEG_NONE = 0, SEG_IDS = 1, SEG_PAIRS = 2;
+
 // ---- buffer loads ---------------------------------------------------------------------------------
 // K/V/Q/dO tiles are fetched with raw buffer loads: the per-thread byte offset inside a tile is computed
 // once, the tile's offset is a scalar, so the per-tile address arithmetic is free, and rows past the end
@@ -349,6 +390,17 @@ struct DmaTile {
     static_assert(PER_WAVE <= 6, "head dim above 192");
   }
 };
+// 4 bytes per lane straight into LDS at dst + 4 * lane (a 64-entry row vector per instruction)
+__device__ __forceinline__ void dma_dword(u32x4 rs, unsigned byte_offset, unsigned char* dst, int lane) {
+  const unsigned d = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
+  byte_offset = __builtin_amdgcn_readfirstlane(byte_offset);
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               :: "s"(d), "v"((unsigned)lane * 4u), "s"(rs), "s"(byte_offset) : "memory", "m0");
+}
+__device__ __forceinline__ void dma_dword_at(u32x4 rs, unsigned byte_offset, unsigned dst, int lane) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               :: "s"(dst), "v"((unsigned)lane * 4u), "s"(rs), "s"(byte_offset) : "memory", "m0");
+}
 // two transposing reads -> one 16-byte MFMA operand: values 0..3 from the first address, 4..7 from the second
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));

@@ -36,19 +36,20 @@ struct FwdArgs {
   // Sliding windows and causal offsets without the other mask extensions run through these kernels.
   int band_lo, band_hi;
   MaskExt mx;
+  PairMask pm;
 };
 
 // Two workgroups per CU (256 registers per lane) where the kernel fits them; the non-causal variants at head dims of
 // 128 and more (run-time buffer index, mask extensions) and the 192-wide heads with segment ids need more registers
 // or LDS and take one workgroup per CU instead of spilling a hundred registers.
-template <int DQK, bool CAUSAL, bool SEG>
+template <int DQK, bool CAUSAL, int SEG>
 constexpr int fwd_blocks_per_cu() { return (DQK >= 128 && !CAUSAL) || (DQK > 128 && SEG) ? 1 : 2; }
 // The tiles are filled by buffer loads that write LDS directly (DmaTile): no staging registers, no LDS stores, and
 // dense swizzled rows instead of padded ones.  For the causal 192-wide heads that is what lets two workgroups share a
 // CU: two double-buffered tile sets of 81920 bytes fill the CU's 160 KB exactly (forward at 128 heads x 4096 rows:
 // 1.16 -> 0.89 ms with K loaded that way, 0.72 ms with V as well).
 
-template <typename T, int DQK, int DV, bool CAUSAL, bool SEG>
+template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
 __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void attn_fwd_kernel(const FwdArgs a) {
   typedef typename MT<T>::v8 v8;
   constexpr int BN = 64;              // kv rows per LDS tile, processed as two halves of 32
@@ -59,7 +60,8 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   typedef DmaTile<DV, true> VD;  // row-major like K; its transposed operand comes out of transposing LDS reads
   constexpr int K_BYTES = KD::BYTES;
   constexpr int V_BYTES = VD::BYTES;
-  constexpr int SEG_BYTES = SEG ? BN * 4 : 0;
+  // per buffer: the tile's segment ids, or the workgroup's rows' pair bits of the tile
+  constexpr int SEG_BYTES = SEG == SEG_PAIRS ? BM * 8 : SEG ? BN * 4 : 0;
   constexpr int BUF_BYTES = K_BYTES + V_BYTES + SEG_BYTES;
   // LDS layout: the two K tiles, then the two V^T tiles, then the two segment-id rows: with the buffer index a
   // constant, every address is a loop-invariant per-lane offset plus an immediate
@@ -87,8 +89,9 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   const T* kb = (const T*)a.k + b * a.ks[0] + hk * a.ks[1];
   const T* vb = (const T*)a.v + b * a.vs[0] + hk * a.vs[1];
   // GEN: the instantiation that also evaluates the mask extensions (and then may run without segment ids)
-  constexpr bool GEN = !CAUSAL && SEG;
-  const bool has_seg = SEG && (!GEN || a.seg != nullptr);
+  constexpr bool GEN = !CAUSAL && SEG == SEG_IDS, PAIRS = SEG == SEG_PAIRS;
+  static_assert(!PAIRS || CAUSAL, "pair masks run with the all-covering band of the causal kernels");
+  const bool has_seg = SEG == SEG_IDS && (!GEN || a.seg != nullptr);
   const bool ext = GEN && a.mx.on;
   const bool capped = GEN && a.mx.cap_in != 0.f;
   const bool biased = GEN && a.mx.bias != nullptr;
@@ -137,7 +140,21 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   const int* ctl = (const int*)(smem + 2 * BUF_BYTES);
   int nact = ntiles - t_first;
   int wqmin = 0, wqmax = 0;
-  if (SEG) {
+  if constexpr (PAIRS) {
+    // every wave builds the same list from the classes of this block's 128 query rows
+    const int* cls = a.pm.qcls + ((int64_t)(a.pm.per_batch ? b : 0) * n_qt + qt) * ntiles;
+    int cnt = 0;
+    for (int base = 0; base < ntiles; base += 64) {
+      const int t = base + lane;
+      const int c4 = t < ntiles ? cls[t] : 0;
+      const unsigned long long m = __ballot(c4 != 0);
+      if (c4 != 0 && wave == 0) *(i32x4*)(smem + 2 * BUF_BYTES + 16 * (cnt + __popcll(m & ((1ull << lane) - 1ull)))) = i32x4{t, c4, 0, 0};
+      cnt += __popcll(m);
+    }
+    nact = cnt;
+    __syncthreads();
+  }
+  if (SEG == SEG_IDS) {
     wqmin = segq; wqmax = segq;
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) {
@@ -197,6 +214,14 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   const unsigned kdst0 = lds_base + (unsigned)K_AT + (unsigned)(wave_s * K_ITEMS * 1024);
   const unsigned vdst0 = lds_base + (unsigned)V_AT + (unsigned)(wave_s * V_ITEMS * 1024);
   int sreg = 0;
+  // pair masks: this wave's 32 rows' words of a tile, 256 bytes, written to LDS by one load
+  const int sqp = n_qt * BM;  // (rows of qbits are padded to the workgroup's 128)
+  const u32x4 brw = make_rsrc_words(PAIRS ? (const void*)(a.pm.qbits + (int64_t)(a.pm.per_batch ? b : 0) * ntiles * sqp) : (const void*)kb,
+                                    PAIRS ? (unsigned)ntiles * (unsigned)sqp * 8u : 0u);
+  auto load_bits = [&](int t, int kbuf) {
+    dma_dword_at(brw, __builtin_amdgcn_readfirstlane(((unsigned)t * (unsigned)sqp + (unsigned)wq0) * 8u),
+                 lds_base + (unsigned)SEG_AT + (unsigned)(wave_s * 256) + (unsigned)(kbuf * SEG_STEP), lane);
+  };
   // piece P of the K_ITEMS + V_ITEMS loads of tile t into buffer kbuf, for issuing between MFMAs
   auto load_piece = [&](auto Pc, int t, int kbuf) {
     constexpr int p = decltype(Pc)::value;
@@ -209,11 +234,12 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   auto load_tile = [&](int t, int kbuf) {
     static_for<0, K_ITEMS + V_ITEMS>([&](auto P) { load_piece(P, t, kbuf); });
     if (has_seg && tid < BN) sreg = segb[min(t * BN + tid, Skv - 1)];
+    if constexpr (PAIRS) load_bits(t, kbuf);
   };
   // what is left to do before the barrier that hands buffer `buf` over: the id row, and the wait for this wave's
   // loads (they are outside the compiler's bookkeeping)
   auto store_tile = [&](int buf) {
-    if (SEG && tid < BN) ((int*)(smem + SEG_AT + buf * SEG_STEP))[tid] = sreg;
+    if (SEG == SEG_IDS && tid < BN) ((int*)(smem + SEG_AT + buf * SEG_STEP))[tid] = sreg;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
 
@@ -309,7 +335,11 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
     // extract and a bit-field insert of -inf instead of its compares.  kbits[hf] is shifted so that value v of the
     // lane's 16 is bit 8 (v / 4) + v % 4.
     unsigned kbits[2] = {0u, 0u};
-    if (MASKED) {
+    if (MASKED && PAIRS) {
+      const u32x2 w = *(const u32x2*)(smem + SEG_AT + buf * SEG_STEP + wave * 256 + ln * 8);
+      kbits[0] = w[0] >> (4 * g);
+      kbits[1] = w[1] >> (4 * g);
+    } else if (MASKED) {
       int lo = 0, hi = min(Skv - kv0, BN);
       if (CAUSAL) {
         hi = min(hi, qrow + band_hi - kv0 + 1);
@@ -321,7 +351,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
       }
       unsigned long long m = 0ull;
       if (hi > lo) m = (~0ull << lo) & (~0ull >> (64 - hi));
-      if (SEG && has_seg) {
+      if (SEG == SEG_IDS && has_seg) {
         const int rowseg = sl[lane];  // lane l: id of the tile's kv row l
         unsigned long long ms = 0ull, todo = ~0ull;
         while (todo) {
@@ -426,6 +456,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
       if constexpr (i < K_ITEMS + V_ITEMS) load_piece(I, t_next, buf ^ 1);
       if constexpr (i == 0) {
         if (has_seg && tid < BN) sreg = segb[min(t_next * BN + tid, Skv - 1)];
+        if constexpr (PAIRS) load_bits(t_next, buf ^ 1);
       }
       // one slot after the last MFMA of a half: mask, running max (the rare rescale of O is a wave-uniform
       // branch), then the exponentials under the following MFMAs
@@ -482,7 +513,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
     const int t_next = has_next ? nxt[0] : t;
     bool skip = CAUSAL && (kv0 > wq_last + band_hi || kv0 + BN - 1 < wq0 - band_lo);
     bool need_mask = (kv0 + BN > Skv) || (CAUSAL && (kv0 + BN - 1 > wq0 + band_hi || kv0 < wq_last - band_lo));
-    if (SEG) {
+    if (SEG == SEG_IDS) {
       const int lo = cur[1], hi = cur[2];
       skip = skip || hi < wqmin || lo > wqmax;
       need_mask = need_mask || !(lo == hi && wqmin == wqmax && lo == wqmin);
@@ -521,10 +552,17 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
       const int t_next = has_next ? nxt[0] : t;
       bool skip = CAUSAL && (kv0 > wq_last + band_hi || kv0 + BN - 1 < wq0 - band_lo);
       bool need_mask = (kv0 + BN > Skv) || (CAUSAL && (kv0 + BN - 1 > wq0 + band_hi || kv0 < wq_last - band_lo));
-      if (SEG) {
+      if (SEG == SEG_IDS) {
         const int lo = cur[1], hi = cur[2];
         skip = skip || hi < wqmin || lo > wqmax;
         need_mask = need_mask || !(lo == hi && wqmin == wqmax && lo == wqmin);
+      }
+      if (PAIRS) {
+        const int cls = (cur[1] >> (8 * wave_s)) & 255;
+        // (added to the band's conditions, which never hold here: with decisions from the class alone the compiler keeps
+        // the two bodies' registers apart and spills)
+        skip = skip || cls == 0;
+        need_mask = need_mask || cls != 2;
       }
       if (ext) {
         // outside every row's band: nothing to do; not inside every row's band (or a soft cap): element-wise path
@@ -575,10 +613,10 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
 // ------------------------------------------------------------------------------------------------
 // host dispatch
 // ------------------------------------------------------------------------------------------------
-template <typename T, int DQK, int DV, bool CAUSAL, bool SEG>
+template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
 static int launch_fwd(const FwdArgs& a, int B, hipStream_t st) {
   constexpr int BN = 64, BM = 128;
-  constexpr int BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES + (SEG ? BN * 4 : 0);
+  constexpr int BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES + (SEG == SEG_PAIRS ? BM * 8 : SEG ? BN * 4 : 0);
   const int ntiles_max = (a.Skv + BN - 1) / BN;
   const size_t smem = 2 * (size_t)BUF + (SEG ? (size_t)16 * ntiles_max : 0);  // (the id ranges borrow the tile buffers)
   TP_REQUIRE(smem <= 160 * 1024 && (!SEG || (size_t)(2 * ntiles_max + 16) * 4 <= 2 * (size_t)BUF), TP_ERR_UNSUPPORTED, "tp_attn_fwd: Skv=%d needs %zu bytes of LDS (max 163840)", a.Skv, smem);
@@ -596,6 +634,7 @@ static int launch_fwd(const FwdArgs& a, int B, hipStream_t st) {
 
 template <typename T, int DQK, int DV>
 static int dispatch_fwd(const FwdArgs& a, int B, int causal, hipStream_t st) {
+  if (a.pm.qbits) return launch_fwd<T, DQK, DV, true, SEG_PAIRS>(a, B, st);
   if (a.mx.on) {
     if (band_only(a.mx)) {
       // a window and / or a causal offset and nothing else: the causal kernels, with that band instead of (-inf, 0]
@@ -603,15 +642,15 @@ static int dispatch_fwd(const FwdArgs& a, int B, int causal, hipStream_t st) {
       b.band_lo = a.mx.lo_off;
       b.band_hi = a.mx.hi_off;
       b.mx = no_mask_ext();
-      if (a.seg) return launch_fwd<T, DQK, DV, true, true>(b, B, st);
-      return launch_fwd<T, DQK, DV, true, false>(b, B, st);
+      if (a.seg) return launch_fwd<T, DQK, DV, true, SEG_IDS>(b, B, st);
+      return launch_fwd<T, DQK, DV, true, SEG_NONE>(b, B, st);
     }
     // the other mask extensions: the general instantiation (causality is part of the band then)
-    return launch_fwd<T, DQK, DV, false, true>(a, B, st);
+    return launch_fwd<T, DQK, DV, false, SEG_IDS>(a, B, st);
   }
   if (causal) {
-    if (a.seg) return launch_fwd<T, DQK, DV, true, true>(a, B, st);
-    return launch_fwd<T, DQK, DV, true, false>(a, B, st);
+    if (a.seg) return launch_fwd<T, DQK, DV, true, SEG_IDS>(a, B, st);
+    return launch_fwd<T, DQK, DV, true, SEG_NONE>(a, B, st);
   }
   // no causality and no mask extension: the causal kernels with a band that covers every key.  (The instantiation
   // without causality ran the same tiles 1.8 times slower at the benchmark's shape, 5.03 against 2.76 ms, with bit-identical
@@ -619,8 +658,8 @@ static int dispatch_fwd(const FwdArgs& a, int B, int causal, hipStream_t st) {
   FwdArgs b = a;
   b.band_lo = BAND_INF;
   b.band_hi = BAND_INF;
-  if (a.seg) return launch_fwd<T, DQK, DV, true, true>(b, B, st);
-  return launch_fwd<T, DQK, DV, true, false>(b, B, st);
+  if (a.seg) return launch_fwd<T, DQK, DV, true, SEG_IDS>(b, B, st);
+  return launch_fwd<T, DQK, DV, true, SEG_NONE>(b, B, st);
 }
 
 // One element type and head-dim pair per translation unit, as in attn_bwd.hip; the unit without a pair holds the C
@@ -650,7 +689,8 @@ using namespace tp;
 static int attn_fwd_impl(const void* q, const void* k, const void* v, const int32_t* seg, void* out, float* lse,
                          int B, int Hq, int Hkv, int Sq, int Skv, int Dqk, int Dv, const int64_t q_strides[3],
                          const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
-                         float sm_scale, int causal, int dtype, void* stream, const MaskExt& mx) {
+                         float sm_scale, int causal, int dtype, void* stream, const MaskExt& mx,
+                         const PairMask& pm = no_pair_mask()) {
   TP_REQUIRE(q && k && v && out && lse && q_strides && k_strides && v_strides && o_strides, TP_ERR_BAD_ARG,
              "tp_attn_fwd: null pointer");
   TP_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Sq > 0 && Skv > 0, TP_ERR_BAD_ARG, "tp_attn_fwd: non-positive size");
@@ -677,8 +717,9 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, const int3
              TP_ERR_UNSUPPORTED, "tp_attn_fwd: one (batch, head) slice of k or v spans 2 GiB or more");
   a.scale_log2 = sm_scale * LOG2E;
   a.mx = mx;
-  a.band_lo = BAND_INF;  // plain causality (used by the causal kernels only)
-  a.band_hi = 0;
+  a.pm = pm;
+  a.band_lo = BAND_INF;  // plain causality (used by the causal kernels only); a pair mask's band covers every key
+  a.band_hi = pm.qbits ? BAND_INF : 0;
   hipStream_t st = (hipStream_t)stream;
   const bool bf = dtype == TP_BF16;
   if (Dqk == 128 && Dv == 128) return (bf ? fwd_bf16_128_128 : fwd_f16_128_128)(a, B, causal, st);
@@ -724,5 +765,18 @@ extern "C" int tp_attn_fwd_biased(const void* q, const void* k, const void* v, c
                        causal, dtype, stream,
                        make_mask_ext(q_positions, causal, causal_offset, window_left, window_right, logits_soft_cap, sm_scale, bias,
                                      bias_strides));
+}
+
+extern "C" int tp_attn_fwd_pairs(const void* q, const void* k, const void* v, const void* pairs, int mask_batches, void* out, float* lse,
+                                 int B, int Hq, int Hkv, int Sq, int Skv, int Dqk, int Dv, const int64_t q_strides[3],
+                                 const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3], float sm_scale,
+                                 int dtype, void* stream) {
+  TP_REQUIRE(pairs && (mask_batches == 1 || mask_batches == B), TP_ERR_BAD_ARG, "tp_attn_fwd_pairs: null mask or %d masks for %d batches",
+             mask_batches, B);
+  TP_REQUIRE(Sq > 0 && Skv > 0, TP_ERR_BAD_ARG, "tp_attn_fwd_pairs: non-positive size");
+  TP_REQUIRE(dtype == TP_BF16 || dtype == TP_F16, TP_ERR_UNSUPPORTED, "tp_attn_fwd_pairs: dtype %d (bf16 and fp16 only)", dtype);
+  TP_REQUIRE((int64_t)((Sq + 127) / 128) * 128 * ((Skv + 63) / 64) * 8 < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_fwd_pairs: mask too large");
+  return attn_fwd_impl(q, k, v, nullptr, out, lse, B, Hq, Hkv, Sq, Skv, Dqk, Dv, q_strides, k_strides, v_strides, o_strides, sm_scale, 0,
+                       dtype, stream, no_mask_ext(), pair_mask(pairs, mask_batches, Sq, Skv));
 }
 #endif  // !TP_FWD_UNIT

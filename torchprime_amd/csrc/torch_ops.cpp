@@ -151,6 +151,8 @@ TP_OP(attn_fwd_masked, T2(const Tensor&, const Tensor&, const Tensor&, OptTensor
                           double, OptTensor))
 TP_OP(attn_bwd_masked, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, OptTensor, OptTensor,
                           double, bool, int64_t, int64_t, int64_t, double, OptTensor))
+TP_OP(attn_fwd_pairs, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, double))
+TP_OP(attn_bwd_pairs, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, int64_t, double))
 TP_OP(l2norm_fwd, T2(const Tensor&, double))
 TP_OP(l2norm_bwd, Tensor(const Tensor&, const Tensor&, const Tensor&))
 TP_OP(scale_rows, Tensor(const Tensor&, const Tensor&))
@@ -600,6 +602,78 @@ T2 attn_fwd_masked_autograd(const Tensor& q, const Tensor& k, const Tensor& v, O
   return r;
 }
 
+// additive masks that only drop pairs (tp_mask_pairs): a (1|B, 1, Sq, Skv) mask in any of the three dtypes
+struct PairsIn { Tensor mask; int batches; std::array<int64_t, 2> strides; };
+PairsIn prep_pairs(const Tensor& mask, int64_t Sq, int64_t Skv) {
+  TORCH_CHECK_VALUE(mask.dim() == 4 && mask.size(1) == 1 && mask.size(2) == Sq && mask.size(3) == Skv, "mask must have shape (1|batch, 1, ", Sq,
+                    ", ", Skv, "), got (", mask.sizes(), ")");
+  const Tensor m = mask.stride(3) != 1 ? mask.contiguous() : mask;
+  return {m, (int)m.size(0), {m.size(0) == 1 ? 0 : m.stride(0), m.stride(2)}};
+}
+Tensor make_pairs(const PairsIn& m, int64_t Sq, int64_t Skv, bool verdict, void* stream) {
+  Tensor pairs = at::empty({(int64_t)tp_mask_pairs_bytes(m.batches, (int)Sq, (int)Skv) / 4}, m.mask.options().dtype(at::kInt));
+  if (verdict) pairs.slice(0, 0, 16).zero_();
+  check(tp_mask_pairs(m.mask.data_ptr(), m.strides.data(), m.batches, (int)Sq, (int)Skv, dtype_code(m.mask.scalar_type()), pairs.data_ptr(),
+                      (int)verdict, stream), "tp_mask_pairs");
+  return pairs;
+}
+// (out, lse, pairs): the bits are made once per forward and kept for the backward
+T3 attn_fwd_pairs_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& mask, double sm_scale) {
+  const c10::Device dev = require_gpu(q_, k_, v_, mask);
+  const AttnShape s = check_attn(q_, k_, v_, undef());
+  TORCH_CHECK_VALUE(mask.size(0) == 1 || mask.size(0) == s.B, "mask batch ", mask.size(0), " does not broadcast to ", s.B);
+  c10::DeviceGuard guard(dev);
+  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_);
+  const PairsIn m = prep_pairs(mask, s.Sq, s.Skv);
+  const Tensor pairs = make_pairs(m, s.Sq, s.Skv, false, stream_of(dev));
+  Tensor out = empty_like_heads(q, s.Dv), lse = empty_f32({s.B, s.Hq, s.Sq}, q);
+  const Strides3 qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out);
+  check(tp_attn_fwd_pairs(q.data_ptr(), k.data_ptr(), v.data_ptr(), pairs.data_ptr(), m.batches, out.data_ptr(), (float*)lse.data_ptr(), s.B, s.Hq,
+                          s.Hkv, s.Sq, s.Skv, s.Dqk, s.Dv, qs.data(), ks.data(), vs.data(), os.data(), (float)sm_scale,
+                          dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_fwd_pairs");
+  return {out, lse, pairs};
+}
+T3 attn_bwd_pairs_cuda(const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
+                       const Tensor& pairs, int64_t mask_batches, double sm_scale) {
+  const c10::Device dev = require_gpu(dout_, q_, k_, v_, out_, lse_, pairs);
+  const AttnShape s = check_attn(q_, k_, v_, undef());
+  TORCH_CHECK_VALUE(pairs.is_contiguous() && pairs.scalar_type() == at::kInt && mask_batches > 0 &&
+                    pairs.numel() == (int64_t)tp_mask_pairs_bytes((int)mask_batches, s.Sq, s.Skv) / 4, "pairs were not made for this problem");
+  c10::DeviceGuard guard(dev);
+  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), out = prep_heads(out_), dout = prep_heads(dout_);
+  const Tensor lse = lse_.contiguous();
+  Tensor dq = empty_like_heads(q, s.Dqk), dk = empty_like_heads(k, s.Dqk), dv = empty_like_heads(v, s.Dv);
+  Tensor ws = empty_f32({(int64_t)tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq) / 4}, q);
+  const Strides3 gs = strides3(dout), qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out), dqs = strides3(dq),
+                 dks = strides3(dk), dvs = strides3(dv);
+  check(tp_attn_bwd_pairs(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (const float*)lse.data_ptr(),
+                          pairs.data_ptr(), (int)mask_batches, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)ws.data_ptr(), s.B, s.Hq, s.Hkv,
+                          s.Sq, s.Skv, s.Dqk, s.Dv, gs.data(), qs.data(), ks.data(), vs.data(), os.data(), dqs.data(), dks.data(), dvs.data(),
+                          (float)sm_scale, dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_bwd_pairs");
+  return {dq, dk, dv};
+}
+struct AttnPairsNode : OpNode {
+  int64_t mask_batches;
+  double sm_scale;
+  std::string name() const override { return "TprimeAttnPairsBackward"; }
+  variable_list bwd(variable_list&& g) override {
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    T3 r = op_attn_bwd_pairs()(g[0], get(0), get(1), get(2), get(3), get(4), get(5), mask_batches, sm_scale);
+    return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
+  }
+};
+T3 attn_fwd_pairs_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+  auto node = make_node<AttnPairsNode>(q, k, v);
+  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_attn_fwd_pairs()(q, k, v, mask, sm_scale); }();
+  if (node) {
+    torch::autograd::set_history(std::get<0>(r), node);
+    node->keep(q); node->keep(k); node->keep(v); node->keep(std::get<0>(r), true); node->keep(std::get<1>(r)); node->keep(std::get<2>(r));
+    node->mask_batches = mask.size(0);
+    node->sm_scale = sm_scale;
+  }
+  return r;
+}
+
 // ---- L2 norm, temperature scale ----------------------------------------------------------------------------------
 T2 l2norm_fwd_cuda(const Tensor& x, double eps) {
   const c10::Device dev = require_gpu(x);
@@ -790,6 +864,23 @@ Tensor py_attention_masked(const Tensor& q, const Tensor& k, const Tensor& v, Op
   require_gpu(q, k, v, seg, qpos, bias);
   return std::get<0>(op_attn_fwd_masked()(q, k, v, seg, qpos, sm_scale, causal, causal_offset, window_left, window_right, soft_cap, bias));
 }
+Tensor py_attention_pairs(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+  require_gpu(q, k, v, mask);
+  return std::get<0>(op_attn_fwd_pairs()(q, k, v, mask, sm_scale));
+}
+// What a (1|B, 1, Sq, Skv) mask is: 1 the exact causal mask, 2 one that only drops pairs, 0 anything else.  Two short
+// kernels and one synchronisation.
+int64_t py_mask_kind(const Tensor& mask) {
+  const c10::Device dev = require_gpu(mask);
+  TORCH_CHECK_VALUE(mask.dim() == 4, "expected a 4-D mask");
+  if (mask.numel() == 0) return 0;
+  c10::DeviceGuard guard(dev);
+  at::AutoDispatchBelowADInplaceOrView below;
+  const PairsIn m = prep_pairs(mask, mask.size(2), mask.size(3));
+  const Tensor flags = make_pairs(m, mask.size(2), mask.size(3), true, stream_of(dev)).slice(0, 0, 16).cpu();
+  const int* f = flags.const_data_ptr<int>();
+  return !f[1] ? 1 : (!f[0] && !f[2]) ? 2 : 0;
+}
 Tensor py_l2norm(const Tensor& x, double eps) { return std::get<0>(op_l2norm_fwd()(x, eps)); }
 Tensor py_swiglu(const Tensor& g, const Tensor& u) { return op_swiglu_fwd()(g, u); }
 Tensor py_cross_entropy(const Tensor& l, const Tensor& y, int64_t ignore) { return std::get<0>(op_cross_entropy_fwd()(l, y, ignore)); }
@@ -810,6 +901,9 @@ TORCH_LIBRARY(tprime, m) {
         "int window_left, int window_right, float soft_cap, Tensor? bias=None) -> (Tensor, Tensor)");
   m.def("attn_bwd_masked(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor? seg, Tensor? qpos, float sm_scale, "
         "bool causal, int causal_offset, int window_left, int window_right, float soft_cap, Tensor? bias=None) -> (Tensor, Tensor, Tensor)");
+  m.def("attn_fwd_pairs(Tensor q, Tensor k, Tensor v, Tensor mask, float sm_scale) -> (Tensor, Tensor, Tensor)");
+  m.def("attn_bwd_pairs(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor pairs, int mask_batches, float sm_scale) "
+        "-> (Tensor, Tensor, Tensor)");
   m.def("l2norm_fwd(Tensor x, float eps) -> (Tensor, Tensor)");
   m.def("l2norm_bwd(Tensor dy, Tensor x, Tensor rstd) -> Tensor");
   m.def("scale_rows(Tensor x, Tensor scale) -> Tensor");
@@ -830,6 +924,8 @@ TORCH_LIBRARY_IMPL(tprime, CUDA, m) {
   m.impl("attn_bwd", attn_bwd_cuda);
   m.impl("attn_fwd_masked", attn_fwd_masked_cuda);
   m.impl("attn_bwd_masked", attn_bwd_masked_cuda);
+  m.impl("attn_fwd_pairs", attn_fwd_pairs_cuda);
+  m.impl("attn_bwd_pairs", attn_bwd_pairs_cuda);
   m.impl("l2norm_fwd", l2norm_fwd_cuda);
   m.impl("l2norm_bwd", l2norm_bwd_cuda);
   m.impl("scale_rows", scale_rows_cuda);
@@ -845,12 +941,13 @@ TORCH_LIBRARY_IMPL(tprime, Autograd, m) {
   m.impl("rope_apply", rope_apply_autograd);
   m.impl("attn_fwd", attn_fwd_autograd);
   m.impl("attn_fwd_masked", attn_fwd_masked_autograd);
+  m.impl("attn_fwd_pairs", attn_fwd_pairs_autograd);
   m.impl("l2norm_fwd", l2norm_fwd_autograd);
   m.impl("scale_rows", scale_rows_autograd);
   m.impl("swiglu_fwd", swiglu_fwd_autograd);
   m.impl("cross_entropy_fwd", cross_entropy_fwd_autograd);
-  for (const char* name : {"rope_table", "rmsnorm_bwd", "add_rmsnorm_bwd", "attn_bwd", "attn_bwd_masked", "l2norm_bwd", "swiglu_bwd",
-                           "cross_entropy_bwd"})
+  for (const char* name : {"rope_table", "rmsnorm_bwd", "add_rmsnorm_bwd", "attn_bwd", "attn_bwd_masked", "attn_bwd_pairs", "l2norm_bwd",
+                           "swiglu_bwd", "cross_entropy_bwd"})
     m.impl(name, torch::autograd::autogradNotImplementedFallback());
 }
 
@@ -861,6 +958,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_apply", &py_rope_apply);
   m.def("attention", &py_attention);
   m.def("attention_masked", &py_attention_masked);
+  m.def("attention_pairs", &py_attention_pairs);
+  m.def("mask_kind", &py_mask_kind);
+  m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
   m.def("l2norm", &py_l2norm);
   m.def("swiglu", &py_swiglu);
   m.def("cross_entropy", &py_cross_entropy);

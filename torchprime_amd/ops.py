@@ -46,6 +46,7 @@ add_rmsnorm_fwd, add_rmsnorm_bwd = _ops.add_rmsnorm_fwd.default, _ops.add_rmsnor
 rope_table, rope_apply_op = _ops.rope_table.default, _ops.rope_apply.default
 attn_fwd, attn_bwd = _ops.attn_fwd.default, _ops.attn_bwd.default
 attn_fwd_masked, attn_bwd_masked = _ops.attn_fwd_masked.default, _ops.attn_bwd_masked.default
+attn_fwd_pairs, attn_bwd_pairs = _ops.attn_fwd_pairs.default, _ops.attn_bwd_pairs.default
 l2norm_fwd, l2norm_bwd = _ops.l2norm_fwd.default, _ops.l2norm_bwd.default
 scale_rows = _ops.scale_rows.default
 swiglu_fwd, swiglu_bwd = _ops.swiglu_fwd.default, _ops.swiglu_bwd.default
@@ -121,6 +122,18 @@ def _(q, k, v, seg, qpos, sm_scale, causal, causal_offset, window_left, window_r
 
 @torch.library.register_fake("tprime::attn_bwd_masked")
 def _(dout, q, k, v, out, lse, seg, qpos, sm_scale, causal, causal_offset, window_left, window_right, soft_cap, bias=None):
+  return _empty_like_heads(q), _empty_like_heads(k), _empty_like_heads(v)
+
+
+@torch.library.register_fake("tprime::attn_fwd_pairs")
+def _(q, k, v, mask, sm_scale):
+  B, Hq, Sq, _ = q.shape
+  words = _native.mask_pairs_words(mask.shape[0], Sq, k.shape[2])
+  return _empty_like_heads(q, v.shape[-1]), q.new_empty((B, Hq, Sq), dtype=torch.float32), q.new_empty((words,), dtype=torch.int32)
+
+
+@torch.library.register_fake("tprime::attn_bwd_pairs")
+def _(dout, q, k, v, out, lse, pairs, mask_batches, sm_scale):
   return _empty_like_heads(q), _empty_like_heads(k), _empty_like_heads(v)
 
 
@@ -245,6 +258,25 @@ def attention(
     bias = bias.detach()
   args = (q, k, v, segment_ids, q_positions, sm_scale, causal, causal_offset, wl, wr, float(soft_cap or 0.0), bias)
   return attn_fwd_masked(*args)[0] if is_compiling() else _native.attention_masked(*args)
+
+
+# kinds of additive masks (mask_kind)
+MASK_GENERAL, MASK_CAUSAL, MASK_PAIRS = 0, 1, 2
+
+
+def mask_kind(mask: Tensor) -> int:
+  """What a (1|B, 1, Sq, Skv) additive mask is: ``MASK_CAUSAL`` (exactly 0 on and below the diagonal, -inf above),
+  ``MASK_PAIRS`` (every entry 0 or one that lets its pair drop out of the softmax, and no row of finite such entries
+  only: causality + padding) or ``MASK_GENERAL``.  Waits for the device."""
+  return _native.mask_kind(mask)
+
+
+def attention_pairs(q: Tensor, k: Tensor, v: Tensor, mask: Tensor, sm_scale: float) -> Tensor:
+  """Attention under an additive mask of kind ``MASK_PAIRS`` (1|B, 1, Sq, Skv): as ``attention(bias=mask)``, with the
+  mask as one bit per pair, tiles without a pair left out and tiles with every pair unmasked.  bfloat16 and float16."""
+  if is_compiling():
+    return attn_fwd_pairs(q, k, v, mask, sm_scale)[0]
+  return _native.attention_pairs(q, k, v, mask, sm_scale)
 
 
 def l2norm(x: Tensor, eps: float) -> Tensor:
