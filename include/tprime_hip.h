@@ -336,6 +336,29 @@ int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float*
                          int64_t labels_b_stride, int64_t dlogits_b_stride, int64_t dlogits_s_stride,
                          int ignore_index, int dtype, void* stream);
 
+/* ------------------------------------------------------------------------------------------------
+ * Small matrix products, up to four in one launch: c[m, n] = sum over segments j and k of a_j(m, k) b_j(n, k),
+ * fp32 accumulation, one rounding.  The projections of small models (nn.Linear without bias,
+ * torchprime/torch_xla_models/model/llama/model.py:125-139, 189-238), forward and backward.
+ *   a_kmajor != 0   a(m, k) = a[m*lda + k], else a[k*lda + m];   b likewise with n
+ *                   (built: both k-major, a only, neither)
+ *   c               row stride ldc; rows of a multiple of 4 values, 16-byte aligned; operand rows 16-byte
+ *                   aligned; a k-major contraction is a multiple of 16 bytes
+ * dtype: TP_BF16, TP_F16 or TP_F32 for a, b and c alike.
+ * ---------------------------------------------------------------------------------------------- */
+typedef struct tp_linear_problem {
+  const void* a[3];
+  const void* b[3];
+  int64_t lda[3], ldb[3];
+  int k[3];
+  int segments; /* 1..3 */
+  int a_kmajor, b_kmajor;
+  int m, n;
+  void* c;
+  int64_t ldc;
+} tp_linear_problem;
+int tp_linears(const tp_linear_problem* problems, int count, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,69 @@
+"""Grouped small projections (``linear.project``) against float64 products: edges of the 64 x 64 tiles and of the 64- / 32-
+value steps of the contraction, one to three weights with a summed input gradient, gradients that are strided views or
+missing.  Bound: the operands are exact, sums are float32, so an element is off by its one rounding (2^-9 relative for
+bfloat16, 2^-12 for float16) and by at most K 2^-24 of the sum of magnitudes; on normal data both are far below
+``2^-8`` / ``2^-11`` / ``1e-5`` of the tensor in the 2-norm."""
+
+import pytest
+import torch
+from torch import nn
+
+from tests.util import randn
+from torchprime_amd.linear import project
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+REL = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 1e-5}
+
+
+def _close(got, ref, dtype, name):
+  got, ref = got.double().cpu(), ref.double()
+  assert torch.isfinite(got).all(), name
+  err = ((got - ref).norm() / ref.norm()).item()
+  assert err <= REL[dtype], f"{name}: {err:.3e} > {REL[dtype]:.3e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,K,Ns", [(1, 64, (64,)), (16, 8, (8,)), (63, 72, (64, 8)), (65, 512, (512, 128, 128)), (130, 136, (72, 200)),
+                                    (300, 512, (64, 64)), (513, 64, (512,))])  # fmt: skip
+def test_forward_and_gradients(M, K, Ns, dtype):
+  x = randn((M, K), 1, dtype)
+  ws = [randn((n, K), 10 + i, dtype) for i, n in enumerate(Ns)]
+  gs = [randn((M, n), 20 + i, dtype) for i, n in enumerate(Ns)]
+  mods = [nn.Linear(K, n, bias=False, device=DEV, dtype=dtype) for n in Ns]
+  with torch.no_grad():
+    for m, w in zip(mods, ws):
+      m.weight.copy_(w)
+  xd = x.to(DEV).requires_grad_(True)
+  outs = project(xd.view(1, M, K), *mods)
+  assert all(o.grad_fn.name() == "TprimeLinearsBackward" and o.shape == (1, M, n) for o, n in zip(outs, Ns))
+  for o, w in zip(outs, ws):
+    _close(o[0], x.double() @ w.double().T, dtype, "out")
+  # gradients as a caller may hand them over: contiguous, and the first as a strided view
+  wide = torch.cat([gs[0], gs[0]], 1).to(DEV)
+  grads = [wide[:, : Ns[0]][None]] + [g.to(DEV)[None] for g in gs[1:]]
+  got = torch.autograd.grad(outs, [xd] + [m.weight for m in mods], grads, retain_graph=True)
+  _close(got[0], sum(g.double() @ w.double() for g, w in zip(gs, ws)), dtype, "dx")
+  for d, g in zip(got[1:], gs):
+    _close(d, g.double().T @ x.double(), dtype, "dw")
+  # only the last output used; only the input asked for
+  (dx,) = torch.autograd.grad(outs[-1], xd, grads[-1])
+  _close(dx, gs[-1].double() @ ws[-1].double(), dtype, "dx of one output")
+
+
+def test_what_the_modules_have_to_see_themselves():
+  """Hooks, a bias, autocast, a recorded backward: the results are the modules' own."""
+  x = randn((7, 64), 1, torch.float32).to(DEV).requires_grad_(True)
+  m, b = nn.Linear(64, 64, bias=False, device=DEV), nn.Linear(64, 64, device=DEV)
+  seen = []
+  h = m.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+  project(x, m)
+  assert seen == [(7, 64)]
+  h.remove()
+  assert torch.equal(project(x, b)[0], b(x))
+  with torch.autocast("cuda", dtype=torch.bfloat16):
+    assert project(x, m)[0].dtype == torch.bfloat16
+  (g,) = torch.autograd.grad(project(x, m)[0].pow(2).sum(), x, create_graph=True)
+  (gg,) = torch.autograd.grad(g.sum(), x)
+  w = m.weight.detach().double().cpu()
+  _close(gg, 2.0 * torch.ones(7, 64, dtype=torch.float64) @ w.T @ w, torch.float32, "second derivative")

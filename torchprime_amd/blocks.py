@@ -1,6 +1,7 @@
 """Attention blocks that call the hot path the way the reference's models do.  They exist so tests
 and the benchmark can drive RMSNorm -> projections -> RoPE -> attention -> output projection with the
-reference's tensor layouts; the projections are stock ``nn.Linear`` (GEMMs are outside the path).
+reference's tensor layouts; the projections are stock ``nn.Linear`` modules
+(``linear.project`` calls them).
 
 * LlamaAttention        torchprime/torch_xla_models/model/llama/model.py:156-238
 * MixtralAttention      model/mixtral/model.py:159-243
@@ -15,6 +16,7 @@ import torch
 from torch import nn
 
 from .attention import AttentionModule
+from .linear import project
 from .norm import DeepseekV3RMSNorm
 from .rotary import MixtralRotaryEmbedding, apply_rotary_pos_emb, apply_rotary_pos_emb_interleave
 
@@ -43,14 +45,15 @@ class LlamaAttention(nn.Module):
 
   def forward(self, hidden_states, position_embeddings, attention_mask=None, position_ids=None):
     bsz, q_len, _ = hidden_states.size()
-    q = self.q_proj(hidden_states).view(bsz, q_len, self.num_heads, self.head_dim).transpose(1, 2)
-    k = self.k_proj(hidden_states).view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
-    v = self.v_proj(hidden_states).view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
+    q, k, v = project(hidden_states, self.q_proj, self.k_proj, self.v_proj)
+    q = q.view(bsz, q_len, self.num_heads, self.head_dim).transpose(1, 2)
+    k = k.view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
+    v = v.view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
     cos, sin = position_embeddings
     q, k = apply_rotary_pos_emb(q, k, cos, sin)
     out = self.attention_block(q, k, v, attention_mask)
     out = out.transpose(1, 2).contiguous().reshape(bsz, q_len, self.hidden_size)
-    return self.o_proj(out)
+    return project(out, self.o_proj)[0]
 
 
 class MixtralAttention(nn.Module):
@@ -81,14 +84,15 @@ class MixtralAttention(nn.Module):
 
   def forward(self, hidden_states, attention_mask=None, position_ids=None):
     bsz, q_len, _ = hidden_states.size()
-    q = self.q_proj(hidden_states).view(bsz, q_len, self.num_heads, self.head_dim).transpose(1, 2)
-    k = self.k_proj(hidden_states).view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
-    v = self.v_proj(hidden_states).view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
+    q, k, v = project(hidden_states, self.q_proj, self.k_proj, self.v_proj)
+    q = q.view(bsz, q_len, self.num_heads, self.head_dim).transpose(1, 2)
+    k = k.view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
+    v = v.view(bsz, q_len, self.num_key_value_heads, self.head_dim).transpose(1, 2)
     cos, sin = self.rotary_emb(v, seq_len=k.shape[-2])
     q, k = apply_rotary_pos_emb(q, k, cos, sin, position_ids)
     out = self.attention_block(q, k, v, attention_mask)
     out = out.transpose(1, 2).contiguous().reshape(bsz, q_len, self.hidden_size)
-    return self.o_proj(out)
+    return project(out, self.o_proj)[0]
 
 
 class DeepseekV3Attention(nn.Module):
@@ -144,7 +148,7 @@ class DeepseekV3Attention(nn.Module):
     k = torch.cat((k_pass, k_rot), dim=-1)
     out = self.attention_block(q, k, v, attention_mask)
     out = out.transpose(1, 2).contiguous().reshape(bsz, q_len, -1)
-    return self.o_proj(out)
+    return project(out, self.o_proj)[0]
 
 
 class Llama4TextAttention(nn.Module):
@@ -186,9 +190,10 @@ class Llama4TextAttention(nn.Module):
     from .llama4 import apply_attn_temperature, apply_rotary_emb
 
     bsz, q_len, _ = hidden_states.size()
-    q = self.q_proj(hidden_states).view(bsz, q_len, -1, self.head_dim)
-    k = self.k_proj(hidden_states).view(bsz, q_len, -1, self.head_dim)
-    v = self.v_proj(hidden_states).view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
+    q, k, v = project(hidden_states, self.q_proj, self.k_proj, self.v_proj)
+    q = q.view(bsz, q_len, -1, self.head_dim)
+    k = k.view(bsz, q_len, -1, self.head_dim)
+    v = v.view(bsz, q_len, -1, self.head_dim).transpose(1, 2)
     if self.use_rope:
       q, k = apply_rotary_emb(q, k, position_embeddings)
     if hasattr(self, "qk_norm"):
@@ -197,7 +202,7 @@ class Llama4TextAttention(nn.Module):
       q = apply_attn_temperature(q, self.floor_scale, self.attn_scale)
     out = self.attention_block(q.transpose(1, 2), k.transpose(1, 2), v, attention_mask)
     out = out.transpose(1, 2).contiguous().reshape(bsz, q_len, self.hidden_size)
-    return self.o_proj(out)
+    return project(out, self.o_proj)[0]
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -329,7 +334,7 @@ class LlamaForCausalLM(nn.Module):
     from .loss import cross_entropy_loss
 
     hidden_states = self.model(input_ids=input_ids, attention_mask=attention_mask)
-    logits = self.lm_head(hidden_states).float()
+    logits = project(hidden_states, self.lm_head)[0].float()
     if labels is None:
       return logits, None
     return logits, cross_entropy_loss(logits, labels=labels, vocab_size=self.config.vocab_size)

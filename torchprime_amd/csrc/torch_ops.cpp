@@ -16,6 +16,7 @@
 #include <torch/extension.h>
 #include <torch/library.h>
 
+#include <ATen/autocast_mode.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -839,6 +840,153 @@ T3 cross_entropy_fwd_autograd(const Tensor& logits, const Tensor& labels, int64_
   return r;
 }
 
+// ---- projections -------------------------------------------------------------------------------------------------
+// One input through one to three nn.Linear weights (no bias): tp_linears where the products are small, at::linear where
+// they are not, or where anything but plain eager tensors is involved.
+//
+// No mode, transform, autocast or tensor subclass is to see these calls: they do not go through the dispatcher.
+bool plain_eager(const Tensor& t) {
+  static const c10::DispatchKeySet usual({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
+  const c10::DispatchKeySet on = c10::impl::tls_local_dispatch_key_set().included_;
+  return (on - usual).empty() && !at::autocast::is_autocast_enabled(at::kCUDA) && t.is_cuda() && !t.unsafeGetTensorImpl()->is_python_dispatch() && t.layout() == at::kStrided;
+}
+// The line between the two, in multiply-adds of the whole group.  Measured with the host's time, us, tp_linears against
+// at::linear, forward | forward + backward:  bf16 512 x 512 through three 512 x 512: 8 : 62 | 83 : 296;  1024 x 1024 through
+// three 1024 x 1024 (3.2e9): 17 : 60 | 81 : 291;  1024 x 2048 through 2048 x 2048 (4.3e9): 18 : 20 | 52 : 114.  Beyond that
+// the library's larger tiles win on the device.  fp32: 2048 x 512 through three 512 x 512 (1.6e9): 39 : 60 | 126 : 287;
+// 3.2e9: 69 : 60 | 208 : 290;  4.3e9: 76 : 62 | 270 : 188.
+int64_t lin_max_work(at::ScalarType t) { return t == at::kFloat ? 1ll << 31 : 1ll << 32; }
+bool linears_take(const Tensor& x, const std::vector<Tensor>& ws) {
+  const auto t = x.scalar_type();
+  if (ws.empty() || ws.size() > 3 || x.dim() < 1 || x.numel() == 0 || !plain_eager(x)) return false;
+  if (t != at::kBFloat16 && t != at::kHalf && t != at::kFloat) return false;
+  const int64_t k = x.size(-1), m = x.numel() / k, vec = 16 / x.element_size();
+  int64_t n = 0;
+  for (const auto& w : ws) {
+    if (!plain_eager(w) || w.dim() != 2 || w.scalar_type() != t || w.device() != x.device() || w.size(1) != k || !w.is_contiguous()) return false;
+    if (w.size(0) == 0 || w.size(0) % vec || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) return false;
+    n += w.size(0);
+  }
+  return k % vec == 0 && m * n * k <= lin_max_work(t);
+}
+
+struct LinearsNode : torch::autograd::Node {
+  SavedVariable x;
+  std::vector<SavedVariable> ws;
+  std::string name() const override { return "TprimeLinearsBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    x.reset_data();
+    for (auto& w : ws) w.reset_data();
+  }
+  variable_list apply(variable_list&& g) override;
+};
+tp_linear_problem lin_problem(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k, bool a_kmajor, bool b_kmajor, int64_t m,
+                              int64_t n, const Tensor& c) {
+  tp_linear_problem p{};
+  p.a[0] = a; p.b[0] = b; p.lda[0] = lda; p.ldb[0] = ldb; p.k[0] = (int)k; p.segments = 1;
+  p.a_kmajor = a_kmajor; p.b_kmajor = b_kmajor; p.m = (int)m; p.n = (int)n; p.c = c.data_ptr(); p.ldc = n;
+  return p;
+}
+variable_list LinearsNode::apply(variable_list&& g) {
+  std::lock_guard<std::mutex> lock(mutex_);
+  const size_t nw = ws.size();
+  variable_list out(1 + nw);
+  const Tensor xt = x.unpack();
+  std::vector<Tensor> wt;
+  for (auto& w : ws) wt.push_back(w.unpack());
+  bool plain = !at::GradMode::is_enabled();
+  for (const auto& t : g) plain = plain && (!t.defined() || (plain_eager(t) && t.scalar_type() == xt.scalar_type()));
+  if (!plain) {  // a graph of the backward is being recorded, or the gradients are not plain tensors
+    for (size_t i = 0; i < nw; i++) {
+      if (!g[i].defined()) continue;
+      const Tensor g2 = g[i].reshape({-1, g[i].size(-1)});
+      if (task_should_compute_output(0)) {
+        const Tensor d = at::matmul(g[i], wt[i]);
+        out[0] = out[0].defined() ? out[0] + d : d;
+      }
+      if (task_should_compute_output(1 + i)) out[1 + i] = at::mm(g2.t(), xt.reshape({-1, xt.size(-1)}));
+    }
+    return out;
+  }
+  at::AutoDispatchBelowADInplaceOrView below;
+  c10::DeviceGuard guard(xt.device());
+  const Rows xr = rows_of(xt, true);
+  std::vector<Rows> gr;  // (keep copies of strided gradients alive until the launch)
+  gr.reserve(nw);
+  std::array<tp_linear_problem, 4> p;
+  int n = 0, dx = -1;
+  for (size_t i = 0; i < nw; i++) {
+    if (!g[i].defined()) continue;
+    gr.push_back(rows_of(g[i], true));
+    const Rows& r = gr.back();
+    const int64_t nf = wt[i].size(0);
+    if (task_should_compute_output(0)) {
+      if (dx < 0) {
+        out[0] = at::empty(xt.sizes(), xt.options());
+        dx = n++;
+        p[dx] = lin_problem(r.ptr(), r.stride, wt[i].data_ptr(), xr.cols, nf, true, false, r.rows, xr.cols, out[0]);
+      } else {
+        const int s = p[dx].segments++;
+        p[dx].a[s] = r.ptr(); p[dx].lda[s] = r.stride; p[dx].b[s] = wt[i].data_ptr(); p[dx].ldb[s] = xr.cols; p[dx].k[s] = (int)nf;
+      }
+    }
+  }
+  size_t j = 0;
+  for (size_t i = 0; i < nw; i++) {
+    if (!g[i].defined()) continue;
+    const Rows& r = gr[j++];
+    if (!task_should_compute_output(1 + i)) continue;
+    out[1 + i] = at::empty(wt[i].sizes(), wt[i].options());
+    p[n++] = lin_problem(r.ptr(), r.stride, xr.ptr(), xr.stride, r.rows, false, false, wt[i].size(0), xr.cols, out[1 + i]);
+  }
+  if (n) check(tp_linears(p.data(), n, dtype_code(xt.scalar_type()), stream_of(xt.device())), "tp_linears");
+  return out;
+}
+
+std::vector<Tensor> py_linears(const Tensor& x, const std::vector<Tensor>& ws) {
+  std::vector<Tensor> out;
+  out.reserve(ws.size());
+  if (!linears_take(x, ws)) {
+    for (const auto& w : ws) out.push_back(at::linear(x, w));
+    return out;
+  }
+  std::shared_ptr<LinearsNode> node;
+  bool req = at::GradMode::is_enabled() && x.requires_grad();
+  for (const auto& w : ws) {
+    TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(w), "the tprime operators have no forward-mode derivative");
+    req = req || (at::GradMode::is_enabled() && w.requires_grad());
+  }
+  TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(x), "the tprime operators have no forward-mode derivative");
+  if (req) {
+    node = std::shared_ptr<LinearsNode>(new LinearsNode(), torch::autograd::deleteNode);
+    torch::autograd::edge_list edges{torch::autograd::impl::gradient_edge(x)};
+    for (const auto& w : ws) edges.push_back(torch::autograd::impl::gradient_edge(w));
+    node->set_next_edges(std::move(edges));
+  }
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::DeviceGuard guard(x.device());
+    const Rows xr = rows_of(x, true);
+    std::array<tp_linear_problem, 4> p;
+    auto sizes = x.sizes().vec();
+    for (size_t i = 0; i < ws.size(); i++) {
+      sizes.back() = ws[i].size(0);
+      out.push_back(at::empty(sizes, x.options()));
+      p[i] = lin_problem(xr.ptr(), xr.stride, ws[i].data_ptr(), xr.cols, xr.cols, true, true, xr.rows, ws[i].size(0), out[i]);
+    }
+    check(tp_linears(p.data(), (int)ws.size(), dtype_code(x.scalar_type()), stream_of(x.device())), "tp_linears");
+  }
+  if (req) {
+    node->x = SavedVariable(x, false);
+    for (size_t i = 0; i < ws.size(); i++) {
+      node->ws.emplace_back(ws[i], false);
+      torch::autograd::set_history(out[i], node);
+    }
+  }
+  return out;
+}
+
 // ---- Python entry points -----------------------------------------------------------------------------------------
 // What the Python functions of ops.py call: the GPU check with its own message, then the operator.
 Tensor py_rmsnorm(const Tensor& x, const Tensor& w, double eps) { require_gpu(x, w); return std::get<0>(op_rmsnorm_fwd()(x, w, eps)); }
@@ -961,6 +1109,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention_pairs", &py_attention_pairs);
   m.def("mask_kind", &py_mask_kind);
   m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
+  m.def("linears", &py_linears);
   m.def("l2norm", &py_l2norm);
   m.def("swiglu", &py_swiglu);
   m.def("cross_entropy", &py_cross_entropy);

@@ -1,11 +1,13 @@
 """LlamaMLP (torchprime/torch_xla_models/model/llama/model.py:125-139) with the activation and the gate product in
-one HIP kernel (``tprime::swiglu_fwd``); the three projections stay stock ``nn.Linear`` GEMMs."""
+one HIP kernel (``tprime::swiglu_fwd``); the three projections stay stock ``nn.Linear``
+modules (``linear.project``)."""
 
 from __future__ import annotations
 
 from torch import nn
 
 from . import ops
+from .linear import project
 
 
 class LlamaMLP(nn.Module):
@@ -22,4 +24,5 @@ class LlamaMLP(nn.Module):
       raise NotImplementedError(f"hidden_act={act!r}: the fused kernel implements SiLU (every shipped Llama config uses it)")
 
   def forward(self, x):
-    return self.down_proj(ops.swiglu(self.gate_proj(x), self.up_proj(x)))
+    gate, up = project(x, self.gate_proj, self.up_proj)
+    return project(ops.swiglu(gate, up), self.down_proj)[0]
