@@ -150,9 +150,9 @@ int tp_attn_fwd(const void* q, const void* k, const void* v, const int32_t* seg,
  *   verdict       non-zero: also set the int32 flags at the start of `pairs`, which the caller has cleared:
  *                 [0] some entry is neither 0 nor drops its pair, [1] the mask is not the exact causal mask
  *                 (0 / -inf), [2] a row without a pair has entries other than -inf.  The attention entry
- *                 points below give the eager formula's results if [0] and [2] are 0.
- * tp_attn_fwd_pairs / tp_attn_bwd_pairs   tp_attn_fwd / tp_attn_bwd (no segment ids, no causality of their
- *   own) over the pairs of `pairs`, made for mask_batches (1 or B) masks.  bf16 and fp16.
+ *                 points give the eager formula's results if [0] and [2] are 0.
+ * tp_attn_fwd_pairs   tp_attn_fwd (no segment ids, no causality of its own) over the pairs of `pairs`, made for
+ *   mask_batches (1 or B) masks.  bf16 and fp16.  Backward: tp_attn_bwd_run with `pairs`.
  * ---------------------------------------------------------------------------------------------- */
 size_t tp_mask_pairs_bytes(int mask_batches, int Sq, int Skv);
 int tp_mask_pairs(const void* mask, const int64_t mask_strides[2], int mask_batches, int Sq, int Skv, int dtype, void* pairs,
@@ -161,11 +161,6 @@ int tp_attn_fwd_pairs(const void* q, const void* k, const void* v, const void* p
                       int B, int Hq, int Hkv, int Sq, int Skv, int Dqk, int Dv, const int64_t q_strides[3],
                       const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3], float sm_scale,
                       int dtype, void* stream);
-int tp_attn_bwd_pairs(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
-                      const void* pairs, int mask_batches, void* dq, void* dk, void* dv, float* ws, int B, int Hq, int Hkv, int Sq,
-                      int Skv, int Dqk, int Dv, const int64_t do_strides[3], const int64_t q_strides[3], const int64_t k_strides[3],
-                      const int64_t v_strides[3], const int64_t o_strides[3], const int64_t dq_strides[3],
-                      const int64_t dk_strides[3], const int64_t dv_strides[3], float sm_scale, int dtype, void* stream);
 
 /* Bytes of fp32 workspace tp_attn_bwd needs (two floats per query row: rowsum(dO o O) and the LSE in
  * log2 units). */
@@ -335,6 +330,37 @@ int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float*
                          int V, int64_t logits_b_stride, int64_t logits_s_stride,
                          int64_t labels_b_stride, int64_t dlogits_b_stride, int64_t dlogits_s_stride,
                          int ignore_index, int dtype, void* stream);
+
+/* ------------------------------------------------------------------------------------------------
+ * The attention backward as one struct: everything tp_attn_bwd / _masked / _biased take (fields that do not
+ * apply: NULL, windows -1, soft_cap 0), a pair mask, and workspace for problems with few key tiles.
+ *   pairs, mask_batches   see tp_mask_pairs; goes with no other mask
+ *   parts, parts_bytes    tp_attn_bwd_parts_bytes() bytes, 16-byte aligned, or NULL / 0.  With it the walk of a
+ *                         key tile over its queries is split over several workgroups where one each would
+ *                         leave CUs idle; 0 bytes are asked for where it would not pay
+ * ---------------------------------------------------------------------------------------------- */
+typedef struct tp_attn_bwd_problem {
+  const void *dout, *q, *k, *v, *out;
+  const float* lse;
+  const int32_t* seg;
+  const int32_t* q_positions;
+  const float* bias;
+  int64_t bias_strides[3];
+  const void* pairs;
+  int mask_batches;
+  void *dq, *dk, *dv;
+  float* ws;
+  void* parts;
+  size_t parts_bytes;
+  int B, Hq, Hkv, Sq, Skv, Dqk, Dv;
+  int64_t do_strides[3], q_strides[3], k_strides[3], v_strides[3], o_strides[3], dq_strides[3], dk_strides[3], dv_strides[3];
+  float sm_scale;
+  int causal, causal_offset, window_left, window_right;
+  float soft_cap;
+  int dtype;
+} tp_attn_bwd_problem;
+size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* problem);
+int tp_attn_bwd_run(const tp_attn_bwd_problem* problem, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Small matrix products, up to four in one launch: c[m, n] = sum over segments j and k of a_j(m, k) b_j(n, k),

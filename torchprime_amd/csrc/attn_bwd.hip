@@ -26,6 +26,8 @@
 // about 1.3 TB/s on this part, an order of magnitude short of what accumulating dQ tiles would need.
 #include <type_traits>
 
+#include <string.h>
+
 #include "attn_common.hpp"
 
 namespace tp {
@@ -61,7 +63,7 @@ struct BwdArgs {
   void* dk;
   void* dv;
   float* delta;
-  int B, Hq, Hkv, Sq, Skv, n_rep;
+  int B, Hq, Hkv, Sq, Skv, n_rep, dqk, dv_dim;
   int64_t qs[3], ks[3], vs[3], os[3], dos[3], dqs[3], dks[3], dvs[3];
   float scale_log2;  // sm_scale * log2(e)
   float sm_scale;
@@ -70,7 +72,83 @@ struct BwdArgs {
   int band_lo, band_hi;
   MaskExt mx;
   PairMask pm;
+  int interleave;  // order of the workgroups (xcd_map)
+  // dK/dV: partial results of the splits of a kv tile's work (split_plan), NULL: no tile is split
+  float* parts;
+  size_t parts_bytes;
+  int split;                      // the plan below is in use
+  unsigned short split_first[65]; // per XCD: number of workgroups before kv tile t
 };
+
+// ------------------------------------------------------------------------------------------------
+// splitting a kv tile's work
+// ------------------------------------------------------------------------------------------------
+// A dK/dV workgroup walks every query tile of every query head of its group: with few kv tiles (one sequence of a few
+// thousand tokens and eight kv heads) that is one workgroup for every second CU or fewer, each with the longest chain
+// there can be.  Such a tile's walk is cut into pieces of at most `cap` iterations, one workgroup each, which leave
+// their sums as fp32 in a workspace for a short kernel to add up in order (deterministic).  The cap is the one for which
+// the estimate below is least; pieces cost their start-up and 2 x 128 x (dqk + dv) x 4 bytes of traffic each.
+// Measured (bf16, 32q/8kv heads of 128, B1): dK/dV of a 1024-key window over 2047 rows 116 -> see the table of figures
+// at the launch.
+struct SplitPlan {
+  bool on;
+  int n_tiles, n_gl;
+  unsigned short first[65];
+  size_t bytes;
+};
+static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk, int Dv, int band_lo, int band_hi) {
+  SplitPlan p;
+  p.on = false;
+  p.bytes = 0;
+  p.n_tiles = (Skv + 127) / 128;
+  const int groups = B * Hkv;
+  p.n_gl = (groups + NUM_XCD - 1) / NUM_XCD;
+  const bool two = Dqk <= 64;  // workgroups per CU
+  const int slots = CUS_PER_XCD * (two ? 2 : 1);
+  // (four rounds and more balance themselves)
+  if (p.n_tiles > 64 || (int64_t)p.n_tiles * p.n_gl >= 4 * slots) return p;
+  // time of an iteration and of a workgroup's start, us (measured: a chain of iterations on an otherwise idle chip)
+  const float ti = Dqk <= 64 ? 1.0f : Dqk <= 128 ? 1.4f : 2.0f, start = 4.f;
+  const int nqt = (Sq + 63) / 64;
+  int per[64], longest = 0;
+  int64_t total = 0;
+  for (int t = 0; t < p.n_tiles; t++) {
+    const int64_t lo = (int64_t)t * 128 - band_hi, hi = (int64_t)t * 128 + 127 + band_lo;
+    const int q0 = (int)((lo > 0 ? lo : 0) / 64), q1 = hi < 0 ? 0 : (int)(hi / 64 + 1 < nqt ? hi / 64 + 1 : nqt);
+    per[t] = (q1 > q0 ? q1 - q0 : 0) * n_rep;
+    longest = per[t] > longest ? per[t] : longest;
+    total += per[t];
+  }
+  const float wg_mb = 128.f * (Dqk + Dv) * 4.f * 2.f * 1e-6f;  // a partial tile, written and read
+  float best = 0.f;
+  int best_cap = 0;
+  for (int s = 1; s <= 16 && s <= longest; s++) {
+    const int cap = (longest + s - 1) / s;
+    int64_t wgs = 0, parts = 0;
+    for (int t = 0; t < p.n_tiles; t++) {
+      const int n = per[t] > cap ? (per[t] + cap - 1) / cap : 1;
+      wgs += n;
+      parts += n > 1 ? n : 0;
+    }
+    wgs *= p.n_gl;
+    const float rounds = (float)((wgs + slots - 1) / slots), share = (float)total * p.n_gl / slots;
+    const float chain = wgs <= slots ? (float)cap : (share + 0.5f * cap > cap ? share + 0.5f * cap : (float)cap);
+    const float est = start * rounds + ti * chain + (parts ? 5.f + parts * p.n_gl * NUM_XCD * wg_mb / 4.f : 0.f);
+    if (s == 1 || est < best * (best_cap == longest ? 0.9f : 1.f)) { best = est; best_cap = cap; }
+  }
+  if (best_cap == longest) return p;
+  int at = 0, last = 0;
+  for (int t = 0; t < p.n_tiles; t++) {
+    p.first[t] = (unsigned short)at;
+    const int n = per[t] > best_cap ? (per[t] + best_cap - 1) / best_cap : 1;
+    at += n * p.n_gl;
+    if (n > 1) last = at;
+  }
+  p.first[p.n_tiles] = (unsigned short)at;
+  p.on = true;
+  p.bytes = (size_t)last * NUM_XCD * 128 * (Dqk + Dv) * 4;  // one slot per workgroup up to the last split tile
+  return p;
+}
 
 // ------------------------------------------------------------------------------------------------
 // delta = rowsum(dO o O)
@@ -219,8 +297,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
-  int tile, inner, group;
-  if (!xcd_map((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group)) return;
+  int tile, inner, group, n_split = 1, split = 0;
+  if (a.split) {
+    // tile after tile, groups inside, pieces inside those; a lane per tile finds the workgroup's tile
+    const int n_tiles = (a.Skv + BNK - 1) / BNK, r = blockIdx.x / NUM_XCD;
+    const bool before = lane < n_tiles && r >= (int)a.split_first[lane + 1];
+    tile = (int)__popcll(__ballot(before));
+    const int n_gl = (a.B * a.Hkv + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
+    n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
+    const int gl = (r - f) / n_split;
+    split = (r - f) - gl * n_split;
+    group = gl * NUM_XCD + blockIdx.x % NUM_XCD;
+    if (group >= a.B * a.Hkv) return;
+  } else if (!xcd_map((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
   const int b = group / a.Hkv, hk = group - b * a.Hkv;
   const int kv0 = tile * BNK;  // low kv tiles see the most queries: they start first
   const int wkv0 = kv0 + wave * 32;
@@ -320,7 +409,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     }
     __syncthreads();
   }
-  const int n_iter = nact * a.n_rep;
+  // this workgroup's piece of the walk: iterations it_first .. it_first + n_iter - 1
+  const int n_walk = nact * a.n_rep;
+  const int it_first = n_split > 1 ? split * n_walk / n_split : 0;
+  const int n_iter = n_split > 1 ? (split + 1) * n_walk / n_split - it_first : n_walk;
 
   // ---- staging: every piece of a query tile (Q, dO row-major; log2-scaled LSE, delta, segment ids of its
   // rows) is written into LDS by the loads themselves; the transposed copies are made LDS-to-LDS
@@ -430,7 +522,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     //                                  -> tile t+1 has landed for everybody, everybody is done with tile t-1
     //   part 2 (dV, dK: transposing reads of buffer t % 3), with the loads of tile t+2 issued between its MFMAs
     //   into the buffer tile t-1 used
-    int c_hl = 0, c_idx = 0, n_hl = 0, n_idx = 0;  // tile being computed, tile whose loads are issued next
+    const int hl_first = n_split > 1 ? it_first / max(nact, 1) : 0, idx_first = it_first - hl_first * nact;
+    int c_hl = hl_first, c_idx = idx_first, n_hl = hl_first, n_idx = idx_first;  // tile being computed, tile whose loads are issued next
     // Per-lane LDS byte addresses of the operands inside a tile (base of the workgroup's LDS included), each an
     // opaque register: every read below is such a register plus an immediate.  (Formed from the `smem` symbol, the
     // same addresses cost an add per read whenever the constant part happens to be zero, and the compiler
@@ -476,7 +569,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
       return i32x4{__builtin_amdgcn_readfirstlane(v[0]), __builtin_amdgcn_readfirstlane(v[1]),
                    __builtin_amdgcn_readfirstlane(v[2]), __builtin_amdgcn_readfirstlane(v[3])};
     };
-    i32x4 cur = scalar4(entry(0));
+    i32x4 cur = scalar4(entry(c_idx));
     int nq_cur = __builtin_amdgcn_readfirstlane(entry(n_idx)[0]);
     // all earlier loads (the K/V fragments, the first tiles) have landed
     __builtin_amdgcn_s_waitcnt(0);
@@ -807,6 +900,27 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
   if constexpr (DVB > 2) asm volatile("" : "+a"(dvacc[2]), "+a"(dvacc[3]));
   // ---- epilogue: lane = kv row, 4 consecutive head-dim values per store
   const int row = wkv0 + ln;
+  if (n_split > 1) {
+    // a piece: its sums as they are, [row][dk | dv], for attn_bwd_parts_kernel
+    if (row < Skv) {
+      float* pp = a.parts + ((int64_t)blockIdx.x * BNK + wave * 32 + ln) * (DQK + DV) + 4 * g;
+#pragma unroll
+      for (int d = 0; d < DKB; d++)
+#pragma unroll
+        for (int vq = 0; vq < 4; vq++) {
+          const f32x16& o = dkacc[d];
+          *(f32x4*)(pp + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+        }
+#pragma unroll
+      for (int d = 0; d < DVB; d++)
+#pragma unroll
+        for (int vq = 0; vq < 4; vq++) {
+          const f32x16& o = dvacc[d];
+          *(f32x4*)(pp + DQK + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+        }
+    }
+    return;
+  }
   if (row < Skv) {
     T* dkp = (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row * a.dks[2];
     T* dvp = (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row * a.dvs[2];
@@ -835,6 +949,33 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
 // NW = waves per workgroup.  With 8 (head dims up to 128) two waves share a SIMD, 256 registers each: a wave
 // issues at most one instruction every four cycles, and at ~600 instructions for 48 MFMAs per tile a single
 // wave per SIMD leaves the matrix unit idle most of the time, whatever the order of its instructions.
+
+// sums of the pieces of the split kv tiles: one thread per four values of a row, pieces in order
+template <typename T, int DQK, int DV>
+__global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
+  constexpr int BNK = 128, W = (DQK + DV) / 4, PER_TILE = BNK * W / 256;  // workgroups per (tile, group)
+  static_assert(BNK * W % 256 == 0, "whole workgroups");
+  const int n_groups = a.B * a.Hkv;
+  const int item = blockIdx.x % PER_TILE * 256 + threadIdx.x, tg = blockIdx.x / PER_TILE;
+  const int tile = tg / n_groups, group = tg - tile * n_groups;
+  const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
+  const int n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
+  const int r = item / W, d = (item - r * W) * 4, row = tile * BNK + r;
+  if (n_split == 1 || row >= a.Skv) return;
+  const float* p = a.parts + (((int64_t)(f + group / NUM_XCD * n_split) * NUM_XCD + group % NUM_XCD) * BNK + r) * (DQK + DV) + d;
+  f32x4 acc = *(const f32x4*)p;
+  for (int s = 1; s < n_split; s++) {
+    p += (int64_t)NUM_XCD * BNK * (DQK + DV);
+    const f32x4 x = *(const f32x4*)p;
+    acc[0] += x[0]; acc[1] += x[1]; acc[2] += x[2]; acc[3] += x[3];
+  }
+  const int b = group / a.Hkv, hk = group - b * a.Hkv;
+  const float sc = d < DQK ? a.sm_scale : 1.f;
+  T* o = d < DQK ? (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row * a.dks[2] + d
+                 : (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row * a.dvs[2] + (d - DQK);
+  *(u32x2*)o = pack4<T>(acc[0] * sc, acc[1] * sc, acc[2] * sc, acc[3] * sc);
+}
+
 template <typename T, int DQK, int DV, int NW, bool CAUSAL, int SEG>
 __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
   typedef typename MT<T>::v8 v8;
@@ -855,7 +996,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group)) return;
+  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
   const int qt = n_qt - 1 - tile;
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM, wq0 = q0 + wave * 32;
@@ -1458,7 +1599,7 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group)) return;
+  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
   const int qt = n_qt - 1 - tile;  // the longest rows first
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM, wq0 = q0 + wave * 32;
@@ -1874,8 +2015,17 @@ struct LeanDq {
   static bool taken(int Skv) { return BUILT && lds_bytes(Skv) <= 160 * 1024; }
 };
 
+// the plan of a problem as the dK/dV kernel sees it: its band (all keys where the mask is something else)
+static SplitPlan bwd_split_plan(const BwdArgs& a, bool causal) {
+  const int lo = causal ? a.band_lo : a.mx.on && !a.mx.qpos ? a.mx.lo_off : BAND_INF;
+  const int hi = causal ? a.band_hi : a.mx.on && !a.mx.qpos ? a.mx.hi_off : BAND_INF;
+  return split_plan(a.B, a.Hkv, a.n_rep, a.Sq, a.Skv, a.dqk, a.dv_dim, lo, hi);
+}
+
 template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
-static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
+static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
+  BwdArgs a = args;
+  const int groups = a.B * a.Hkv;
   typedef LeanDq<DQK, DV, CAUSAL, SEG> Lean;
   const bool lean = Lean::taken(a.Skv);
   // dK/dV: three row-major buffers of Q and dO tiles, the row vectors, the tile list (checked before anything is launched)
@@ -1906,7 +2056,8 @@ static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
         if (rc) return rc;
         attr_set = true;
       }
-      kern<<<dim3(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, a.B * a.Hkv)), dim3(256), Lean::lds_bytes(a.Skv), st>>>(a);
+      a.interleave = interleave_groups((a.Sq + BM - 1) / BM, a.n_rep, groups, DQK == DV ? 2 : 1);
+      kern<<<dim3(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, groups)), dim3(256), Lean::lds_bytes(a.Skv), st>>>(a);
       int rc = check_launch("tp_attn_bwd(dq)");
       if (rc) return rc;
       mark(ev, 3, st);
@@ -1921,9 +2072,22 @@ static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
       if (rc) return rc;
       attr_set = true;
     }
-    kern<<<dim3(xcd_grid((a.Skv + DKDV_BNK - 1) / DKDV_BNK, 1, a.B * a.Hkv)), dim3(256), dkdv_smem, st>>>(a);
+    const int n_tiles = (a.Skv + DKDV_BNK - 1) / DKDV_BNK;
+    SplitPlan plan;
+    plan.on = false;
+    if (a.parts) plan = bwd_split_plan(a, CAUSAL);
+    a.split = plan.on && plan.bytes <= a.parts_bytes;
+    if (a.split) memcpy(a.split_first, plan.first, sizeof(a.split_first));
+    a.interleave = interleave_groups(n_tiles, 1, groups, DQK <= 64 ? 2 : 1);
+    kern<<<dim3(a.split ? NUM_XCD * plan.first[n_tiles] : xcd_grid(n_tiles, 1, groups)), dim3(256), dkdv_smem, st>>>(a);
     int rc = check_launch("tp_attn_bwd(dkdv)");
     if (rc) return rc;
+    if (a.split) {
+      constexpr int PER_TILE = DKDV_BNK * (DQK + DV) / 4 / 256;
+      attn_bwd_parts_kernel<T, DQK, DV><<<dim3((unsigned)(n_tiles * groups * PER_TILE)), dim3(256), 0, st>>>(a);
+      rc = check_launch("tp_attn_bwd(parts)");
+      if (rc) return rc;
+    }
   }
   mark(ev, 2, st);
   // dQ, the general kernel
@@ -1945,7 +2109,8 @@ static int launch_bwd(const BwdArgs& a, hipStream_t st, void* const* ev) {
       if (rc) return rc;
       attr_set = true;
     }
-    kern<<<dim3(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, a.B * a.Hkv)), dim3(64 * NW), smem, st>>>(a);
+    a.interleave = 0;
+    kern<<<dim3(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, groups)), dim3(64 * NW), smem, st>>>(a);
     int rc = check_launch("tp_attn_bwd(dq)");
     if (rc) return rc;
     }
@@ -2060,7 +2225,8 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
                          const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                          const int64_t o_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
                          const int64_t dv_strides[3], float sm_scale, int causal, int dtype, void* stream,
-                         void* const* events, const MaskExt& mx, const PairMask& pm = no_pair_mask()) {
+                         void* const* events, const MaskExt& mx, const PairMask& pm = no_pair_mask(),
+                         void* parts = nullptr, size_t parts_bytes = 0) {
   TP_REQUIRE(dout && q && k && v && out && lse && dq && dk && dv && ws, TP_ERR_BAD_ARG, "tp_attn_bwd: null pointer");
   TP_REQUIRE(do_strides && q_strides && k_strides && v_strides && o_strides && dq_strides && dk_strides && dv_strides,
              TP_ERR_BAD_ARG, "tp_attn_bwd: null stride array");
@@ -2080,7 +2246,8 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   BwdArgs a;
   a.q = q; a.k = k; a.v = v; a.out = out; a.dout = dout; a.lse = lse; a.seg = seg;
   a.dq = dq; a.dk = dk; a.dv = dv; a.delta = ws;
-  a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv; a.n_rep = Hq / Hkv;
+  a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv; a.n_rep = Hq / Hkv; a.dqk = Dqk; a.dv_dim = Dv;
+  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.interleave = 0;
   bool ok = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(dout) && aligned16(dq) &&
             aligned16(dk) && aligned16(dv);
   for (int i = 0; i < 3; i++) {
@@ -2173,19 +2340,47 @@ extern "C" int tp_attn_bwd(const void* dout, const void* q, const void* k, const
                         nullptr);
 }
 
-extern "C" int tp_attn_bwd_pairs(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
-                                 const void* pairs, int mask_batches, void* dq, void* dk, void* dv, float* ws, int B, int Hq, int Hkv,
-                                 int Sq, int Skv, int Dqk, int Dv, const int64_t do_strides[3], const int64_t q_strides[3],
-                                 const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
-                                 const int64_t dq_strides[3], const int64_t dk_strides[3], const int64_t dv_strides[3], float sm_scale,
-                                 int dtype, void* stream) {
-  TP_REQUIRE(pairs && (mask_batches == 1 || mask_batches == B), TP_ERR_BAD_ARG, "tp_attn_bwd_pairs: null mask or %d masks for %d batches",
-             mask_batches, B);
-  TP_REQUIRE(Sq > 0 && Skv > 0, TP_ERR_BAD_ARG, "tp_attn_bwd_pairs: non-positive size");
-  TP_REQUIRE(dtype == TP_BF16 || dtype == TP_F16, TP_ERR_UNSUPPORTED, "tp_attn_bwd_pairs: dtype %d (bf16 and fp16 only)", dtype);
-  TP_REQUIRE((int64_t)((Sq + 127) / 128 + 1) * 128 * ((Skv + 127) / 128 + 1) * 16 < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_bwd_pairs: mask too large");
-  return attn_bwd_impl(dout, q, k, v, out, lse, nullptr, dq, dk, dv, ws, B, Hq, Hkv, Sq, Skv, Dqk, Dv, do_strides, q_strides, k_strides,
-                       v_strides, o_strides, dq_strides, dk_strides, dv_strides, sm_scale, 0, dtype, stream, nullptr, no_mask_ext(),
-                       pair_mask(pairs, mask_batches, Sq, Skv));
+// the mask of a problem: extensions, or pairs
+static MaskExt problem_mask(const tp_attn_bwd_problem& p) {
+  const bool plain = !p.q_positions && !p.bias && p.window_left < 0 && p.window_right < 0 && !(p.soft_cap > 0.f) && (!p.causal || p.causal_offset == 0);
+  if (p.pairs || plain) return no_mask_ext();
+  return make_mask_ext(p.q_positions, p.causal, p.causal_offset, p.window_left, p.window_right, p.soft_cap, p.sm_scale, p.bias, p.bias_strides);
+}
+
+extern "C" size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* p) {
+  if (!p || (p->dtype != TP_BF16 && p->dtype != TP_F16) || p->B <= 0 || p->Hkv <= 0 || p->Hq <= 0 || p->Sq <= 0 || p->Skv <= 0) return 0;
+  const MaskExt mx = problem_mask(*p);
+  int lo = BAND_INF, hi = BAND_INF;
+  if (mx.on) {
+    if (!mx.qpos) { lo = mx.lo_off; hi = mx.hi_off; }
+  } else if (p->causal && !p->pairs) {
+    hi = 0;
+  }
+  const SplitPlan plan = split_plan(p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi);
+  return plan.on ? plan.bytes : 0;
+}
+
+extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {
+  TP_REQUIRE(p, TP_ERR_BAD_ARG, "tp_attn_bwd_run: null problem");
+  TP_REQUIRE(p->sm_scale > 0.f, TP_ERR_BAD_ARG, "tp_attn_bwd_run: sm_scale must be positive");
+  TP_REQUIRE(p->window_left < BAND_INF && p->window_right < BAND_INF && p->causal_offset > -BAND_INF && p->causal_offset < BAND_INF, TP_ERR_BAD_ARG,
+             "tp_attn_bwd_run: window or offset out of range");
+  TP_REQUIRE(!p->bias || (p->bias_strides[0] >= 0 && p->bias_strides[1] >= 0 && p->bias_strides[2] >= 0), TP_ERR_BAD_ARG,
+             "tp_attn_bwd_run: negative bias stride");
+  TP_REQUIRE((p->parts != nullptr) == (p->parts_bytes != 0) && aligned16(p->parts), TP_ERR_BAD_ARG, "tp_attn_bwd_run: parts and parts_bytes disagree");
+  PairMask pm = no_pair_mask();
+  if (p->pairs) {
+    TP_REQUIRE(!p->seg && !p->bias && !p->q_positions && !p->causal && p->window_left < 0 && p->window_right < 0 && !(p->soft_cap > 0.f), TP_ERR_BAD_ARG,
+               "tp_attn_bwd_run: pairs go with no other mask");
+    TP_REQUIRE(p->mask_batches == 1 || p->mask_batches == p->B, TP_ERR_BAD_ARG, "tp_attn_bwd_run: %d masks for %d batches", p->mask_batches, p->B);
+    TP_REQUIRE(p->Sq > 0 && p->Skv > 0, TP_ERR_BAD_ARG, "tp_attn_bwd_run: non-positive size");
+    TP_REQUIRE(p->dtype == TP_BF16 || p->dtype == TP_F16, TP_ERR_UNSUPPORTED, "tp_attn_bwd_run: pairs: dtype %d (bf16 and fp16 only)", p->dtype);
+    TP_REQUIRE((int64_t)((p->Sq + 127) / 128 + 1) * 128 * ((p->Skv + 127) / 128 + 1) * 16 < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_bwd_run: mask too large");
+    pm = pair_mask(p->pairs, p->mask_batches, p->Sq, p->Skv);
+  }
+  const MaskExt mx = problem_mask(*p);
+  return attn_bwd_impl(p->dout, p->q, p->k, p->v, p->out, p->lse, p->seg, p->dq, p->dk, p->dv, p->ws, p->B, p->Hq, p->Hkv, p->Sq, p->Skv, p->Dqk,
+                       p->Dv, p->do_strides, p->q_strides, p->k_strides, p->v_strides, p->o_strides, p->dq_strides, p->dk_strides, p->dv_strides,
+                       p->sm_scale, p->causal, p->dtype, stream, nullptr, mx, pm, p->parts, p->parts_bytes);
 }
 #endif  // !TP_BWD_UNIT

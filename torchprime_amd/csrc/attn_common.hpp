@@ -230,17 +230,36 @@ __device__ __forceinline__ unsigned span_bytes(int rows, int64_t stride, int row
 // Q/dO) slice - one (batch, kv head) "group" - lands on the same XCD and runs at about the same time:
 //     id = (group_local * per_group + r) * 8 + xcd,   group = group_local * 8 + xcd,
 //     r  = tile * n_inner + inner   (tiles outer so the heaviest tiles start first).
+// With group after group the last group's heaviest tile starts when nearly everything else is done.  Where an XCD gets
+// only a few rounds of workgroups that tail is a good part of the launch (dK/dV of 64 groups of 10 causal tiles: a
+// third), and there the groups take turns tile by tile instead (`interleave`; the host's rule is interleave_groups); with
+// many rounds the tail is small and the groups' sharing of an L2 is worth more.
 // Returns false for the padding ids of a group count that is not a multiple of 8.
-constexpr int NUM_XCD = 8;
-__device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group) {
+constexpr int NUM_XCD = 8, CUS_PER_XCD = 32;
+__device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, bool interleave = false) {
   const int n = blockIdx.x;
   const int xcd = n % NUM_XCD, slot = n / NUM_XCD;
-  const int per_group = n_tiles * n_inner;
-  const int gl = slot / per_group, r = slot - gl * per_group;
+  int gl, r;
+  if (interleave) {
+    const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, per_tile = n_gl * n_inner;
+    tile = slot / per_tile;
+    r = slot - tile * per_tile;
+    gl = r / n_inner;
+    inner = r - gl * n_inner;
+  } else {
+    const int per_group = n_tiles * n_inner;
+    gl = slot / per_group;
+    r = slot - gl * per_group;
+    tile = r / n_inner;
+    inner = r - tile * n_inner;
+  }
   group = gl * NUM_XCD + xcd;
-  tile = r / n_inner;
-  inner = r - tile * n_inner;
   return group < n_groups;
+}
+// fewer than four rounds of workgroups on an XCD (per_cu of them share a CU), and more than one group to order
+inline bool interleave_groups(int n_tiles, int n_inner, int n_groups, int per_cu) {
+  const int64_t n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD;
+  return n_gl > 1 && n_gl * n_tiles * n_inner < 4 * CUS_PER_XCD * per_cu;
 }
 inline unsigned xcd_grid(int n_tiles, int n_inner, int n_groups) {
   return (unsigned)(NUM_XCD * ((n_groups + NUM_XCD - 1) / NUM_XCD) * n_tiles * n_inner);

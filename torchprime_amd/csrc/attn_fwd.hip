@@ -37,6 +37,7 @@ struct FwdArgs {
   int band_lo, band_hi;
   MaskExt mx;
   PairMask pm;
+  int interleave;  // order of the workgroups (xcd_map)
 };
 
 // Two workgroups per CU (256 registers per lane) where the kernel fits them; the non-causal variants at head dims of
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group)) return;
+  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
   const int qt = n_qt - 1 - tile;  // longest (latest) query tiles are scheduled first
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM;
@@ -614,7 +615,8 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
 // host dispatch
 // ------------------------------------------------------------------------------------------------
 template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
-static int launch_fwd(const FwdArgs& a, int B, hipStream_t st) {
+static int launch_fwd(const FwdArgs& args, int B, hipStream_t st) {
+  FwdArgs a = args;
   constexpr int BN = 64, BM = 128;
   constexpr int BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES + (SEG == SEG_PAIRS ? BM * 8 : SEG ? BN * 4 : 0);
   const int ntiles_max = (a.Skv + BN - 1) / BN;
@@ -627,6 +629,7 @@ static int launch_fwd(const FwdArgs& a, int B, hipStream_t st) {
     TP_REQUIRE(e == hipSuccess, TP_ERR_LAUNCH, "tp_attn_fwd: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     attr_set = true;
   }
+  a.interleave = interleave_groups((a.Sq + BM - 1) / BM, a.n_rep, B * a.Hkv, fwd_blocks_per_cu<DQK, CAUSAL, SEG>());
   const dim3 grid(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, B * a.Hkv)), block(256);
   kern<<<grid, block, smem, st>>>(a);
   return check_launch("tp_attn_fwd");

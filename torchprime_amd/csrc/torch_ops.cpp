@@ -474,23 +474,49 @@ T2 attn_fwd_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, OptTensor
   return {out, lse};
 }
 
-T3 attn_bwd_cuda(const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
-                 OptTensor seg_, double sm_scale, bool causal) {
-  const c10::Device dev = require_gpu(dout_, q_, k_, v_, out_, lse_, seg_);
-  const AttnShape s = check_attn(q_, k_, v_, val(seg_));
-  c10::DeviceGuard guard(dev);
-  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), out = prep_heads(out_), dout = prep_heads(dout_);
-  const Tensor lse = lse_.contiguous(), seg = prep_ids(val(seg_));
-  Tensor dq = empty_like_heads(q, s.Dqk), dk = empty_like_heads(k, s.Dqk), dv = empty_like_heads(v, s.Dv);
-  if (dq.numel() == 0 || dk.numel() == 0) return {dq.zero_(), dk.zero_(), dv.zero_()};
-  Tensor ws = empty_f32({(int64_t)tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq) / 4}, q);
-  const Strides3 gs = strides3(dout), qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out), dqs = strides3(dq),
-                 dks = strides3(dk), dvs = strides3(dv);
-  check(tp_attn_bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (const float*)lse.data_ptr(),
-                    (const int32_t*)opt_ptr(seg), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)ws.data_ptr(), s.B, s.Hq, s.Hkv, s.Sq,
-                    s.Skv, s.Dqk, s.Dv, gs.data(), qs.data(), ks.data(), vs.data(), os.data(), dqs.data(), dks.data(), dvs.data(),
-                    (float)sm_scale, (int)causal, dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_bwd");
-  return {dq, dk, dv};
+// the parts of a backward problem that do not depend on its mask, and the launch
+struct BwdCall {
+  c10::Device dev;
+  AttnShape s;
+  c10::DeviceGuard guard;
+  Tensor q, k, v, out, dout, lse, dq, dk, dv;
+  tp_attn_bwd_problem p{};
+  BwdCall(c10::Device device, const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
+          const Tensor& seg_, double sm_scale)
+      : dev(device), s(check_attn(q_, k_, v_, seg_)), guard(device), q(prep_heads(q_)), k(prep_heads(k_)), v(prep_heads(v_)),
+        out(prep_heads(out_)), dout(prep_heads(dout_)), lse(lse_.contiguous()), dq(empty_like_heads(q, s.Dqk)), dk(empty_like_heads(k, s.Dqk)),
+        dv(empty_like_heads(v, s.Dv)) {
+    p.dout = dout.data_ptr(); p.q = q.data_ptr(); p.k = k.data_ptr(); p.v = v.data_ptr(); p.out = out.data_ptr();
+    p.lse = (const float*)lse.data_ptr();
+    p.dq = dq.data_ptr(); p.dk = dk.data_ptr(); p.dv = dv.data_ptr();
+    p.B = s.B; p.Hq = s.Hq; p.Hkv = s.Hkv; p.Sq = s.Sq; p.Skv = s.Skv; p.Dqk = s.Dqk; p.Dv = s.Dv;
+    const auto st = [](int64_t (&d)[3], const Tensor& t) { for (int i = 0; i < 3; i++) d[i] = t.stride(i); };
+    st(p.do_strides, dout); st(p.q_strides, q); st(p.k_strides, k); st(p.v_strides, v); st(p.o_strides, out);
+    st(p.dq_strides, dq); st(p.dk_strides, dk); st(p.dv_strides, dv);
+    p.sm_scale = (float)sm_scale;
+    p.window_left = p.window_right = -1;
+    p.dtype = dtype_code(q.scalar_type());
+  }
+  T3 run() {
+    if (dq.numel() == 0 || dk.numel() == 0) return {dq.zero_(), dk.zero_(), dv.zero_()};
+    // one workspace: the row vectors, then the pieces of split key tiles (none for most problems)
+    const size_t rows = tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq), at = (rows + 255) / 256 * 256;
+    p.parts_bytes = tp_attn_bwd_parts_bytes(&p);
+    const Tensor ws = empty_f32({(int64_t)((p.parts_bytes ? at + p.parts_bytes : rows) / 4)}, q);
+    p.ws = (float*)ws.data_ptr();
+    p.parts = p.parts_bytes ? (char*)ws.data_ptr() + at : nullptr;
+    check(tp_attn_bwd_run(&p, stream_of(dev)), "tp_attn_bwd_run");
+    return {dq, dk, dv};
+  }
+};
+
+T3 attn_bwd_cuda(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse, OptTensor seg_,
+                 double sm_scale, bool causal) {
+  BwdCall c(require_gpu(dout, q, k, v, out, lse, seg_), dout, q, k, v, out, lse, val(seg_), sm_scale);
+  const Tensor seg = prep_ids(val(seg_));
+  c.p.seg = (const int32_t*)opt_ptr(seg);
+  c.p.causal = causal;
+  return c.run();
 }
 
 struct AttnNode : OpNode {
@@ -542,31 +568,22 @@ T2 attn_fwd_masked_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, Op
   return {out, lse};
 }
 
-T3 attn_bwd_masked_cuda(const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
+T3 attn_bwd_masked_cuda(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
                         OptTensor seg_, OptTensor qpos_, double sm_scale, bool causal, int64_t causal_offset, int64_t window_left,
                         int64_t window_right, double soft_cap, OptTensor bias_) {
-  const c10::Device dev = require_gpu(dout_, q_, k_, v_, out_, lse_, seg_, qpos_, bias_);
-  const AttnShape s = check_attn(q_, k_, v_, val(seg_));
-  c10::DeviceGuard guard(dev);
-  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), out = prep_heads(out_), dout = prep_heads(dout_);
-  const Tensor lse = lse_.contiguous(), seg = prep_ids(val(seg_)), qpos = prep_qpos(val(qpos_), s.Sq);
-  Tensor dq = empty_like_heads(q, s.Dqk), dk = empty_like_heads(k, s.Dqk), dv = empty_like_heads(v, s.Dv);
-  if (dq.numel() == 0 || dk.numel() == 0) return {dq.zero_(), dk.zero_(), dv.zero_()};
-  Tensor ws = empty_f32({(int64_t)tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq) / 4}, q);
+  BwdCall c(require_gpu(dout, q, k, v, out, lse, seg_, qpos_, bias_), dout, q, k, v, out, lse, val(seg_), sm_scale);
   Strides3 bs{};
-  const Tensor bias = prep_bias(val(bias_), s, bs);
-  const Strides3 gs = strides3(dout), qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out), dqs = strides3(dq),
-                 dks = strides3(dk), dvs = strides3(dv);
-  const auto launch = [&](auto fn, const char* name, auto... bias_args) {
-    check(fn(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (const float*)lse.data_ptr(),
-             (const int32_t*)opt_ptr(seg), (const int32_t*)opt_ptr(qpos), bias_args..., dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-             (float*)ws.data_ptr(), s.B, s.Hq, s.Hkv, s.Sq, s.Skv, s.Dqk, s.Dv, gs.data(), qs.data(), ks.data(), vs.data(), os.data(),
-             dqs.data(), dks.data(), dvs.data(), (float)sm_scale, (int)causal, (int)causal_offset, (int)window_left, (int)window_right,
-             (float)soft_cap, dtype_code(q.scalar_type()), stream_of(dev)), name);
-  };
-  if (bias.defined()) launch(tp_attn_bwd_biased, "tp_attn_bwd_biased", (const float*)bias.data_ptr(), (const int64_t*)bs.data());
-  else launch(tp_attn_bwd_masked, "tp_attn_bwd_masked");
-  return {dq, dk, dv};
+  const Tensor seg = prep_ids(val(seg_)), qpos = prep_qpos(val(qpos_), c.s.Sq), bias = prep_bias(val(bias_), c.s, bs);
+  c.p.seg = (const int32_t*)opt_ptr(seg);
+  c.p.q_positions = (const int32_t*)opt_ptr(qpos);
+  c.p.bias = (const float*)opt_ptr(bias);
+  std::copy(bs.begin(), bs.end(), c.p.bias_strides);
+  c.p.causal = causal;
+  c.p.causal_offset = (int)causal_offset;
+  c.p.window_left = (int)window_left;
+  c.p.window_right = (int)window_right;
+  c.p.soft_cap = (float)soft_cap;
+  return c.run();
 }
 
 struct AttnMaskedNode : OpNode {
@@ -634,24 +651,14 @@ T3 attn_fwd_pairs_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, con
                           dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_fwd_pairs");
   return {out, lse, pairs};
 }
-T3 attn_bwd_pairs_cuda(const Tensor& dout_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& out_, const Tensor& lse_,
+T3 attn_bwd_pairs_cuda(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
                        const Tensor& pairs, int64_t mask_batches, double sm_scale) {
-  const c10::Device dev = require_gpu(dout_, q_, k_, v_, out_, lse_, pairs);
-  const AttnShape s = check_attn(q_, k_, v_, undef());
+  BwdCall c(require_gpu(dout, q, k, v, out, lse, pairs), dout, q, k, v, out, lse, undef(), sm_scale);
   TORCH_CHECK_VALUE(pairs.is_contiguous() && pairs.scalar_type() == at::kInt && mask_batches > 0 &&
-                    pairs.numel() == (int64_t)tp_mask_pairs_bytes((int)mask_batches, s.Sq, s.Skv) / 4, "pairs were not made for this problem");
-  c10::DeviceGuard guard(dev);
-  const Tensor q = prep_heads(q_), k = prep_heads(k_), v = prep_heads(v_), out = prep_heads(out_), dout = prep_heads(dout_);
-  const Tensor lse = lse_.contiguous();
-  Tensor dq = empty_like_heads(q, s.Dqk), dk = empty_like_heads(k, s.Dqk), dv = empty_like_heads(v, s.Dv);
-  Tensor ws = empty_f32({(int64_t)tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq) / 4}, q);
-  const Strides3 gs = strides3(dout), qs = strides3(q), ks = strides3(k), vs = strides3(v), os = strides3(out), dqs = strides3(dq),
-                 dks = strides3(dk), dvs = strides3(dv);
-  check(tp_attn_bwd_pairs(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (const float*)lse.data_ptr(),
-                          pairs.data_ptr(), (int)mask_batches, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (float*)ws.data_ptr(), s.B, s.Hq, s.Hkv,
-                          s.Sq, s.Skv, s.Dqk, s.Dv, gs.data(), qs.data(), ks.data(), vs.data(), os.data(), dqs.data(), dks.data(), dvs.data(),
-                          (float)sm_scale, dtype_code(q.scalar_type()), stream_of(dev)), "tp_attn_bwd_pairs");
-  return {dq, dk, dv};
+                    pairs.numel() == (int64_t)tp_mask_pairs_bytes((int)mask_batches, c.s.Sq, c.s.Skv) / 4, "pairs were not made for this problem");
+  c.p.pairs = pairs.data_ptr();
+  c.p.mask_batches = (int)mask_batches;
+  return c.run();
 }
 struct AttnPairsNode : OpNode {
   int64_t mask_batches;
