@@ -22,9 +22,11 @@ template <> constexpr float Dropped<f16_t> = -65504.f;
 // without a pair whose entries are not all -inf
 constexpr int F_OTHER = 0, F_NOT_CAUSAL = 1, F_EMPTY_FINITE = 2;
 
-// One wave per 64 x 64 block: 64 coalesced row reads, a ballot per row gives the row's word (kept by lane r), the lane
-// gathers its own column's word.  Bound by reading the mask once (bf16, 4 x 1000 x 1000: 8 MB); words are written 512
-// contiguous bytes at a time, in the order in which the attention kernels fetch them.
+// One wave per 64 x 64 block.  Lane r reads its row's 64 entries, 128 or 256 contiguous bytes, in 16-byte loads that are
+// all in flight together, and builds the row's word; the columns' words are 64 ballots over the rows' words.  (A lane
+// per column with 64 row reads one after the other, two bytes a lane, took 15-37 us at the sizes below.)  The last tile of
+// a row is read entry by entry.  Bound by latency below a few thousand rows; words are written 512 contiguous bytes at a
+// time, in the order in which the attention kernels fetch them.
 template <typename T>
 __global__ __launch_bounds__(256) void mask_bits_kernel(const T* __restrict__ mask, int64_t bs, int64_t rs, int Sq, int Skv, int nqt,
                                                         int nkt, int nqb, int nkb, unsigned long long* __restrict__ qbits,
@@ -33,24 +35,38 @@ __global__ __launch_bounds__(256) void mask_bits_kernel(const T* __restrict__ ma
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kt = blockIdx.x * 4 + wave, qt = blockIdx.y, b = blockIdx.z;
   if (kt >= 2 * nkb) return;
-  const int key = kt * 64 + lane, q0 = qt * 64;
-  const T* mb = mask + b * bs + key;
-  unsigned long long roww = 0ull, colw = 0ull;
+  const int k0 = kt * 64, key = k0 + lane, q0 = qt * 64, row = q0 + lane;
+  unsigned long long roww = 0ull;
   bool other = false, ncausal = false;
-  const int rows = min(64, Sq - q0);  // (<= 0 in the padding of the last block)
-#pragma unroll 16
-  for (int r = 0; r < 64; r++) {
-    const bool valid = r < rows && key < Skv;
-    const float x = valid ? (float)mb[(int64_t)(q0 + r) * rs] : -INFINITY;
-    const bool keep = !(x <= Dropped<T>);  // (a NaN is kept, and is not 0)
-    const unsigned long long w = __ballot(keep);
-    roww = lane == r ? w : roww;
-    colw |= (unsigned long long)keep << r;
-    other = other || (keep && x != 0.f);
-    ncausal = ncausal || (valid && (key <= q0 + r ? x != 0.f : x != -INFINITY));
+  if (row < Sq) {
+    const T* mr = mask + b * bs + row * rs + k0;
+    auto take = [&](T v, int j) {
+      const float x = (float)v;
+      const bool keep = !(x <= Dropped<T>);  // (a NaN is kept, and is not 0)
+      roww |= (unsigned long long)keep << j;
+      other = other || (keep && x != 0.f);
+      ncausal = ncausal || (k0 + j <= row ? x != 0.f : x != -INFINITY);
+    };
+    if (k0 + 64 <= Skv) {
+      constexpr int PER = 16 / sizeof(T);
+      typedef T Chunk __attribute__((ext_vector_type(PER), aligned(sizeof(T))));  // (rows are aligned to an entry only)
+      Chunk c[64 / PER];
+#pragma unroll
+      for (int i = 0; i < 64 / PER; i++) c[i] = *(const Chunk*)(mr + i * PER);
+#pragma unroll
+      for (int j = 0; j < 64; j++) take(c[j / PER][j % PER], j);
+    } else {
+      for (int j = 0; j < Skv - k0; j++) take(mr[j], j);
+    }
+  }
+  unsigned long long colw = 0ull;
+#pragma unroll
+  for (int j = 0; j < 64; j++) {
+    const unsigned long long w = __ballot((roww >> j) & 1ull);
+    colw = lane == j ? w : colw;
   }
   // words: rows up to the padding of the last block of 128
-  if (kt < nkt) qbits[((int64_t)b * nkt + kt) * (nqb * 128) + q0 + lane] = roww;
+  if (kt < nkt) qbits[((int64_t)b * nkt + kt) * (nqb * 128) + row] = roww;
   if (qt < nqt) kbits[((int64_t)b * nqt + qt) * (nkb * 128) + key] = colw;
   // classes of the two halves of 32 rows: 0 no pair, 2 every pair (rows past the end do not count), 1 otherwise
   auto classes = [&](unsigned long long w, bool past) -> unsigned short {
@@ -58,7 +74,7 @@ __global__ __launch_bounds__(256) void mask_bits_kernel(const T* __restrict__ ma
     const unsigned a0 = (unsigned)any, a1 = (unsigned)(any >> 32), f0 = (unsigned)full, f1 = (unsigned)(full >> 32);
     return (unsigned short)((a0 == 0u ? 0 : f0 == ~0u ? 2 : 1) | ((a1 == 0u ? 0 : f1 == ~0u ? 2 : 1) << 8));
   };
-  const unsigned short qc = classes(roww, q0 + lane >= Sq), kc = classes(colw, key >= Skv);
+  const unsigned short qc = classes(roww, row >= Sq), kc = classes(colw, key >= Skv);
   if (lane == 0) {
     if (kt < nkt) qcls[(((int64_t)b * nqb + (qt >> 1)) * nkt + kt) * 2 + (qt & 1)] = qc;
     if (qt < nqt) kcls[(((int64_t)b * nkb + (kt >> 1)) * nqt + qt) * 2 + (kt & 1)] = kc;
