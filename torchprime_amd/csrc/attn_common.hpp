@@ -442,4 +442,52 @@ __device__ __forceinline__ u32x4 make_rsrc_words(const void* base, unsigned byte
   return r;
 }
 
+// ---- fp32 kernels ----------------------------------------------------------------------------------
+// Sum of the four waves' accumulators, in wave 0: (w0 + w2) + (w1 + w3).  red: 2 x N x 16 x 64 floats of LDS, free to use
+// again after the next barrier.
+template <int N>
+__device__ __forceinline__ void sum_waves(f32x16 (&acc)[N], float* red, int wave, int lane) {
+  auto put = [&](float* r) {
+#pragma unroll
+    for (int d = 0; d < N; d++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) r[(d * 16 + v) * 64 + lane] = acc[d][v];
+  };
+  auto add = [&](const float* r) {
+#pragma unroll
+    for (int d = 0; d < N; d++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[d][v] += r[(d * 16 + v) * 64 + lane];
+  };
+  if (wave >= 2) put(red + (wave - 2) * N * 1024);
+  __syncthreads();
+  if (wave < 2) add(red + wave * N * 1024);
+  __syncthreads();
+  if (wave == 1) put(red);
+  __syncthreads();
+  if (wave == 0) add(red);
+}
+// HD consecutive floats
+template <int HD>
+__device__ __forceinline__ void load_row32(float (&x)[HD], const float* p) {
+#pragma unroll
+  for (int s = 0; s < HD; s += 4) {
+    const f32x4 t = *(const f32x4*)(p + s);
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[s + e] = t[e];
+  }
+}
+// rows r0 + 8 (v / 4) + 4 g + v % 4 (v = 0..15) of a row-major matrix, column d * 32 + lane % 32 for d < DB: what a "C-fed"
+// product pairs with an accumulator's values.  Rows past n are zeros.
+template <int DB>
+__device__ __forceinline__ void load_cols32(float (&x)[16][DB], const float* base, int64_t stride, int r0, int n, int g, int ln) {
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    const int r = r0 + 8 * (v / 4) + 4 * g + (v % 4);
+    const float* p = base + (int64_t)min(r, n - 1) * stride + ln;
+#pragma unroll
+    for (int d = 0; d < DB; d++) x[v][d] = r < n ? p[d * 32] : 0.f;
+  }
+}
+
 }  // namespace tp

@@ -4,7 +4,14 @@
 // softmax) is what its own CPU tests run the small configurations in
 // (torchprime/torch_xla_models/tests/test_llama.py:143-188); the 16-bit kernels cannot meet those tolerances.  This
 // kernel is the same algorithm as attn_fwd.hip without any 16-bit rounding: causal / full, segment ids, GQA, explicit
-// scale, LSE out.  It is sized for correctness at small shapes, not tuned like the 16-bit kernels.
+// scale, LSE out.
+//
+// At the sizes this is used for (sequences of a few hundred, eight heads) there are few query rows to go round and the
+// chain of kv tiles is what takes the time.  So a workgroup owns 32 query rows only, its four waves take the kv tiles in
+// turn, each with an online softmax of its own, and the four partial results meet in LDS at the end; operands come
+// straight from memory in the layout the MFMA wants (K and Q rows as contiguous pieces, V rows as coalesced columns: every
+// byte of a line is used), so no wave waits for another inside the loop, and V's loads fly under the S products.
+// B2 S128, 8 heads of 64: 26 us with 128 rows a workgroup and staged tiles.
 //
 // v_mfma_f32_32x32x2_f32 (wave64; ln = lane % 32, g = lane / 32):
 //   A (32 x 2): lane holds row ln, k = g        B (2 x 32): lane holds column ln, k = g
@@ -37,44 +44,34 @@ typedef float f32x1 __attribute__((ext_vector_type(1)));
 
 template <int D>
 __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
-  constexpr int BN = 32, BM = 128, DB = D / 32, HD = D / 2;
-  constexpr int KSTRIDE = D + 4;  // floats per LDS row of K: 16-byte aligned rows, consecutive rows 4 banks apart
-  constexpr int VSTRIDE = D + 1;
-  __shared__ __align__(16) float ksm[BN * KSTRIDE];
-  __shared__ float vsm[BN * VSTRIDE];
-  __shared__ int ssm[BN];
+  constexpr int BN = 32, BM = 32, DB = D / 32, HD = D / 2;
+  __shared__ __align__(16) float red[2 * DB * 1024];
+  __shared__ float msm[4][64], lsm[4][64];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
-  const int qt = blockIdx.x % n_qt;
+  const int qt = n_qt - 1 - blockIdx.x % n_qt;  // the longest rows first
   const int bh = blockIdx.x / n_qt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.n_rep;
-  const int q0 = qt * BM, wq0 = q0 + wave * 32;
+  const int q0 = qt * BM;
   const int Sq = a.Sq, Skv = a.Skv;
-  const int qrow = wq0 + ln;
-  const float* qb = a.q + b * a.qs[0] + h * a.qs[1];
+  const int qrow = q0 + ln, qrow_c = min(qrow, Sq - 1);
   const float* kb = a.k + b * a.ks[0] + hk * a.ks[1];
   const float* vb = a.v + b * a.vs[0] + hk * a.vs[1];
   const int32_t* segb = a.seg ? a.seg + (int64_t)b * Skv : nullptr;
-  const int segq = segb ? segb[min(qrow, Sq - 1)] : 0;
+  const int segq = segb ? segb[qrow_c] : 0;
   // mask extensions: this lane's query row may see key positions qp - lo_off .. qp + hi_off (causality is part of
   // the band then, and a.causal is off)
-  const int qp = a.mx.on ? (a.mx.qpos ? a.mx.qpos[min(qrow, Sq - 1)] : qrow) : 0;
+  const int qp = a.mx.on ? (a.mx.qpos ? a.mx.qpos[qrow_c] : qrow) : 0;
   const int band_lo = a.mx.on ? qp - a.mx.lo_off : -BAND_INF, band_hi = a.mx.on ? qp + a.mx.hi_off : BAND_INF;
-  const float* bias_row =
-      a.mx.bias ? a.mx.bias + b * a.mx.bias_s[0] + h * a.mx.bias_s[1] + (int64_t)min(qrow, Sq - 1) * a.mx.bias_s[2] : nullptr;
+  const float* bias_row = a.mx.bias ? a.mx.bias + b * a.mx.bias_s[0] + h * a.mx.bias_s[1] + (int64_t)qrow_c * a.mx.bias_s[2] : nullptr;
 
   // Q^T fragments: lane (query column ln, group g) holds Q[q][g*HD + s] for s = 0..HD-1, pre-multiplied by the
   // scale in log2 units (an fp32 product: no precision is lost that the fp32 reference keeps)
   float qf[HD];
-  {
-    const float* qp = qb + (int64_t)min(qrow, Sq - 1) * a.qs[2] + g * HD;
+  load_row32(qf, a.q + b * a.qs[0] + h * a.qs[1] + (int64_t)qrow_c * a.qs[2] + g * HD);
 #pragma unroll
-    for (int s = 0; s < HD; s += 4) {
-      const f32x4 t = *(const f32x4*)(qp + s);
-      qf[s] = t[0] * a.scale_log2; qf[s + 1] = t[1] * a.scale_log2; qf[s + 2] = t[2] * a.scale_log2; qf[s + 3] = t[3] * a.scale_log2;
-    }
-  }
+  for (int s = 0; s < HD; s++) qf[s] *= a.scale_log2;
 
   f32x16 oacc[DB];
 #pragma unroll
@@ -85,42 +82,23 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
 
   const int kv_end = a.causal ? min(Skv, q0 + BM) : Skv;
   const int ntiles = (kv_end + BN - 1) / BN;
-  for (int t = 0; t < ntiles; t++) {
+  for (int t = wave; t < ntiles; t += 4) {
     const int kv0 = t * BN;
-    __syncthreads();  // everyone is done with the previous tile
-    // stage K and V rows kv0 .. kv0+31 (rows past Skv as zeros): 16-byte chunks, thread -> (row, chunk)
-    for (int c = tid; c < BN * (D / 4); c += 256) {
-      const int r = c / (D / 4), cc = (c % (D / 4)) * 4;
-      f32x4 kvv = {0.f, 0.f, 0.f, 0.f}, vvv = {0.f, 0.f, 0.f, 0.f};
-      if (kv0 + r < Skv) {
-        kvv = *(const f32x4*)(kb + (int64_t)(kv0 + r) * a.ks[2] + cc);
-        vvv = *(const f32x4*)(vb + (int64_t)(kv0 + r) * a.vs[2] + cc);
-      }
-      *(f32x4*)(ksm + r * KSTRIDE + cc) = kvv;
-      vsm[r * VSTRIDE + cc] = vvv[0]; vsm[r * VSTRIDE + cc + 1] = vvv[1]; vsm[r * VSTRIDE + cc + 2] = vvv[2]; vsm[r * VSTRIDE + cc + 3] = vvv[3];
-    }
-    if (segb && tid < BN) ssm[tid] = segb[min(kv0 + tid, Skv - 1)];
-    __syncthreads();
-    if (a.causal && kv0 > wq0 + 31) continue;  // the whole tile lies above this wave's diagonal (uniform per wave)
-
+    float kf[HD], vf[16][DB];
+    load_row32(kf, kb + (int64_t)min(kv0 + ln, Skv - 1) * a.ks[2] + g * HD);
+    load_cols32(vf, vb, a.vs[2], kv0, Skv, g, ln);
     // S^T = K Q^T: row = kv (ln of the A operand), column = query
     f32x16 s;
 #pragma unroll
     for (int v = 0; v < 16; v++) s[v] = 0.f;
-    const float* kr = ksm + ln * KSTRIDE + g * HD;
 #pragma unroll
-    for (int st = 0; st < HD; st += 4) {
-      const f32x4 k4 = *(const f32x4*)(kr + st);
-#pragma unroll
-      for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[e], qf[st + e], s, 0, 0, 0);
-    }
+    for (int st = 0; st < HD; st++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[st], qf[st], s, 0, 0, 0);
     // mask, online softmax (log2 units)
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < 16; v++) {
-      const int kvl = 8 * (v / 4) + 4 * g + (v % 4);
-      const int kv = kv0 + kvl;
-      const bool ok = kv < Skv && (!a.causal || kv <= qrow) && (!segb || ssm[kvl] == segq) && kv >= band_lo && kv <= band_hi;
+      const int kv = kv0 + 8 * (v / 4) + 4 * g + (v % 4);
+      const bool ok = kv < Skv && (!a.causal || kv <= qrow) && (!segb || segb[min(kv, Skv - 1)] == segq) && kv >= band_lo && kv <= band_hi;
       if (a.cap2 != 0.f) s[v] = a.cap2 * tanhf(s[v] / a.cap2);  // cap * tanh(score / cap), in log2 units
       if (bias_row) s[v] += LOG2E * bias_row[min(kv, Skv - 1)];  // additive mask (-inf stays -inf)
       s[v] = ok ? s[v] : -INFINITY;
@@ -144,18 +122,29 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
       for (int v = 0; v < 16; v++) oacc[d][v] *= alpha;
     // O^T += V^T P^T: step v pairs kv row 8*(v/4) + 4*g + v%4 of V with the lane's value v of P^T
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int kvl = 8 * (v / 4) + 4 * g + (v % 4);
+    for (int v = 0; v < 16; v++)
 #pragma unroll
-      for (int d = 0; d < DB; d++) oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vsm[kvl * VSTRIDE + d * 32 + ln], s[v], oacc[d], 0, 0, 0);
-    }
+      for (int d = 0; d < DB; d++) oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[v][d], s[v], oacc[d], 0, 0, 0);
   }
 
+  // the waves' shares: brought to the largest of the four maxima, then added
+  msm[wave][lane] = m_run;
+  __syncthreads();
+  const float m_all = fmaxf(fmaxf(msm[0][lane], msm[1][lane]), fmaxf(msm[2][lane], msm[3][lane]));
+  const float share = m_run == -INFINITY ? 0.f : exp2f(m_run - m_all);
+  lsm[wave][lane] = l_run * share;
+#pragma unroll
+  for (int d = 0; d < DB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) oacc[d][v] *= share;
+  sum_waves(oacc, red, wave, lane);
+  if (wave != 0) return;
+
   // epilogue: lane = query, value v of block d is output column d*32 + 8*(v/4) + 4*g + v%4
-  const float l = half_sum(l_run);
+  const float l = half_sum((lsm[0][lane] + lsm[2][lane]) + (lsm[1][lane] + lsm[3][lane]));
   const float inv = l > 0.f ? 1.f / l : 0.f;
   if (qrow < Sq) {
-    if (g == 0) a.lse[((int64_t)b * a.Hq + h) * Sq + qrow] = l > 0.f ? (m_run + log2f(l)) * LN2 : -INFINITY;
+    if (g == 0) a.lse[((int64_t)b * a.Hq + h) * Sq + qrow] = l > 0.f ? (m_all + log2f(l)) * LN2 : -INFINITY;
     float* op = a.out + b * a.os[0] + h * a.os[1] + (int64_t)qrow * a.os[2];
 #pragma unroll
     for (int d = 0; d < DB; d++)
@@ -186,7 +175,7 @@ int attn_fwd_f32(const void* q, const void* k, const void* v, const int32_t* seg
   a.causal = mx.on ? 0 : causal;
   a.mx = mx;
   a.cap2 = mx.cap_in != 0.f ? mx.cap_out * sm_scale * LOG2E : 0.f;
-  const int64_t blocks = (int64_t)B * Hq * ((Sq + 127) / 128);
+  const int64_t blocks = (int64_t)B * Hq * ((Sq + 31) / 32);
   TP_REQUIRE(blocks < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_fwd: too many workgroups");
   if (Dqk == 64) attn_fwd_f32_kernel<64><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
   else attn_fwd_f32_kernel<128><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
