@@ -64,6 +64,23 @@ class AttentionModule(nn.Module):
     self.kernel_config = kernel_config
     self.partition_spec = None
 
+  def plain_causal(self, seq_len: int, attention_mask: torch.Tensor | None):
+    """What ``forward`` computes for ``seq_len`` queries and keys where that is plain attention: True causal, False over
+    all pairs; None where it is neither (another mask, load-balanced context parallelism, dropout)."""
+    config = self.config
+    kernel = config.attention_kernel
+    if kernel == "splash_attention" and has_key(config, "load_balance_cp") and config.load_balance_cp:
+      return None
+    if kernel in ("splash_attention", "flash_attention"):
+      return True
+    if getattr(config, "attention_dropout", 0.0) and self.training:
+      return None
+    if attention_mask is None:
+      return False
+    if self.kernel_config and self.kernel_config.get("assume_causal_mask"):
+      return True
+    return True if _mask_verdict(attention_mask, seq_len, seq_len) == ops.MASK_CAUSAL else None
+
   def forward(
     self,
     query_states: torch.Tensor,  # (batch_size, num_heads, q_len, head_dim)

@@ -14,10 +14,13 @@ from __future__ import annotations
 
 import torch
 from torch import nn
+from torch.compiler import is_compiling
 
 from .attention import AttentionModule
-from .linear import project
-from .norm import DeepseekV3RMSNorm
+from .linear import global_hooks, plain, project, weight_of
+from .mlp import LlamaMLP
+from .norm import DeepseekV3RMSNorm, LlamaRMSNorm, add_rms_norm
+from .ops import _native
 from .rotary import MixtralRotaryEmbedding, apply_rotary_pos_emb, apply_rotary_pos_emb_interleave
 
 
@@ -212,9 +215,6 @@ class LlamaDecoderLayer(nn.Module):
 
   def __init__(self, config, layer_idx: int):
     super().__init__()
-    from .mlp import LlamaMLP
-    from .norm import LlamaRMSNorm
-
     self.hidden_size = config.hidden_size
     self.self_attn = LlamaAttention(config=config, layer_idx=layer_idx)
     self.mlp = LlamaMLP(config)
@@ -222,8 +222,6 @@ class LlamaDecoderLayer(nn.Module):
     self.post_attention_layernorm = LlamaRMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
   def forward(self, hidden_states, attention_mask=None, position_ids=None, position_embeddings=None):
-    from .norm import add_rms_norm
-
     residual = hidden_states
     hidden_states = self.input_layernorm(hidden_states)
     hidden_states = self.self_attn(hidden_states, position_embeddings, attention_mask, position_ids)
@@ -232,6 +230,33 @@ class LlamaDecoderLayer(nn.Module):
     hidden_states = self.mlp(hidden_states)
     return residual + hidden_states
 
+  def _one_call(self, x, residual, attention_mask, position_embeddings):
+    """``forward_deferred`` of a small layer as one native call (``llama_layer`` in csrc/torch_ops.cpp), or None: where a
+    module of the layer has to see its own call (hooks, a bias, another class, a patched forward), where the attention is
+    not plain causal or full attention, or where the projections are large (nothing is gained there)."""
+    if is_compiling() or global_hooks():
+      return None
+    mods = self.__dict__["_modules"]
+    attn, mlp, n1, n2 = mods["self_attn"], mods["mlp"], mods["input_layernorm"], mods["post_attention_layernorm"]
+    if not (plain(attn, LlamaAttention) and plain(mlp, LlamaMLP) and plain(n1, LlamaRMSNorm) and plain(n2, LlamaRMSNorm)):
+      return None
+    am, mm = attn.__dict__["_modules"], mlp.__dict__["_modules"]
+    block = am["attention_block"]
+    if not plain(block, AttentionModule):
+      return None
+    ws = [weight_of(am[n]) for n in ("q_proj", "k_proj", "v_proj", "o_proj")]
+    ws += [weight_of(mm[n]) for n in ("gate_proj", "up_proj", "down_proj")]
+    if any(w is None for w in ws):
+      return None
+    causal = block.plain_causal(x.shape[1], attention_mask)
+    if causal is None:
+      return None
+    w1, w2 = n1.__dict__["_parameters"]["weight"], n2.__dict__["_parameters"]["weight"]
+    cos, sin = position_embeddings
+    return _native.llama_layer(
+      x, residual, [w1, *ws[:4], w2, *ws[4:]], cos, sin, attn.num_heads, attn.num_key_value_heads, n1.variance_epsilon,
+      n2.variance_epsilon, causal,
+    )  # fmt: skip
 
 
   def forward_deferred(self, x, residual, attention_mask=None, position_ids=None, position_embeddings=None):
@@ -239,7 +264,9 @@ class LlamaDecoderLayer(nn.Module):
     ``x + residual`` (``residual`` None: ``x`` itself), added inside the first norm's kernel; the return value is
     ``(mlp_out, h)`` whose sum is the layer's output, for the next layer (or the model's final norm) to add the same
     way.  Same values as ``forward``, bit for bit, with one pass over the hidden states less per layer."""
-    from .norm import add_rms_norm
+    fused = self._one_call(x, residual, attention_mask, position_embeddings)
+    if fused:
+      return fused
 
     if residual is None:
       residual, hidden_states = x, self.input_layernorm(x)
@@ -261,7 +288,6 @@ class LlamaModel(nn.Module):
 
   def __init__(self, config):
     super().__init__()
-    from .norm import LlamaRMSNorm
     from .rope import RopeScaling
     from .rotary import LlamaRotaryEmbedding
 
@@ -294,8 +320,6 @@ class LlamaModel(nn.Module):
     return causal
 
   def forward(self, input_ids, attention_mask=None):
-    from .norm import add_rms_norm
-
     inputs_embeds = self.embed_tokens(input_ids)
     seq_length = inputs_embeds.size(1)
     position_ids = torch.arange(seq_length, device=inputs_embeds.device).unsqueeze(0).float()

@@ -26,6 +26,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <tuple>
 #include <unordered_map>
@@ -994,6 +995,253 @@ std::vector<Tensor> py_linears(const Tensor& x, const std::vector<Tensor>& ws) {
   return out;
 }
 
+// ---- a decoder layer ---------------------------------------------------------------------------------------------
+// The Llama decoder layer with its residual adds deferred (blocks.LlamaDecoderLayer.forward_deferred) as one call and one
+// autograd node, for layers whose projections are small (linears_take): norm, q / k / v, rotary, attention, output
+// projection, add + norm, gate / up, SwiGLU, down, the same kernels in the same order with the same roundings as the
+// modules, so the results are theirs bit for bit.  A layer of that size is 21 launches of 3 to 12 us; taken module by
+// module the host spent 30 us per launch on them (Python, one autograd node and its edges per operator, views, a tensor
+// per intermediate).  Intermediates lie in one allocation, the rotary runs in place, the backward's in another.
+struct LayerShape { int64_t B, S, H, Hq, Hkv, D, I, rows; int dtype; bool causal, residual; double eps1, eps2; };
+enum LayerParam { LP_N1, LP_Q, LP_K, LP_V, LP_O, LP_N2, LP_G, LP_U, LP_D, LP_COUNT };
+
+// offsets of the forward's intermediates in one buffer
+struct LayerBuf {
+  size_t h, n1, q, k, v, attn, n2, gate, up, act, rstd1, rstd2, lse, bytes;
+  explicit LayerBuf(const LayerShape& s) {
+    const size_t e = s.dtype == TP_F32 ? 4 : 2;
+    size_t at = 0;
+    const auto take = [&](size_t n) { const size_t o = at; at += (n + 255) / 256 * 256; return o; };
+    h = take(s.residual ? s.rows * s.H * e : 0);
+    n1 = take(s.rows * s.H * e);
+    q = take(s.rows * s.Hq * s.D * e); k = take(s.rows * s.Hkv * s.D * e); v = take(s.rows * s.Hkv * s.D * e);
+    attn = take(s.rows * s.Hq * s.D * e);
+    n2 = take(s.rows * s.H * e);
+    gate = take(s.rows * s.I * e); up = take(s.rows * s.I * e); act = take(s.rows * s.I * e);
+    rstd1 = take(s.rows * 4); rstd2 = take(s.rows * 4); lse = take(s.rows * s.Hq * 4);
+    bytes = at;
+  }
+};
+tp_linear_problem raw_linear(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k, bool akm, bool bkm, int64_t m, int64_t n, void* c) {
+  tp_linear_problem p{};
+  p.a[0] = a; p.b[0] = b; p.lda[0] = lda; p.ldb[0] = ldb; p.k[0] = (int)k; p.segments = 1;
+  p.a_kmajor = akm; p.b_kmajor = bkm; p.m = (int)m; p.n = (int)n; p.c = c; p.ldc = n;
+  return p;
+}
+void add_segment(tp_linear_problem& p, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k) {
+  const int i = p.segments++;
+  p.a[i] = a; p.b[i] = b; p.lda[i] = lda; p.ldb[i] = ldb; p.k[i] = (int)k;
+}
+// (batch, head, seq) strides of heads side by side in a row
+Strides3 head_strides(const LayerShape& s, int64_t heads) { return {s.S * heads * s.D, s.D, heads * s.D}; }
+// cos / sin rows: batch stride (0: one table for all batches)
+int64_t table_stride(const Tensor& cos, const LayerShape& s) { return cos.size(0) == s.B && s.B > 1 ? cos.stride(0) : 0; }
+
+void layer_rope(const LayerShape& s, void* q, void* k, const Tensor& cos, const Tensor& sin, bool backward, void* st) {
+  const Strides3 qs = head_strides(s, s.Hq), ks = head_strides(s, s.Hkv);
+  check(tp_rope_apply(q, k, cos.data_ptr(), sin.data_ptr(), nullptr, q, k, (int)s.B, (int)s.Hq, (int)s.Hkv, (int)s.S, (int)s.D, qs.data(),
+                      ks.data(), qs.data(), ks.data(), table_stride(cos, s), cos.stride(1), 0, 0, 0, (int)backward, s.dtype, st), "tp_rope_apply");
+}
+
+struct LayerNode : torch::autograd::Node {
+  LayerShape s;
+  SavedVariable x, buf, h2, cos, sin;
+  std::vector<SavedVariable> params;
+  std::string name() const override { return "TprimeLlamaLayerBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto* v : {&x, &buf, &h2, &cos, &sin}) v->reset_data();
+    for (auto& p : params) p.reset_data();
+  }
+  variable_list apply(variable_list&& g) override;
+};
+
+variable_list LayerNode::apply(variable_list&& g) {
+  std::lock_guard<std::mutex> lock(mutex_);
+  TORCH_CHECK_NOT_IMPLEMENTED(!at::GradMode::is_enabled(), "derivative for a decoder layer's backward is not implemented");
+  variable_list out(2 + LP_COUNT);  // x, residual, the parameters
+  if (!g[0].defined() && !g[1].defined()) return out;
+  const Tensor B = buf.unpack(), H2 = h2.unpack(shared_from_this()), C = cos.unpack(), Sn = sin.unpack();
+  const Tensor X = s.residual ? Tensor() : x.unpack();
+  std::array<Tensor, LP_COUNT> w;
+  for (int i = 0; i < LP_COUNT; i++) w[i] = params[i].unpack();
+  at::AutoDispatchBelowADInplaceOrView below;
+  c10::DeviceGuard guard(B.device());
+  void* st = stream_of(B.device());
+  const LayerBuf f(s);
+  char* base = (char*)B.data_ptr();
+  const int64_t R = s.rows, NQ = s.Hq * s.D, NK = s.Hkv * s.D;
+  const size_t e = s.dtype == TP_F32 ? 4 : 2;
+  const auto opts = H2.options();
+  const Tensor go = g[0].defined() ? g[0].to(H2.scalar_type()).contiguous() : at::zeros(H2.sizes(), opts);
+  const Tensor gh = g[1].defined() ? g[1].to(H2.scalar_type()).contiguous() : at::zeros(H2.sizes(), opts);
+  const auto need = [&](int i) { return task_should_compute_output(2 + i); };
+  const auto grad_of = [&](int i) { return out[2 + i] = at::empty(w[i].sizes(), w[i].options()); };
+  // scratch
+  const size_t ws_rows = tp_attn_bwd_workspace_bytes((int)s.B, (int)s.Hq, (int)s.S), ws_norm = tp_rmsnorm_bwd_workspace_bytes(R, (int)s.H);
+  tp_attn_bwd_problem ab{};
+  ab.B = (int)s.B; ab.Hq = (int)s.Hq; ab.Hkv = (int)s.Hkv; ab.Sq = ab.Skv = (int)s.S; ab.Dqk = ab.Dv = (int)s.D;
+  ab.causal = s.causal; ab.window_left = ab.window_right = -1; ab.dtype = s.dtype; ab.sm_scale = (float)(1.0 / std::sqrt((double)s.D));
+  ab.parts_bytes = tp_attn_bwd_parts_bytes(&ab);
+  size_t at = 0;
+  const auto take = [&](size_t n) { const size_t o = at; at += (n + 255) / 256 * 256; return o; };
+  const size_t o_act = take(R * s.I * e), o_dg = take(R * s.I * e), o_du = take(R * s.I * e), o_dn = take(R * s.H * e), o_ds = take(R * s.H * e);
+  const size_t o_da = take(R * NQ * e), o_dq = take(R * NQ * e), o_dk = take(R * NK * e), o_dv = take(R * NK * e);
+  const size_t o_ws = take(ws_rows), o_norm = take(ws_norm), o_parts = take(ab.parts_bytes), o_dw = take(s.H * e);
+  const Tensor scratch = at::empty({(int64_t)at}, opts.dtype(at::kByte));
+  char* t = (char*)scratch.data_ptr();
+  std::array<tp_linear_problem, 4> p;
+  const auto run = [&](int n) { check(tp_linears(p.data(), n, s.dtype, st), "tp_linears"); };
+  const auto wgrad = [&](int i, const void* gr, int64_t nf, const void* in, int64_t k) { return raw_linear(gr, nf, in, k, R, false, false, nf, k, grad_of(i).data_ptr()); };
+  int n = 0;
+  // down projection
+  p[n++] = raw_linear(go.data_ptr(), s.H, w[LP_D].data_ptr(), s.I, s.H, true, false, R, s.I, t + o_act);
+  if (need(LP_D)) p[n++] = wgrad(LP_D, go.data_ptr(), s.H, base + f.act, s.I);
+  run(n);
+  check(tp_swiglu_bwd(t + o_act, base + f.gate, base + f.up, t + o_dg, t + o_du, R, (int)s.I, s.I, s.I, s.I, s.I, s.I, s.dtype, st), "tp_swiglu_bwd");
+  // gate, up
+  n = 0;
+  p[n] = raw_linear(t + o_dg, s.I, w[LP_G].data_ptr(), s.H, s.I, true, false, R, s.H, t + o_dn);
+  add_segment(p[n++], t + o_du, s.I, w[LP_U].data_ptr(), s.H, s.I);
+  if (need(LP_G)) p[n++] = wgrad(LP_G, t + o_dg, s.I, base + f.n2, s.H);
+  if (need(LP_U)) p[n++] = wgrad(LP_U, t + o_du, s.I, base + f.n2, s.H);
+  run(n);
+  // norm 2 and the residual's gradient
+  const auto norm_bwd = [&](int i, const void* dy, const void* dh, const void* hh, size_t rstd, void* dx) {
+    void* dw = need(i) ? grad_of(i).data_ptr() : t + o_dw;
+    check(tp_add_rmsnorm_bwd(dy, dh, hh, w[i].data_ptr(), (const float*)(base + rstd), dx, dw, (float*)(t + o_norm), R, (int)s.H, s.H, s.H, s.H, s.H,
+                             s.dtype, s.dtype, st), "tp_add_rmsnorm_bwd");
+  };
+  norm_bwd(LP_N2, t + o_dn, gh.data_ptr(), H2.data_ptr(), f.rstd2, t + o_ds);
+  // output projection
+  n = 0;
+  p[n++] = raw_linear(t + o_ds, s.H, w[LP_O].data_ptr(), NQ, s.H, true, false, R, NQ, t + o_da);
+  if (need(LP_O)) p[n++] = wgrad(LP_O, t + o_ds, s.H, base + f.attn, NQ);
+  run(n);
+  // attention, rotary
+  ab.dout = t + o_da; ab.q = base + f.q; ab.k = base + f.k; ab.v = base + f.v; ab.out = base + f.attn; ab.lse = (const float*)(base + f.lse);
+  ab.dq = t + o_dq; ab.dk = t + o_dk; ab.dv = t + o_dv; ab.ws = (float*)(t + o_ws);
+  ab.parts = ab.parts_bytes ? t + o_parts : nullptr;
+  const Strides3 qs = head_strides(s, s.Hq), ks = head_strides(s, s.Hkv);
+  for (int i = 0; i < 3; i++) {
+    ab.do_strides[i] = ab.q_strides[i] = ab.o_strides[i] = ab.dq_strides[i] = qs[i];
+    ab.k_strides[i] = ab.v_strides[i] = ab.dk_strides[i] = ab.dv_strides[i] = ks[i];
+  }
+  check(tp_attn_bwd_run(&ab, st), "tp_attn_bwd_run");
+  layer_rope(s, t + o_dq, t + o_dk, C, Sn, true, st);
+  // q, k, v
+  n = 0;
+  p[n] = raw_linear(t + o_dq, NQ, w[LP_Q].data_ptr(), s.H, NQ, true, false, R, s.H, t + o_dn);
+  add_segment(p[n], t + o_dk, NK, w[LP_K].data_ptr(), s.H, NK);
+  add_segment(p[n++], t + o_dv, NK, w[LP_V].data_ptr(), s.H, NK);
+  if (need(LP_Q)) p[n++] = wgrad(LP_Q, t + o_dq, NQ, base + f.n1, s.H);
+  if (need(LP_K)) p[n++] = wgrad(LP_K, t + o_dk, NK, base + f.n1, s.H);
+  if (need(LP_V)) p[n++] = wgrad(LP_V, t + o_dv, NK, base + f.n1, s.H);
+  run(n);
+  // norm 1; x and the residual get the same gradient
+  const Tensor dx = at::empty(H2.sizes(), opts);
+  norm_bwd(LP_N1, t + o_dn, t + o_ds, s.residual ? base + f.h : (char*)X.data_ptr(), f.rstd1, dx.data_ptr());
+  out[0] = dx;
+  if (s.residual) out[1] = dx;
+  return out;
+}
+
+// (mlp output, residual), or nothing where this layer is one for the modules
+std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const std::vector<Tensor>& w, const Tensor& cos, const Tensor& sin,
+                                   int64_t Hq, int64_t Hkv, double eps1, double eps2, bool causal) {
+  const Tensor& residual = val(residual_);
+  if (w.size() != LP_COUNT || x.dim() != 3 || !x.is_contiguous() || x.numel() == 0) return {};
+  const auto dt = x.scalar_type();
+  LayerShape s;
+  s.B = x.size(0); s.S = x.size(1); s.H = x.size(2); s.Hq = Hq; s.Hkv = Hkv; s.rows = s.B * s.S; s.causal = causal; s.eps1 = eps1; s.eps2 = eps2;
+  s.residual = residual.defined();
+  const auto rows_ok = [&](const Tensor& t) { return t.dim() == 1 && t.size(0) == s.H && t.scalar_type() == dt && t.is_contiguous() && plain_eager(t) && t.device() == x.device(); };
+  if (!linears_take(x, {w[LP_Q], w[LP_K], w[LP_V]}) || !linears_take(x, {w[LP_G], w[LP_U]}) || !rows_ok(w[LP_N1]) || !rows_ok(w[LP_N2])) return {};
+  if (s.residual && (residual.sizes() != x.sizes() || residual.scalar_type() != dt || !residual.is_contiguous() || !plain_eager(residual) || residual.device() != x.device())) return {};
+  s.dtype = dtype_code(dt);
+  s.I = w[LP_G].size(0);
+  const int64_t NQ = w[LP_Q].size(0), NK = w[LP_K].size(0), vec = 16 / x.element_size();
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || NQ % Hq) return {};
+  s.D = NQ / Hq;
+  if ((s.D != 64 && s.D != 128) || NK != Hkv * s.D || w[LP_V].size(0) != NK || w[LP_U].size(0) != s.I || s.H % vec) return {};
+  // the two projections whose input is made here: shape, layout, and the same line on size
+  const auto lin_ok = [&](const Tensor& t, int64_t n, int64_t k) {
+    return t.dim() == 2 && t.size(0) == n && t.size(1) == k && t.scalar_type() == dt && t.is_contiguous() && plain_eager(t) && t.device() == x.device() &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && s.rows * n * k <= lin_max_work(dt);
+  };
+  if (!lin_ok(w[LP_O], s.H, NQ) || !lin_ok(w[LP_D], s.H, s.I)) return {};
+  for (const Tensor* t : {&cos, &sin})
+    if (t->dim() != 3 || (t->size(0) != 1 && t->size(0) != s.B) || t->size(1) != s.S || t->size(2) != s.D || t->scalar_type() != dt ||
+        !t->is_contiguous() || !plain_eager(*t) || t->device() != x.device() || t->requires_grad()) return {};
+  for (const Tensor* t : {&x, &residual})
+    if (t->defined() && (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 || torch::autograd::isFwGradDefined(*t))) return {};
+
+  std::shared_ptr<LayerNode> node;
+  if (at::GradMode::is_enabled()) {
+    bool req = x.requires_grad() || (s.residual && residual.requires_grad());
+    for (const auto& t : w) req = req || t.requires_grad();
+    if (req) {
+      node = std::shared_ptr<LayerNode>(new LayerNode(), torch::autograd::deleteNode);
+      torch::autograd::edge_list edges;
+      edges.reserve(2 + LP_COUNT);
+      edges.push_back(torch::autograd::impl::gradient_edge(x));
+      edges.push_back(s.residual ? torch::autograd::impl::gradient_edge(residual) : torch::autograd::Edge());
+      for (const auto& t : w) edges.push_back(torch::autograd::impl::gradient_edge(t));
+      node->set_next_edges(std::move(edges));
+    }
+  }
+  Tensor out, h2, buf;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::DeviceGuard guard(x.device());
+    void* st = stream_of(x.device());
+    const LayerBuf f(s);
+    buf = at::empty({(int64_t)f.bytes}, x.options().dtype(at::kByte));
+    out = at::empty(x.sizes(), x.options());
+    h2 = at::empty(x.sizes(), x.options());
+    char* b = (char*)buf.data_ptr();
+    const int64_t R = s.rows;
+    std::array<tp_linear_problem, 4> p;
+    const auto lin = [&](int i, const void* in, int64_t k, int wi, void* c) { p[i] = raw_linear(in, k, w[wi].data_ptr(), k, k, true, true, R, w[wi].size(0), c); };
+    const auto run = [&](int n) { check(tp_linears(p.data(), n, s.dtype, st), "tp_linears"); };
+    if (s.residual)
+      check(tp_add_rmsnorm_fwd(x.data_ptr(), residual.data_ptr(), w[LP_N1].data_ptr(), b + f.h, b + f.n1, (float*)(b + f.rstd1), R, (int)s.H, s.H, s.H,
+                               s.H, s.H, (float)eps1, s.dtype, s.dtype, st), "tp_add_rmsnorm_fwd");
+    else
+      check(tp_rmsnorm_fwd(x.data_ptr(), w[LP_N1].data_ptr(), b + f.n1, (float*)(b + f.rstd1), R, (int)s.H, s.H, s.H, (float)eps1, s.dtype, s.dtype, st),
+            "tp_rmsnorm_fwd");
+    lin(0, b + f.n1, s.H, LP_Q, b + f.q); lin(1, b + f.n1, s.H, LP_K, b + f.k); lin(2, b + f.n1, s.H, LP_V, b + f.v);
+    run(3);
+    layer_rope(s, b + f.q, b + f.k, cos, sin, false, st);
+    const Strides3 qs = head_strides(s, s.Hq), ks = head_strides(s, s.Hkv);
+    check(tp_attn_fwd(b + f.q, b + f.k, b + f.v, nullptr, b + f.attn, (float*)(b + f.lse), (int)s.B, (int)s.Hq, (int)s.Hkv, (int)s.S, (int)s.S, (int)s.D,
+                      (int)s.D, qs.data(), ks.data(), ks.data(), qs.data(), (float)(1.0 / std::sqrt((double)s.D)), (int)causal, s.dtype, st), "tp_attn_fwd");
+    lin(0, b + f.attn, NQ, LP_O, out.data_ptr());  // (the output's memory is free until the last projection)
+    run(1);
+    const void* h = s.residual ? (const void*)(b + f.h) : x.data_ptr();
+    check(tp_add_rmsnorm_fwd(out.data_ptr(), h, w[LP_N2].data_ptr(), h2.data_ptr(), b + f.n2, (float*)(b + f.rstd2), R, (int)s.H, s.H, s.H, s.H, s.H,
+                             (float)eps2, s.dtype, s.dtype, st), "tp_add_rmsnorm_fwd");
+    lin(0, b + f.n2, s.H, LP_G, b + f.gate); lin(1, b + f.n2, s.H, LP_U, b + f.up);
+    run(2);
+    check(tp_swiglu_fwd(b + f.gate, b + f.up, b + f.act, R, (int)s.I, s.I, s.I, s.I, s.dtype, st), "tp_swiglu_fwd");
+    lin(0, b + f.act, s.I, LP_D, out.data_ptr());
+    run(1);
+  }
+  if (node) {
+    node->s = s;
+    torch::autograd::set_history(out, node);
+    torch::autograd::set_history(h2, node);
+    if (!s.residual) node->x = SavedVariable(x, false);
+    node->buf = SavedVariable(buf, false);
+    node->h2 = SavedVariable(h2, true);
+    node->cos = SavedVariable(cos, false);
+    node->sin = SavedVariable(sin, false);
+    node->params.reserve(LP_COUNT);
+    for (const auto& t : w) node->params.emplace_back(t, false);
+  }
+  return {out, h2};
+}
+
 // ---- Python entry points -----------------------------------------------------------------------------------------
 // What the Python functions of ops.py call: the GPU check with its own message, then the operator.
 Tensor py_rmsnorm(const Tensor& x, const Tensor& w, double eps) { require_gpu(x, w); return std::get<0>(op_rmsnorm_fwd()(x, w, eps)); }
@@ -1117,6 +1365,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mask_kind", &py_mask_kind);
   m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
   m.def("linears", &py_linears);
+  m.def("llama_layer", &py_llama_layer);
   m.def("l2norm", &py_l2norm);
   m.def("swiglu", &py_swiglu);
   m.def("cross_entropy", &py_cross_entropy);

@@ -17,22 +17,30 @@ _GLOBAL_HOOKS = (
 )  # fmt: skip
 
 
-def _weight(m: nn.Module):
-  """The weight of a module that is nothing but ``x @ weight.T``, else None: a bias, hooks, a subclass or a patched
-  ``forward`` have to see the call."""
-  if type(m) is not nn.Linear:
-    return None
+def plain(m: nn.Module, cls: type) -> bool:
+  """``m`` is exactly a ``cls`` and nothing has to see its call: no hooks, no patched ``forward``."""
   d = m.__dict__
-  p = d["_parameters"]
-  if p.get("bias") is not None or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]:
+  return type(m) is cls and not (
+    d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d
+  )
+
+
+def global_hooks() -> bool:
+  return any(_GLOBAL_HOOKS)
+
+
+def weight_of(m: nn.Module):
+  """The weight of a module that is nothing but ``x @ weight.T``, else None."""
+  if not plain(m, nn.Linear):
     return None
-  return None if "forward" in d else p.get("weight")
+  p = m.__dict__["_parameters"]
+  return None if p.get("bias") is not None else p.get("weight")
 
 
 def project(x: torch.Tensor, *modules: nn.Module) -> list[torch.Tensor]:
   """``[m(x) for m in modules]``."""
-  if not is_compiling() and not any(_GLOBAL_HOOKS):
-    ws = [_weight(m) for m in modules]
+  if not is_compiling() and not global_hooks():
+    ws = [weight_of(m) for m in modules]
     if all(w is not None for w in ws):
       return _native.linears(x, ws)
   return [m(x) for m in modules]
