@@ -251,6 +251,81 @@ __global__ __launch_bounds__(64 * (WAVES > 4 ? WAVES : 4)) void rmsnorm_bwd_vec(
   }
 }
 
+// backward for few rows, one launch: a wave per row for dx, and beside them workgroups that own 4 vectors of columns and
+// walk all rows for dw.  dw needs no row sum (1 / rms is kept from the forward), so nothing has to wait for anything; x
+// and dy are read twice, out of cache.  With the row-walking kernel the same problem was two launches and a fp32 partial
+// row per row of x (512 rows of 512: 4.2 + 3.7 us and the gap between them).
+template <typename XT, typename WT, typename OT, int NV, bool RES>
+__global__ __launch_bounds__(256) void rmsnorm_bwd_few(const OT* __restrict__ dy, const XT* __restrict__ x, const WT* __restrict__ w,
+                                                       const float* __restrict__ rstd, XT* __restrict__ dx, WT* __restrict__ dw, int rows,
+                                                       int hidden, int64_t dys, int64_t xs, int64_t dxs, const XT* __restrict__ dres,
+                                                       int64_t drs, int row_blocks) {
+  constexpr int E = 16 / sizeof(XT);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nvec = hidden / E;
+  if ((int)blockIdx.x < row_blocks) {
+    const int row = blockIdx.x * 4 + wave;
+    if (row >= rows) return;
+    const float r = rstd[row];
+    float n[NV][E], g[NV][E], c = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      const int v = lane + 64 * i, off = (v < nvec ? v : nvec - 1) * E;
+      float wv[E];
+      load_f<XT, E>(x + row * xs + off, n[i]);
+      load_f<OT, E>(dy + row * dys + off, g[i]);
+      load_f<WT, E>(w + off, wv);
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        n[i][e] *= r;
+        g[i][e] *= wv[e];
+        if (v < nvec) c += g[i][e] * n[i][e];
+      }
+    }
+    c = wave_sum(c) * (1.f / (float)hidden);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      const int v = lane + 64 * i;
+      if (v >= nvec) continue;
+      float o[E];
+#pragma unroll
+      for (int e = 0; e < E; e++) o[e] = r * (g[i][e] - n[i][e] * c);
+      if (RES) {
+        float a[E];
+        load_f<XT, E>(dres + row * drs + v * E, a);
+#pragma unroll
+        for (int e = 0; e < E; e++) o[e] = round_to<XT>(o[e]) + a[e];  // (each addend rounded first, as in rmsnorm_bwd_vec)
+      }
+      store_f<XT, E>(dx + row * dxs + v * E, o);
+    }
+    return;
+  }
+  // dw: thread = (row group of 64, one of 4 vectors)
+  __shared__ float red[64][4 * E + 1];
+  const int vl = threadIdx.x & 3, rg = threadIdx.x >> 2, v = ((int)blockIdx.x - row_blocks) * 4 + vl, off = (v < nvec ? v : nvec - 1) * E;
+  float acc[E];
+#pragma unroll
+  for (int e = 0; e < E; e++) acc[e] = 0.f;
+#pragma unroll 4
+  for (int row = rg; row < rows; row += 64) {
+    float n[E], g[E];
+    load_f<XT, E>(x + row * xs + off, n);
+    load_f<OT, E>(dy + row * dys + off, g);
+    const float r = rstd[row];
+#pragma unroll
+    for (int e = 0; e < E; e++) acc[e] += g[e] * round_to<XT>(n[e] * r);
+  }
+#pragma unroll
+  for (int e = 0; e < E; e++) red[rg][vl * E + e] = acc[e];
+  __syncthreads();
+  if (threadIdx.x < 4 * E) {
+    const int col = ((int)blockIdx.x - row_blocks) * 4 * E + threadIdx.x;
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < 64; k++) s += red[k][threadIdx.x];
+    if (col < hidden) dw[col] = Elem<WT>::from_f(s);
+  }
+}
+
 // backward dx, any hidden / alignment
 template <typename XT, typename WT, typename OT>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_dx_generic(const OT* __restrict__ dy, const XT* __restrict__ x,
@@ -360,6 +435,23 @@ static int bwd_typed(const void* dy, const void* x, const void* w, const float* 
   const bool vec = hidden % E == 0 && aligned16(dy) && aligned16(x) && aligned16(w) && aligned16(dx) &&
                    (dys * sizeof(OT)) % 16 == 0 && (xs * sizeof(XT)) % 16 == 0 && (dxs * sizeof(XT)) % 16 == 0 &&
                    aligned16(dres) && (drs * sizeof(XT)) % 16 == 0 && nvec <= 256 * 8;
+  // few rows: one launch (x and dy twice through the caches).  Up to 1024 rows, where dw's walk (16 rows a thread) is as
+  // short as dx's row, and rows of up to 512 vectors
+  if (vec && rows <= 1024 && nvec <= 512) {
+    const int row_blocks = (int)(rows + 3) / 4;
+    const dim3 grid(row_blocks + (nvec + 3) / 4), block(256);
+#define TP_RMS_FEW(NV)                                                                                                                  \
+  do {                                                                                                                                  \
+    if (drp) rmsnorm_bwd_few<XT, WT, OT, NV, true><<<grid, block, 0, st>>>(gp, xp, wp, rstd, dxp, (WT*)dw, (int)rows, hidden, dys, xs, dxs, drp, drs, row_blocks); \
+    else rmsnorm_bwd_few<XT, WT, OT, NV, false><<<grid, block, 0, st>>>(gp, xp, wp, rstd, dxp, (WT*)dw, (int)rows, hidden, dys, xs, dxs, drp, drs, row_blocks);    \
+  } while (0)
+    if (nvec <= 64) TP_RMS_FEW(1);
+    else if (nvec <= 128) TP_RMS_FEW(2);
+    else if (nvec <= 256) TP_RMS_FEW(4);
+    else TP_RMS_FEW(8);
+#undef TP_RMS_FEW
+    return check_launch("tp_rmsnorm_bwd");
+  }
   if (vec) {
 #define TP_RMS_BWD(NV, WAVES)                                                                             \
   do {                                                                                                    \
