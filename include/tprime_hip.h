@@ -324,6 +324,11 @@ int tp_cross_entropy_fwd(const void* logits, const int64_t* labels, float* lse, 
                          float* loss_and_count, int B, int S, int V, int64_t logits_b_stride,
                          int64_t logits_s_stride, int64_t labels_b_stride, int ignore_index, int dtype,
                          void* stream);
+/* The same; the loss is also written to loss[0] (NULL: not). */
+int tp_cross_entropy_fwd_loss(const void* logits, const int64_t* labels, float* lse, float* row_loss,
+                         float* loss_and_count, float* loss, int B, int S, int V, int64_t logits_b_stride,
+                         int64_t logits_s_stride, int64_t labels_b_stride, int ignore_index, int dtype,
+                         void* stream);
 /* dlogits = dloss / count * (softmax(logits) - onehot(label)) on scored rows, 0 elsewhere; dloss (1) fp32 */
 int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float* lse,
                          const float* loss_and_count, const float* dloss, void* dlogits, int B, int S,
@@ -382,7 +387,18 @@ typedef struct tp_linear_problem {
   int m, n;
   void* c;
   int64_t ldc;
+  int c_float; /* 16-bit dtypes: c is float, each value rounded to the dtype first */
 } tp_linear_problem;
+/* ------------------------------------------------------------------------------------------------
+ * Embedding rows and their gradient for small vocabularies (torch_xla_models/model/llama/model.py:311, 340).
+ *   fwd   out[i, :] = table[ids[i], :]; an id outside the table gives a row of NaN
+ *   bwd   dtable[v, :] = sum of dout[i, :] over the i with ids[i] == v, in order, fp32, one rounding; every row of
+ *         dtable is written.  One workgroup per row of the table looks through all ids: for vocab * n up to about 2^24.
+ * Rows are `hidden` elements without gaps; hidden must be even.
+ * ---------------------------------------------------------------------------------------------- */
+int tp_embedding_fwd(const void* table, const int64_t* ids, void* out, int64_t n, int vocab, int hidden, int dtype, void* stream);
+int tp_embedding_bwd(const void* dout, const int64_t* ids, void* dtable, int64_t n, int vocab, int hidden, int dtype, void* stream);
+
 int tp_linears(const tp_linear_problem* problems, int count, int dtype, void* stream);
 
 #ifdef __cplusplus

@@ -73,3 +73,67 @@ def test_frozen_parameters_and_unused_outputs():
   one = torch.autograd.grad(layer.forward_deferred(x, None, position_embeddings=cs)[0], leaves, g)
   both = torch.autograd.grad(layer.forward_deferred(x, None, position_embeddings=cs), leaves, [g, torch.zeros_like(g)])
   assert all(torch.equal(a, b) for a, b in zip(one, both))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_model_ends_equal_the_modules(dtype):
+  """Embedding, final norm + lm_head + .float(): logits and gradients of the model against the same model with hooks on
+  its body and its layers' mlp (the modules' own calls, over the same projection kernels)."""
+  cfg = tpa.Config(vocab_size=136, num_hidden_layers=2, max_position_embeddings=512, hidden_size=256, intermediate_size=64,
+                   num_attention_heads=4, num_key_value_heads=2, hidden_act="silu", initializer_range=0.02, rms_norm_eps=1e-5,
+                   attention_dropout=False, attention_bias=False, rope_theta=500000.0, attention_kernel="splash_attention")  # fmt: skip
+  model = tpa.LlamaForCausalLM(cfg).to(DEV).to(dtype)
+  ids = torch.randint(136, (2, 37), generator=torch.Generator().manual_seed(1)).to(DEV)
+  params = list(model.parameters())
+  logits, loss = model(ids, labels=ids)
+  assert logits.grad_fn.name() == "TprimeLlamaHeadBackward" and logits.dtype == torch.float32
+  got = torch.autograd.grad(loss, params)
+  for m in [model.model] + [layer.mlp for layer in model.model.layers]:
+    m.register_forward_hook(lambda m, a, o: None)
+  want_logits, want_loss = model(ids, labels=ids)
+  assert want_logits.grad_fn.name() == "ToCopyBackward0" or dtype == torch.float32
+  want = torch.autograd.grad(want_loss, params)
+  assert torch.equal(logits, want_logits) and torch.equal(loss, want_loss)
+  for (name, _), a, b in zip(model.named_parameters(), got, want):
+    if "embed" in name:  # (its gradient is the first layer's input gradient: one rounding instead of two, see above)
+      assert (a.double() - b.double()).abs().max() <= 4 * ULP[dtype] * b.double().abs().max()
+    else:
+      assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,vocab,hidden", [(1, 3, 2), (255, 7, 510), (257, 300, 514), (1000, 2, 64)])
+def test_embedding_of_a_small_vocabulary(n, vocab, hidden, dtype):
+  """Rows exactly; the gradient against a float64 scatter: fp32 sums of up to n rows (n 2^-24 relative to the sum of
+  magnitudes) and one rounding, half a unit in the last place: 2^-8 of the value for bfloat16's 8 significant bits, 2^-11
+  for float16, 2^-24 for fp32 (a first version of this bound had halved them once more)."""
+  from torchprime_amd.linear import embed
+
+  m = torch.nn.Embedding(vocab, hidden, device=DEV, dtype=dtype)
+  ids = torch.randint(vocab, (1, n), generator=torch.Generator().manual_seed(n)).to(DEV)
+  out = embed(m, ids)
+  assert out.grad_fn.name() == "TprimeEmbeddingBackward" and torch.equal(out, torch.nn.functional.embedding(ids, m.weight))
+  g = randn(out.shape, 2, dtype).to(DEV)
+  (dw,) = torch.autograd.grad(out, m.weight, g)
+  zero = torch.zeros((vocab, hidden), dtype=torch.float64, device=DEV)
+  ref = zero.index_add(0, ids[0], g[0].double())
+  mag = zero.index_add(0, ids[0], g[0].double().abs())
+  assert ((dw.double() - ref).abs() <= ULP[dtype] * ref.abs() + n * 2.0**-24 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("rows", [1, 3, 63, 65, 1024, 1025])
+@pytest.mark.parametrize("hidden", [8, 72, 1000, 4096])
+def test_norm_backward_of_few_rows(rows, hidden):
+  """Both sides of the line between the one-launch backward and the row-walking one, against float64.  Bound: bfloat16
+  results of fp32 arithmetic on bfloat16 inputs; dw also carries the normalised value's rounding."""
+  x, r, w = randn((rows, hidden), 1, torch.bfloat16), randn((rows, hidden), 2, torch.bfloat16), 1 + randn((hidden,), 3, torch.bfloat16, 0.1)
+  dy, dh = randn((rows, hidden), 4, torch.bfloat16), randn((rows, hidden), 5, torch.bfloat16)
+  xs = [t.to(DEV).requires_grad_(True) for t in (x, r, w)]
+  got = torch.autograd.grad(tpa.ops.add_rmsnorm(*xs, 1e-5), xs, [dy.to(DEV), dh.to(DEV)])
+  h = (x + r).double().requires_grad_(True)
+  wd = w.double().requires_grad_(True)
+  y = wd * (h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5))
+  dxr, dwr = torch.autograd.grad(y, [h, wd], dy.double())
+  for a, b in ((got[0], dxr + dh.double()), (got[1], dxr + dh.double()), (got[2], dwr)):
+    a = a.double().cpu()
+    assert ((a - b).norm() / b.norm()).item() <= 1e-2

@@ -17,7 +17,7 @@ from torch import nn
 from torch.compiler import is_compiling
 
 from .attention import AttentionModule
-from .linear import global_hooks, plain, project, weight_of
+from .linear import embed, global_hooks, plain, project, weight_of
 from .mlp import LlamaMLP
 from .norm import DeepseekV3RMSNorm, LlamaRMSNorm, add_rms_norm
 from .ops import _native
@@ -319,19 +319,22 @@ class LlamaModel(nn.Module):
       causal = causal * attention_mask[:, None, None, :]
     return causal
 
-  def forward(self, input_ids, attention_mask=None):
-    inputs_embeds = self.embed_tokens(input_ids)
+  def deferred(self, input_ids, attention_mask=None):
+    """``(x, residual)`` whose sum the final norm takes (``residual`` None: ``x`` itself)."""
+    inputs_embeds = embed(self.embed_tokens, input_ids)
     seq_length = inputs_embeds.size(1)
-    position_ids = torch.arange(seq_length, device=inputs_embeds.device).unsqueeze(0).float()
+    position_ids = torch.arange(seq_length, device=inputs_embeds.device, dtype=torch.float32).unsqueeze(0)
     causal_mask = self._mask(seq_length, attention_mask, inputs_embeds.device)
     position_embeddings = self.rotary_emb(inputs_embeds, position_ids)
     x, residual = inputs_embeds, None
     for layer in self.layers:
       x, residual = layer.forward_deferred(x, residual, attention_mask=causal_mask, position_ids=position_ids,
                                            position_embeddings=position_embeddings)
-    if residual is None:
-      return self.norm(x)
-    return add_rms_norm(x, residual, self.norm)[0]
+    return x, residual
+
+  def forward(self, input_ids, attention_mask=None):
+    x, residual = self.deferred(input_ids, attention_mask)
+    return self.norm(x) if residual is None else add_rms_norm(x, residual, self.norm)[0]
 
 
 class LlamaForCausalLM(nn.Module):
@@ -354,11 +357,25 @@ class LlamaForCausalLM(nn.Module):
       if getattr(module, "bias", None) is not None:
         module.bias.data.zero_()
 
+  def _logits(self, input_ids, attention_mask):
+    model, head = self.model, None
+    if not is_compiling() and not global_hooks() and plain(model, LlamaModel) and plain(model.norm, LlamaRMSNorm):
+      head = weight_of(self.lm_head)
+    if head is None:
+      return project(model(input_ids=input_ids, attention_mask=attention_mask), self.lm_head)[0].float()
+    x, residual = model.deferred(input_ids, attention_mask)
+    norm = model.norm
+    if residual is not None:  # norm of the sum, lm_head and .float() in one native call where the projection is small
+      logits = _native.llama_head(x, residual, norm.weight, norm.variance_epsilon, head)
+      if logits is not None:
+        return logits
+    hidden_states = norm(x) if residual is None else add_rms_norm(x, residual, norm)[0]
+    return project(hidden_states, self.lm_head)[0].float()
+
   def forward(self, input_ids, labels=None, attention_mask=None):
     from .loss import cross_entropy_loss
 
-    hidden_states = self.model(input_ids=input_ids, attention_mask=attention_mask)
-    logits = project(hidden_states, self.lm_head)[0].float()
+    logits = self._logits(input_ids, attention_mask)
     if labels is None:
       return logits, None
     return logits, cross_entropy_loss(logits, labels=labels, vocab_size=self.config.vocab_size)

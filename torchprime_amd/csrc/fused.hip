@@ -242,8 +242,8 @@ __global__ __launch_bounds__(256) void xent_fwd_kernel(const T* __restrict__ log
 
 // loss = sum(row_loss) / count(valid targets), one block, fixed order; also stores the count for the backward
 __global__ __launch_bounds__(256) void xent_mean_kernel(const float* __restrict__ row_loss, const int64_t* __restrict__ labels,
-                                                        float* __restrict__ out, int B, int S, int V, int64_t lab_b,
-                                                        int ignore_index) {
+                                                        float* __restrict__ out, float* __restrict__ loss, int B, int S, int V,
+                                                        int64_t lab_b, int ignore_index) {
   __shared__ double sl[256];
   __shared__ int sc[256];
   double acc = 0.0;
@@ -270,6 +270,7 @@ __global__ __launch_bounds__(256) void xent_mean_kernel(const float* __restrict_
   if (threadIdx.x == 0) {
     out[0] = (float)(sl[0] / (double)sc[0]);  // no valid target: 0 / 0 = NaN, as CrossEntropyLoss gives
     out[1] = (float)sc[0];
+    if (loss) loss[0] = out[0];
   }
 }
 
@@ -335,6 +336,89 @@ __global__ __launch_bounds__(256) void xent_bwd_kernel(const T* __restrict__ log
     const float x = lab < 0 ? 0.f : Elem<T>::to_f(lr[c]);
     dr[c] = Elem<T>::from_f(lab < 0 ? 0.f : scale * (__expf(x - l) - (c == lab ? 1.f : 0.f)));
   }
+}
+
+// ------------------------------------------------------------------------------------------------
+// embedding of a small vocabulary
+// ------------------------------------------------------------------------------------------------
+// two elements per thread
+template <typename T>
+__global__ __launch_bounds__(256) void embedding_fwd_kernel(const T* __restrict__ table, const int64_t* __restrict__ ids, T* __restrict__ out,
+                                                            int64_t n, int vocab, int hidden) {
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  const int half = hidden / 2;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= n * half) return;
+  const int64_t row = idx / half;
+  const int c = (int)(idx - row * half) * 2;
+  const int64_t id = ids[row];
+  v2 x;
+  if (id >= 0 && id < vocab) x = *(const v2*)(table + id * hidden + c);
+  else x[0] = x[1] = (T)NAN;
+  *(v2*)(out + row * hidden + c) = x;
+}
+// One workgroup per table row and 512 columns: 256 ids at a time, the matching positions collected in order (a ballot per
+// wave), their rows added by all threads.  No atomics and no sort: at a vocabulary of a few hundred the library's sort,
+// zero fill and scatter took 35 us for 512 tokens.
+template <typename T>
+__global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict__ dout, const int64_t* __restrict__ ids, T* __restrict__ dtable,
+                                                            int64_t n, int hidden) {
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  __shared__ int hit[256], wave_hits[4];
+  const int v = blockIdx.x, c = blockIdx.y * 512 + threadIdx.x * 2, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool live = c < hidden;
+  float a0 = 0.f, a1 = 0.f;
+  for (int64_t i0 = 0; i0 < n; i0 += 256) {
+    const int64_t i = i0 + threadIdx.x;
+    const bool mine = i < n && ids[i] == v;
+    const unsigned long long m = __ballot(mine);
+    if (lane == 0) wave_hits[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      before += w < wave ? wave_hits[w] : 0;
+      total += wave_hits[w];
+    }
+    if (mine) hit[before + __popcll(m & ((1ull << lane) - 1ull))] = threadIdx.x;
+    __syncthreads();
+    if (live) {
+      for (int k = 0; k < total; k++) {
+        const v2 x = *(const v2*)(dout + (i0 + hit[k]) * hidden + c);
+        a0 += Elem<T>::to_f(x[0]);
+        a1 += Elem<T>::to_f(x[1]);
+      }
+    }
+    // (the next round's first barrier comes after its ballots: wave_hits must not change before everybody has read it)
+    __syncthreads();
+  }
+  if (live) {
+    v2 o;
+    o[0] = Elem<T>::from_f(a0);
+    o[1] = Elem<T>::from_f(a1);
+    *(v2*)(dtable + (int64_t)v * hidden + c) = o;
+  }
+}
+
+template <typename T>
+static void embedding_launch(bool backward, const void* src, const int64_t* ids, void* dst, int64_t n, int vocab, int hidden, hipStream_t st) {
+  if (backward)
+    embedding_bwd_kernel<T><<<dim3(vocab, (hidden + 511) / 512), dim3(256), 0, st>>>((const T*)src, ids, (T*)dst, n, hidden);
+  else
+    embedding_fwd_kernel<T><<<dim3((unsigned)((n * (hidden / 2) + 255) / 256)), dim3(256), 0, st>>>((const T*)src, ids, (T*)dst, n, vocab, hidden);
+}
+static int embedding_run(bool backward, const void* src, const int64_t* ids, void* dst, int64_t n, int vocab, int hidden, int dtype, void* stream,
+                         const char* name) {
+  TP_REQUIRE(src && ids && dst, TP_ERR_BAD_ARG, "%s: null pointer", name);
+  TP_REQUIRE(n > 0 && vocab > 0 && hidden > 0 && hidden % 2 == 0, TP_ERR_BAD_ARG, "%s: bad shape", name);
+  TP_REQUIRE(((size_t)src | (size_t)dst) % (dtype == TP_F32 ? 8 : 4) == 0, TP_ERR_BAD_ARG, "%s: misaligned pointer", name);
+  TP_REQUIRE((n * (hidden / 2) + 255) / 256 < (1ll << 31) && hidden <= 512 * 65535, TP_ERR_UNSUPPORTED, "%s: too large", name);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == TP_BF16) embedding_launch<bf16_t>(backward, src, ids, dst, n, vocab, hidden, st);
+  else if (dtype == TP_F16) embedding_launch<f16_t>(backward, src, ids, dst, n, vocab, hidden, st);
+  else if (dtype == TP_F32) embedding_launch<float>(backward, src, ids, dst, n, vocab, hidden, st);
+  else TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "%s: dtype %d", name, dtype);
+  return check_launch(name);
 }
 
 }  // namespace tp
@@ -440,7 +524,7 @@ extern "C" int tp_swiglu_bwd(const void* dout, const void* gate, const void* up,
   TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "tp_swiglu_bwd: unsupported dtype %d", dtype);
 }
 
-extern "C" int tp_cross_entropy_fwd(const void* logits, const int64_t* labels, float* lse, float* row_loss, float* loss_and_count,
+extern "C" int tp_cross_entropy_fwd_loss(const void* logits, const int64_t* labels, float* lse, float* row_loss, float* loss_and_count, float* loss,
                                     int B, int S, int V, int64_t logits_b_stride, int64_t logits_s_stride,
                                     int64_t labels_b_stride, int ignore_index, int dtype, void* stream) {
   TP_REQUIRE(logits && labels && lse && row_loss && loss_and_count, TP_ERR_BAD_ARG, "tp_cross_entropy_fwd: null pointer");
@@ -453,8 +537,15 @@ extern "C" int tp_cross_entropy_fwd(const void* logits, const int64_t* labels, f
     xent_fwd_kernel<bf16_t><<<grid, block, 0, st>>>((const bf16_t*)logits, labels, lse, row_loss, S, V, logits_b_stride, logits_s_stride, labels_b_stride, ignore_index);
   else
     TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "tp_cross_entropy_fwd: dtype %d (fp32 and bf16 logits only)", dtype);
-  xent_mean_kernel<<<dim3(1), block, 0, st>>>(row_loss, labels, loss_and_count, B, S, V, labels_b_stride, ignore_index);
+  xent_mean_kernel<<<dim3(1), block, 0, st>>>(row_loss, labels, loss_and_count, loss, B, S, V, labels_b_stride, ignore_index);
   return check_launch("tp_cross_entropy_fwd");
+}
+
+extern "C" int tp_cross_entropy_fwd(const void* logits, const int64_t* labels, float* lse, float* row_loss, float* loss_and_count,
+                                    int B, int S, int V, int64_t logits_b_stride, int64_t logits_s_stride,
+                                    int64_t labels_b_stride, int ignore_index, int dtype, void* stream) {
+  return tp_cross_entropy_fwd_loss(logits, labels, lse, row_loss, loss_and_count, nullptr, B, S, V, logits_b_stride, logits_s_stride,
+                                   labels_b_stride, ignore_index, dtype, stream);
 }
 
 extern "C" int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float* lse, const float* loss_and_count,
@@ -476,4 +567,11 @@ extern "C" int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, c
   else
     TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "tp_cross_entropy_bwd: dtype %d (fp32 and bf16 logits only)", dtype);
   return check_launch("tp_cross_entropy_bwd");
+}
+
+extern "C" int tp_embedding_fwd(const void* table, const int64_t* ids, void* out, int64_t n, int vocab, int hidden, int dtype, void* stream) {
+  return embedding_run(false, table, ids, out, n, vocab, hidden, dtype, stream, "tp_embedding_fwd");
+}
+extern "C" int tp_embedding_bwd(const void* dout, const int64_t* ids, void* dtable, int64_t n, int vocab, int hidden, int dtype, void* stream) {
+  return embedding_run(true, dout, ids, dtable, n, vocab, hidden, dtype, stream, "tp_embedding_bwd");
 }

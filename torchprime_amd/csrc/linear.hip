@@ -30,9 +30,23 @@ struct LinSeg { const void* a; const void* b; int k, lda, ldb; };
 struct LinProb {
   LinSeg seg[LIN_SEGS];
   void* c;
-  int m, n, ldc, nseg, a_kmajor, b_kmajor, tiles_n, tile_end;  // tile_end: one past its last tile in the launch
+  int m, n, ldc, nseg, a_kmajor, b_kmajor, c_float, tiles_n, tile_end;  // tile_end: one past its last tile in the launch
 };
 struct LinArgs { LinProb p[LIN_MAX]; };
+
+// four consecutive values of a row of c; c_float: rounded to the element type, stored as fp32 (a projection followed by
+// .float(), without the pass in between)
+template <typename E>
+__device__ __forceinline__ void lin_store(const LinProb& p, int m, int n, float x0, float x1, float x2, float x3) {
+  if (n >= p.n) return;
+  const int64_t at = (int64_t)m * p.ldc + n;
+  if constexpr (sizeof(E) == 2) {
+    if (p.c_float) *(f32x4*)((float*)p.c + at) = f32x4{round_to<E>(x0), round_to<E>(x1), round_to<E>(x2), round_to<E>(x3)};
+    else *(u32x2*)((E*)p.c + at) = pack4<E>(x0, x1, x2, x3);
+  } else {
+    *(f32x4*)((float*)p.c + at) = f32x4{x0, x1, x2, x3};
+  }
+}
 
 // One operand's LDS tile of a step, 8 KB: its loads and its fragments.  E: element type; KM: rows hold the contraction.
 //   KM:   64 rows (m or n) x 128 bytes of k, chunks of 16 bytes XOR-swizzled by the row (DmaTile)
@@ -164,15 +178,8 @@ __device__ __forceinline__ void linear_tile(const LinProb& p, int tile, unsigned
   // lane: row m, four consecutive n per group of values
   const int m = m0 + wm + (lane & 31), g = lane >> 5;
   if (m < p.m) {
-    E* c = (E*)p.c + (int64_t)m * p.ldc;
 #pragma unroll
-    for (int vq = 0; vq < 4; vq++) {
-      const int n = n0 + wn + 8 * vq + 4 * g;
-      if (n < p.n) {
-        if constexpr (sizeof(E) == 2) *(u32x2*)(c + n) = pack4<E>(acc[4 * vq], acc[4 * vq + 1], acc[4 * vq + 2], acc[4 * vq + 3]);
-        else *(f32x4*)(c + n) = f32x4{acc[4 * vq], acc[4 * vq + 1], acc[4 * vq + 2], acc[4 * vq + 3]};
-      }
-    }
+    for (int vq = 0; vq < 4; vq++) lin_store<E>(p, m, n0 + wn + 8 * vq + 4 * g, acc[4 * vq], acc[4 * vq + 1], acc[4 * vq + 2], acc[4 * vq + 3]);
   }
 }
 
@@ -316,15 +323,8 @@ __device__ __forceinline__ void linear_tile_split(const LinProb& p, int tile, un
   sum_waves(acc, (float*)smem, wave_s, lane);
   const int m = m0 + (lane & 31), g = lane >> 5;
   if (wave_s == 0 && m < p.m) {
-    E* c = (E*)p.c + (int64_t)m * p.ldc;
 #pragma unroll
-    for (int vq = 0; vq < 4; vq++) {
-      const int n = n0 + 8 * vq + 4 * g;
-      if (n < p.n) {
-        if constexpr (sizeof(E) == 2) *(u32x2*)(c + n) = pack4<E>(acc[0][4 * vq], acc[0][4 * vq + 1], acc[0][4 * vq + 2], acc[0][4 * vq + 3]);
-        else *(f32x4*)(c + n) = f32x4{acc[0][4 * vq], acc[0][4 * vq + 1], acc[0][4 * vq + 2], acc[0][4 * vq + 3]};
-      }
-    }
+    for (int vq = 0; vq < 4; vq++) lin_store<E>(p, m, n0 + 8 * vq + 4 * g, acc[0][4 * vq], acc[0][4 * vq + 1], acc[0][4 * vq + 2], acc[0][4 * vq + 3]);
   }
 }
 
@@ -389,7 +389,7 @@ extern "C" int tp_linears(const tp_linear_problem* problems, int count_, int dty
       d.seg[j] = LinSeg{s.a[j], s.b[j], (int)k, (int)lda, (int)ldb};
     }
     for (int j = s.segments; j < LIN_SEGS; j++) d.seg[j] = d.seg[0];
-    d.c = s.c; d.m = s.m; d.n = s.n; d.ldc = (int)s.ldc; d.nseg = s.segments; d.a_kmajor = s.a_kmajor != 0; d.b_kmajor = s.b_kmajor != 0;
+    d.c = s.c; d.m = s.m; d.n = s.n; d.ldc = (int)s.ldc; d.nseg = s.segments; d.a_kmajor = s.a_kmajor != 0; d.b_kmajor = s.b_kmajor != 0; d.c_float = s.c_float != 0;
     d.tiles_n = (s.n + edge - 1) / edge;
     tiles += (int64_t)((s.m + edge - 1) / edge) * d.tiles_n;
     TP_REQUIRE(tiles < (1ll << 30), TP_ERR_UNSUPPORTED, "tp_linears: too many tiles");

@@ -809,11 +809,12 @@ T3 cross_entropy_fwd_cuda(const Tensor& logits_, const Tensor& labels_, int64_t 
   c10::DeviceGuard guard(dev);
   const int64_t B = logits_.size(0), S = logits_.size(1), V = logits_.size(2);
   const Tensor logits = logits_.stride(2) != 1 ? logits_.contiguous() : logits_, labels = prep_labels(labels_);
-  Tensor lse = empty_f32({B * S}, logits), row_loss = empty_f32({B * S}, logits), lc = empty_f32({2}, logits);
-  check(tp_cross_entropy_fwd(logits.data_ptr(), (const int64_t*)labels.data_ptr(), (float*)lse.data_ptr(), (float*)row_loss.data_ptr(),
-                             (float*)lc.data_ptr(), (int)B, (int)S, (int)V, logits.stride(0), logits.stride(1), labels.stride(0),
-                             (int)ignore_index, dtype_code(logits.scalar_type()), stream_of(dev)), "tp_cross_entropy_fwd");
-  return {lc.select(0, 0).clone(), lse, lc};
+  Tensor lse = empty_f32({B * S}, logits), row_loss = empty_f32({B * S}, logits), lc = empty_f32({2}, logits), loss = empty_f32({}, logits);
+  check(tp_cross_entropy_fwd_loss(logits.data_ptr(), (const int64_t*)labels.data_ptr(), (float*)lse.data_ptr(), (float*)row_loss.data_ptr(),
+                                  (float*)lc.data_ptr(), (float*)loss.data_ptr(), (int)B, (int)S, (int)V, logits.stride(0), logits.stride(1),
+                                  labels.stride(0), (int)ignore_index, dtype_code(logits.scalar_type()), stream_of(dev)),
+        "tp_cross_entropy_fwd_loss");
+  return {loss, lse, lc};
 }
 Tensor cross_entropy_bwd_cuda(const Tensor& dloss, const Tensor& logits_, const Tensor& labels_, const Tensor& lse, const Tensor& lc,
                               int64_t ignore_index) {
@@ -1242,6 +1243,143 @@ std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const s
   return {out, h2};
 }
 
+// ---- the two ends of a small model ---------------------------------------------------------------------------------
+// Embedding rows: the library's where the vocabulary or the batch is not small, or anything but plain tensors is involved.
+struct EmbeddingNode : torch::autograd::Node {
+  SavedVariable ids;
+  int64_t vocab, hidden;
+  at::TensorOptions opts;
+  std::string name() const override { return "TprimeEmbeddingBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    ids.reset_data();
+  }
+  variable_list apply(variable_list&& g) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (!g[0].defined()) return {Tensor()};
+    const Tensor i = ids.unpack();
+    if (at::GradMode::is_enabled() || !plain_eager(g[0])) return {at::embedding_dense_backward(g[0], i, vocab, -1, false)};
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::DeviceGuard guard(i.device());
+    const Tensor dy = g[0].to(opts.dtype().toScalarType()).contiguous();
+    Tensor dt = at::empty({vocab, hidden}, opts);
+    check(tp_embedding_bwd(dy.data_ptr(), (const int64_t*)i.data_ptr(), dt.data_ptr(), i.numel(), (int)vocab, (int)hidden,
+                           dtype_code(dt.scalar_type()), stream_of(i.device())), "tp_embedding_bwd");
+    return {dt};
+  }
+};
+Tensor py_embedding(const Tensor& ids, const Tensor& table) {
+  const auto t = table.scalar_type();
+  const bool small = plain_eager(table) && plain_eager(ids) && ids.device() == table.device() && table.dim() == 2 && table.is_contiguous() &&
+                     (t == at::kBFloat16 || t == at::kHalf || t == at::kFloat) && ids.scalar_type() == at::kLong && ids.numel() > 0 &&
+                     table.size(0) > 0 && table.size(1) > 0 && table.size(1) % 2 == 0 && table.size(0) * ids.numel() <= (1ll << 24) &&
+                     ids.numel() * table.size(1) <= (1ll << 24) && !torch::autograd::isFwGradDefined(table);
+  if (!small) return at::embedding(table, ids);
+  auto node = make_node<EmbeddingNode>(table);
+  Tensor out;
+  const Tensor i = ids.contiguous();
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::DeviceGuard guard(table.device());
+    auto sizes = ids.sizes().vec();
+    sizes.push_back(table.size(1));
+    out = at::empty(sizes, table.options());
+    check(tp_embedding_fwd(table.data_ptr(), (const int64_t*)i.data_ptr(), out.data_ptr(), i.numel(), (int)table.size(0), (int)table.size(1),
+                           dtype_code(t), stream_of(table.device())), "tp_embedding_fwd");
+  }
+  if (node) {
+    torch::autograd::set_history(out, node);
+    node->ids = SavedVariable(i, false);
+    node->vocab = table.size(0);
+    node->hidden = table.size(1);
+    node->opts = table.options();
+  }
+  return out;
+}
+
+// final add + norm, lm_head, .float(): fp32 logits rounded through the model's type.  An undefined tensor where the
+// projection is one for the library.
+struct HeadNode : torch::autograd::Node {
+  SavedVariable h, n, rstd, norm_w, lm_w;
+  std::string name() const override { return "TprimeLlamaHeadBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto* v : {&h, &n, &rstd, &norm_w, &lm_w}) v->reset_data();
+  }
+  variable_list apply(variable_list&& g) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    TORCH_CHECK_NOT_IMPLEMENTED(!at::GradMode::is_enabled(), "derivative for a model head's backward is not implemented");
+    variable_list out(4);  // x, residual, norm weight, lm_head weight
+    if (!g[0].defined()) return out;
+    const Tensor H = h.unpack(), N = n.unpack(), R = rstd.unpack(), nw = norm_w.unpack(), lw = lm_w.unpack();
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::DeviceGuard guard(H.device());
+    void* st = stream_of(H.device());
+    const int64_t k = H.size(-1), rows = H.numel() / k, V = lw.size(0);
+    const int code = dtype_code(H.scalar_type());
+    const Tensor go = g[0].to(H.scalar_type()).contiguous();
+    const bool dx = task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2);
+    Tensor dn;
+    std::array<tp_linear_problem, 2> p;
+    int c = 0;
+    if (dx) {
+      dn = at::empty(H.sizes(), H.options());
+      p[c++] = raw_linear(go.data_ptr(), V, lw.data_ptr(), k, V, true, false, rows, k, dn.data_ptr());
+    }
+    if (task_should_compute_output(3)) {
+      out[3] = at::empty(lw.sizes(), lw.options());
+      p[c++] = raw_linear(go.data_ptr(), V, N.data_ptr(), k, rows, false, false, V, k, out[3].data_ptr());
+    }
+    if (c) check(tp_linears(p.data(), c, code, st), "tp_linears");
+    if (dx) {
+      const Tensor ws = empty_f32({(int64_t)tp_rmsnorm_bwd_workspace_bytes(rows, (int)k) / 4}, H);
+      out[0] = at::empty(H.sizes(), H.options());
+      out[2] = at::empty(nw.sizes(), nw.options());
+      check(tp_rmsnorm_bwd(dn.data_ptr(), H.data_ptr(), nw.data_ptr(), (const float*)R.data_ptr(), out[0].data_ptr(), out[2].data_ptr(),
+                           (float*)ws.data_ptr(), rows, (int)k, k, k, k, code, code, st), "tp_rmsnorm_bwd");
+      out[1] = out[0];
+    }
+    return out;
+  }
+};
+std::optional<Tensor> py_llama_head(const Tensor& x, const Tensor& residual, const Tensor& norm_w, double eps, const Tensor& lm_w) {
+  const auto dt = x.scalar_type();
+  if (!linears_take(x, {lm_w}) || !x.is_contiguous() || !residual.is_contiguous() || residual.sizes() != x.sizes() || residual.scalar_type() != dt ||
+      !plain_eager(residual) || residual.device() != x.device() || norm_w.dim() != 1 || norm_w.size(0) != x.size(-1) || norm_w.scalar_type() != dt ||
+      !norm_w.is_contiguous() || !plain_eager(norm_w) || norm_w.device() != x.device()) return std::nullopt;
+  for (const Tensor* t : {&x, &residual})
+    if (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16) return std::nullopt;
+  auto node = make_node<HeadNode>(x, residual, norm_w, lm_w);
+  Tensor h, n, rstd, logits;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    c10::DeviceGuard guard(x.device());
+    void* st = stream_of(x.device());
+    const int64_t k = x.size(-1), rows = x.numel() / k, V = lm_w.size(0);
+    const int code = dtype_code(dt);
+    h = at::empty(x.sizes(), x.options());
+    n = at::empty(x.sizes(), x.options());
+    rstd = empty_f32({rows}, x);
+    auto sizes = x.sizes().vec();
+    sizes.back() = V;
+    logits = empty_f32(sizes, x);
+    check(tp_add_rmsnorm_fwd(x.data_ptr(), residual.data_ptr(), norm_w.data_ptr(), h.data_ptr(), n.data_ptr(), (float*)rstd.data_ptr(), rows, (int)k,
+                             k, k, k, k, (float)eps, code, code, st), "tp_add_rmsnorm_fwd");
+    tp_linear_problem p = raw_linear(n.data_ptr(), k, lm_w.data_ptr(), k, k, true, true, rows, V, logits.data_ptr());
+    p.c_float = 1;
+    check(tp_linears(&p, 1, code, st), "tp_linears");
+  }
+  if (node) {
+    torch::autograd::set_history(logits, node);
+    node->h = SavedVariable(h, false);
+    node->n = SavedVariable(n, false);
+    node->rstd = SavedVariable(rstd, false);
+    node->norm_w = SavedVariable(norm_w, false);
+    node->lm_w = SavedVariable(lm_w, false);
+  }
+  return logits;
+}
+
 // ---- Python entry points -----------------------------------------------------------------------------------------
 // What the Python functions of ops.py call: the GPU check with its own message, then the operator.
 Tensor py_rmsnorm(const Tensor& x, const Tensor& w, double eps) { require_gpu(x, w); return std::get<0>(op_rmsnorm_fwd()(x, w, eps)); }
@@ -1366,6 +1504,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
   m.def("linears", &py_linears);
   m.def("llama_layer", &py_llama_layer);
+  m.def("llama_head", &py_llama_head);
+  m.def("embedding", &py_embedding);
   m.def("l2norm", &py_l2norm);
   m.def("swiglu", &py_swiglu);
   m.def("cross_entropy", &py_cross_entropy);

@@ -1,4 +1,4 @@
-"""Projections of one input through several ``nn.Linear`` modules (q, k, v; gate, up), as one call.
+"""Projections of one input through several ``nn.Linear`` modules (q, k, v; gate, up), as one call, and embedding lookups.
 
 Small ones run as one HIP launch forward and one backward (``csrc/linear.hip``), large ones as the modules' own GEMMs;
 the modules and their parameters stay what they are."""
@@ -44,3 +44,12 @@ def project(x: torch.Tensor, *modules: nn.Module) -> list[torch.Tensor]:
     if all(w is not None for w in ws):
       return _native.linears(x, ws)
   return [m(x) for m in modules]
+
+
+def embed(module: nn.Module, ids: torch.Tensor) -> torch.Tensor:
+  """``module(ids)`` of an ``nn.Embedding``."""
+  if not is_compiling() and plain(module, nn.Embedding) and not global_hooks():
+    d = module.__dict__
+    if d["padding_idx"] is None and d["max_norm"] is None and not d["scale_grad_by_freq"] and not d["sparse"]:
+      return _native.embedding(ids, d["_parameters"]["weight"])
+  return module(ids)
