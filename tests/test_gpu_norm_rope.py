@@ -129,6 +129,27 @@ def test_rope_apply_backward():
   assert_close(kd.grad, k64.grad, "dk", scale_abs=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("interleave", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(2, 5, 1, 67, 64), (1, 4, 2, 33, 128), (1, 3, 3, 129, 96)])
+def test_rope_whole_and_partial_lines(B, Hq, Hkv, S, D, interleave, dtype):
+  """Heads whose halves are whole 128-byte lines, and those where they are not, in both orders: the same bits as the eager
+  expression forward; the backward is the transposed rotation."""
+  q, k, cos, sin = _rope_inputs(B, Hq, Hkv, S, D, dtype)
+  mine, eager = ((tpa.apply_rotary_pos_emb_interleave, orc.apply_rotary_pos_emb_interleave) if interleave
+                 else (tpa.apply_rotary_pos_emb, orc.apply_rotary_pos_emb))  # fmt: skip
+  qd, kd = q.to(DEV).requires_grad_(True), k.to(DEV).requires_grad_(True)
+  qo, ko = mine(qd, kd, cos.to(DEV), sin.to(DEV))
+  qr, kr = eager(q, k, cos, sin)
+  assert torch.equal(qo.cpu(), qr) and torch.equal(ko.cpu(), kr)
+  gq, gk = randn(q.shape, 33, dtype), randn(k.shape, 34, dtype)
+  torch.autograd.backward((qo, ko), (gq.to(DEV), gk.to(DEV)))
+  q64, k64 = q.double().requires_grad_(True), k.double().requires_grad_(True)
+  torch.autograd.backward(eager(q64, k64, cos.double(), sin.double()), (gq.double(), gk.double()))
+  assert_close(qd.grad, q64.grad, "dq", scale_abs=True)
+  assert_close(kd.grad, k64.grad, "dk", scale_abs=True)
+
+
 def test_rope_interleave_deepseek_layout():
   # q_rot (B,128,S,64) is the tail of a 192-wide head; k_rot (B,1,S,64) the tail of the 576-wide latent
   B, S = 1, 200

@@ -79,7 +79,24 @@ struct RopeArgs {
 // [x0,x1,x2,...] -> [evens | odds] and the output stays in that order (DeepSeek).  MODE 2: adjacent pairs
 // (x[2i], x[2i+1]) are rotated by angle i and written back in place, using the first half of the cos/sin row for both
 // members of a pair (Llama-4 apply_rotary_emb, model/llama4/model.py:364-409).
-template <typename T, int MODE, bool BACKWARD, bool WIDE>
+// LINES: what a wave's instruction touches are whole 128-byte lines (a half of a head is a multiple of one and the two
+// chunks of a thread lie in different halves).  Only then are the accesses non-temporal; where two instructions share a
+// line (heads of 64 in 16 bits, or interleaved pairs, whose chunks are neighbours) the caches have to hold it from one to
+// the other.  us, non-temporal : cached, forward | backward, bf16:
+//   interleaved, 128 + 1 heads of 64:  4096 tokens 28.8 : 25.9 | 33.6 : 26.0;  32768 tokens 214 : 188 | 260 : 189
+//   rotate-half, 8 + 8 heads of 64, 32768 tokens 29.2 : 25.5 | 29.8 : 25.0;  32 + 8 heads of 128, 8192 tokens 27.9 : 30.2 |
+//   28.2 : 30.6,  32768 tokens 104.8 : 113.5 | 104.3 : 113.5
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void rope_load(const T* p, float (&out)[N]) {
+  if constexpr (NT) load_f_nt<T, N>(p, out);
+  else load_f<T, N>(p, out);
+}
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void rope_store(T* p, const float (&in)[N]) {
+  if constexpr (NT) store_f_nt<T, N>(p, in);
+  else store_f<T, N>(p, in);
+}
+template <typename T, int MODE, bool BACKWARD, bool WIDE, bool LINES>
 __global__ __launch_bounds__(256) void rope_apply_kernel(RopeArgs a) {
   constexpr bool LOAD_PAIRS = MODE == 1 && !BACKWARD;   // de-interleave while loading
   constexpr bool STORE_PAIRS = MODE == 1 && BACKWARD;   // re-interleave while storing
@@ -123,7 +140,7 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(RopeArgs a) {
     for (int ch = 0; ch < 2; ch++) {
       const int eoff = ch * half + j * E, poff = ch * (half / 2) + j * P;
       float v[E], c[P], sn[P], o[E];
-      load_f_nt<T, E>(xp + eoff, v);
+      rope_load<T, E, LINES>(xp + eoff, v);
       load_f<T, P>(cp + poff, c);
       load_f<T, P>(sp + poff, sn);
 #pragma unroll
@@ -137,7 +154,7 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(RopeArgs a) {
           o[2 * e + 1] = round_to<T>(y * c[e]) + round_to<T>(-x * sn[e]);
         }
       }
-      store_f_nt<T, E>(yp + eoff, o);
+      rope_store<T, E, LINES>(yp + eoff, o);
     }
     return;
   }
@@ -149,13 +166,13 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(RopeArgs a) {
 
   float x1[E], x2[E], o1[E], o2[E];
   if (!LOAD_PAIRS) {
-    load_f_nt<T, E>(xp + j * E, x1);
-    load_f_nt<T, E>(xp + half + j * E, x2);
+    rope_load<T, E, LINES>(xp + j * E, x1);
+    rope_load<T, E, LINES>(xp + half + j * E, x2);
   } else {
     // permuted input: first-half element i is x[2i], second-half element i is x[2i+1]
     float lo[E], hi[E];
-    load_f_nt<T, E>(xp + 2 * j * E, lo);
-    load_f_nt<T, E>(xp + 2 * j * E + E, hi);
+    rope_load<T, E, LINES>(xp + 2 * j * E, lo);
+    rope_load<T, E, LINES>(xp + 2 * j * E + E, hi);
 #pragma unroll
     for (int e = 0; e < E / 2; e++) {
       x1[e] = lo[2 * e];
@@ -178,8 +195,8 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(RopeArgs a) {
     }
   }
   if (!STORE_PAIRS) {
-    store_f_nt<T, E>(yp + j * E, o1);
-    store_f_nt<T, E>(yp + half + j * E, o2);
+    rope_store<T, E, LINES>(yp + j * E, o1);
+    rope_store<T, E, LINES>(yp + half + j * E, o2);
   } else {
     // inverse permutation: dx[2i] = d_first[i], dx[2i+1] = d_second[i]
     float lo[E], hi[E];
@@ -190,20 +207,20 @@ __global__ __launch_bounds__(256) void rope_apply_kernel(RopeArgs a) {
       hi[2 * e] = o1[E / 2 + e];
       hi[2 * e + 1] = o2[E / 2 + e];
     }
-    store_f_nt<T, E>(yp + 2 * j * E, lo);
-    store_f_nt<T, E>(yp + 2 * j * E + E, hi);
+    rope_store<T, E, LINES>(yp + 2 * j * E, lo);
+    rope_store<T, E, LINES>(yp + 2 * j * E + E, hi);
   }
 }
 
-template <typename T, bool WIDE>
+template <typename T, bool WIDE, bool LINES>
 static void rope_launch(const RopeArgs& a, int interleaved, int backward, dim3 grid, hipStream_t st) {
   const dim3 block(256);
-  if (interleaved == 0 && !backward) rope_apply_kernel<T, 0, false, WIDE><<<grid, block, 0, st>>>(a);
-  else if (interleaved == 0 && backward) rope_apply_kernel<T, 0, true, WIDE><<<grid, block, 0, st>>>(a);
-  else if (interleaved == 1 && !backward) rope_apply_kernel<T, 1, false, WIDE><<<grid, block, 0, st>>>(a);
-  else if (interleaved == 1 && backward) rope_apply_kernel<T, 1, true, WIDE><<<grid, block, 0, st>>>(a);
-  else if (!backward) rope_apply_kernel<T, 2, false, WIDE><<<grid, block, 0, st>>>(a);
-  else rope_apply_kernel<T, 2, true, WIDE><<<grid, block, 0, st>>>(a);
+  if (interleaved == 0 && !backward) rope_apply_kernel<T, 0, false, WIDE, LINES><<<grid, block, 0, st>>>(a);
+  else if (interleaved == 0 && backward) rope_apply_kernel<T, 0, true, WIDE, LINES><<<grid, block, 0, st>>>(a);
+  else if (interleaved == 1 && !backward) rope_apply_kernel<T, 1, false, WIDE, false><<<grid, block, 0, st>>>(a);
+  else if (interleaved == 1 && backward) rope_apply_kernel<T, 1, true, WIDE, false><<<grid, block, 0, st>>>(a);
+  else if (!backward) rope_apply_kernel<T, 2, false, WIDE, LINES><<<grid, block, 0, st>>>(a);
+  else rope_apply_kernel<T, 2, true, WIDE, LINES><<<grid, block, 0, st>>>(a);
 }
 
 template <typename T>
@@ -227,8 +244,11 @@ static int rope_typed(RopeArgs& a, int interleaved, int backward, hipStream_t st
   for (int w = 0; w < 2 && narrow; w++)
     narrow = a.H[w] * a.xs[w][1] + a.S * a.xs[w][2] < lim && a.H[w] * a.ys[w][1] + a.S * a.ys[w][2] < lim;
   const dim3 grid(nb0 + nb1, (unsigned)a.B);
-  if (narrow) rope_launch<T, false>(a, interleaved, backward, grid, st);
-  else rope_launch<T, true>(a, interleaved, backward, grid, st);
+  const bool lines = a.D / 2 * sizeof(T) % 128 == 0;
+  if (narrow && lines) rope_launch<T, false, true>(a, interleaved, backward, grid, st);
+  else if (narrow) rope_launch<T, false, false>(a, interleaved, backward, grid, st);
+  else if (lines) rope_launch<T, true, true>(a, interleaved, backward, grid, st);
+  else rope_launch<T, true, false>(a, interleaved, backward, grid, st);
   return check_launch("tp_rope_apply");
 }
 
