@@ -324,10 +324,11 @@ int tp_cross_entropy_fwd(const void* logits, const int64_t* labels, float* lse, 
                          float* loss_and_count, int B, int S, int V, int64_t logits_b_stride,
                          int64_t logits_s_stride, int64_t labels_b_stride, int ignore_index, int dtype,
                          void* stream);
-/* The same; the loss is also written to loss[0] (NULL: not). */
+/* The same; the loss is also written to loss[0] (NULL: not).  With scored_only the rows without a target are not read:
+ * their lse is 0. */
 int tp_cross_entropy_fwd_loss(const void* logits, const int64_t* labels, float* lse, float* row_loss,
                          float* loss_and_count, float* loss, int B, int S, int V, int64_t logits_b_stride,
-                         int64_t logits_s_stride, int64_t labels_b_stride, int ignore_index, int dtype,
+                         int64_t logits_s_stride, int64_t labels_b_stride, int ignore_index, int scored_only, int dtype,
                          void* stream);
 /* dlogits = dloss / count * (softmax(logits) - onehot(label)) on scored rows, 0 elsewhere; dloss (1) fp32 */
 int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float* lse,

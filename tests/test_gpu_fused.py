@@ -199,3 +199,36 @@ def test_cross_entropy_with_a_masked_vocabulary_range(dtype):
   assert ld.grad[:, :, :2100].abs().max().item() == 0 and ld.grad[:, :, 3000:3300].abs().max().item() == 0
   assert_close(ld.grad, l64.grad, "dlogits", max_abs=1e-7 if dtype == torch.float32 else 1e-4, rel_l2=1e-5 if dtype == torch.float32 else 5e-3)
 
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [5, 2044, 2048, 2052, 4097])
+def test_cross_entropy_rows_without_a_target(V, dtype):
+  """Rows without a target (a prompt, labels outside the vocabulary, the last position) are not read: NaN there reaches
+  neither the loss nor the gradient, which is 0 on them.  The operator itself still gives every row's LSE unless it is told
+  otherwise.  V: around one block's vectors of the backward (512 of 16 bytes)."""
+  B, S = 2, 11
+  logits = randn((B, S, V), 81, dtype, 3.0)
+  labels = torch.randint(0, V, (B, S), generator=torch.Generator().manual_seed(82))
+  labels[0, :6] = -100
+  labels[1, 4] = V
+  scored = torch.zeros((B, S), dtype=torch.bool)
+  scored[:, :-1] = (labels[:, 1:] >= 0) & (labels[:, 1:] < V)
+  l64 = logits.double().requires_grad_(True)
+  rows = (torch.logsumexp(l64, -1)[:, :-1] - l64[:, :-1].gather(-1, labels[:, 1:].clamp(0, V - 1)[..., None])[..., 0])[scored[:, :-1]]
+  ref = rows.mean()
+  ref.backward()
+
+  lse = tpa.ops.cross_entropy_fwd(logits.to(DEV), labels.to(DEV), -100)[1].view(B, S).cpu().double()
+  want = torch.logsumexp(logits.double(), -1)
+  assert (lse - want).abs().max().item() <= 2e-6 * want.abs().max().item()  # fp32: a few roundings of the sum and the log
+  few = tpa.ops.cross_entropy_fwd(logits.to(DEV), labels.to(DEV), -100, True)[1].view(B, S).cpu().double()
+  assert torch.equal(few[scored], lse[scored]) and few[~scored].abs().max().item() == 0
+
+  ld = torch.where(scored[..., None], logits, float("nan")).to(dtype).to(DEV).requires_grad_(True)
+  loss = tpa.cross_entropy_loss(ld, labels.to(DEV), V)
+  loss.backward()
+  assert abs(loss.item() - ref.item()) <= 2e-6 * max(1.0, abs(ref.item()))
+  assert ld.grad.cpu()[~scored].abs().max().item() == 0
+  bounds = dict(max_abs=1e-6, rel_l2=1e-5) if dtype == torch.float32 else dict(max_abs=1e-3, rel_l2=5e-3)
+  assert_close(ld.grad, l64.grad, "dlogits", **bounds)

@@ -51,7 +51,7 @@ SIGNATURES = {
   "tp_swiglu_fwd": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_int64, c_int64, c_int64, c_int, c_void_p]),
   "tp_swiglu_bwd": (c_int, [c_void_p] * 5 + [c_int64, c_int] + [c_int64] * 5 + [c_int, c_void_p]),
   "tp_cross_entropy_fwd": (c_int, [c_void_p] * 5 + [c_int] * 3 + [c_int64] * 3 + [c_int, c_int, c_void_p]),
-  "tp_cross_entropy_fwd_loss": (c_int, [c_void_p] * 6 + [c_int] * 3 + [c_int64] * 3 + [c_int, c_int, c_void_p]),
+  "tp_cross_entropy_fwd_loss": (c_int, [c_void_p] * 6 + [c_int] * 3 + [c_int64] * 3 + [c_int, c_int, c_int, c_void_p]),
   "tp_embedding_fwd": (c_int, [c_void_p] * 3 + [c_int64] + [c_int] * 3 + [c_void_p]),
   "tp_embedding_bwd": (c_int, [c_void_p] * 3 + [c_int64] + [c_int] * 3 + [c_void_p]),
   "tp_cross_entropy_bwd": (c_int, [c_void_p] * 6 + [c_int] * 3 + [c_int64] * 5 + [c_int, c_int, c_void_p]),

@@ -178,12 +178,23 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(const T* __restrict__ d
 template <typename T>
 __global__ __launch_bounds__(256) void xent_fwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ labels,
                                                        float* __restrict__ lse, float* __restrict__ row_loss, int S, int V,
-                                                       int64_t ls_b, int64_t ls_s, int64_t lab_b, int ignore_index) {
+                                                       int64_t ls_b, int64_t ls_s, int64_t lab_b, int ignore_index, int scored_only) {
   constexpr int E = 16 / sizeof(T);
   __shared__ float sm[256], ss[256];
   const int row = blockIdx.x;
   const int b = row / S, s = row - b * S;
   const T* lr = logits + b * ls_b + s * ls_s;
+  int64_t lab = -1;
+  if (s < S - 1) {
+    lab = labels[b * lab_b + s + 1];
+    if (lab == ignore_index || lab < 0 || lab >= V) lab = -1;
+  }
+  // a row without a target (a prompt, padding, the last position) is not read where nobody asks for its LSE: the loss and
+  // its gradient use none.  4096 rows of 128256 in fp32, an eighth of them a prompt: 325 -> 285 us
+  if (scored_only && lab < 0) {
+    if (threadIdx.x == 0) lse[row] = row_loss[row] = 0.f;
+    return;
+  }
   float m = -INFINITY, acc = 0.f;
   const int nvec = V / E;
   const bool vec = (((size_t)lr) & 15) == 0;
@@ -231,25 +242,22 @@ __global__ __launch_bounds__(256) void xent_fwd_kernel(const T* __restrict__ log
   if (threadIdx.x == 0) {
     const float l = sm[0] + logf(ss[0]);
     lse[row] = l;
-    float loss = 0.f;
-    if (s < S - 1) {
-      const int64_t lab = labels[b * lab_b + s + 1];
-      if (lab != ignore_index && lab >= 0 && lab < V) loss = l - Elem<T>::to_f(lr[lab]);
-    }
-    row_loss[row] = loss;
+    row_loss[row] = lab < 0 ? 0.f : l - Elem<T>::to_f(lr[lab]);
   }
 }
 
-// loss = sum(row_loss) / count(valid targets), one block, fixed order; also stores the count for the backward
-__global__ __launch_bounds__(256) void xent_mean_kernel(const float* __restrict__ row_loss, const int64_t* __restrict__ labels,
+// loss = sum(row_loss) / count(valid targets), one block, fixed order; also stores the count for the backward (a thread for
+// every few rows: with 256 threads the chain of loads took 8.5 us for 4096 rows)
+constexpr int XENT_MEAN_THREADS = 1024;
+__global__ __launch_bounds__(XENT_MEAN_THREADS) void xent_mean_kernel(const float* __restrict__ row_loss, const int64_t* __restrict__ labels,
                                                         float* __restrict__ out, float* __restrict__ loss, int B, int S, int V,
                                                         int64_t lab_b, int ignore_index) {
-  __shared__ double sl[256];
-  __shared__ int sc[256];
+  __shared__ double sl[XENT_MEAN_THREADS];
+  __shared__ int sc[XENT_MEAN_THREADS];
   double acc = 0.0;
   int cnt = 0;
   const int n = B * S;
-  for (int i = threadIdx.x; i < n; i += 256) {
+  for (int i = threadIdx.x; i < n; i += XENT_MEAN_THREADS) {
     const int b = i / S, s = i - b * S;
     acc += (double)row_loss[i];
     if (s < S - 1) {
@@ -260,7 +268,7 @@ __global__ __launch_bounds__(256) void xent_mean_kernel(const float* __restrict_
   sl[threadIdx.x] = acc;
   sc[threadIdx.x] = cnt;
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
+  for (int o = XENT_MEAN_THREADS / 2; o > 0; o >>= 1) {
     if ((int)threadIdx.x < o) {
       sl[threadIdx.x] += sl[threadIdx.x + o];
       sc[threadIdx.x] += sc[threadIdx.x + o];
@@ -275,7 +283,7 @@ __global__ __launch_bounds__(256) void xent_mean_kernel(const float* __restrict_
 }
 
 // dlogits[b, s, c] = dloss / count * (softmax(logits[b, s])[c] - [c == label]) for rows with a target, else 0
-constexpr int XENT_BWD_U = 1;
+constexpr int XENT_BWD_U = 2;
 template <typename T>
 __global__ __launch_bounds__(256) void xent_bwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ labels,
                                                        const float* __restrict__ lse, const float* __restrict__ loss_and_count,
@@ -302,8 +310,8 @@ __global__ __launch_bounds__(256) void xent_bwd_kernel(const T* __restrict__ log
   const bool vec = ((((size_t)lr) | ((size_t)dr)) & 15) == 0;
   if (vec) {
     // XENT_BWD_U vectors per thread, all loads first, and one such step per block (`chunks` blocks per row): the card
-    // sees many short blocks instead of a loop per row.  Measured at 8192 rows x 128256 fp32: a loop per row 5.1 TB/s,
-    // 4 vectors per thread in short blocks 5.7 TB/s, 1 vector per thread 5.9 TB/s
+    // sees many short blocks instead of a loop per row.  4096 rows x 128256 fp32, an eighth of them without a target, us:
+    // one vector per thread 686, two 641, three 672, four 718, eight 715
     constexpr int U = XENT_BWD_U;
     for (int v0 = chunk * (256 * U) + threadIdx.x; v0 < nvec; v0 += chunks * 256 * U) {
       float x[U][E];
@@ -526,18 +534,18 @@ extern "C" int tp_swiglu_bwd(const void* dout, const void* gate, const void* up,
 
 extern "C" int tp_cross_entropy_fwd_loss(const void* logits, const int64_t* labels, float* lse, float* row_loss, float* loss_and_count, float* loss,
                                     int B, int S, int V, int64_t logits_b_stride, int64_t logits_s_stride,
-                                    int64_t labels_b_stride, int ignore_index, int dtype, void* stream) {
+                                    int64_t labels_b_stride, int ignore_index, int scored_only, int dtype, void* stream) {
   TP_REQUIRE(logits && labels && lse && row_loss && loss_and_count, TP_ERR_BAD_ARG, "tp_cross_entropy_fwd: null pointer");
   TP_REQUIRE(B > 0 && S > 0 && V > 0 && (int64_t)B * S < (1ll << 31), TP_ERR_BAD_ARG, "tp_cross_entropy_fwd: bad shape");
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)(B * S)), block(256);
   if (dtype == TP_F32)
-    xent_fwd_kernel<float><<<grid, block, 0, st>>>((const float*)logits, labels, lse, row_loss, S, V, logits_b_stride, logits_s_stride, labels_b_stride, ignore_index);
+    xent_fwd_kernel<float><<<grid, block, 0, st>>>((const float*)logits, labels, lse, row_loss, S, V, logits_b_stride, logits_s_stride, labels_b_stride, ignore_index, scored_only);
   else if (dtype == TP_BF16)
-    xent_fwd_kernel<bf16_t><<<grid, block, 0, st>>>((const bf16_t*)logits, labels, lse, row_loss, S, V, logits_b_stride, logits_s_stride, labels_b_stride, ignore_index);
+    xent_fwd_kernel<bf16_t><<<grid, block, 0, st>>>((const bf16_t*)logits, labels, lse, row_loss, S, V, logits_b_stride, logits_s_stride, labels_b_stride, ignore_index, scored_only);
   else
     TP_REQUIRE(false, TP_ERR_UNSUPPORTED, "tp_cross_entropy_fwd: dtype %d (fp32 and bf16 logits only)", dtype);
-  xent_mean_kernel<<<dim3(1), block, 0, st>>>(row_loss, labels, loss_and_count, loss, B, S, V, labels_b_stride, ignore_index);
+  xent_mean_kernel<<<dim3(1), dim3(XENT_MEAN_THREADS), 0, st>>>(row_loss, labels, loss_and_count, loss, B, S, V, labels_b_stride, ignore_index);
   return check_launch("tp_cross_entropy_fwd");
 }
 
@@ -545,7 +553,7 @@ extern "C" int tp_cross_entropy_fwd(const void* logits, const int64_t* labels, f
                                     int B, int S, int V, int64_t logits_b_stride, int64_t logits_s_stride,
                                     int64_t labels_b_stride, int ignore_index, int dtype, void* stream) {
   return tp_cross_entropy_fwd_loss(logits, labels, lse, row_loss, loss_and_count, nullptr, B, S, V, logits_b_stride, logits_s_stride,
-                                   labels_b_stride, ignore_index, dtype, stream);
+                                   labels_b_stride, ignore_index, 0, dtype, stream);
 }
 
 extern "C" int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float* lse, const float* loss_and_count,

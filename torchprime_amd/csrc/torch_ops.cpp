@@ -160,7 +160,7 @@ TP_OP(l2norm_bwd, Tensor(const Tensor&, const Tensor&, const Tensor&))
 TP_OP(scale_rows, Tensor(const Tensor&, const Tensor&))
 TP_OP(swiglu_fwd, Tensor(const Tensor&, const Tensor&))
 TP_OP(swiglu_bwd, T2(const Tensor&, const Tensor&, const Tensor&))
-TP_OP(cross_entropy_fwd, T3(const Tensor&, const Tensor&, int64_t))
+TP_OP(cross_entropy_fwd, T3(const Tensor&, const Tensor&, int64_t, bool))
 TP_OP(cross_entropy_bwd, Tensor(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, int64_t))
 
 // ---- autograd plumbing -----------------------------------------------------------------------------------------
@@ -799,8 +799,9 @@ Tensor prep_labels(const Tensor& labels) {
   Tensor l = labels.to(at::kLong);
   return l.stride(1) != 1 ? l.contiguous() : l;
 }
-// (loss (scalar fp32), lse (B*S), loss_and_count (2)) of the shifted next-token cross entropy
-T3 cross_entropy_fwd_cuda(const Tensor& logits_, const Tensor& labels_, int64_t ignore_index) {
+// (loss (scalar fp32), lse (B*S), loss_and_count (2)) of the shifted next-token cross entropy; scored_only: the lse of rows
+// without a target is 0 (they are not read)
+T3 cross_entropy_fwd_cuda(const Tensor& logits_, const Tensor& labels_, int64_t ignore_index, bool scored_only) {
   const c10::Device dev = require_gpu(logits_, labels_);
   TORCH_CHECK_VALUE(logits_.dim() == 3 && labels_.dim() == 2 && labels_.size(0) == logits_.size(0) && labels_.size(1) == logits_.size(1),
                     "expected logits (batch, seq, vocab) and labels (batch, seq), got (", logits_.sizes(), ") and (", labels_.sizes(), ")");
@@ -812,7 +813,7 @@ T3 cross_entropy_fwd_cuda(const Tensor& logits_, const Tensor& labels_, int64_t 
   Tensor lse = empty_f32({B * S}, logits), row_loss = empty_f32({B * S}, logits), lc = empty_f32({2}, logits), loss = empty_f32({}, logits);
   check(tp_cross_entropy_fwd_loss(logits.data_ptr(), (const int64_t*)labels.data_ptr(), (float*)lse.data_ptr(), (float*)row_loss.data_ptr(),
                                   (float*)lc.data_ptr(), (float*)loss.data_ptr(), (int)B, (int)S, (int)V, logits.stride(0), logits.stride(1),
-                                  labels.stride(0), (int)ignore_index, dtype_code(logits.scalar_type()), stream_of(dev)),
+                                  labels.stride(0), (int)ignore_index, (int)scored_only, dtype_code(logits.scalar_type()), stream_of(dev)),
         "tp_cross_entropy_fwd_loss");
   return {loss, lse, lc};
 }
@@ -838,9 +839,9 @@ struct CrossEntropyNode : OpNode {
     return {op_cross_entropy_bwd()(g[0], get(0), get(1), get(2), get(3), ignore_index)};
   }
 };
-T3 cross_entropy_fwd_autograd(const Tensor& logits, const Tensor& labels, int64_t ignore_index) {
+T3 cross_entropy_fwd_autograd(const Tensor& logits, const Tensor& labels, int64_t ignore_index, bool scored_only) {
   auto node = make_node<CrossEntropyNode>(logits);
-  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_cross_entropy_fwd()(logits, labels, ignore_index); }();
+  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_cross_entropy_fwd()(logits, labels, ignore_index, scored_only); }();
   if (node) {
     torch::autograd::set_history(std::get<0>(r), node);
     node->keep(logits); node->keep(labels); node->keep(std::get<1>(r)); node->keep(std::get<2>(r));
@@ -1424,7 +1425,7 @@ int64_t py_mask_kind(const Tensor& mask) {
 }
 Tensor py_l2norm(const Tensor& x, double eps) { return std::get<0>(op_l2norm_fwd()(x, eps)); }
 Tensor py_swiglu(const Tensor& g, const Tensor& u) { return op_swiglu_fwd()(g, u); }
-Tensor py_cross_entropy(const Tensor& l, const Tensor& y, int64_t ignore) { return std::get<0>(op_cross_entropy_fwd()(l, y, ignore)); }
+Tensor py_cross_entropy(const Tensor& l, const Tensor& y, int64_t ignore) { return std::get<0>(op_cross_entropy_fwd()(l, y, ignore, true)); }
 
 }  // namespace
 
@@ -1450,7 +1451,7 @@ TORCH_LIBRARY(tprime, m) {
   m.def("scale_rows(Tensor x, Tensor scale) -> Tensor");
   m.def("swiglu_fwd(Tensor gate, Tensor up) -> Tensor");
   m.def("swiglu_bwd(Tensor dout, Tensor gate, Tensor up) -> (Tensor, Tensor)");
-  m.def("cross_entropy_fwd(Tensor logits, Tensor labels, int ignore_index) -> (Tensor, Tensor, Tensor)");
+  m.def("cross_entropy_fwd(Tensor logits, Tensor labels, int ignore_index, bool scored_only=False) -> (Tensor, Tensor, Tensor)");
   m.def("cross_entropy_bwd(Tensor dloss, Tensor logits, Tensor labels, Tensor lse, Tensor loss_and_count, int ignore_index) -> Tensor");
 }
 

@@ -163,7 +163,7 @@ def _(dout, gate, up):
 
 
 @torch.library.register_fake("tprime::cross_entropy_fwd")
-def _(logits, labels, ignore_index):
+def _(logits, labels, ignore_index, scored_only=False):
   B, S, _ = logits.shape
   return logits.new_empty((), dtype=torch.float32), logits.new_empty((B * S,), dtype=torch.float32), logits.new_empty((2,), dtype=torch.float32)
 
@@ -291,4 +291,4 @@ def swiglu(gate: Tensor, up: Tensor) -> Tensor:
 
 def cross_entropy(logits: Tensor, labels: Tensor, ignore_index: int) -> Tensor:
   """Mean of ``logsumexp(logits[b, s]) - logits[b, s, labels[b, s+1]]`` over the labels that are not ``ignore_index``."""
-  return cross_entropy_fwd(logits, labels, ignore_index)[0] if is_compiling() else _native.cross_entropy(logits, labels, ignore_index)
+  return cross_entropy_fwd(logits, labels, ignore_index, True)[0] if is_compiling() else _native.cross_entropy(logits, labels, ignore_index)
