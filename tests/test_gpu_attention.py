@@ -534,3 +534,31 @@ def test_llama3_8b_packed_segments_closed_forms():
 
 def test_deepseek_v3_shape_closed_forms():
   _closed_form_check(1, 128, 128, 4096, 192, 128, None, 4323)
+
+
+@pytest.mark.parametrize("seg", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,S,Dqk,Dv", [
+  (3, 48, 12, 1601, 64, 64),     # forward, dQ: five groups on an XCD (the last one half padding), three of them in turns
+  (3, 26, 26, 1601, 128, 128),   # dK/dV: ten groups, five in turns
+  (3, 26, 26, 1601, 192, 128),   # forward, dK/dV and dQ
+])  # fmt: skip
+def test_every_group_is_done_once_where_the_last_ones_take_turns(B, Hq, Hkv, S, Dqk, Dv, seg):
+  """Many workgroups per XCD, the last groups' tiles interleaved: the same results as one batch element at a time (another
+  order of workgroups).  Forward and dQ are the same bits; dK / dV of one element may be summed in pieces, which moves the
+  last rounding: one unit of bf16, 2^-8 of the value."""
+  dt = torch.bfloat16
+  q, k, v = heads_view(B, Hq, S, Dqk, 1, dt, 1.0), heads_view(B, Hkv, S, Dqk, 2, dt, 1.0), heads_view(B, Hkv, S, Dv, 3, dt, 1.0)
+  do = heads_view(B, Hq, S, Dv, 4, dt, 1.0)
+  ids = packed_segment_ids(B, S, 64, 900, 5)[0] if seg else None
+  scale = 1.0 / math.sqrt(Dv)
+  out, lse, dq, dk, dv = _run(q, k, v, do, ids, True, scale)
+  for b in range(B):
+    one = slice(b, b + 1)
+    o1, l1, dq1, dk1, dv1 = _run(q[one], k[one], v[one], do[one], None if ids is None else ids[one], True, scale)
+    assert torch.equal(out[one], o1) and torch.equal(lse[one], l1) and torch.equal(dq[one], dq1)
+    for name, got, want in (("dk", dk[one], dk1), ("dv", dv[one], dv1)):
+      assert_close(got, want.cpu().double(), name, scale_abs=True, rel_l2=2.0**-8)
+  h = Hq // Hkv  # one group against the oracle
+  o_ref = orc.attention_grads_ref(q[B - 1 :, -h:], k[B - 1 :, -1:], v[B - 1 :, -1:], do[B - 1 :, -h:], None if ids is None else ids[B - 1 :], True,
+                                  scale, torch.float64)[0]  # fmt: skip
+  assert_close(out[B - 1 :, -h:], o_ref, "out")

@@ -72,7 +72,7 @@ struct BwdArgs {
   int band_lo, band_hi;
   MaskExt mx;
   PairMask pm;
-  int interleave;  // order of the workgroups (xcd_map)
+  int turns;       // order of the workgroups (xcd_map)
   // dK/dV: partial results of the splits of a kv tile's work (split_plan), NULL: no tile is split
   float* parts;
   size_t parts_bytes;
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     split = (r - f) - gl * n_split;
     group = gl * NUM_XCD + blockIdx.x % NUM_XCD;
     if (group >= a.B * a.Hkv) return;
-  } else if (!xcd_map((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
+  } else if (!xcd_map((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int b = group / a.Hkv, hk = group - b * a.Hkv;
   const int kv0 = tile * BNK;  // low kv tiles see the most queries: they start first
   const int wkv0 = kv0 + wave * 32;
@@ -996,7 +996,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
+  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM, wq0 = q0 + wave * 32;
@@ -1599,7 +1599,7 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
+  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;  // the longest rows first
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM, wq0 = q0 + wave * 32;
@@ -2056,7 +2056,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
         if (rc) return rc;
         attr_set = true;
       }
-      a.interleave = interleave_groups((a.Sq + BM - 1) / BM, a.n_rep, groups, DQK == DV ? 2 : 1);
+      a.turns = groups_in_turns((a.Sq + BM - 1) / BM, a.n_rep, groups, DQK == DV ? 2 : 1);
       kern<<<dim3(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, groups)), dim3(256), Lean::lds_bytes(a.Skv), st>>>(a);
       int rc = check_launch("tp_attn_bwd(dq)");
       if (rc) return rc;
@@ -2078,7 +2078,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
     if (a.parts) plan = bwd_split_plan(a, CAUSAL);
     a.split = plan.on && plan.bytes <= a.parts_bytes;
     if (a.split) memcpy(a.split_first, plan.first, sizeof(a.split_first));
-    a.interleave = interleave_groups(n_tiles, 1, groups, DQK <= 64 ? 2 : 1);
+    a.turns = groups_in_turns(n_tiles, 1, groups, DQK <= 64 ? 2 : 1);
     kern<<<dim3(a.split ? NUM_XCD * plan.first[n_tiles] : xcd_grid(n_tiles, 1, groups)), dim3(256), dkdv_smem, st>>>(a);
     int rc = check_launch("tp_attn_bwd(dkdv)");
     if (rc) return rc;
@@ -2109,7 +2109,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
       if (rc) return rc;
       attr_set = true;
     }
-    a.interleave = 0;
+    a.turns = 0;
     kern<<<dim3(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, groups)), dim3(64 * NW), smem, st>>>(a);
     int rc = check_launch("tp_attn_bwd(dq)");
     if (rc) return rc;
@@ -2247,7 +2247,7 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   a.q = q; a.k = k; a.v = v; a.out = out; a.dout = dout; a.lse = lse; a.seg = seg;
   a.dq = dq; a.dk = dk; a.dv = dv; a.delta = ws;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv; a.n_rep = Hq / Hkv; a.dqk = Dqk; a.dv_dim = Dv;
-  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.interleave = 0;
+  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.turns = 0;
   bool ok = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(dout) && aligned16(dq) &&
             aligned16(dk) && aligned16(dv);
   for (int i = 0; i < 3; i++) {

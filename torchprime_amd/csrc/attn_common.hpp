@@ -11,6 +11,7 @@
 // 16h + 8a + 4g + e (a = 0..1, e = 0..3), and the other operand is laid out in LDS so that a lane's
 // 16 bytes hold exactly those rows ("quad-swapped" order, see vt_offset).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -230,24 +231,25 @@ __device__ __forceinline__ unsigned span_bytes(int rows, int64_t stride, int row
 // Q/dO) slice - one (batch, kv head) "group" - lands on the same XCD and runs at about the same time:
 //     id = (group_local * per_group + r) * 8 + xcd,   group = group_local * 8 + xcd,
 //     r  = tile * n_inner + inner   (tiles outer so the heaviest tiles start first).
-// With group after group the last group's heaviest tile starts when nearly everything else is done.  Where an XCD gets
-// only a few rounds of workgroups that tail is a good part of the launch (dK/dV of 64 groups of 10 causal tiles: a
-// third), and there the groups take turns tile by tile instead (`interleave`; the host's rule is interleave_groups); with
-// many rounds the tail is small and the groups' sharing of an L2 is worth more.
+// With group after group the last group's heaviest tile starts when nearly everything else is done.  The last groups of
+// an XCD therefore take turns tile by tile (`turns` of them; the host's rule is groups_in_turns), heaviest tiles of all
+// of them first; the ones before run group after group, which shares an L2 best.
 // Returns false for the padding ids of a group count that is not a multiple of 8.
 constexpr int NUM_XCD = 8, CUS_PER_XCD = 32;
-__device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, bool interleave = false) {
+__device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns = 0) {
   const int n = blockIdx.x;
-  const int xcd = n % NUM_XCD, slot = n / NUM_XCD;
-  int gl, r;
-  if (interleave) {
-    const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, per_tile = n_gl * n_inner;
+  const int xcd = n % NUM_XCD;
+  int slot = n / NUM_XCD, gl, r;
+  const int per_group = n_tiles * n_inner, first = (n_groups + NUM_XCD - 1) / NUM_XCD - turns;
+  if (turns && slot >= first * per_group) {
+    const int per_tile = turns * n_inner;
+    slot -= first * per_group;
     tile = slot / per_tile;
     r = slot - tile * per_tile;
     gl = r / n_inner;
     inner = r - gl * n_inner;
+    gl += first;
   } else {
-    const int per_group = n_tiles * n_inner;
     gl = slot / per_group;
     r = slot - gl * per_group;
     tile = r / n_inner;
@@ -256,10 +258,16 @@ __device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, 
   group = gl * NUM_XCD + xcd;
   return group < n_groups;
 }
-// fewer than four rounds of workgroups on an XCD (per_cu of them share a CU), and more than one group to order
-inline bool interleave_groups(int n_tiles, int n_inner, int n_groups, int per_cu) {
-  const int64_t n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD;
-  return n_gl > 1 && n_gl * n_tiles * n_inner < 4 * CUS_PER_XCD * per_cu;
+// How many groups: all where an XCD gets fewer than four rounds of workgroups (per_cu of them share a CU), else the last
+// ones that make up two rounds; 0 where one group has that many by itself.  More of them in turns balances better still
+// and loses more in the L2 than that gains.  us, none | two rounds | four | all in turns, bf16, causal:
+//   forward, 128 heads of (192,128): B1 S4096 684 | 657 | 671 | 677;  B2 S2048 405 | 362 | 391 | 437
+//   forward + backward: B8 8 heads of 64 S4096 718 | 629 | 621 | 634;  B8 32q/8kv of 128 S2048 1321 | 1261 | 1252 | 1267
+//   packed documents: B4 32q/8kv of 128 S4096 1085 | 1039 | 1084 | 1090;  S8192 (one group is two rounds) 3556 | - | 3628 | 3812
+inline int groups_in_turns(int n_tiles, int n_inner, int n_groups, int per_cu) {
+  const int64_t n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, per_group = (int64_t)n_tiles * n_inner, round = CUS_PER_XCD * per_cu;
+  const int64_t n = n_gl * per_group < 4 * round ? n_gl : std::min(n_gl, (2 * round + per_group - 1) / per_group);
+  return n > 1 ? (int)n : 0;
 }
 inline unsigned xcd_grid(int n_tiles, int n_inner, int n_groups) {
   return (unsigned)(NUM_XCD * ((n_groups + NUM_XCD - 1) / NUM_XCD) * n_tiles * n_inner);

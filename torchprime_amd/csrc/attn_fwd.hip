@@ -37,7 +37,7 @@ struct FwdArgs {
   int band_lo, band_hi;
   MaskExt mx;
   PairMask pm;
-  int interleave;  // order of the workgroups (xcd_map)
+  int turns;       // order of the workgroups (xcd_map)
 };
 
 // Two workgroups per CU (256 registers per lane) where the kernel fits them; the non-causal variants at head dims of
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.interleave)) return;
+  if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;  // longest (latest) query tiles are scheduled first
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM;
@@ -629,7 +629,7 @@ static int launch_fwd(const FwdArgs& args, int B, hipStream_t st) {
     TP_REQUIRE(e == hipSuccess, TP_ERR_LAUNCH, "tp_attn_fwd: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     attr_set = true;
   }
-  a.interleave = interleave_groups((a.Sq + BM - 1) / BM, a.n_rep, B * a.Hkv, fwd_blocks_per_cu<DQK, CAUSAL, SEG>());
+  a.turns = groups_in_turns((a.Sq + BM - 1) / BM, a.n_rep, B * a.Hkv, fwd_blocks_per_cu<DQK, CAUSAL, SEG>());
   const dim3 grid(xcd_grid((a.Sq + BM - 1) / BM, a.n_rep, B * a.Hkv)), block(256);
   kern<<<grid, block, smem, st>>>(a);
   return check_launch("tp_attn_fwd");
