@@ -88,8 +88,7 @@ struct BwdArgs {
 // there can be.  Such a tile's walk is cut into pieces of at most `cap` iterations, one workgroup each, which leave
 // their sums as fp32 in a workspace for a short kernel to add up in order (deterministic).  The cap is the one for which
 // the estimate below is least; pieces cost their start-up and 2 x 128 x (dqk + dv) x 4 bytes of traffic each.
-// Measured (bf16, 32q/8kv heads of 128, B1): dK/dV of a 1024-key window over 2047 rows 116 -> see the table of figures
-// at the launch.
+// Measured (bf16, 32q/8kv heads of 128, B1): dK/dV of a 1024-key window over 2047 rows 116 -> 71 us and 7 us for the sums.
 struct SplitPlan {
   bool on;
   int n_tiles, n_gl;
