@@ -137,3 +137,23 @@ def test_norm_backward_of_few_rows(rows, hidden):
   for a, b in ((got[0], dxr + dh.double()), (got[1], dxr + dh.double()), (got[2], dwr)):
     a = a.double().cpu()
     assert ((a - b).norm() / b.norm()).item() <= 1e-2
+
+
+def test_a_recorded_backward_gives_the_gradients_and_no_second_ones():
+  """create_graph: the same gradients as without it; differentiating through them raises."""
+  cfg = tpa.Config(vocab_size=136, num_hidden_layers=2, max_position_embeddings=512, hidden_size=128, intermediate_size=64,
+                   num_attention_heads=2, num_key_value_heads=2, hidden_act="silu", initializer_range=0.02, rms_norm_eps=1e-5,
+                   attention_dropout=False, attention_bias=False, rope_theta=500000.0, attention_kernel="splash_attention")  # fmt: skip
+  model = tpa.LlamaForCausalLM(cfg).to(DEV)
+  ids = torch.randint(136, (1, 37), generator=torch.Generator().manual_seed(1)).to(DEV)
+  params = list(model.parameters())
+  logits, loss = model(ids, labels=ids)
+  assert logits.grad_fn.name() == "TprimeLlamaHeadBackward"
+  want = torch.autograd.grad(loss, params)
+  got = torch.autograd.grad(model(ids, labels=ids)[1], params, create_graph=True)
+  for (name, _), a, b in zip(model.named_parameters(), got, want):
+    # (the embedding's gradient is the library's scatter then: fp32 sums in another order)
+    same = (a - b).abs().max() <= 1e-5 * b.abs().max() if "embed" in name else torch.equal(a, b)
+    assert same and a.requires_grad, name
+  with pytest.raises((NotImplementedError, RuntimeError), match="not implemented"):
+    torch.autograd.grad(sum(g.sum() for g in got), params)

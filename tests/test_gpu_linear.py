@@ -67,3 +67,17 @@ def test_what_the_modules_have_to_see_themselves():
   (gg,) = torch.autograd.grad(g.sum(), x)
   w = m.weight.detach().double().cpu()
   _close(gg, 2.0 * torch.ones(7, 64, dtype=torch.float64) @ w.T @ w, torch.float32, "second derivative")
+
+
+def test_forward_mode_goes_to_the_modules():
+  """Tangents of the input and of a weight: the library's product rule, not a product without it."""
+  x, m = randn((7, 64), 1, torch.float32).to(DEV), nn.Linear(64, 64, bias=False, device=DEV)
+  w, tx, tw = m.weight.detach(), randn((7, 64), 2, torch.float32).to(DEV), randn((64, 64), 3, torch.float32).to(DEV)
+  with torch.autograd.forward_ad.dual_level():
+    del m.weight
+    m.register_parameter("weight", None)
+    m._parameters["weight"] = torch.autograd.forward_ad.make_dual(w, tw)
+    y = project(torch.autograd.forward_ad.make_dual(x, tx), m)[0]
+    got = torch.autograd.forward_ad.unpack_dual(y).tangent
+  assert got is not None
+  _close(got, tx.double().cpu() @ w.double().cpu().T + x.double().cpu() @ tw.double().cpu().T, torch.float32, "tangent")

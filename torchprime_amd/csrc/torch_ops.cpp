@@ -858,7 +858,26 @@ T3 cross_entropy_fwd_autograd(const Tensor& logits, const Tensor& labels, int64_
 bool plain_eager(const Tensor& t) {
   static const c10::DispatchKeySet usual({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
   const c10::DispatchKeySet on = c10::impl::tls_local_dispatch_key_set().included_;
-  return (on - usual).empty() && !at::autocast::is_autocast_enabled(at::kCUDA) && t.is_cuda() && !t.unsafeGetTensorImpl()->is_python_dispatch() && t.layout() == at::kStrided;
+  return (on - usual).empty() && !at::autocast::is_autocast_enabled(at::kCUDA) && t.is_cuda() && !t.unsafeGetTensorImpl()->is_python_dispatch() &&
+         t.layout() == at::kStrided && !torch::autograd::isFwGradDefined(t);
+}
+
+// The native nodes below have no second derivative.  A backward that records a graph (create_graph) gets its gradients all
+// the same; only differentiating through them raises, as for the operators' own backwards.
+struct NoDerivative : torch::autograd::Node {
+  const char* what;
+  std::string name() const override { return "TprimeNoDerivative"; }
+  variable_list apply(variable_list&&) override { TORCH_CHECK_NOT_IMPLEMENTED(false, "derivative for the backward of ", what, " is not implemented"); }
+};
+void end_of_graph(const char* what, const variable_list& grads, const torch::autograd::Node& from, variable_list& outs) {
+  if (!at::GradMode::is_enabled()) return;
+  std::shared_ptr<NoDerivative> n(new NoDerivative(), torch::autograd::deleteNode);
+  n->what = what;
+  torch::autograd::edge_list edges = from.next_edges();
+  for (const auto& g : grads) edges.push_back(g.defined() ? torch::autograd::impl::gradient_edge(g) : torch::autograd::Edge());
+  n->set_next_edges(std::move(edges));
+  for (auto& o : outs)
+    if (o.defined() && !o.requires_grad()) torch::autograd::set_history(o, n);  // (two inputs may share one gradient)
 }
 // The line between the two, in multiply-adds of the whole group.  Measured with the host's time, us, tp_linears against
 // at::linear, forward | forward + backward:  bf16 512 x 512 through three 512 x 512: 8 : 62 | 83 : 296;  1024 x 1024 through
@@ -963,11 +982,7 @@ std::vector<Tensor> py_linears(const Tensor& x, const std::vector<Tensor>& ws) {
   }
   std::shared_ptr<LinearsNode> node;
   bool req = at::GradMode::is_enabled() && x.requires_grad();
-  for (const auto& w : ws) {
-    TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(w), "the tprime operators have no forward-mode derivative");
-    req = req || (at::GradMode::is_enabled() && w.requires_grad());
-  }
-  TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(x), "the tprime operators have no forward-mode derivative");
+  for (const auto& w : ws) req = req || (at::GradMode::is_enabled() && w.requires_grad());
   if (req) {
     node = std::shared_ptr<LinearsNode>(new LinearsNode(), torch::autograd::deleteNode);
     torch::autograd::edge_list edges{torch::autograd::impl::gradient_edge(x)};
@@ -1060,7 +1075,6 @@ struct LayerNode : torch::autograd::Node {
 
 variable_list LayerNode::apply(variable_list&& g) {
   std::lock_guard<std::mutex> lock(mutex_);
-  TORCH_CHECK_NOT_IMPLEMENTED(!at::GradMode::is_enabled(), "derivative for a decoder layer's backward is not implemented");
   variable_list out(2 + LP_COUNT);  // x, residual, the parameters
   if (!g[0].defined() && !g[1].defined()) return out;
   const Tensor B = buf.unpack(), H2 = h2.unpack(shared_from_this()), C = cos.unpack(), Sn = sin.unpack();
@@ -1145,6 +1159,7 @@ variable_list LayerNode::apply(variable_list&& g) {
   norm_bwd(LP_N1, t + o_dn, t + o_ds, s.residual ? base + f.h : (char*)X.data_ptr(), f.rstd1, dx.data_ptr());
   out[0] = dx;
   if (s.residual) out[1] = dx;
+  end_of_graph("a decoder layer", g, *this, out);
   return out;
 }
 
@@ -1176,7 +1191,7 @@ std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const s
     if (t->dim() != 3 || (t->size(0) != 1 && t->size(0) != s.B) || t->size(1) != s.S || t->size(2) != s.D || t->scalar_type() != dt ||
         !t->is_contiguous() || !plain_eager(*t) || t->device() != x.device() || t->requires_grad()) return {};
   for (const Tensor* t : {&x, &residual})
-    if (t->defined() && (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 || torch::autograd::isFwGradDefined(*t))) return {};
+    if (t->defined() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16) return {};
 
   std::shared_ptr<LayerNode> node;
   if (at::GradMode::is_enabled()) {
@@ -1274,7 +1289,7 @@ Tensor py_embedding(const Tensor& ids, const Tensor& table) {
   const bool small = plain_eager(table) && plain_eager(ids) && ids.device() == table.device() && table.dim() == 2 && table.is_contiguous() &&
                      (t == at::kBFloat16 || t == at::kHalf || t == at::kFloat) && ids.scalar_type() == at::kLong && ids.numel() > 0 &&
                      table.size(0) > 0 && table.size(1) > 0 && table.size(1) % 2 == 0 && table.size(0) * ids.numel() <= (1ll << 24) &&
-                     ids.numel() * table.size(1) <= (1ll << 24) && !torch::autograd::isFwGradDefined(table);
+                     ids.numel() * table.size(1) <= (1ll << 24);
   if (!small) return at::embedding(table, ids);
   auto node = make_node<EmbeddingNode>(table);
   Tensor out;
@@ -1309,7 +1324,6 @@ struct HeadNode : torch::autograd::Node {
   }
   variable_list apply(variable_list&& g) override {
     std::lock_guard<std::mutex> lock(mutex_);
-    TORCH_CHECK_NOT_IMPLEMENTED(!at::GradMode::is_enabled(), "derivative for a model head's backward is not implemented");
     variable_list out(4);  // x, residual, norm weight, lm_head weight
     if (!g[0].defined()) return out;
     const Tensor H = h.unpack(), N = n.unpack(), R = rstd.unpack(), nw = norm_w.unpack(), lw = lm_w.unpack();
@@ -1340,6 +1354,7 @@ struct HeadNode : torch::autograd::Node {
                            (float*)ws.data_ptr(), rows, (int)k, k, k, k, code, code, st), "tp_rmsnorm_bwd");
       out[1] = out[0];
     }
+    end_of_graph("a model head", g, *this, out);
     return out;
   }
 };
