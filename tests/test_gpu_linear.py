@@ -51,6 +51,31 @@ def test_forward_and_gradients(M, K, Ns, dtype):
   _close(dx, gs[-1].double() @ ws[-1].double(), dtype, "dx of one output")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_far_apart_or_shared(dtype):
+  """Rows whose span is past the launch's 32-bit offsets (the last token of each long sequence of a batch) and gradients
+  whose rows are one row expanded: the results of the same values side by side, bit for bit."""
+  K, N = 4096, 64
+  m = nn.Linear(K, N, bias=False, device=DEV, dtype=dtype)
+  far = torch.empty((2, 4096, K), dtype=dtype, device=DEV)
+  far[:, -1] = randn((2, K), 1, dtype).to(DEV)
+  x, near = (t.detach().requires_grad_(True) for t in (far[:, -1:], far[:, -1:].contiguous()))
+  assert (2 + 64) * x.stride(0) * x.element_size() >= 2**31
+  g = randn((1, 1, N), 2, dtype).to(DEV).expand(2, 1, N)
+  got, want = project(x, m)[0], project(near, m)[0]
+  assert got.grad_fn.name() == "TprimeLinearsBackward" and torch.equal(got, want)
+  for a, b in zip(torch.autograd.grad(got, [x, m.weight], g), torch.autograd.grad(want, [near, m.weight], g.contiguous())):
+    assert torch.equal(a, b)
+
+
+def test_a_weight_past_the_offsets_is_the_library_s():
+  """2 GiB of weight and one token: little work, but more than the launch's 32-bit offsets reach."""
+  m = nn.Linear(8192, 131072, bias=False, device=DEV, dtype=torch.bfloat16)
+  x = randn((1, 8192), 1, torch.bfloat16).to(DEV)
+  with torch.no_grad():
+    assert torch.equal(project(x, m)[0], m(x))
+
+
 def test_what_the_modules_have_to_see_themselves():
   """Hooks, a bias, autocast, a recorded backward: the results are the modules' own."""
   x = randn((7, 64), 1, torch.float32).to(DEV).requires_grad_(True)

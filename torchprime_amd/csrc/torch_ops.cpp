@@ -885,6 +885,17 @@ void end_of_graph(const char* what, const variable_list& grads, const torch::aut
 // the library's larger tiles win on the device.  fp32: 2048 x 512 through three 512 x 512 (1.6e9): 39 : 60 | 126 : 287;
 // 3.2e9: 69 : 60 | 208 : 290;  4.3e9: 76 : 62 | 270 : 188.
 int64_t lin_max_work(at::ScalarType t) { return t == at::kFloat ? 1ll << 31 : 1ll << 32; }
+// tp_linears addresses an operand with 32-bit byte offsets, up to 64 rows past its end
+bool lin_reach(int64_t rows, int64_t stride, int64_t esize) { return (rows + 64) * stride * esize < (1ll << 31); }
+// The matrices of one product m x k by n x k, its output and that output's gradient, stored row after row, are in reach.
+bool lin_fits(int64_t m, int64_t n, int64_t k, int64_t esize) { return lin_reach(m, k, esize) && lin_reach(n, k, esize) && lin_reach(m, n, esize); }
+// x as rows that tp_linears reads, for matrices that lin_fits: a copy where the view's rows lie too far apart (the last token
+// of every sequence of a batch) or on top of each other (the expanded gradient of a sum).
+Rows lin_rows(const Tensor& x) {
+  Rows r = rows_of(x, true);
+  if (r.stride >= r.cols && lin_reach(r.rows, r.stride, x.element_size())) return r;
+  return {r.t.reshape({r.rows, r.cols}).clone(at::MemoryFormat::Contiguous), r.rows, r.cols, r.cols};
+}
 bool linears_take(const Tensor& x, const std::vector<Tensor>& ws) {
   const auto t = x.scalar_type();
   if (ws.empty() || ws.size() > 3 || x.dim() < 1 || x.numel() == 0 || !plain_eager(x)) return false;
@@ -894,6 +905,7 @@ bool linears_take(const Tensor& x, const std::vector<Tensor>& ws) {
   for (const auto& w : ws) {
     if (!plain_eager(w) || w.dim() != 2 || w.scalar_type() != t || w.device() != x.device() || w.size(1) != k || !w.is_contiguous()) return false;
     if (w.size(0) == 0 || w.size(0) % vec || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) return false;
+    if (!lin_fits(m, w.size(0), k, x.element_size())) return false;
     n += w.size(0);
   }
   return k % vec == 0 && m * n * k <= lin_max_work(t);
@@ -940,14 +952,14 @@ variable_list LinearsNode::apply(variable_list&& g) {
   }
   at::AutoDispatchBelowADInplaceOrView below;
   c10::DeviceGuard guard(xt.device());
-  const Rows xr = rows_of(xt, true);
+  const Rows xr = lin_rows(xt);
   std::vector<Rows> gr;  // (keep copies of strided gradients alive until the launch)
   gr.reserve(nw);
   std::array<tp_linear_problem, 4> p;
   int n = 0, dx = -1;
   for (size_t i = 0; i < nw; i++) {
     if (!g[i].defined()) continue;
-    gr.push_back(rows_of(g[i], true));
+    gr.push_back(lin_rows(g[i]));
     const Rows& r = gr.back();
     const int64_t nf = wt[i].size(0);
     if (task_should_compute_output(0)) {
@@ -992,7 +1004,7 @@ std::vector<Tensor> py_linears(const Tensor& x, const std::vector<Tensor>& ws) {
   {
     at::AutoDispatchBelowADInplaceOrView below;
     c10::DeviceGuard guard(x.device());
-    const Rows xr = rows_of(x, true);
+    const Rows xr = lin_rows(x);
     std::array<tp_linear_problem, 4> p;
     auto sizes = x.sizes().vec();
     for (size_t i = 0; i < ws.size(); i++) {
@@ -1184,7 +1196,7 @@ std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const s
   // the two projections whose input is made here: shape, layout, and the same line on size
   const auto lin_ok = [&](const Tensor& t, int64_t n, int64_t k) {
     return t.dim() == 2 && t.size(0) == n && t.size(1) == k && t.scalar_type() == dt && t.is_contiguous() && plain_eager(t) && t.device() == x.device() &&
-           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && s.rows * n * k <= lin_max_work(dt);
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && s.rows * n * k <= lin_max_work(dt) && lin_fits(s.rows, n, k, x.element_size());
   };
   if (!lin_ok(w[LP_O], s.H, NQ) || !lin_ok(w[LP_D], s.H, s.I)) return {};
   for (const Tensor* t : {&cos, &sin})
