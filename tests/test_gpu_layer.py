@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import torchprime_amd as tpa
-from tests.util import randn
+from tests.util import off_address, randn
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -73,6 +73,33 @@ def test_frozen_parameters_and_unused_outputs():
   one = torch.autograd.grad(layer.forward_deferred(x, None, position_embeddings=cs)[0], leaves, g)
   both = torch.autograd.grad(layer.forward_deferred(x, None, position_embeddings=cs), leaves, [g, torch.zeros_like(g)])
   assert all(torch.equal(a, b) for a, b in zip(one, both))
+
+
+def test_gradients_at_odd_addresses():
+  """Gradients of a layer, of the logits and of embedding rows that are contiguous but off the 16-byte addresses (pieces of
+  a concatenation): the gradients of the same values at an allocation's start."""
+  from torchprime_amd.linear import embed
+
+  layer = _layer(128, 2, 2, 64, "splash_attention", torch.float32)
+  x = randn((1, 20, 128), 1).to(DEV).requires_grad_(True)
+  cs = tpa.LlamaRotaryEmbedding(64, 500000.0).to(DEV)(x, torch.arange(20, device=DEV)[None].float())
+  g = [randn((1, 20, 128), 2).to(DEV), randn((1, 20, 128), 3).to(DEV)]
+  for a, b in zip(_run(layer, x, None, None, cs, [off_address(t) for t in g])[1], _run(layer, x, None, None, cs, g)[1]):
+    assert torch.equal(a, b)
+  cfg = tpa.Config(vocab_size=136, num_hidden_layers=1, max_position_embeddings=512, hidden_size=128, intermediate_size=64,
+                   num_attention_heads=2, num_key_value_heads=2, hidden_act="silu", initializer_range=0.02, rms_norm_eps=1e-5,
+                   attention_dropout=False, attention_bias=False, rope_theta=500000.0, attention_kernel="splash_attention")  # fmt: skip
+  model = tpa.LlamaForCausalLM(cfg).to(DEV)
+  ids = torch.randint(136, (2, 37), generator=torch.Generator().manual_seed(1)).to(DEV)
+  params, gl = list(model.parameters()), randn((2, 37, 136), 4).to(DEV)
+  got, want = (torch.autograd.grad(model(ids)[0], params, t) for t in (off_address(gl), gl))
+  assert all(torch.equal(a, b) for a, b in zip(got, want))
+  m = torch.nn.Embedding(7, 64, device=DEV)
+  ge = randn((2, 37, 64), 5).to(DEV)
+  got, want = (torch.autograd.grad(embed(m, ids % 7), m.weight, t)[0] for t in (off_address(ge), ge))
+  assert torch.equal(got, want)
+  m.weight = torch.nn.Parameter(off_address(m.weight.detach()))
+  assert torch.equal(embed(m, ids % 7), m(ids % 7))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

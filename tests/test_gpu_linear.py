@@ -8,7 +8,7 @@ import pytest
 import torch
 from torch import nn
 
-from tests.util import randn
+from tests.util import off_address, randn
 from torchprime_amd.linear import project
 
 pytestmark = pytest.mark.gpu
@@ -66,6 +66,20 @@ def test_rows_far_apart_or_shared(dtype):
   assert got.grad_fn.name() == "TprimeLinearsBackward" and torch.equal(got, want)
   for a, b in zip(torch.autograd.grad(got, [x, m.weight], g), torch.autograd.grad(want, [near, m.weight], g.contiguous())):
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_contiguous_at_an_odd_address(dtype):
+  """Input and gradients that are contiguous pieces of larger tensors, off the 16-byte addresses: the results of the same
+  values at an allocation's start, bit for bit."""
+  a, b = (nn.Linear(64, n, bias=False, device=DEV, dtype=dtype) for n in (64, 8))
+  leaves = [f(randn((3, 5, 64), 1, dtype).to(DEV)).detach().requires_grad_(True) for f in (off_address, torch.clone)]
+  grads = [randn((3, 5, n), 2, dtype).to(DEV) for n in (64, 8)]
+  got, want = (project(x, a, b) for x in leaves)
+  assert all(o.grad_fn.name() == "TprimeLinearsBackward" for o in got) and all(torch.equal(s, t) for s, t in zip(got, want))
+  for s, t in zip(torch.autograd.grad(got, [leaves[0], a.weight, b.weight], [off_address(g) for g in grads]),
+                  torch.autograd.grad(want, [leaves[1], a.weight, b.weight], grads)):
+    assert torch.equal(s, t)
 
 
 def test_a_weight_past_the_offsets_is_the_library_s():

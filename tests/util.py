@@ -82,3 +82,12 @@ def packed_segment_ids(B, S, lo, hi, seed):
       ls.append(L)
     lengths.append(ls)
   return seg, lengths
+
+
+def off_address(t: torch.Tensor) -> torch.Tensor:
+  """A contiguous copy of ``t`` one element past a 16-byte address, as a piece of a concatenation may lie."""
+  n = torch.empty(t.numel() + 16 // t.element_size(), dtype=t.dtype, device=t.device)
+  v = n[1 : 1 + t.numel()].view(t.shape)
+  v.copy_(t)
+  assert v.is_contiguous() and v.data_ptr() % 16
+  return v

@@ -108,6 +108,15 @@ Rows rows_of(const Tensor& x, bool align16) {
   return {x2, x2.size(0), h, x2.size(0) > 1 ? x2.stride(0) : h};
 }
 
+bool at16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+// t with its elements side by side from a 16-byte address, copied only if they are not: for launches that are handed a
+// bare pointer.  (A gradient may be a contiguous piece of a larger tensor at any address; a tensor that comes back through
+// a saved-tensor hook may have other strides than the one that went in.)
+Tensor packed16(const Tensor& t) {
+  const Tensor c = t.contiguous();
+  return at16(c) ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
 // New (B,H,S,D') tensor.  Head-minor inputs (the (B,S,H,D)-memory views the attention modules build with
 // .view(B,S,H,D).transpose(1,2)) get the same head-minor memory order, so the caller's transpose(1,2).contiguous()
 // afterwards is free; anything else gets plain contiguous memory.
@@ -890,10 +899,10 @@ bool lin_reach(int64_t rows, int64_t stride, int64_t esize) { return (rows + 64)
 // The matrices of one product m x k by n x k, its output and that output's gradient, stored row after row, are in reach.
 bool lin_fits(int64_t m, int64_t n, int64_t k, int64_t esize) { return lin_reach(m, k, esize) && lin_reach(n, k, esize) && lin_reach(m, n, esize); }
 // x as rows that tp_linears reads, for matrices that lin_fits: a copy where the view's rows lie too far apart (the last token
-// of every sequence of a batch) or on top of each other (the expanded gradient of a sum).
+// of every sequence of a batch), on top of each other (the expanded gradient of a sum) or off the 16-byte addresses.
 Rows lin_rows(const Tensor& x) {
   Rows r = rows_of(x, true);
-  if (r.stride >= r.cols && lin_reach(r.rows, r.stride, x.element_size())) return r;
+  if (at16(r.t) && r.stride >= r.cols && lin_reach(r.rows, r.stride, x.element_size())) return r;
   return {r.t.reshape({r.rows, r.cols}).clone(at::MemoryFormat::Contiguous), r.rows, r.cols, r.cols};
 }
 bool linears_take(const Tensor& x, const std::vector<Tensor>& ws) {
@@ -904,7 +913,7 @@ bool linears_take(const Tensor& x, const std::vector<Tensor>& ws) {
   int64_t n = 0;
   for (const auto& w : ws) {
     if (!plain_eager(w) || w.dim() != 2 || w.scalar_type() != t || w.device() != x.device() || w.size(1) != k || !w.is_contiguous()) return false;
-    if (w.size(0) == 0 || w.size(0) % vec || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) return false;
+    if (w.size(0) == 0 || w.size(0) % vec || !at16(w)) return false;
     if (!lin_fits(m, w.size(0), k, x.element_size())) return false;
     n += w.size(0);
   }
@@ -952,6 +961,7 @@ variable_list LinearsNode::apply(variable_list&& g) {
   }
   at::AutoDispatchBelowADInplaceOrView below;
   c10::DeviceGuard guard(xt.device());
+  for (auto& w : wt) w = packed16(w);
   const Rows xr = lin_rows(xt);
   std::vector<Rows> gr;  // (keep copies of strided gradients alive until the launch)
   gr.reserve(nw);
@@ -1089,10 +1099,10 @@ variable_list LayerNode::apply(variable_list&& g) {
   std::lock_guard<std::mutex> lock(mutex_);
   variable_list out(2 + LP_COUNT);  // x, residual, the parameters
   if (!g[0].defined() && !g[1].defined()) return out;
-  const Tensor B = buf.unpack(), H2 = h2.unpack(shared_from_this()), C = cos.unpack(), Sn = sin.unpack();
-  const Tensor X = s.residual ? Tensor() : x.unpack();
+  const Tensor B = packed16(buf.unpack()), H2 = packed16(h2.unpack(shared_from_this())), C = packed16(cos.unpack()), Sn = packed16(sin.unpack());
+  const Tensor X = s.residual ? Tensor() : packed16(x.unpack());
   std::array<Tensor, LP_COUNT> w;
-  for (int i = 0; i < LP_COUNT; i++) w[i] = params[i].unpack();
+  for (int i = 0; i < LP_COUNT; i++) w[i] = packed16(params[i].unpack());
   at::AutoDispatchBelowADInplaceOrView below;
   c10::DeviceGuard guard(B.device());
   void* st = stream_of(B.device());
@@ -1101,8 +1111,8 @@ variable_list LayerNode::apply(variable_list&& g) {
   const int64_t R = s.rows, NQ = s.Hq * s.D, NK = s.Hkv * s.D;
   const size_t e = s.dtype == TP_F32 ? 4 : 2;
   const auto opts = H2.options();
-  const Tensor go = g[0].defined() ? g[0].to(H2.scalar_type()).contiguous() : at::zeros(H2.sizes(), opts);
-  const Tensor gh = g[1].defined() ? g[1].to(H2.scalar_type()).contiguous() : at::zeros(H2.sizes(), opts);
+  const Tensor go = g[0].defined() ? packed16(g[0].to(H2.scalar_type())) : at::zeros(H2.sizes(), opts);
+  const Tensor gh = g[1].defined() ? packed16(g[1].to(H2.scalar_type())) : at::zeros(H2.sizes(), opts);
   const auto need = [&](int i) { return task_should_compute_output(2 + i); };
   const auto grad_of = [&](int i) { return out[2 + i] = at::empty(w[i].sizes(), w[i].options()); };
   // scratch
@@ -1196,14 +1206,14 @@ std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const s
   // the two projections whose input is made here: shape, layout, and the same line on size
   const auto lin_ok = [&](const Tensor& t, int64_t n, int64_t k) {
     return t.dim() == 2 && t.size(0) == n && t.size(1) == k && t.scalar_type() == dt && t.is_contiguous() && plain_eager(t) && t.device() == x.device() &&
-           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && s.rows * n * k <= lin_max_work(dt) && lin_fits(s.rows, n, k, x.element_size());
+           at16(t) && s.rows * n * k <= lin_max_work(dt) && lin_fits(s.rows, n, k, x.element_size());
   };
   if (!lin_ok(w[LP_O], s.H, NQ) || !lin_ok(w[LP_D], s.H, s.I)) return {};
   for (const Tensor* t : {&cos, &sin})
     if (t->dim() != 3 || (t->size(0) != 1 && t->size(0) != s.B) || t->size(1) != s.S || t->size(2) != s.D || t->scalar_type() != dt ||
         !t->is_contiguous() || !plain_eager(*t) || t->device() != x.device() || t->requires_grad()) return {};
   for (const Tensor* t : {&x, &residual})
-    if (t->defined() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16) return {};
+    if (t->defined() && !at16(*t)) return {};
 
   std::shared_ptr<LayerNode> node;
   if (at::GradMode::is_enabled()) {
@@ -1285,11 +1295,11 @@ struct EmbeddingNode : torch::autograd::Node {
   variable_list apply(variable_list&& g) override {
     std::lock_guard<std::mutex> lock(mutex_);
     if (!g[0].defined()) return {Tensor()};
-    const Tensor i = ids.unpack();
-    if (at::GradMode::is_enabled() || !plain_eager(g[0])) return {at::embedding_dense_backward(g[0], i, vocab, -1, false)};
+    const Tensor kept = ids.unpack();
+    if (at::GradMode::is_enabled() || !plain_eager(g[0])) return {at::embedding_dense_backward(g[0], kept, vocab, -1, false)};
     at::AutoDispatchBelowADInplaceOrView below;
-    c10::DeviceGuard guard(i.device());
-    const Tensor dy = g[0].to(opts.dtype().toScalarType()).contiguous();
+    c10::DeviceGuard guard(kept.device());
+    const Tensor dy = packed16(g[0].to(opts.dtype().toScalarType())), i = packed16(kept);
     Tensor dt = at::empty({vocab, hidden}, opts);
     check(tp_embedding_bwd(dy.data_ptr(), (const int64_t*)i.data_ptr(), dt.data_ptr(), i.numel(), (int)vocab, (int)hidden,
                            dtype_code(dt.scalar_type()), stream_of(i.device())), "tp_embedding_bwd");
@@ -1300,7 +1310,7 @@ Tensor py_embedding(const Tensor& ids, const Tensor& table) {
   const auto t = table.scalar_type();
   const bool small = plain_eager(table) && plain_eager(ids) && ids.device() == table.device() && table.dim() == 2 && table.is_contiguous() &&
                      (t == at::kBFloat16 || t == at::kHalf || t == at::kFloat) && ids.scalar_type() == at::kLong && ids.numel() > 0 &&
-                     table.size(0) > 0 && table.size(1) > 0 && table.size(1) % 2 == 0 && table.size(0) * ids.numel() <= (1ll << 24) &&
+                     table.size(0) > 0 && table.size(1) > 0 && at16(table) && table.size(1) % 2 == 0 && table.size(0) * ids.numel() <= (1ll << 24) &&
                      ids.numel() * table.size(1) <= (1ll << 24);
   if (!small) return at::embedding(table, ids);
   auto node = make_node<EmbeddingNode>(table);
@@ -1338,13 +1348,13 @@ struct HeadNode : torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     variable_list out(4);  // x, residual, norm weight, lm_head weight
     if (!g[0].defined()) return out;
-    const Tensor H = h.unpack(), N = n.unpack(), R = rstd.unpack(), nw = norm_w.unpack(), lw = lm_w.unpack();
+    const Tensor H = packed16(h.unpack()), N = packed16(n.unpack()), R = packed16(rstd.unpack()), nw = packed16(norm_w.unpack()), lw = packed16(lm_w.unpack());
     at::AutoDispatchBelowADInplaceOrView below;
     c10::DeviceGuard guard(H.device());
     void* st = stream_of(H.device());
     const int64_t k = H.size(-1), rows = H.numel() / k, V = lw.size(0);
     const int code = dtype_code(H.scalar_type());
-    const Tensor go = g[0].to(H.scalar_type()).contiguous();
+    const Tensor go = packed16(g[0].to(H.scalar_type()));
     const bool dx = task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2);
     Tensor dn;
     std::array<tp_linear_problem, 2> p;
@@ -1376,7 +1386,7 @@ std::optional<Tensor> py_llama_head(const Tensor& x, const Tensor& residual, con
       !plain_eager(residual) || residual.device() != x.device() || norm_w.dim() != 1 || norm_w.size(0) != x.size(-1) || norm_w.scalar_type() != dt ||
       !norm_w.is_contiguous() || !plain_eager(norm_w) || norm_w.device() != x.device()) return std::nullopt;
   for (const Tensor* t : {&x, &residual})
-    if (reinterpret_cast<uintptr_t>(t->data_ptr()) % 16) return std::nullopt;
+    if (!at16(*t)) return std::nullopt;
   auto node = make_node<HeadNode>(x, residual, norm_w, lm_w);
   Tensor h, n, rstd, logits;
   {
