@@ -166,6 +166,28 @@ def test_norm_backward_of_few_rows(rows, hidden):
     assert ((a - b).norm() / b.norm()).item() <= 1e-2
 
 
+def test_a_function_mode_sees_the_modules():
+  """Under an active function mode the model runs module by module, so that the mode sees every projection and lookup; the
+  logits are the same but for the order of fp32 sums."""
+  cfg = tpa.Config(vocab_size=136, num_hidden_layers=2, max_position_embeddings=512, hidden_size=128, intermediate_size=64,
+                   num_attention_heads=2, num_key_value_heads=2, hidden_act="silu", initializer_range=0.02, rms_norm_eps=1e-5,
+                   attention_dropout=False, attention_bias=False, rope_theta=500000.0, attention_kernel="splash_attention")  # fmt: skip
+  model = tpa.LlamaForCausalLM(cfg).to(DEV)
+  ids = torch.randint(136, (1, 37), generator=torch.Generator().manual_seed(1)).to(DEV)
+  names = []
+
+  class Seen(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+      names.append(getattr(func, "__name__", str(func)))
+      return func(*args, **(kwargs or {}))
+
+  want, _ = model(ids)
+  with Seen():
+    got, _ = model(ids)
+  assert names.count("linear") == 2 * 7 + 1 and names.count("embedding") == 1
+  assert ((got - want).norm() / want.norm()).item() <= 1e-5  # (the library's fp32 products: sums in another order)
+
+
 def test_a_recorded_backward_gives_the_gradients_and_no_second_ones():
   """create_graph: the same gradients as without it; differentiating through them raises."""
   cfg = tpa.Config(vocab_size=136, num_hidden_layers=2, max_position_embeddings=512, hidden_size=128, intermediate_size=64,

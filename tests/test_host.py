@@ -79,6 +79,60 @@ def test_ops_reject_cpu_tensors_and_bad_shapes():
     tpa.ops._check_attn(q, q, q, torch.zeros(1, 4, dtype=torch.int32))
 
 
+class _Seen(torch.overrides.TorchFunctionMode):
+  """Notes the name of every call; answers the tprime operators itself (they have no CPU kernels)."""
+
+  def __init__(self):
+    super().__init__()
+    self.names = []
+
+  def __torch_function__(self, func, types, args=(), kwargs=None):
+    name = str(func) if "tprime" in str(func) else getattr(func, "__name__", str(func))
+    self.names.append(name)
+    return (f"{name}[0]", f"{name}[1]", f"{name}[2]") if name.startswith("tprime") else func(*args, **(kwargs or {}))
+
+
+def test_function_modes_and_subclasses_see_projections_and_lookups():
+  from torchprime_amd.linear import embed, project
+
+  a, b, e = torch.nn.Linear(8, 16, bias=False), torch.nn.Linear(8, 8, bias=False), torch.nn.Embedding(5, 8)
+  x, ids = torch.randn(2, 3, 8), torch.tensor([[1, 4]])
+  with _Seen() as seen:
+    outs = project(x, a, b)
+  assert seen.names.count("linear") == 2 and all(torch.equal(o, m(x)) for o, m in zip(outs, (a, b)))
+  with _Seen() as seen:
+    out = embed(e, ids)
+  assert "embedding" in seen.names and torch.equal(out, e(ids))
+
+  class Marked(torch.Tensor):
+    pass
+
+  assert all(type(o) is Marked for o in project(x.as_subclass(Marked), a, b)) and type(embed(e, ids.as_subclass(Marked))) is Marked
+  a.weight = torch.nn.Parameter(a.weight.detach().as_subclass(Marked))
+  assert type(project(x, a)[0]) is Marked
+
+
+def test_function_modes_see_the_operators():
+  o, x, h, m = tpa.ops, torch.ones(2, 8), torch.ones(1, 2, 4, 64), torch.zeros(1, 1, 4, 4)
+  for name, call in (
+    ("rmsnorm_fwd", lambda: o.rmsnorm(x, x[0], 1e-5)), ("add_rmsnorm_fwd", lambda: o.add_rmsnorm(x, x, x[0], 1e-5)),
+    ("rope_table", lambda: o.rope_table_like(x[0], x, 1.0, x)), ("rope_apply", lambda: o.rope_apply(h, h, x, x)),
+    ("attn_fwd", lambda: o.attention(h, h, h)), ("attn_fwd_masked", lambda: o.attention(h, h, h, window=(2, 0))),
+    ("attn_fwd_pairs", lambda: o.attention_pairs(h, h, h, m, 1.0)), ("l2norm_fwd", lambda: o.l2norm(x, 1e-5)),
+    ("swiglu_fwd", lambda: o.swiglu(x, x)), ("cross_entropy_fwd", lambda: o.cross_entropy(h[0], x.long(), -100)),
+  ):  # fmt: skip
+    with _Seen() as seen:
+      call()
+    assert [n for n in seen.names if "tprime" in n] == [f"tprime.{name}.default"], (name, seen.names)
+
+
+def test_mlp_traces_symbolically():
+  g = torch.fx.symbolic_trace(tpa.LlamaMLP(tpa.Config(hidden_size=64, intermediate_size=128)))
+  called = [(n.op, str(n.target)) for n in g.graph.nodes if n.op.startswith("call")]
+  assert [t for k, t in called if k == "call_module"] == ["gate_proj", "up_proj", "down_proj"]
+  assert [t for k, t in called if k == "call_function" and "tprime" in t] == ["tprime.swiglu_fwd.default"]
+
+
 def test_reference_surface_names_and_signatures():
   sig = inspect.signature(tpa.AttentionModule.forward)
   assert list(sig.parameters) == ["self", "query_states", "key_states", "value_states", "attention_mask"]

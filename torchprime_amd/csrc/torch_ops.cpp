@@ -863,7 +863,9 @@ T3 cross_entropy_fwd_autograd(const Tensor& logits, const Tensor& labels, int64_
 // One input through one to three nn.Linear weights (no bias): tp_linears where the products are small, at::linear where
 // they are not, or where anything but plain eager tensors is involved.
 //
-// No mode, transform, autocast or tensor subclass is to see these calls: they do not go through the dispatcher.
+// These calls do not go through the dispatcher: nothing that acts there (dispatch modes, transforms, autocast, tensors with
+// __torch_dispatch__) may be waiting for them.  What acts on Python calls (__torch_function__) is asked for in linear.py
+// and blocks.py, before a tensor becomes a C++ argument.
 bool plain_eager(const Tensor& t) {
   static const c10::DispatchKeySet usual({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
   const c10::DispatchKeySet on = c10::impl::tls_local_dispatch_key_set().included_;

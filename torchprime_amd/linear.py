@@ -9,6 +9,7 @@ import torch
 from torch import nn
 from torch.compiler import is_compiling
 from torch.nn.modules import module as _module
+from torch.overrides import has_torch_function
 
 from .ops import _native
 
@@ -41,7 +42,8 @@ def project(x: torch.Tensor, *modules: nn.Module) -> list[torch.Tensor]:
   """``[m(x) for m in modules]``."""
   if not is_compiling() and not global_hooks():
     ws = [weight_of(m) for m in modules]
-    if all(w is not None for w in ws):
+    # (nor may the call be overridden: fx proxies, tensor subclasses and function modes see the modules' own calls)
+    if all(w is not None for w in ws) and not has_torch_function((x, *ws)):
       return _native.linears(x, ws)
   return [m(x) for m in modules]
 
@@ -50,6 +52,7 @@ def embed(module: nn.Module, ids: torch.Tensor) -> torch.Tensor:
   """``module(ids)`` of an ``nn.Embedding``."""
   if not is_compiling() and plain(module, nn.Embedding) and not global_hooks():
     d = module.__dict__
-    if d["padding_idx"] is None and d["max_norm"] is None and not d["scale_grad_by_freq"] and not d["sparse"]:
-      return _native.embedding(ids, d["_parameters"]["weight"])
+    w = d["_parameters"]["weight"]
+    if d["padding_idx"] is None and d["max_norm"] is None and not d["scale_grad_by_freq"] and not d["sparse"] and not has_torch_function((ids, w)):
+      return _native.embedding(ids, w)
   return module(ids)
