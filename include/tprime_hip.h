@@ -153,8 +153,11 @@ int tp_attn_fwd(const void* q, const void* k, const void* v, const int32_t* seg,
  *                 points give the eager formula's results if [0] and [2] are 0.
  * tp_attn_fwd_pairs   tp_attn_fwd (no segment ids, no causality of its own) over the pairs of `pairs`, made for
  *   mask_batches (1 or B) masks.  bf16 and fp16.  Backward: tp_attn_bwd_run with `pairs`.
+ * tp_attn_pairs_fit   non-zero where all three take masks and heads of these sizes (for head dims (128,128) up to
+ *   about 131000 x 131000, for (192,128) up to 92700 queries); larger masks go through tp_attn_fwd_biased
  * ---------------------------------------------------------------------------------------------- */
 size_t tp_mask_pairs_bytes(int mask_batches, int Sq, int Skv);
+int tp_attn_pairs_fit(int mask_batches, int Sq, int Skv, int Dqk, int Dv);
 int tp_mask_pairs(const void* mask, const int64_t mask_strides[2], int mask_batches, int Sq, int Skv, int dtype, void* pairs,
                   int verdict, void* stream);
 int tp_attn_fwd_pairs(const void* q, const void* k, const void* v, const void* pairs, int mask_batches, void* out, float* lse,

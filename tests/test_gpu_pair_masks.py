@@ -75,3 +75,20 @@ def test_kind(dtype):
   assert kind(empty) == K.MASK_PAIRS
   empty[..., 64, :] = low  # ... of finite entries: uniform weights
   assert kind(empty) == K.MASK_GENERAL
+
+
+def test_more_masks_than_one_launch_takes():
+  """65537 sequences of 4 tokens, each with its padding: kinds over all of them, and the last one's attention."""
+  B, S, low = 65537, 4, float("-inf")
+  causal = torch.full((S, S), low).triu(1)
+  mask = causal.expand(B, 1, S, S).to(DEV, torch.bfloat16)
+  assert tpa.ops.mask_kind(mask) == tpa.ops.MASK_CAUSAL
+  mask = mask.clone()
+  mask[-1, :, 3, 2] = low
+  assert tpa.ops.mask_kind(mask) == tpa.ops.MASK_PAIRS
+  q = heads_view(B, 1, S, 64, 1, torch.bfloat16).to(DEV)
+  m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=1, num_key_value_heads=1))
+  ref = orc.eager_attention(*(q[-1:].float().cpu(),) * 3, mask[-1:].float().cpu())
+  assert_close(m(q, q, q, mask)[-1:], ref, "out")
+  mask[-1, :, 3, 1] = 0.5
+  assert tpa.ops.mask_kind(mask) == tpa.ops.MASK_GENERAL

@@ -228,6 +228,33 @@ def test_attention_module_cpu_side_errors():
     tpa.tpu_splash_attention_jax_call_wrapper(None, q, q, q, "{}", None, True, attn_logits_soft_cap=-1.0)
 
 
+@pytest.mark.parametrize("Dqk,Dv,Sq,Skv,fits", [
+  (128, 128, 8192, 8192, True), (128, 128, 130000, 130000, True), (128, 128, 131200, 131200, False), (192, 128, 92000, 92000, True),
+  (192, 128, 93000, 93000, False), (192, 128, 93000, 4096, False), (64, 64, 130000, 130000, True), (64, 64, 4096, 300000, False)])  # fmt: skip
+def test_masks_too_large_for_bits_are_added(Dqk, Dv, Sq, Skv, fits, monkeypatch):
+  """The module asks whether the pair kernels, forward and backward, take a mask of this size before it hands them one."""
+  assert bool(_lib.load().tp_attn_pairs_fit(1, Sq, Skv, Dqk, Dv)) is fits
+  went = []
+  monkeypatch.setattr(tpa.ops, "mask_kind", lambda m: tpa.ops.MASK_PAIRS)
+  out = lambda q, v: q.new_empty(1).expand(*q.shape[:3], v.shape[3])  # noqa: E731
+  monkeypatch.setattr(tpa.ops, "attention", lambda q, k, v, *a, **kw: went.append("added") or out(q, v))
+  monkeypatch.setattr(tpa.ops, "attention_pairs", lambda q, k, v, *a, **kw: went.append("bits") or out(q, v))
+  t = lambda *shape: torch.zeros((1,) * len(shape), dtype=torch.bfloat16).expand(shape)  # noqa: E731
+  m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=2, num_key_value_heads=2))
+  m(t(1, 2, Sq, Dqk), t(1, 2, Skv, Dqk), t(1, 2, Skv, Dv), t(1, 1, Sq, Skv))
+  assert went == ["bits" if fits else "added"]
+
+
+def test_pair_kernels_take_no_more_than_they_say():
+  """Past tp_attn_pairs_fit an entry point refuses on the host, before any launch (so this runs without a GPU)."""
+  lib, buf = _lib.load(), ctypes.create_string_buffer(64)
+  p = ctypes.addressof(buf) + (-ctypes.addressof(buf)) % 16
+  z2 = (ctypes.c_int64 * 2)(0, 0)
+  for b, sq, skv in ((65536, 8, 8), (1, 128 * 32768, 8)):
+    assert not lib.tp_attn_pairs_fit(b, sq, skv, 128, 128) and lib.tp_mask_pairs(p, z2, b, sq, skv, 0, p, 0, None) == -2
+  assert b"too large" in lib.tp_last_error()
+
+
 def test_ops_trace_with_fake_tensors():
   """register_fake shapes/dtypes/layouts: what AOT tracing (torchprime's remat tooling) relies on."""
   from torch._subclasses.fake_tensor import FakeTensorMode

@@ -87,6 +87,7 @@ SIGNATURES = {
   ),
   "tp_linears": (c_int, [c_void_p, c_int, c_int, c_void_p]),
   "tp_mask_pairs_bytes": (c_size_t, [c_int] * 3),
+  "tp_attn_pairs_fit": (c_int, [c_int] * 5),
   "tp_mask_pairs": (c_int, [c_void_p, c_int64 * 2] + [c_int] * 4 + [c_void_p, c_int, c_void_p]),
   "tp_attn_fwd_pairs": (c_int, [c_void_p] * 4 + [c_int] + [c_void_p] * 2 + [c_int] * 7 + [_I64x3] * 4 + [c_float, c_int, c_void_p]),
   "tp_attn_bwd_parts_bytes": (c_size_t, [c_void_p]),

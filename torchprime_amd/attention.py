@@ -141,7 +141,7 @@ class AttentionModule(nn.Module):
         # (a float16 mask's lowest value drops a pair for float16 logits only; fp32 has no kernels for pair bits)
         by_bits = kind == ops.MASK_PAIRS and bias.shape[0] in (1, bsz) and (
           query_states.dtype == torch.bfloat16 and bias.dtype != torch.float16 or query_states.dtype == torch.float16
-        )
+        ) and ops.attention_pairs_fit(query_states, key_states, value_states, bias)
         if by_bits:
           attn_output = ops.attention_pairs(query_states, key_states, value_states, bias.detach(), scale)
         else:

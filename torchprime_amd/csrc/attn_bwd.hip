@@ -2014,6 +2014,18 @@ struct LeanDq {
   static bool taken(int Skv) { return BUILT && lds_bytes(Skv) <= 160 * 1024; }
 };
 
+// LDS of the dK/dV kernel: three row-major buffers of Q and dO tiles, the row vectors (pair masks: and the rows' bits), the
+// tile list; the id ranges borrow the tile buffers
+template <int DQK, int DV, int SEG>
+struct DkdvLds {
+  static constexpr int NBUF = 3, BMQ = 64, BNK = 128;
+  static constexpr size_t BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES;
+  static_assert(NBUF * BUF <= 144 * 1024, "the three buffers must leave room for the row vectors and the tile list");
+  static size_t tiles(int Sq) { return (size_t)((Sq + BMQ - 1) / BMQ); }
+  static size_t bytes(int Sq) { return NBUF * BUF + 3 * (BMQ * 16 + (SEG == SEG_PAIRS ? BNK * 8 : 0)) + (SEG ? (6 * tiles(Sq) + 8 + 4) * 4 : 0); }
+  static bool fits(int Sq) { return bytes(Sq) <= 160 * 1024 && 3 * tiles(Sq) * 4 <= NBUF * BUF; }
+};
+
 // the plan of a problem as the dK/dV kernel sees it: its band (all keys where the mask is something else)
 static SplitPlan bwd_split_plan(const BwdArgs& a, bool causal) {
   const int lo = causal ? a.band_lo : a.mx.on && !a.mx.qpos ? a.mx.lo_off : BAND_INF;
@@ -2027,14 +2039,10 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
   const int groups = a.B * a.Hkv;
   typedef LeanDq<DQK, DV, CAUSAL, SEG> Lean;
   const bool lean = Lean::taken(a.Skv);
-  // dK/dV: three row-major buffers of Q and dO tiles, the row vectors, the tile list (checked before anything is launched)
-  constexpr int DKDV_NBUF = 3, DKDV_BMQ = 64, DKDV_BNK = 128;
-  constexpr int DKDV_BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES;
-  static_assert(DKDV_NBUF * DKDV_BUF <= 144 * 1024, "the three buffers must leave room for the row vectors and the tile list");
-  const int nqt = (a.Sq + DKDV_BMQ - 1) / DKDV_BMQ;
-  const size_t dkdv_smem = (size_t)DKDV_NBUF * DKDV_BUF + 3 * (DKDV_BMQ * 16 + (SEG == SEG_PAIRS ? DKDV_BNK * 8 : 0)) + (SEG ? (size_t)(6 * nqt + 8 + 4) * 4 : 0);
-  TP_REQUIRE(dkdv_smem <= 160 * 1024 && (size_t)3 * nqt * 4 <= (size_t)DKDV_NBUF * DKDV_BUF, TP_ERR_UNSUPPORTED,
-             "tp_attn_bwd: Sq=%d needs %zu bytes of LDS (max 163840)", a.Sq, dkdv_smem);
+  typedef DkdvLds<DQK, DV, SEG> Dkdv;
+  constexpr int DKDV_NBUF = Dkdv::NBUF, DKDV_BNK = Dkdv::BNK;
+  const size_t dkdv_smem = Dkdv::bytes(a.Sq);  // (checked before anything is launched)
+  TP_REQUIRE(Dkdv::fits(a.Sq), TP_ERR_UNSUPPORTED, "tp_attn_bwd: Sq=%d needs %zu bytes of LDS (max 163840)", a.Sq, dkdv_smem);
   mark(ev, 0, st);
   if (!lean) {
     // delta
@@ -2202,6 +2210,13 @@ extern "C" int tp_attn_bwd_dq_first(int Skv, int Dqk, int Dv, int causal, int ha
   if (Dqk == 64 && Dv == 64) return pick(I64{}, I64{});
   if (Dqk == 192 && Dv == 128) return pick(I192{}, I128{});
   return 0;
+}
+
+extern "C" int tp_attn_pairs_fit(int mask_batches, int Sq, int Skv, int Dqk, int Dv) {
+  if (!pair_mask_sizes_ok(mask_batches, Sq, Skv) || !pair_bits_in_reach(Sq, Skv) || !attn_fwd_pairs_lists_fit(Skv, Dqk, Dv)) return 0;
+  if (Dqk == 128 && Dv == 128) return LeanDq<128, 128, true, SEG_PAIRS>::taken(Skv) && DkdvLds<128, 128, SEG_PAIRS>::fits(Sq);
+  if (Dqk == 64 && Dv == 64) return LeanDq<64, 64, true, SEG_PAIRS>::taken(Skv) && DkdvLds<64, 64, SEG_PAIRS>::fits(Sq);
+  return LeanDq<192, 128, true, SEG_PAIRS>::taken(Skv) && DkdvLds<192, 128, SEG_PAIRS>::fits(Sq);
 }
 
 extern "C" size_t tp_attn_bwd_workspace_bytes(int B, int Hq, int Sq) {
@@ -2374,7 +2389,7 @@ extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {
     TP_REQUIRE(p->mask_batches == 1 || p->mask_batches == p->B, TP_ERR_BAD_ARG, "tp_attn_bwd_run: %d masks for %d batches", p->mask_batches, p->B);
     TP_REQUIRE(p->Sq > 0 && p->Skv > 0, TP_ERR_BAD_ARG, "tp_attn_bwd_run: non-positive size");
     TP_REQUIRE(p->dtype == TP_BF16 || p->dtype == TP_F16, TP_ERR_UNSUPPORTED, "tp_attn_bwd_run: pairs: dtype %d (bf16 and fp16 only)", p->dtype);
-    TP_REQUIRE((int64_t)((p->Sq + 127) / 128 + 1) * 128 * ((p->Skv + 127) / 128 + 1) * 16 < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_bwd_run: mask too large");
+    TP_REQUIRE(pair_bits_in_reach(p->Sq, p->Skv), TP_ERR_UNSUPPORTED, "tp_attn_bwd_run: mask too large");
     pm = pair_mask(p->pairs, p->mask_batches, p->Sq, p->Skv);
   }
   const MaskExt mx = problem_mask(*p);

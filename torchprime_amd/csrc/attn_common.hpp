@@ -199,6 +199,15 @@ struct PairLayout {
     bytes = at;
   }
 };
+// The sizes that can be bits: what the kernel that makes them takes (its grid), and the 32-bit byte offsets into one mask
+// with which the attention kernels read them (dK/dV up to a block past the end).
+inline bool pair_mask_sizes_ok(int Bm, int Sq, int Skv) {
+  return Bm > 0 && Sq > 0 && Skv > 0 && Bm < 65536 && (Sq + 127) / 128 < 32768 && (int64_t)Sq * Skv < (1ll << 40);
+}
+inline bool pair_bits_in_reach(int Sq, int Skv) {
+  return (int64_t)((Sq + 127) / 128 + 1) * 128 * ((Skv + 127) / 128 + 1) * 16 < (1ll << 31);
+}
+bool attn_fwd_pairs_lists_fit(int Skv, int Dqk, int Dv);  // (attn_fwd.hip)
 inline PairMask no_pair_mask() { return PairMask{nullptr, nullptr, nullptr, nullptr, 0}; }
 inline PairMask pair_mask(const void* pairs, int Bm, int Sq, int Skv) {
   const PairLayout l(Bm, Sq, Skv);

@@ -614,14 +614,23 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
 // ------------------------------------------------------------------------------------------------
 // host dispatch
 // ------------------------------------------------------------------------------------------------
+// LDS of a launch: the two tile buffers, then the list of tiles; the id ranges borrow the tile buffers
+template <int DQK, int DV, int SEG>
+struct FwdLds {
+  static constexpr int BN = 64, BM = 128;
+  static constexpr size_t BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES + (SEG == SEG_PAIRS ? BM * 8 : SEG ? BN * 4 : 0);
+  static size_t tiles(int Skv) { return (size_t)((Skv + BN - 1) / BN); }
+  static size_t bytes(int Skv) { return 2 * BUF + (SEG ? 16 * tiles(Skv) : 0); }
+  static bool fits(int Skv) { return bytes(Skv) <= 160 * 1024 && (!SEG || (2 * tiles(Skv) + 16) * 4 <= 2 * BUF); }
+};
+
 template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
 static int launch_fwd(const FwdArgs& args, int B, hipStream_t st) {
   FwdArgs a = args;
-  constexpr int BN = 64, BM = 128;
-  constexpr int BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES + (SEG == SEG_PAIRS ? BM * 8 : SEG ? BN * 4 : 0);
-  const int ntiles_max = (a.Skv + BN - 1) / BN;
-  const size_t smem = 2 * (size_t)BUF + (SEG ? (size_t)16 * ntiles_max : 0);  // (the id ranges borrow the tile buffers)
-  TP_REQUIRE(smem <= 160 * 1024 && (!SEG || (size_t)(2 * ntiles_max + 16) * 4 <= 2 * (size_t)BUF), TP_ERR_UNSUPPORTED, "tp_attn_fwd: Skv=%d needs %zu bytes of LDS (max 163840)", a.Skv, smem);
+  typedef FwdLds<DQK, DV, SEG> Lds;
+  constexpr int BM = Lds::BM;
+  const size_t smem = Lds::bytes(a.Skv);
+  TP_REQUIRE(Lds::fits(a.Skv), TP_ERR_UNSUPPORTED, "tp_attn_fwd: Skv=%d needs %zu bytes of LDS (max 163840)", a.Skv, smem);
   auto kern = attn_fwd_kernel<T, DQK, DV, CAUSAL, SEG>;
   static bool attr_set = false;  // benign race: every thread sets the same value
   if (!attr_set) {
@@ -768,6 +777,12 @@ extern "C" int tp_attn_fwd_biased(const void* q, const void* k, const void* v, c
                        causal, dtype, stream,
                        make_mask_ext(q_positions, causal, causal_offset, window_left, window_right, logits_soft_cap, sm_scale, bias,
                                      bias_strides));
+}
+
+bool tp::attn_fwd_pairs_lists_fit(int Skv, int Dqk, int Dv) {
+  if (Dqk == 128 && Dv == 128) return FwdLds<128, 128, SEG_PAIRS>::fits(Skv);
+  if (Dqk == 64 && Dv == 64) return FwdLds<64, 64, SEG_PAIRS>::fits(Skv);
+  return Dqk == 192 && Dv == 128 && FwdLds<192, 128, SEG_PAIRS>::fits(Skv);
 }
 
 extern "C" int tp_attn_fwd_pairs(const void* q, const void* k, const void* v, const void* pairs, int mask_batches, void* out, float* lse,

@@ -130,7 +130,7 @@ extern "C" int tp_mask_pairs(const void* mask, const int64_t mask_strides[2], in
   TP_REQUIRE(mask_batches > 0 && Sq > 0 && Skv > 0, TP_ERR_BAD_ARG, "tp_mask_pairs: non-positive size");
   TP_REQUIRE(mask_strides[0] >= 0 && mask_strides[1] >= 0, TP_ERR_BAD_ARG, "tp_mask_pairs: negative stride");
   TP_REQUIRE(aligned16(pairs), TP_ERR_BAD_ARG, "tp_mask_pairs: pairs must be 16-byte aligned");
-  TP_REQUIRE(mask_batches < 65536 && (Sq + 127) / 128 < 32768 && (int64_t)Sq * Skv < (1ll << 40), TP_ERR_UNSUPPORTED, "tp_mask_pairs: mask too large");
+  TP_REQUIRE(pair_mask_sizes_ok(mask_batches, Sq, Skv), TP_ERR_UNSUPPORTED, "tp_mask_pairs: mask too large");
   hipStream_t st = (hipStream_t)stream;
   if (dtype == TP_BF16) return mask_typed<bf16_t>(mask, mask_batches, Sq, Skv, mask_strides, pairs, verdict != 0, st);
   if (dtype == TP_F16) return mask_typed<f16_t>(mask, mask_batches, Sq, Skv, mask_strides, pairs, verdict != 0, st);

@@ -1450,17 +1450,23 @@ Tensor py_attention_pairs(const Tensor& q, const Tensor& k, const Tensor& v, con
   return std::get<0>(op_attn_fwd_pairs()(q, k, v, mask, sm_scale));
 }
 // What a (1|B, 1, Sq, Skv) mask is: 1 the exact causal mask, 2 one that only drops pairs, 0 anything else.  Two short
-// kernels and one synchronisation.
+// kernels and one synchronisation (for each 65535 masks, as many as their grid takes).
 int64_t py_mask_kind(const Tensor& mask) {
   const c10::Device dev = require_gpu(mask);
   TORCH_CHECK_VALUE(mask.dim() == 4, "expected a 4-D mask");
   if (mask.numel() == 0) return 0;
   c10::DeviceGuard guard(dev);
   at::AutoDispatchBelowADInplaceOrView below;
-  const PairsIn m = prep_pairs(mask, mask.size(2), mask.size(3));
-  const Tensor flags = make_pairs(m, mask.size(2), mask.size(3), true, stream_of(dev)).slice(0, 0, 16).cpu();
-  const int* f = flags.const_data_ptr<int>();
-  return !f[1] ? 1 : (!f[0] && !f[2]) ? 2 : 0;
+  constexpr int64_t MOST = 65535;
+  const int64_t Sq = mask.size(2), Skv = mask.size(3);
+  int other = 0, not_causal = 0, empty_finite = 0;
+  for (int64_t b = 0; b < mask.size(0); b += MOST) {
+    const PairsIn m = prep_pairs(mask.size(0) <= MOST ? mask : mask.slice(0, b, b + MOST), Sq, Skv);
+    const Tensor flags = make_pairs(m, Sq, Skv, true, stream_of(dev)).slice(0, 0, 16).cpu();
+    const int* f = flags.const_data_ptr<int>();
+    other |= f[0]; not_causal |= f[1]; empty_finite |= f[2];
+  }
+  return !not_causal ? 1 : (!other && !empty_finite) ? 2 : 0;
 }
 Tensor py_l2norm(const Tensor& x, double eps) { return std::get<0>(op_l2norm_fwd()(x, eps)); }
 Tensor py_swiglu(const Tensor& g, const Tensor& u) { return op_swiglu_fwd()(g, u); }
@@ -1542,6 +1548,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention_pairs", &py_attention_pairs);
   m.def("mask_kind", &py_mask_kind);
   m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
+  m.def("attention_pairs_fit", [](int64_t Bm, int64_t Sq, int64_t Skv, int64_t Dqk, int64_t Dv) {
+    const auto is_int = [](int64_t v) { return v >= 0 && v < (1ll << 31); };
+    return is_int(Bm) && is_int(Sq) && is_int(Skv) && is_int(Dqk) && is_int(Dv) && tp_attn_pairs_fit((int)Bm, (int)Sq, (int)Skv, (int)Dqk, (int)Dv) != 0;
+  });
   m.def("linears", &py_linears);
   m.def("llama_layer", &py_llama_layer);
   m.def("llama_head", &py_llama_head);

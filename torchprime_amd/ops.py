@@ -279,6 +279,12 @@ def mask_kind(mask: Tensor) -> int:
   return _native.mask_kind(mask)
 
 
+def attention_pairs_fit(q: Tensor, k: Tensor, v: Tensor, mask: Tensor) -> bool:
+  """The kernels behind ``attention_pairs``, forward and backward, take problems of these sizes (they keep lists of tiles
+  in LDS and address a mask's bits with 32 bits); ``attention(bias=mask)`` goes further."""
+  return _native.attention_pairs_fit(mask.shape[0], q.shape[2], k.shape[2], q.shape[3], v.shape[3])
+
+
 def attention_pairs(q: Tensor, k: Tensor, v: Tensor, mask: Tensor, sm_scale: float) -> Tensor:
   """Attention under an additive mask of kind ``MASK_PAIRS`` (1|B, 1, Sq, Skv): as ``attention(bias=mask)``, with the
   mask as one bit per pair, tiles without a pair left out and tiles with every pair unmasked.  bfloat16 and float16."""
