@@ -235,7 +235,7 @@ def test_masks_too_large_for_bits_are_added(Dqk, Dv, Sq, Skv, fits, monkeypatch)
   """The module asks whether the pair kernels, forward and backward, take a mask of this size before it hands them one."""
   assert bool(_lib.load().tp_attn_pairs_fit(1, Sq, Skv, Dqk, Dv)) is fits
   went = []
-  monkeypatch.setattr(tpa.ops, "mask_kind", lambda m: tpa.ops.MASK_PAIRS)
+  monkeypatch.setattr(tpa.attention, "_mask_verdict", lambda *a: tpa.ops.MASK_PAIRS)
   out = lambda q, v: q.new_empty(1).expand(*q.shape[:3], v.shape[3])  # noqa: E731
   monkeypatch.setattr(tpa.ops, "attention", lambda q, k, v, *a, **kw: went.append("added") or out(q, v))
   monkeypatch.setattr(tpa.ops, "attention_pairs", lambda q, k, v, *a, **kw: went.append("bits") or out(q, v))
@@ -243,6 +243,19 @@ def test_masks_too_large_for_bits_are_added(Dqk, Dv, Sq, Skv, fits, monkeypatch)
   m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=2, num_key_value_heads=2))
   m(t(1, 2, Sq, Dqk), t(1, 2, Skv, Dqk), t(1, 2, Skv, Dv), t(1, 1, Sq, Skv))
   assert went == ["bits" if fits else "added"]
+
+
+def test_causal_masks_are_known_wherever_they_lie(monkeypatch):
+  """The kernels do not read a causal mask, so one on the host or in another type is as good (fp64 here)."""
+  went = []
+  monkeypatch.setattr(tpa.ops, "attention", lambda q, k, v, *a, **kw: went.append((a, kw)) or q)
+  m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=2, num_key_value_heads=2))
+  q = torch.zeros(1, 2, 8, 64)
+  for dtype in (torch.float32, torch.float64):
+    mask = orc.causal_additive_mask(8).to(dtype)
+    m(q, q, q, mask)
+    m(q, q, q, mask + torch.ones(8, 8).tril())
+  assert [a[2] for a, kw in went] == [True, False] * 2 and ["bias" in kw for a, kw in went] == [False, True] * 2
 
 
 def test_pair_kernels_take_no_more_than_they_say():

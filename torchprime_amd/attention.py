@@ -47,10 +47,14 @@ def _mask_verdict(mask: torch.Tensor, q_len: int, kv_len: int) -> int:
     return entry[2]
   kind = ops.MASK_GENERAL
   # (per-head masks and other shapes are evaluated element by element)
-  if mask.dim() == 4 and mask.shape[1] == 1 and mask.shape[2] == q_len and mask.shape[3] >= kv_len and mask.dtype in (
-    torch.bfloat16, torch.float16, torch.float32,
-  ):  # fmt: skip
-    kind = ops.mask_kind(mask[:, :, :, :kv_len])
+  if mask.dim() == 4 and mask.shape[1] == 1 and mask.shape[2] == q_len and mask.shape[3] >= kv_len:
+    m = mask[:, :, :, :kv_len]
+    if m.is_cuda and m.dtype in (torch.bfloat16, torch.float16, torch.float32):
+      kind = ops.mask_kind(m)
+    else:  # (a causal mask is not read any further: it may be of any type and on the host)
+      keep = torch.ones((q_len, kv_len), dtype=torch.bool, device=m.device).tril()
+      if bool((((m == 0) == keep) & ((m == float("-inf")) == ~keep)).all()):
+        kind = ops.MASK_CAUSAL
   # the entry leaves with the tensor (its id may be reused afterwards, hence also the identity check above)
   ref = weakref.ref(mask, lambda _r, ident=ident: _MASK_VERDICTS.pop(ident, None))
   _MASK_VERDICTS[ident] = (ref, key, kind)
