@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import torchprime_amd as tpa
-from tests.util import randn
+from tests.util import randn, ticks_during
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -65,3 +65,19 @@ def test_saved_tensor_hooks_and_trace():
   for outs in (hooked, traced):
     assert all(torch.equal(a, b) for a, b in zip(outs, want))
     assert all(torch.equal(a, b) for a, b in zip(grads(outs), g_want))
+
+
+def test_waits_for_the_device_let_other_threads_run():
+  """The kind of a mask and the range of position ids are read back from the device, behind whatever is queued there."""
+  a = randn((8192, 8192), 1, BF).to(DEV)
+  b = torch.empty_like(a)
+  q, pos = _leaf((1, 2, 9, 64), 1), torch.arange(9, device=DEV)[None]
+  table = randn((16, 64), 2, BF).to(DEV)
+  mask = torch.full((9, 9), float("-inf"), device=DEV).triu(1)[None, None]
+  tpa.ops.mask_kind(mask), tpa.ops.rope_apply(q, q, table, table, pos.clone()), torch.mm(a, a, out=b)
+  for call in (lambda: tpa.ops.mask_kind(mask), lambda: tpa.ops.rope_apply(q, q, table, table, pos)):
+    torch.cuda.synchronize()
+    for _ in range(150):  # 0.1 s and more
+      torch.mm(a, a, out=b)
+    n, took = ticks_during(call)
+    assert took > 0.03 and n > 0, (n, took)

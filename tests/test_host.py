@@ -12,6 +12,7 @@ import torch
 
 import torchprime_amd as tpa
 from oracle import tprime_oracle as orc
+from tests.util import ticks_during
 from torchprime_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -124,6 +125,15 @@ def test_function_modes_see_the_operators():
     with _Seen() as seen:
       call()
     assert [n for n in seen.names if "tprime" in n] == [f"tprime.{name}.default"], (name, seen.names)
+
+
+def test_native_calls_let_other_threads_run():
+  from torchprime_amd.linear import project
+
+  m, x = torch.nn.Linear(4096, 4096, bias=False), torch.randn(2048, 4096)
+  with torch.no_grad():
+    n, took = ticks_during(lambda: project(x, m))
+  assert took < 0.03 or n > 0, (n, took)
 
 
 def test_mlp_traces_symbolically():

@@ -2,6 +2,8 @@
 
 import json
 import os
+import threading
+import time
 
 import torch
 
@@ -91,3 +93,26 @@ def off_address(t: torch.Tensor) -> torch.Tensor:
   v.copy_(t)
   assert v.is_contiguous() and v.data_ptr() % 16
   return v
+
+
+def ticks_during(call) -> tuple[int, float]:
+  """How often another Python thread got to run while ``call`` did, a few milliseconds in from both ends, and how long
+  ``call`` took."""
+  stamps, stop = [], threading.Event()
+
+  def tick():
+    while not stop.is_set():
+      stamps.append(time.perf_counter())
+      time.sleep(0.001)
+
+  t = threading.Thread(target=tick)
+  t.start()
+  try:
+    time.sleep(0.01)
+    start = time.perf_counter()
+    call()
+    end = time.perf_counter()
+  finally:
+    stop.set()
+    t.join()
+  return sum(start + 0.005 < s < end - 0.005 for s in stamps), end - start

@@ -1539,24 +1539,27 @@ TORCH_LIBRARY_IMPL(tprime, Autograd, m) {
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("rmsnorm", &py_rmsnorm);
-  m.def("add_rmsnorm", &py_add_rmsnorm);
-  m.def("rope_table", &py_rope_table);
-  m.def("rope_apply", &py_rope_apply);
-  m.def("attention", &py_attention);
-  m.def("attention_masked", &py_attention_masked);
-  m.def("attention_pairs", &py_attention_pairs);
-  m.def("mask_kind", &py_mask_kind);
+  // Other Python threads run meanwhile: some of these wait for the device (mask_kind, rope_apply with positions), and any
+  // launch or allocation may.
+  const py::call_guard<py::gil_scoped_release> no_gil;
+  m.def("rmsnorm", &py_rmsnorm, no_gil);
+  m.def("add_rmsnorm", &py_add_rmsnorm, no_gil);
+  m.def("rope_table", &py_rope_table, no_gil);
+  m.def("rope_apply", &py_rope_apply, no_gil);
+  m.def("attention", &py_attention, no_gil);
+  m.def("attention_masked", &py_attention_masked, no_gil);
+  m.def("attention_pairs", &py_attention_pairs, no_gil);
+  m.def("mask_kind", &py_mask_kind, no_gil);
   m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
   m.def("attention_pairs_fit", [](int64_t Bm, int64_t Sq, int64_t Skv, int64_t Dqk, int64_t Dv) {
     const auto is_int = [](int64_t v) { return v >= 0 && v < (1ll << 31); };
     return is_int(Bm) && is_int(Sq) && is_int(Skv) && is_int(Dqk) && is_int(Dv) && tp_attn_pairs_fit((int)Bm, (int)Sq, (int)Skv, (int)Dqk, (int)Dv) != 0;
   });
-  m.def("linears", &py_linears);
-  m.def("llama_layer", &py_llama_layer);
-  m.def("llama_head", &py_llama_head);
-  m.def("embedding", &py_embedding);
-  m.def("l2norm", &py_l2norm);
-  m.def("swiglu", &py_swiglu);
-  m.def("cross_entropy", &py_cross_entropy);
+  m.def("linears", &py_linears, no_gil);
+  m.def("llama_layer", &py_llama_layer, no_gil);
+  m.def("llama_head", &py_llama_head, no_gil);
+  m.def("embedding", &py_embedding, no_gil);
+  m.def("l2norm", &py_l2norm, no_gil);
+  m.def("swiglu", &py_swiglu, no_gil);
+  m.def("cross_entropy", &py_cross_entropy, no_gil);
 }
