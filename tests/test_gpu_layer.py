@@ -75,6 +75,55 @@ def test_frozen_parameters_and_unused_outputs():
   assert all(torch.equal(a, b) for a, b in zip(one, both))
 
 
+@pytest.mark.parametrize("trained,untouched", [
+  ("down_proj", "q_proj k_proj v_proj o_proj gate_proj up_proj down_proj input_layernorm post_attention_layernorm tables"),
+  ("gate_proj up_proj", "q_proj k_proj v_proj o_proj gate_proj up_proj input_layernorm post_attention_layernorm tables"),
+  ("post_attention_layernorm", "q_proj k_proj v_proj o_proj input_layernorm tables"),
+  ("o_proj", "q_proj k_proj v_proj o_proj input_layernorm tables"), ("k_proj", "q_proj k_proj v_proj input_layernorm"),
+  ("input_layernorm", "")])  # fmt: skip
+@pytest.mark.parametrize("residual", [False, True])
+def test_a_frozen_lower_part_is_left_alone(trained, untouched, residual):
+  """The backward of a layer whose lower part is frozen, from an input without a gradient, forms no gradient there and keeps
+  nothing for it: what lies below may be changed in place after the forward, as with the modules, and the gradients are
+  theirs bit for bit."""
+  layer = _layer(128, 2, 2, 64, "splash_attention", torch.bfloat16)
+  for n, p in layer.named_parameters():
+    p.requires_grad_(any(t in n for t in trained.split()))
+  leaves = [p for p in layer.parameters() if p.requires_grad]
+  x, res = randn((1, 20, 128), 1, torch.bfloat16).to(DEV), randn((1, 20, 128), 2, torch.bfloat16).to(DEV) if residual else None
+  cs = tpa.LlamaRotaryEmbedding(64, 500000.0).to(DEV)(x, torch.arange(20, device=DEV)[None].float())
+  g = [randn((1, 20, 128), 3, torch.bfloat16).to(DEV), randn((1, 20, 128), 4, torch.bfloat16).to(DEV)]
+  outs = layer.forward_deferred(x, res, position_embeddings=cs)
+  assert outs[0].grad_fn.name() == "TprimeLlamaLayerBackward"
+  hook = layer.mlp.register_forward_hook(lambda m, a, o: None)
+  want_outs = layer.forward_deferred(x, res, position_embeddings=cs)
+  hook.remove()
+  used = [i for i, o in enumerate(want_outs) if o.requires_grad]  # (the modules' sum has no gradient if nothing below it has)
+  want = torch.autograd.grad([want_outs[i] for i in used], leaves, [g[i] for i in used])
+  with torch.no_grad():
+    for n, p in layer.named_parameters():
+      if any(t in n for t in untouched.split()):
+        p.zero_()
+    for t in cs if "tables" in untouched else ():
+      t.zero_()
+    if "input_layernorm" in untouched:
+      x.zero_()
+  for a, b in zip(torch.autograd.grad(outs, leaves, g), want):
+    assert torch.equal(a, b)
+
+
+def test_a_head_that_is_tuned_alone_keeps_only_its_input():
+  norm, lm = tpa.LlamaRMSNorm(64).to(DEV).requires_grad_(False), torch.nn.Linear(64, 136, bias=False, device=DEV)
+  x, res = randn((1, 9, 64), 1).to(DEV), randn((1, 9, 64), 2).to(DEV)
+  logits = tpa.ops._native.llama_head(x, res, norm.weight, 1e-6, lm.weight)
+  g = randn((1, 9, 136), 3).to(DEV)
+  (want,) = torch.autograd.grad(logits, lm.weight, g, retain_graph=True)
+  with torch.no_grad():
+    for t in (x, res, norm.weight, lm.weight):
+      t.zero_()
+  assert torch.equal(torch.autograd.grad(logits, lm.weight, g)[0], want)
+
+
 def test_gradients_at_odd_addresses():
   """Gradients of a layer, of the logits and of embedding rows that are contiguous but off the 16-byte addresses (pieces of
   a concatenation): the gradients of the same values at an allocation's start."""

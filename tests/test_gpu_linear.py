@@ -82,6 +82,23 @@ def test_contiguous_at_an_odd_address(dtype):
     assert torch.equal(s, t)
 
 
+def test_what_no_gradient_needs_may_change():
+  """The input of frozen weights and the weight of an input without a gradient are not kept, as with the modules."""
+  m = nn.Linear(64, 64, bias=False, device=DEV)
+  x, g = randn((7, 64), 1).to(DEV).requires_grad_(True), randn((7, 64), 2).to(DEV)
+  want = torch.autograd.grad(project(x, m)[0], [x, m.weight], g)
+  m.weight.requires_grad_(False)
+  h = x * 1
+  y = project(h, m)[0]
+  h.zero_()
+  assert y.grad_fn.name() == "TprimeLinearsBackward" and torch.equal(torch.autograd.grad(y, x, g)[0], want[0])
+  m.weight.requires_grad_(True)
+  y = project(x.detach(), m)[0]
+  with torch.no_grad():
+    m.weight.zero_()
+  assert torch.equal(torch.autograd.grad(y, m.weight, g)[0], want[1])
+
+
 def test_a_weight_past_the_offsets_is_the_library_s():
   """2 GiB of weight and one token: little work, but more than the launch's 32-bit offsets reach."""
   m = nn.Linear(8192, 131072, bias=False, device=DEV, dtype=torch.bfloat16)

@@ -922,9 +922,12 @@ bool linears_take(const Tensor& x, const std::vector<Tensor>& ws) {
   return k % vec == 0 && m * n * k <= lin_max_work(t);
 }
 
+// (x is kept where a weight wants a gradient, the weights where x does: what is not kept may be freed or changed in place)
 struct LinearsNode : torch::autograd::Node {
   SavedVariable x;
   std::vector<SavedVariable> ws;
+  at::TensorOptions opts;
+  std::vector<int64_t> x_sizes, features;
   std::string name() const override { return "TprimeLinearsBackward"; }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -933,67 +936,73 @@ struct LinearsNode : torch::autograd::Node {
   }
   variable_list apply(variable_list&& g) override;
 };
+// c[m, n] = a b over one segment of k; further pairs of operands are added to the sum
 tp_linear_problem lin_problem(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k, bool a_kmajor, bool b_kmajor, int64_t m,
-                              int64_t n, const Tensor& c) {
+                              int64_t n, void* c) {
   tp_linear_problem p{};
   p.a[0] = a; p.b[0] = b; p.lda[0] = lda; p.ldb[0] = ldb; p.k[0] = (int)k; p.segments = 1;
-  p.a_kmajor = a_kmajor; p.b_kmajor = b_kmajor; p.m = (int)m; p.n = (int)n; p.c = c.data_ptr(); p.ldc = n;
+  p.a_kmajor = a_kmajor; p.b_kmajor = b_kmajor; p.m = (int)m; p.n = (int)n; p.c = c; p.ldc = n;
   return p;
+}
+void add_segment(tp_linear_problem& p, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k) {
+  const int i = p.segments++;
+  p.a[i] = a; p.b[i] = b; p.lda[i] = lda; p.ldb[i] = ldb; p.k[i] = (int)k;
 }
 variable_list LinearsNode::apply(variable_list&& g) {
   std::lock_guard<std::mutex> lock(mutex_);
   const size_t nw = ws.size();
   variable_list out(1 + nw);
-  const Tensor xt = x.unpack();
-  std::vector<Tensor> wt;
-  for (auto& w : ws) wt.push_back(w.unpack());
-  bool plain = !at::GradMode::is_enabled();
-  for (const auto& t : g) plain = plain && (!t.defined() || (plain_eager(t) && t.scalar_type() == xt.scalar_type()));
+  const bool want_x = task_should_compute_output(0);
+  const auto want_w = [&](size_t i) { return g[i].defined() && task_should_compute_output(1 + i); };
+  bool any_w = false, plain = !at::GradMode::is_enabled();
+  for (size_t i = 0; i < nw; i++) {
+    any_w = any_w || want_w(i);
+    plain = plain && (!g[i].defined() || (plain_eager(g[i]) && g[i].scalar_type() == opts.dtype().toScalarType()));
+  }
+  const Tensor xt = any_w ? x.unpack() : Tensor();
+  std::vector<Tensor> wt(nw);
+  for (size_t i = 0; i < nw && want_x; i++) wt[i] = ws[i].unpack();
   if (!plain) {  // a graph of the backward is being recorded, or the gradients are not plain tensors
     for (size_t i = 0; i < nw; i++) {
       if (!g[i].defined()) continue;
-      const Tensor g2 = g[i].reshape({-1, g[i].size(-1)});
-      if (task_should_compute_output(0)) {
+      if (want_x) {
         const Tensor d = at::matmul(g[i], wt[i]);
         out[0] = out[0].defined() ? out[0] + d : d;
       }
-      if (task_should_compute_output(1 + i)) out[1 + i] = at::mm(g2.t(), xt.reshape({-1, xt.size(-1)}));
+      if (want_w(i)) out[1 + i] = at::mm(g[i].reshape({-1, g[i].size(-1)}).t(), xt.reshape({-1, xt.size(-1)}));
     }
     return out;
   }
   at::AutoDispatchBelowADInplaceOrView below;
-  c10::DeviceGuard guard(xt.device());
-  for (auto& w : wt) w = packed16(w);
-  const Rows xr = lin_rows(xt);
+  c10::DeviceGuard guard(opts.device());
+  const int64_t k = x_sizes.back();
   std::vector<Rows> gr;  // (keep copies of strided gradients alive until the launch)
   gr.reserve(nw);
   std::array<tp_linear_problem, 4> p;
-  int n = 0, dx = -1;
+  int n = 0;
   for (size_t i = 0; i < nw; i++) {
     if (!g[i].defined()) continue;
     gr.push_back(lin_rows(g[i]));
     const Rows& r = gr.back();
-    const int64_t nf = wt[i].size(0);
-    if (task_should_compute_output(0)) {
-      if (dx < 0) {
-        out[0] = at::empty(xt.sizes(), xt.options());
-        dx = n++;
-        p[dx] = lin_problem(r.ptr(), r.stride, wt[i].data_ptr(), xr.cols, nf, true, false, r.rows, xr.cols, out[0]);
-      } else {
-        const int s = p[dx].segments++;
-        p[dx].a[s] = r.ptr(); p[dx].lda[s] = r.stride; p[dx].b[s] = wt[i].data_ptr(); p[dx].ldb[s] = xr.cols; p[dx].k[s] = (int)nf;
-      }
+    if (!want_x) continue;
+    wt[i] = packed16(wt[i]);
+    if (n == 0) {
+      out[0] = at::empty(x_sizes, opts);
+      p[n++] = lin_problem(r.ptr(), r.stride, wt[i].data_ptr(), k, features[i], true, false, r.rows, k, out[0].data_ptr());
+    } else {
+      add_segment(p[0], r.ptr(), r.stride, wt[i].data_ptr(), k, features[i]);
     }
   }
+  const optional<Rows> xr = any_w ? optional<Rows>(lin_rows(xt)) : std::nullopt;
   size_t j = 0;
   for (size_t i = 0; i < nw; i++) {
     if (!g[i].defined()) continue;
     const Rows& r = gr[j++];
-    if (!task_should_compute_output(1 + i)) continue;
-    out[1 + i] = at::empty(wt[i].sizes(), wt[i].options());
-    p[n++] = lin_problem(r.ptr(), r.stride, xr.ptr(), xr.stride, r.rows, false, false, wt[i].size(0), xr.cols, out[1 + i]);
+    if (!want_w(i)) continue;
+    out[1 + i] = at::empty({features[i], k}, opts);
+    p[n++] = lin_problem(r.ptr(), r.stride, xr->ptr(), xr->stride, r.rows, false, false, features[i], k, out[1 + i].data_ptr());
   }
-  if (n) check(tp_linears(p.data(), n, dtype_code(xt.scalar_type()), stream_of(xt.device())), "tp_linears");
+  if (n) check(tp_linears(p.data(), n, dtype_code(opts.dtype().toScalarType()), stream_of(opts.device())), "tp_linears");
   return out;
 }
 
@@ -1022,14 +1031,20 @@ std::vector<Tensor> py_linears(const Tensor& x, const std::vector<Tensor>& ws) {
     for (size_t i = 0; i < ws.size(); i++) {
       sizes.back() = ws[i].size(0);
       out.push_back(at::empty(sizes, x.options()));
-      p[i] = lin_problem(xr.ptr(), xr.stride, ws[i].data_ptr(), xr.cols, xr.cols, true, true, xr.rows, ws[i].size(0), out[i]);
+      p[i] = lin_problem(xr.ptr(), xr.stride, ws[i].data_ptr(), xr.cols, xr.cols, true, true, xr.rows, ws[i].size(0), out[i].data_ptr());
     }
     check(tp_linears(p.data(), (int)ws.size(), dtype_code(x.scalar_type()), stream_of(x.device())), "tp_linears");
   }
   if (req) {
-    node->x = SavedVariable(x, false);
+    bool any_w = false;
+    for (const auto& w : ws) any_w = any_w || w.requires_grad();
+    if (any_w) node->x = SavedVariable(x, false);
+    node->ws.resize(ws.size());
+    node->opts = x.options();
+    node->x_sizes = x.sizes().vec();
     for (size_t i = 0; i < ws.size(); i++) {
-      node->ws.emplace_back(ws[i], false);
+      if (x.requires_grad()) node->ws[i] = SavedVariable(ws[i], false);
+      node->features.push_back(ws[i].size(0));
       torch::autograd::set_history(out[i], node);
     }
   }
@@ -1063,16 +1078,6 @@ struct LayerBuf {
     bytes = at;
   }
 };
-tp_linear_problem raw_linear(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k, bool akm, bool bkm, int64_t m, int64_t n, void* c) {
-  tp_linear_problem p{};
-  p.a[0] = a; p.b[0] = b; p.lda[0] = lda; p.ldb[0] = ldb; p.k[0] = (int)k; p.segments = 1;
-  p.a_kmajor = akm; p.b_kmajor = bkm; p.m = (int)m; p.n = (int)n; p.c = c; p.ldc = n;
-  return p;
-}
-void add_segment(tp_linear_problem& p, const void* a, int64_t lda, const void* b, int64_t ldb, int64_t k) {
-  const int i = p.segments++;
-  p.a[i] = a; p.b[i] = b; p.lda[i] = lda; p.ldb[i] = ldb; p.k[i] = (int)k;
-}
 // (batch, head, seq) strides of heads side by side in a row
 Strides3 head_strides(const LayerShape& s, int64_t heads) { return {s.S * heads * s.D, s.D, heads * s.D}; }
 // cos / sin rows: batch stride (0: one table for all batches)
@@ -1084,8 +1089,34 @@ void layer_rope(const LayerShape& s, void* q, void* k, const Tensor& cos, const 
                       ks.data(), qs.data(), ks.data(), table_stride(cos, s), cos.stride(1), 0, 0, 0, (int)backward, s.dtype, st), "tp_rope_apply");
 }
 
+// Which gradients a layer's backward forms on its way down, for what is asked for: of the layer's input; of the first
+// norm's output; through attention and rotary; of h, the residual after the attention; of the second norm's output; of gate
+// and up.  With the lower parameters frozen and an input without a gradient the way ends where the modules' would: an MLP
+// that is tuned alone runs neither the attention's backward nor any product below it, and keeps nothing for them.
+struct LayerWants {
+  bool in, n1, attn, h, n2, mlp;
+  template <typename F>
+  LayerWants(bool input, F param) {
+    in = input;
+    n1 = in || param(LP_N1);
+    attn = n1 || param(LP_Q) || param(LP_K) || param(LP_V);
+    h = attn || param(LP_O);
+    n2 = h || param(LP_N2);
+    mlp = n2 || param(LP_G) || param(LP_U);
+  }
+  bool weight(int i) const {
+    switch (i) {
+      case LP_D: return mlp;
+      case LP_G: case LP_U: case LP_N2: return n2;
+      case LP_O: return attn;
+      default: return n1;
+    }
+  }
+};
+
 struct LayerNode : torch::autograd::Node {
   LayerShape s;
+  at::ScalarType scalar;
   SavedVariable x, buf, h2, cos, sin;
   std::vector<SavedVariable> params;
   std::string name() const override { return "TprimeLlamaLayerBackward"; }
@@ -1101,10 +1132,16 @@ variable_list LayerNode::apply(variable_list&& g) {
   std::lock_guard<std::mutex> lock(mutex_);
   variable_list out(2 + LP_COUNT);  // x, residual, the parameters
   if (!g[0].defined() && !g[1].defined()) return out;
-  const Tensor B = packed16(buf.unpack()), H2 = packed16(h2.unpack(shared_from_this())), C = packed16(cos.unpack()), Sn = packed16(sin.unpack());
-  const Tensor X = s.residual ? Tensor() : packed16(x.unpack());
+  const auto need = [&](int i) { return task_should_compute_output(2 + i); };
+  const LayerWants want(task_should_compute_output(0) || task_should_compute_output(1), need);
+  const Tensor B = packed16(buf.unpack());
   std::array<Tensor, LP_COUNT> w;
-  for (int i = 0; i < LP_COUNT; i++) w[i] = packed16(params[i].unpack());
+  for (int i = 0; i < LP_COUNT; i++)
+    if (want.weight(i)) w[i] = packed16(params[i].unpack());
+  Tensor H2, C, Sn, X;
+  if (want.n2) H2 = packed16(h2.unpack(shared_from_this()));
+  if (want.attn) { C = packed16(cos.unpack()); Sn = packed16(sin.unpack()); }
+  if (want.n1 && !s.residual) X = packed16(x.unpack());
   at::AutoDispatchBelowADInplaceOrView below;
   c10::DeviceGuard guard(B.device());
   void* st = stream_of(B.device());
@@ -1112,77 +1149,91 @@ variable_list LayerNode::apply(variable_list&& g) {
   char* base = (char*)B.data_ptr();
   const int64_t R = s.rows, NQ = s.Hq * s.D, NK = s.Hkv * s.D;
   const size_t e = s.dtype == TP_F32 ? 4 : 2;
-  const auto opts = H2.options();
-  const Tensor go = g[0].defined() ? packed16(g[0].to(H2.scalar_type())) : at::zeros(H2.sizes(), opts);
-  const Tensor gh = g[1].defined() ? packed16(g[1].to(H2.scalar_type())) : at::zeros(H2.sizes(), opts);
-  const auto need = [&](int i) { return task_should_compute_output(2 + i); };
-  const auto grad_of = [&](int i) { return out[2 + i] = at::empty(w[i].sizes(), w[i].options()); };
+  const auto opts = B.options().dtype(scalar);
+  const std::array<int64_t, 3> hidden{s.B, s.S, s.H};
+  const auto grad_in = [&](const Tensor& t) { return t.defined() ? packed16(t.to(scalar)) : at::zeros(hidden, opts); };
+  const Tensor go = grad_in(g[0]);
+  const auto grad_of = [&](int i) {
+    const int64_t n[] = {s.H, NQ, NK, NK, s.H, s.H, s.I, s.I, s.H}, k[] = {0, s.H, s.H, s.H, NQ, 0, s.H, s.H, s.I};
+    return out[2 + i] = k[i] ? at::empty({n[i], k[i]}, opts) : at::empty({n[i]}, opts);
+  };
   // scratch
-  const size_t ws_rows = tp_attn_bwd_workspace_bytes((int)s.B, (int)s.Hq, (int)s.S), ws_norm = tp_rmsnorm_bwd_workspace_bytes(R, (int)s.H);
   tp_attn_bwd_problem ab{};
   ab.B = (int)s.B; ab.Hq = (int)s.Hq; ab.Hkv = (int)s.Hkv; ab.Sq = ab.Skv = (int)s.S; ab.Dqk = ab.Dv = (int)s.D;
   ab.causal = s.causal; ab.window_left = ab.window_right = -1; ab.dtype = s.dtype; ab.sm_scale = (float)(1.0 / std::sqrt((double)s.D));
-  ab.parts_bytes = tp_attn_bwd_parts_bytes(&ab);
+  ab.parts_bytes = want.attn ? tp_attn_bwd_parts_bytes(&ab) : 0;
   size_t at = 0;
-  const auto take = [&](size_t n) { const size_t o = at; at += (n + 255) / 256 * 256; return o; };
-  const size_t o_act = take(R * s.I * e), o_dg = take(R * s.I * e), o_du = take(R * s.I * e), o_dn = take(R * s.H * e), o_ds = take(R * s.H * e);
-  const size_t o_da = take(R * NQ * e), o_dq = take(R * NQ * e), o_dk = take(R * NK * e), o_dv = take(R * NK * e);
-  const size_t o_ws = take(ws_rows), o_norm = take(ws_norm), o_parts = take(ab.parts_bytes), o_dw = take(s.H * e);
+  const auto take = [&](bool used, size_t n) { const size_t o = at; at += used ? (n + 255) / 256 * 256 : 0; return o; };
+  const size_t o_act = take(want.mlp, R * s.I * e), o_dg = take(want.mlp, R * s.I * e), o_du = take(want.mlp, R * s.I * e);
+  const size_t o_dn = take(want.n2, R * s.H * e), o_ds = take(want.n2, R * s.H * e);
+  const size_t o_da = take(want.attn, R * NQ * e), o_dq = take(want.attn, R * NQ * e), o_dk = take(want.attn, R * NK * e), o_dv = take(want.attn, R * NK * e);
+  const size_t o_ws = take(want.attn, tp_attn_bwd_workspace_bytes((int)s.B, (int)s.Hq, (int)s.S));
+  const size_t o_norm = take(want.n2, tp_rmsnorm_bwd_workspace_bytes(R, (int)s.H)), o_dw = take(want.n2, s.H * e), o_parts = take(want.attn, ab.parts_bytes);
   const Tensor scratch = at::empty({(int64_t)at}, opts.dtype(at::kByte));
   char* t = (char*)scratch.data_ptr();
   std::array<tp_linear_problem, 4> p;
-  const auto run = [&](int n) { check(tp_linears(p.data(), n, s.dtype, st), "tp_linears"); };
-  const auto wgrad = [&](int i, const void* gr, int64_t nf, const void* in, int64_t k) { return raw_linear(gr, nf, in, k, R, false, false, nf, k, grad_of(i).data_ptr()); };
   int n = 0;
+  const auto wgrad = [&](int i, const void* gr, int64_t nf, const void* in, int64_t k) {
+    if (need(i)) p[n++] = lin_problem(gr, nf, in, k, R, false, false, nf, k, grad_of(i).data_ptr());
+  };
+  const auto run = [&]() { if (n) check(tp_linears(p.data(), n, s.dtype, st), "tp_linears"); n = 0; };
   // down projection
-  p[n++] = raw_linear(go.data_ptr(), s.H, w[LP_D].data_ptr(), s.I, s.H, true, false, R, s.I, t + o_act);
-  if (need(LP_D)) p[n++] = wgrad(LP_D, go.data_ptr(), s.H, base + f.act, s.I);
-  run(n);
-  check(tp_swiglu_bwd(t + o_act, base + f.gate, base + f.up, t + o_dg, t + o_du, R, (int)s.I, s.I, s.I, s.I, s.I, s.I, s.dtype, st), "tp_swiglu_bwd");
+  if (want.mlp) p[n++] = lin_problem(go.data_ptr(), s.H, w[LP_D].data_ptr(), s.I, s.H, true, false, R, s.I, t + o_act);
+  wgrad(LP_D, go.data_ptr(), s.H, base + f.act, s.I);
+  run();
   // gate, up
-  n = 0;
-  p[n] = raw_linear(t + o_dg, s.I, w[LP_G].data_ptr(), s.H, s.I, true, false, R, s.H, t + o_dn);
-  add_segment(p[n++], t + o_du, s.I, w[LP_U].data_ptr(), s.H, s.I);
-  if (need(LP_G)) p[n++] = wgrad(LP_G, t + o_dg, s.I, base + f.n2, s.H);
-  if (need(LP_U)) p[n++] = wgrad(LP_U, t + o_du, s.I, base + f.n2, s.H);
-  run(n);
+  if (want.mlp)
+    check(tp_swiglu_bwd(t + o_act, base + f.gate, base + f.up, t + o_dg, t + o_du, R, (int)s.I, s.I, s.I, s.I, s.I, s.I, s.dtype, st), "tp_swiglu_bwd");
+  if (want.n2) {
+    p[n] = lin_problem(t + o_dg, s.I, w[LP_G].data_ptr(), s.H, s.I, true, false, R, s.H, t + o_dn);
+    add_segment(p[n++], t + o_du, s.I, w[LP_U].data_ptr(), s.H, s.I);
+  }
+  wgrad(LP_G, t + o_dg, s.I, base + f.n2, s.H);
+  wgrad(LP_U, t + o_du, s.I, base + f.n2, s.H);
+  run();
   // norm 2 and the residual's gradient
   const auto norm_bwd = [&](int i, const void* dy, const void* dh, const void* hh, size_t rstd, void* dx) {
     void* dw = need(i) ? grad_of(i).data_ptr() : t + o_dw;
     check(tp_add_rmsnorm_bwd(dy, dh, hh, w[i].data_ptr(), (const float*)(base + rstd), dx, dw, (float*)(t + o_norm), R, (int)s.H, s.H, s.H, s.H, s.H,
                              s.dtype, s.dtype, st), "tp_add_rmsnorm_bwd");
   };
-  norm_bwd(LP_N2, t + o_dn, gh.data_ptr(), H2.data_ptr(), f.rstd2, t + o_ds);
-  // output projection
-  n = 0;
-  p[n++] = raw_linear(t + o_ds, s.H, w[LP_O].data_ptr(), NQ, s.H, true, false, R, NQ, t + o_da);
-  if (need(LP_O)) p[n++] = wgrad(LP_O, t + o_ds, s.H, base + f.attn, NQ);
-  run(n);
-  // attention, rotary
-  ab.dout = t + o_da; ab.q = base + f.q; ab.k = base + f.k; ab.v = base + f.v; ab.out = base + f.attn; ab.lse = (const float*)(base + f.lse);
-  ab.dq = t + o_dq; ab.dk = t + o_dk; ab.dv = t + o_dv; ab.ws = (float*)(t + o_ws);
-  ab.parts = ab.parts_bytes ? t + o_parts : nullptr;
-  const Strides3 qs = head_strides(s, s.Hq), ks = head_strides(s, s.Hkv);
-  for (int i = 0; i < 3; i++) {
-    ab.do_strides[i] = ab.q_strides[i] = ab.o_strides[i] = ab.dq_strides[i] = qs[i];
-    ab.k_strides[i] = ab.v_strides[i] = ab.dk_strides[i] = ab.dv_strides[i] = ks[i];
+  if (want.n2) {
+    const Tensor gh = grad_in(g[1]);
+    norm_bwd(LP_N2, t + o_dn, gh.data_ptr(), H2.data_ptr(), f.rstd2, t + o_ds);
   }
-  check(tp_attn_bwd_run(&ab, st), "tp_attn_bwd_run");
-  layer_rope(s, t + o_dq, t + o_dk, C, Sn, true, st);
+  // output projection
+  if (want.attn) p[n++] = lin_problem(t + o_ds, s.H, w[LP_O].data_ptr(), NQ, s.H, true, false, R, NQ, t + o_da);
+  wgrad(LP_O, t + o_ds, s.H, base + f.attn, NQ);
+  run();
+  if (want.attn) {  // attention, rotary
+    ab.dout = t + o_da; ab.q = base + f.q; ab.k = base + f.k; ab.v = base + f.v; ab.out = base + f.attn; ab.lse = (const float*)(base + f.lse);
+    ab.dq = t + o_dq; ab.dk = t + o_dk; ab.dv = t + o_dv; ab.ws = (float*)(t + o_ws);
+    ab.parts = ab.parts_bytes ? t + o_parts : nullptr;
+    const Strides3 qs = head_strides(s, s.Hq), ks = head_strides(s, s.Hkv);
+    for (int i = 0; i < 3; i++) {
+      ab.do_strides[i] = ab.q_strides[i] = ab.o_strides[i] = ab.dq_strides[i] = qs[i];
+      ab.k_strides[i] = ab.v_strides[i] = ab.dk_strides[i] = ab.dv_strides[i] = ks[i];
+    }
+    check(tp_attn_bwd_run(&ab, st), "tp_attn_bwd_run");
+    layer_rope(s, t + o_dq, t + o_dk, C, Sn, true, st);
+  }
   // q, k, v
-  n = 0;
-  p[n] = raw_linear(t + o_dq, NQ, w[LP_Q].data_ptr(), s.H, NQ, true, false, R, s.H, t + o_dn);
-  add_segment(p[n], t + o_dk, NK, w[LP_K].data_ptr(), s.H, NK);
-  add_segment(p[n++], t + o_dv, NK, w[LP_V].data_ptr(), s.H, NK);
-  if (need(LP_Q)) p[n++] = wgrad(LP_Q, t + o_dq, NQ, base + f.n1, s.H);
-  if (need(LP_K)) p[n++] = wgrad(LP_K, t + o_dk, NK, base + f.n1, s.H);
-  if (need(LP_V)) p[n++] = wgrad(LP_V, t + o_dv, NK, base + f.n1, s.H);
-  run(n);
+  if (want.n1) {
+    p[n] = lin_problem(t + o_dq, NQ, w[LP_Q].data_ptr(), s.H, NQ, true, false, R, s.H, t + o_dn);
+    add_segment(p[n], t + o_dk, NK, w[LP_K].data_ptr(), s.H, NK);
+    add_segment(p[n++], t + o_dv, NK, w[LP_V].data_ptr(), s.H, NK);
+  }
+  wgrad(LP_Q, t + o_dq, NQ, base + f.n1, s.H);
+  wgrad(LP_K, t + o_dk, NK, base + f.n1, s.H);
+  wgrad(LP_V, t + o_dv, NK, base + f.n1, s.H);
+  run();
   // norm 1; x and the residual get the same gradient
-  const Tensor dx = at::empty(H2.sizes(), opts);
-  norm_bwd(LP_N1, t + o_dn, t + o_ds, s.residual ? base + f.h : (char*)X.data_ptr(), f.rstd1, dx.data_ptr());
-  out[0] = dx;
-  if (s.residual) out[1] = dx;
+  if (want.n1) {
+    const Tensor dx = at::empty(hidden, opts);
+    norm_bwd(LP_N1, t + o_dn, t + o_ds, s.residual ? base + f.h : (char*)X.data_ptr(), f.rstd1, dx.data_ptr());
+    if (want.in) out[0] = dx;
+    if (want.in && s.residual) out[1] = dx;
+  }
   end_of_graph("a decoder layer", g, *this, out);
   return out;
 }
@@ -1243,7 +1294,7 @@ std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const s
     char* b = (char*)buf.data_ptr();
     const int64_t R = s.rows;
     std::array<tp_linear_problem, 4> p;
-    const auto lin = [&](int i, const void* in, int64_t k, int wi, void* c) { p[i] = raw_linear(in, k, w[wi].data_ptr(), k, k, true, true, R, w[wi].size(0), c); };
+    const auto lin = [&](int i, const void* in, int64_t k, int wi, void* c) { p[i] = lin_problem(in, k, w[wi].data_ptr(), k, k, true, true, R, w[wi].size(0), c); };
     const auto run = [&](int n) { check(tp_linears(p.data(), n, s.dtype, st), "tp_linears"); };
     if (s.residual)
       check(tp_add_rmsnorm_fwd(x.data_ptr(), residual.data_ptr(), w[LP_N1].data_ptr(), b + f.h, b + f.n1, (float*)(b + f.rstd1), R, (int)s.H, s.H, s.H,
@@ -1270,15 +1321,17 @@ std::vector<Tensor> py_llama_layer(const Tensor& x, OptTensor residual_, const s
   }
   if (node) {
     node->s = s;
+    node->scalar = dt;
     torch::autograd::set_history(out, node);
     torch::autograd::set_history(h2, node);
-    if (!s.residual) node->x = SavedVariable(x, false);
+    const LayerWants want(x.requires_grad() || (s.residual && residual.requires_grad()), [&](int i) { return w[i].requires_grad(); });
     node->buf = SavedVariable(buf, false);
-    node->h2 = SavedVariable(h2, true);
-    node->cos = SavedVariable(cos, false);
-    node->sin = SavedVariable(sin, false);
-    node->params.reserve(LP_COUNT);
-    for (const auto& t : w) node->params.emplace_back(t, false);
+    if (want.n2) node->h2 = SavedVariable(h2, true);
+    if (want.attn) { node->cos = SavedVariable(cos, false); node->sin = SavedVariable(sin, false); }
+    if (want.n1 && !s.residual) node->x = SavedVariable(x, false);
+    node->params.resize(LP_COUNT);
+    for (int i = 0; i < LP_COUNT; i++)
+      if (want.weight(i)) node->params[i] = SavedVariable(w[i], false);
   }
   return {out, h2};
 }
@@ -1341,6 +1394,8 @@ Tensor py_embedding(const Tensor& ids, const Tensor& table) {
 // projection is one for the library.
 struct HeadNode : torch::autograd::Node {
   SavedVariable h, n, rstd, norm_w, lm_w;
+  std::vector<int64_t> sizes;  // of the hidden states
+  at::TensorOptions opts;
   std::string name() const override { return "TprimeLlamaHeadBackward"; }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -1350,30 +1405,33 @@ struct HeadNode : torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     variable_list out(4);  // x, residual, norm weight, lm_head weight
     if (!g[0].defined()) return out;
-    const Tensor H = packed16(h.unpack()), N = packed16(n.unpack()), R = packed16(rstd.unpack()), nw = packed16(norm_w.unpack()), lw = packed16(lm_w.unpack());
+    const bool dx = task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2), dw = task_should_compute_output(3);
+    Tensor H, N, R, nw, lw;
+    if (dx) { H = packed16(h.unpack()); R = packed16(rstd.unpack()); nw = packed16(norm_w.unpack()); lw = packed16(lm_w.unpack()); }
+    if (dw) N = packed16(n.unpack());
     at::AutoDispatchBelowADInplaceOrView below;
-    c10::DeviceGuard guard(H.device());
-    void* st = stream_of(H.device());
-    const int64_t k = H.size(-1), rows = H.numel() / k, V = lw.size(0);
-    const int code = dtype_code(H.scalar_type());
-    const Tensor go = packed16(g[0].to(H.scalar_type()));
-    const bool dx = task_should_compute_output(0) || task_should_compute_output(1) || task_should_compute_output(2);
+    c10::DeviceGuard guard(opts.device());
+    void* st = stream_of(opts.device());
+    const int64_t k = sizes.back(), V = g[0].size(-1), rows = g[0].numel() / V;
+    const auto type = opts.dtype().toScalarType();
+    const int code = dtype_code(type);
+    const Tensor go = packed16(g[0].to(type));
     Tensor dn;
     std::array<tp_linear_problem, 2> p;
     int c = 0;
     if (dx) {
-      dn = at::empty(H.sizes(), H.options());
-      p[c++] = raw_linear(go.data_ptr(), V, lw.data_ptr(), k, V, true, false, rows, k, dn.data_ptr());
+      dn = at::empty(sizes, opts);
+      p[c++] = lin_problem(go.data_ptr(), V, lw.data_ptr(), k, V, true, false, rows, k, dn.data_ptr());
     }
-    if (task_should_compute_output(3)) {
-      out[3] = at::empty(lw.sizes(), lw.options());
-      p[c++] = raw_linear(go.data_ptr(), V, N.data_ptr(), k, rows, false, false, V, k, out[3].data_ptr());
+    if (dw) {
+      out[3] = at::empty({V, k}, opts);
+      p[c++] = lin_problem(go.data_ptr(), V, N.data_ptr(), k, rows, false, false, V, k, out[3].data_ptr());
     }
     if (c) check(tp_linears(p.data(), c, code, st), "tp_linears");
     if (dx) {
       const Tensor ws = empty_f32({(int64_t)tp_rmsnorm_bwd_workspace_bytes(rows, (int)k) / 4}, H);
-      out[0] = at::empty(H.sizes(), H.options());
-      out[2] = at::empty(nw.sizes(), nw.options());
+      out[0] = at::empty(sizes, opts);
+      out[2] = at::empty({k}, opts);
       check(tp_rmsnorm_bwd(dn.data_ptr(), H.data_ptr(), nw.data_ptr(), (const float*)R.data_ptr(), out[0].data_ptr(), out[2].data_ptr(),
                            (float*)ws.data_ptr(), rows, (int)k, k, k, k, code, code, st), "tp_rmsnorm_bwd");
       out[1] = out[0];
@@ -1405,17 +1463,21 @@ std::optional<Tensor> py_llama_head(const Tensor& x, const Tensor& residual, con
     logits = empty_f32(sizes, x);
     check(tp_add_rmsnorm_fwd(x.data_ptr(), residual.data_ptr(), norm_w.data_ptr(), h.data_ptr(), n.data_ptr(), (float*)rstd.data_ptr(), rows, (int)k,
                              k, k, k, k, (float)eps, code, code, st), "tp_add_rmsnorm_fwd");
-    tp_linear_problem p = raw_linear(n.data_ptr(), k, lm_w.data_ptr(), k, k, true, true, rows, V, logits.data_ptr());
+    tp_linear_problem p = lin_problem(n.data_ptr(), k, lm_w.data_ptr(), k, k, true, true, rows, V, logits.data_ptr());
     p.c_float = 1;
     check(tp_linears(&p, 1, code, st), "tp_linears");
   }
   if (node) {
     torch::autograd::set_history(logits, node);
-    node->h = SavedVariable(h, false);
-    node->n = SavedVariable(n, false);
-    node->rstd = SavedVariable(rstd, false);
-    node->norm_w = SavedVariable(norm_w, false);
-    node->lm_w = SavedVariable(lm_w, false);
+    node->sizes = x.sizes().vec();
+    node->opts = x.options();
+    if (x.requires_grad() || residual.requires_grad() || norm_w.requires_grad()) {
+      node->h = SavedVariable(h, false);
+      node->rstd = SavedVariable(rstd, false);
+      node->norm_w = SavedVariable(norm_w, false);
+      node->lm_w = SavedVariable(lm_w, false);
+    }
+    if (lm_w.requires_grad()) node->n = SavedVariable(n, false);
   }
   return logits;
 }
