@@ -81,3 +81,17 @@ def test_waits_for_the_device_let_other_threads_run():
       torch.mm(a, a, out=b)
     n, took = ticks_during(call)
     assert took > 0.03 and n > 0, (n, took)
+
+
+def test_attention_refuses_shapes_it_has_no_kernel_for():
+  """The checks of the operators themselves, forward and (through the mask extensions) general, before any launch."""
+  q = _leaf((1, 4, 8, 64), 1)
+  for kw in ({}, {"soft_cap": 5.0}):
+    for exc, args in ((ValueError, (q, q[:, :3], q[:, :3])), (ValueError, (q, q, q[:, :, :4])), (ValueError, (q[0], q[0], q[0])),
+                      (NotImplementedError, (q[..., :32],) * 3), (TypeError, (q, q.float(), q.float())), (TypeError, (q.double(),) * 3)):
+      with pytest.raises(exc):
+        tpa.ops.attention(*args, sm_scale=0.1, **kw)
+    with pytest.raises(NotImplementedError, match="not built"):
+      tpa.ops.attention(*(torch.zeros((1, 2, 8, d), device=DEV) for d in (192, 192, 128)), **kw)
+    with pytest.raises(AssertionError, match="Sharding along sequence dimension"):
+      tpa.ops.attention(q, q, q, torch.zeros((1, 4), dtype=torch.int32, device=DEV), **kw)

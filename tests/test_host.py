@@ -65,19 +65,16 @@ def test_c_abi_validates_arguments_before_launching():
   assert lib.tp_attn_bwd_workspace_bytes(4, 32, 8192) == 2 * 4 * 32 * 8192 * 4
 
 
-def test_ops_reject_cpu_tensors_and_bad_shapes():
+def test_ops_reject_cpu_tensors_and_bad_types():
   x = torch.ones(2, 8)
   with pytest.raises(RuntimeError, match="no CPU path"):
     _lib.require_gpu(x)
   with pytest.raises(TypeError):
     _lib.dtype_code(torch.int8)
   q = torch.zeros(1, 4, 8, 64, dtype=torch.bfloat16)
-  with pytest.raises(ValueError):
-    tpa.ops._check_attn(q, q[:, :3], q[:, :3], None)  # 4 heads over 3 kv heads
-  with pytest.raises(NotImplementedError):
-    tpa.ops._check_attn(q[..., :32], q[..., :32], q[..., :32], None)
-  with pytest.raises(AssertionError, match="Sharding along sequence dimension"):
-    tpa.ops._check_attn(q, q, q, torch.zeros(1, 4, dtype=torch.int32))
+  for call in (lambda: tpa.ops.attention(q, q, q), lambda: tpa.ops.rmsnorm(x, x[0], 1e-5), lambda: tpa.ops.mask_kind(q[:, :1])):
+    with pytest.raises(RuntimeError, match="no CPU path"):
+      call()
 
 
 class _Seen(torch.overrides.TorchFunctionMode):

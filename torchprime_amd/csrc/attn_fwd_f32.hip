@@ -40,7 +40,6 @@ struct FwdArgs32 {
   float cap2;   // the soft cap in the scores' log2 units (0: none)
 };
 
-typedef float f32x1 __attribute__((ext_vector_type(1)));
 
 template <int D>
 __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {

@@ -211,31 +211,6 @@ def rope_apply(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor, pos: Tensor | Non
   return _native.rope_apply(q, k, cos, sin, pos, int(interleaved))
 
 
-_SUPPORTED_HEAD_DIMS = ((64, 64), (128, 128), (192, 128))
-_SUPPORTED_HEAD_DIMS_F32 = ((64, 64), (128, 128))  # fp32 operands (the small fp32 configurations)
-
-
-def _check_attn(q, k, v, seg):
-  if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-    raise ValueError("attention expects (batch, heads, seq, dim) tensors")
-  B, Hq, Sq, Dqk = q.shape
-  Bk, Hkv, Skv, Dk = k.shape
-  if (Bk, Dk) != (B, Dqk) or v.shape[:3] != k.shape[:3]:
-    raise ValueError(f"q {tuple(q.shape)}, k {tuple(k.shape)}, v {tuple(v.shape)} are inconsistent")
-  if Hkv == 0 or Hq % Hkv != 0:
-    raise ValueError(f"num query heads {Hq} must be a multiple of num kv heads {Hkv}")
-  if q.dtype not in (torch.bfloat16, torch.float16, torch.float32) or k.dtype != q.dtype or v.dtype != q.dtype:
-    raise TypeError(f"attention kernels take bfloat16, float16 or float32 q/k/v of one dtype, got {q.dtype}/{k.dtype}/{v.dtype}")
-  Dv = v.shape[-1]
-  dims = _SUPPORTED_HEAD_DIMS_F32 if q.dtype == torch.float32 else _SUPPORTED_HEAD_DIMS
-  if (Dqk, Dv) not in dims:
-    raise NotImplementedError(f"head dims (qk={Dqk}, v={Dv}) not built for {q.dtype}; supported: {dims}")
-  if seg is not None:
-    # kernel_utils.py:238-241: segment ids must cover the whole (unsharded) sequence
-    assert seg.shape == (B, Skv) and Sq == Skv, "Sharding along sequence dimension not allowed in tpu kernel attention"
-  return B, Hq, Hkv, Sq, Skv, Dqk, Dv
-
-
 def attention(
   q: Tensor, k: Tensor, v: Tensor, segment_ids: Tensor | None = None, sm_scale: float | None = None, causal: bool = True,
   *, window: tuple[int | None, int | None] | None = None, soft_cap: float | None = None,
