@@ -390,6 +390,25 @@ def test_fp32_attention_backward(B, Hq, Hkv, S, Skv, D, causal, use_seg):
     assert_close(got, ref, name, max_abs=2e-5 * max(1.0, ref.abs().max().item()), rel_l2=1e-5)
 
 
+# Workgroups of 128 rows that fill the 256 CUs (fwd_staged and its like): the layout that stages tiles through LDS, from one
+# row past a wave's 32 to ragged last workgroups, for each kernel with and without its neighbours.
+@pytest.mark.parametrize("B,Hq,Hkv,S,Skv,D,causal,use_seg,kw", [
+  (16, 32, 32, 33, 33, 64, True, False, {}), (16, 32, 32, 33, 33, 128, True, False, {}), (16, 32, 8, 100, 100, 64, False, True, {}),
+  (8, 32, 32, 129, 129, 128, False, False, {}), (64, 8, 2, 127, 127, 128, True, True, {}), (16, 32, 8, 128, 65, 64, False, False, {}),
+  (32, 16, 16, 40, 130, 64, False, False, {}), (8, 16, 16, 256, 256, 128, True, False, {"window": (70, 0)}),
+  (16, 32, 16, 97, 97, 64, True, False, {"soft_cap": 3.0}), (8, 32, 32, 130, 130, 64, False, True, {"window": (40, 9)})])  # fmt: skip
+def test_fp32_attention_of_many_rows(B, Hq, Hkv, S, Skv, D, causal, use_seg, kw):
+  q, do = (heads_view(B, Hq, S, D, i, torch.float32) for i in (1, 4))
+  k, v = (heads_view(B, Hkv, Skv, D, i, torch.float32) for i in (2, 3))
+  seg = packed_segment_ids(B, S, 5, 90, seed=8)[0] if use_seg else None
+  qd, kd, vd = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
+  out = tpa.ops.attention(qd, kd, vd, None if seg is None else seg.to(DEV), D**-0.5, causal, **kw)
+  out.backward(do.to(DEV))
+  refs = orc.attention_grads_ref(q, k, v, do, seg, causal, D**-0.5, torch.float64, **kw)
+  for name, got, ref in zip(("out", "dq", "dk", "dv"), (out, qd.grad, kd.grad, vd.grad), refs):  # (bounds as above and for the mask extensions)
+    assert_close(got, ref, name, max_abs=2e-5 * max(1.0, ref.abs().max().item()), rel_l2=2e-5 if kw else 1e-5)
+
+
 def test_long_packed_sequence_65536_rows():
   """S = 65536 with 96 packed documents, one head of 128: 1024 query tiles per workgroup list (the longest the dK/dV
   kernel's LDS holds at this head dim).  A packed row is a set of independent causal problems, so three documents

@@ -303,6 +303,25 @@ def test_additive_mask_fp32_operands(D):
   _check_bias(B, 4, 2, S, D, bias, dtype=torch.float32, seed=2)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_additive_mask_and_row_order_of_many_fp32_rows(D):
+  """The layout for fp32 problems that fill the CUs (16 batches of 32 heads): a per-head bias against the eager formula, and
+  query rows in another order against the same batch alone, which the other layout computes; sums of up to 48 keys in
+  another order, 48 * 2^-24 = 3e-6 of the sum of magnitudes."""
+  B, H, S = 16, 32, 48
+  bias = 2.0 * torch.randn((1, H, S, S), generator=torch.Generator().manual_seed(5))
+  _check_bias(B, H, H, S, D, bias, dtype=torch.float32, seed=2)
+  order = torch.randperm(S, generator=torch.Generator().manual_seed(6)).to(DEV)
+  leaves = [heads_view(B, H, S, D, i, torch.float32).to(DEV).requires_grad_(True) for i in range(3)]
+  do = heads_view(B, H, S, D, 3, torch.float32).to(DEV)
+  out = tpa.ops.attention(*leaves, q_positions=order)
+  got = (out, *torch.autograd.grad(out, leaves, do))
+  one = [t.detach()[5:6].requires_grad_(True) for t in leaves]
+  out = tpa.ops.attention(*one, q_positions=order)
+  for a, b in zip(got, (out, *torch.autograd.grad(out, one, do[5:6]))):
+    assert_close(a[5:6], b, max_abs=2e-5 * max(1.0, b.abs().max().item()), rel_l2=1e-5)
+
+
 def test_additive_mask_with_finite_values_per_head_and_the_causal_flag():
   """A per-head finite bias (ALiBi-like slopes plus noise), broadcast over the batch; once with causality inside the
   mask and once through the kernel's own causal flag: both are the eager formula with the summed mask."""

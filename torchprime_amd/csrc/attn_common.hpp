@@ -519,4 +519,22 @@ __device__ __forceinline__ void load_cols32(float (&x)[16][DB], const float* bas
   }
 }
 
+// rows r0 .. r0+31 of a row-major matrix of D columns into LDS rows of STRIDE floats, by 256 threads (zeros past n)
+template <int D, int STRIDE>
+__device__ __forceinline__ void stage_rows32(float* dst, const float* src, int64_t stride, int r0, int n, int tid) {
+  for (int c = tid; c < 32 * (D / 4); c += 256) {
+    const int r = c / (D / 4), cc = (c % (D / 4)) * 4;
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+    if (r0 + r < n) x = *(const f32x4*)(src + (int64_t)(r0 + r) * stride + cc);
+    *(f32x4*)(dst + r * STRIDE + cc) = x;
+  }
+}
+// For the fp32 kernels' choice of layout (fwd_staged in attn_fwd_f32.hip has the figures).  full_rounds: workgroups of 128
+// rows, one a CU at a time, make at least one round, and all rounds together are at least 8/9 full.  staged_triangle: not a
+// triangle so long that a workgroup waits for its last rows (up to 1024 where the 32-row tiles divide the CUs: there
+// every CU meets the same tile of each head, and the small workgroups gain nothing from causality).
+constexpr int CUS = NUM_XCD * CUS_PER_XCD;
+inline bool full_rounds(int64_t workgroups) { return workgroups >= CUS && (workgroups + CUS - 1) / CUS * CUS * 8 <= workgroups * 9; }
+inline bool staged_triangle(int rows) { return rows <= 768 || (rows <= 1024 && CUS % ((rows + 31) / 32) == 0); }
+
 }  // namespace tp

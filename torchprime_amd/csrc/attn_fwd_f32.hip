@@ -11,7 +11,12 @@
 // turn, each with an online softmax of its own, and the four partial results meet in LDS at the end; operands come
 // straight from memory in the layout the MFMA wants (K and Q rows as contiguous pieces, V rows as coalesced columns: every
 // byte of a line is used), so no wave waits for another inside the loop, and V's loads fly under the S products.
-// B2 S128, 8 heads of 64: 26 us with 128 rows a workgroup and staged tiles.
+// B2 S128, 8 heads of 64: 22 us with 128 rows a workgroup and staged tiles, 10 us so.
+//
+// Where there are enough query rows to fill the chip anyway that costs more than it gives: every 32 rows fetch all keys and
+// values, four times the reads, and the sums over the waves come on top.  STAGED is the layout for those: 128 rows a
+// workgroup, 32 a wave, tiles of keys and values staged through LDS and read by all four waves, two barriers a tile
+// (fwd_staged has the line and the figures).
 //
 // v_mfma_f32_32x32x2_f32 (wave64; ln = lane % 32, g = lane / 32):
 //   A (32 x 2): lane holds row ln, k = g        B (2 x 32): lane holds column ln, k = g
@@ -40,21 +45,25 @@ struct FwdArgs32 {
   float cap2;   // the soft cap in the scores' log2 units (0: none)
 };
 
-
-template <int D>
+template <int D, bool STAGED>
 __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
-  constexpr int BN = 32, BM = 32, DB = D / 32, HD = D / 2;
-  __shared__ __align__(16) float red[2 * DB * 1024];
+  constexpr int BN = 32, BM = STAGED ? 128 : 32, DB = D / 32, HD = D / 2;
+  constexpr int KSTRIDE = D + 4;  // floats per LDS row of K: 16-byte aligned rows, consecutive rows 4 banks apart
+  constexpr int VSTRIDE = D + 1;
+  __shared__ __align__(16) float smem[STAGED ? BN * (KSTRIDE + VSTRIDE) : 2 * DB * 1024];  // K and V tile, or the waves' sums
   __shared__ float msm[4][64], lsm[4][64];
+  __shared__ int ssm[BN];  // STAGED: the tile's segment ids
+  float* const ksm = smem;
+  float* const vsm = smem + BN * KSTRIDE;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   const int qt = n_qt - 1 - blockIdx.x % n_qt;  // the longest rows first
   const int bh = blockIdx.x / n_qt;
   const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.n_rep;
-  const int q0 = qt * BM;
+  const int q0 = qt * BM, wq0 = q0 + (STAGED ? wave * 32 : 0);
   const int Sq = a.Sq, Skv = a.Skv;
-  const int qrow = q0 + ln, qrow_c = min(qrow, Sq - 1);
+  const int qrow = wq0 + ln, qrow_c = min(qrow, Sq - 1);
   const float* kb = a.k + b * a.ks[0] + hk * a.ks[1];
   const float* vb = a.v + b * a.vs[0] + hk * a.vs[1];
   const int32_t* segb = a.seg ? a.seg + (int64_t)b * Skv : nullptr;
@@ -81,23 +90,50 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
 
   const int kv_end = a.causal ? min(Skv, q0 + BM) : Skv;
   const int ntiles = (kv_end + BN - 1) / BN;
-  for (int t = wave; t < ntiles; t += 4) {
+  for (int t = STAGED ? 0 : wave; t < ntiles; t += STAGED ? 1 : 4) {
     const int kv0 = t * BN;
-    float kf[HD], vf[16][DB];
-    load_row32(kf, kb + (int64_t)min(kv0 + ln, Skv - 1) * a.ks[2] + g * HD);
-    load_cols32(vf, vb, a.vs[2], kv0, Skv, g, ln);
-    // S^T = K Q^T: row = kv (ln of the A operand), column = query
     f32x16 s;
 #pragma unroll
     for (int v = 0; v < 16; v++) s[v] = 0.f;
+    float vf[16][DB];  // (not STAGED)
+    // S^T = K Q^T: row = kv (ln of the A operand), column = query
+    if constexpr (STAGED) {
+      __syncthreads();  // everyone is done with the previous tile
+      // K and V rows kv0 .. kv0+31 (rows past Skv as zeros): 16-byte chunks, thread -> (row, chunk), both loads in flight
+      for (int c = tid; c < BN * (D / 4); c += 256) {
+        const int r = c / (D / 4), cc = (c % (D / 4)) * 4;
+        f32x4 kvv = {0.f, 0.f, 0.f, 0.f}, vvv = {0.f, 0.f, 0.f, 0.f};
+        if (kv0 + r < Skv) {
+          kvv = *(const f32x4*)(kb + (int64_t)(kv0 + r) * a.ks[2] + cc);
+          vvv = *(const f32x4*)(vb + (int64_t)(kv0 + r) * a.vs[2] + cc);
+        }
+        *(f32x4*)(ksm + r * KSTRIDE + cc) = kvv;
 #pragma unroll
-    for (int st = 0; st < HD; st++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[st], qf[st], s, 0, 0, 0);
+        for (int e = 0; e < 4; e++) vsm[r * VSTRIDE + cc + e] = vvv[e];
+      }
+      if (segb && tid < BN) ssm[tid] = segb[min(kv0 + tid, Skv - 1)];
+      __syncthreads();
+      if (a.causal && kv0 > wq0 + 31) continue;  // the whole tile lies above this wave's diagonal (uniform per wave)
+      const float* kr = ksm + ln * KSTRIDE + g * HD;
+#pragma unroll
+      for (int st = 0; st < HD; st += 4) {
+        const f32x4 k4 = *(const f32x4*)(kr + st);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[e], qf[st + e], s, 0, 0, 0);
+      }
+    } else {
+      float kf[HD];
+      load_row32(kf, kb + (int64_t)min(kv0 + ln, Skv - 1) * a.ks[2] + g * HD);
+      load_cols32(vf, vb, a.vs[2], kv0, Skv, g, ln);
+#pragma unroll
+      for (int st = 0; st < HD; st++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[st], qf[st], s, 0, 0, 0);
+    }
     // mask, online softmax (log2 units)
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < 16; v++) {
-      const int kv = kv0 + 8 * (v / 4) + 4 * g + (v % 4);
-      const bool ok = kv < Skv && (!a.causal || kv <= qrow) && (!segb || segb[min(kv, Skv - 1)] == segq) && kv >= band_lo && kv <= band_hi;
+      const int kvl = 8 * (v / 4) + 4 * g + (v % 4), kv = kv0 + kvl;
+      const bool ok = kv < Skv && (!a.causal || kv <= qrow) && (!segb || (STAGED ? ssm[kvl] : segb[min(kv, Skv - 1)]) == segq) && kv >= band_lo && kv <= band_hi;
       if (a.cap2 != 0.f) s[v] = a.cap2 * tanhf(s[v] / a.cap2);  // cap * tanh(score / cap), in log2 units
       if (bias_row) s[v] += LOG2E * bias_row[min(kv, Skv - 1)];  // additive mask (-inf stays -inf)
       s[v] = ok ? s[v] : -INFINITY;
@@ -121,26 +157,33 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
       for (int v = 0; v < 16; v++) oacc[d][v] *= alpha;
     // O^T += V^T P^T: step v pairs kv row 8*(v/4) + 4*g + v%4 of V with the lane's value v of P^T
 #pragma unroll
-    for (int v = 0; v < 16; v++)
+    for (int v = 0; v < 16; v++) {
+      const int kvl = 8 * (v / 4) + 4 * g + (v % 4);
 #pragma unroll
-      for (int d = 0; d < DB; d++) oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[v][d], s[v], oacc[d], 0, 0, 0);
+      for (int d = 0; d < DB; d++)
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(STAGED ? vsm[kvl * VSTRIDE + d * 32 + ln] : vf[v][d], s[v], oacc[d], 0, 0, 0);
+    }
   }
 
-  // the waves' shares: brought to the largest of the four maxima, then added
-  msm[wave][lane] = m_run;
-  __syncthreads();
-  const float m_all = fmaxf(fmaxf(msm[0][lane], msm[1][lane]), fmaxf(msm[2][lane], msm[3][lane]));
-  const float share = m_run == -INFINITY ? 0.f : exp2f(m_run - m_all);
-  lsm[wave][lane] = l_run * share;
+  float m_all = m_run, l = l_run;
+  if constexpr (!STAGED) {
+    // the waves' shares: brought to the largest of the four maxima, then added
+    msm[wave][lane] = m_run;
+    __syncthreads();
+    m_all = fmaxf(fmaxf(msm[0][lane], msm[1][lane]), fmaxf(msm[2][lane], msm[3][lane]));
+    const float share = m_run == -INFINITY ? 0.f : exp2f(m_run - m_all);
+    lsm[wave][lane] = l_run * share;
 #pragma unroll
-  for (int d = 0; d < DB; d++)
+    for (int d = 0; d < DB; d++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) oacc[d][v] *= share;
-  sum_waves(oacc, red, wave, lane);
-  if (wave != 0) return;
+      for (int v = 0; v < 16; v++) oacc[d][v] *= share;
+    sum_waves(oacc, smem, wave, lane);
+    if (wave != 0) return;
+    l = (lsm[0][lane] + lsm[2][lane]) + (lsm[1][lane] + lsm[3][lane]);
+  }
 
   // epilogue: lane = query, value v of block d is output column d*32 + 8*(v/4) + 4*g + v%4
-  const float l = half_sum((lsm[0][lane] + lsm[2][lane]) + (lsm[1][lane] + lsm[3][lane]));
+  l = half_sum(l);
   const float inv = l > 0.f ? 1.f / l : 0.f;
   if (qrow < Sq) {
     if (g == 0) a.lse[((int64_t)b * a.Hq + h) * Sq + qrow] = l > 0.f ? (m_all + log2f(l)) * LN2 : -INFINITY;
@@ -153,6 +196,18 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdArgs32 a) {
         *(f32x4*)(op + d * 32 + 8 * vq + 4 * g) = f32x4{o[4 * vq] * inv, o[4 * vq + 1] * inv, o[4 * vq + 2] * inv, o[4 * vq + 3] * inv};
       }
   }
+}
+
+// Which layout: staged where its workgroups of 128 rows fill the CUs by themselves.  Head dim 128 keeps one workgroup a CU
+// busy with its MFMAs, so rounds count whole; at head dim 64 two share a CU, and staging pays from two of them on.  Not for
+// long causal sequences (the 128 rows of a workgroup wait for its last ones, and four times fewer workgroups balance the
+// triangle worse), nor where a workgroup would have rows for one wave only.  us, 32 rows : staged, B Hq/Hkv S:
+//   64, full:    1 8/8 4096  470 : 640;  2 32/8 768  149 : 169;  2 32/8 1024  254 : 225;  64 8/8 100  53 : 34;  2 32/8 4096  3560 : 2930
+//   64, causal:  16 8/8 384  72 : 79;  4 32/8 512  130 : 113;  64 8/8 640  543 : 433;  16 8/8 900  265 : 392;  4 32/8 2048  1380 : 1521
+//   128, full:   2 8/8 1024  148 : 251;  2 32/8 512  155 : 134;  2 32/8 768  327 : 382;  4 32/32 256  96 : 69;  4 32/8 2048  4573 : 4114
+//   128, causal: 16 8/8 384  149 : 162;  64 8/8 128  111 : 75;  4 32/8 768  489 : 494;  4 32/8 1024  1118 : 973;  2 32/8 2048  1673 : 1898
+static bool fwd_staged(int D, int64_t workgroups, int Sq, bool causal) {
+  return Sq > 32 && (!causal || staged_triangle(Sq)) && (D == 64 ? workgroups >= 2 * CUS : full_rounds(workgroups));
 }
 
 // called by tp_attn_fwd for TP_F32 inputs (arguments already validated there)
@@ -176,8 +231,13 @@ int attn_fwd_f32(const void* q, const void* k, const void* v, const int32_t* seg
   a.cap2 = mx.cap_in != 0.f ? mx.cap_out * sm_scale * LOG2E : 0.f;
   const int64_t blocks = (int64_t)B * Hq * ((Sq + 31) / 32);
   TP_REQUIRE(blocks < (1ll << 31), TP_ERR_UNSUPPORTED, "tp_attn_fwd: too many workgroups");
-  if (Dqk == 64) attn_fwd_f32_kernel<64><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
-  else attn_fwd_f32_kernel<128><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
+  const int64_t staged_blocks = (int64_t)B * Hq * ((Sq + 127) / 128);
+  const bool staged = fwd_staged(Dqk, staged_blocks, Sq, a.causal);
+  const dim3 grid((unsigned)(staged ? staged_blocks : blocks)), block(256);
+  if (Dqk == 64 && staged) attn_fwd_f32_kernel<64, true><<<grid, block, 0, st>>>(a);
+  else if (Dqk == 64) attn_fwd_f32_kernel<64, false><<<grid, block, 0, st>>>(a);
+  else if (staged) attn_fwd_f32_kernel<128, true><<<grid, block, 0, st>>>(a);
+  else attn_fwd_f32_kernel<128, false><<<grid, block, 0, st>>>(a);
   return check_launch("tp_attn_fwd(fp32)");
 }
 
