@@ -15,7 +15,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 from torch.compiler import is_compiling
-from torch.overrides import has_torch_function
+from torch.overrides import has_torch_function_variadic as overridden
 
 from .attention import AttentionModule
 from .linear import embed, global_hooks, plain, project, weight_of
@@ -255,7 +255,7 @@ class LlamaDecoderLayer(nn.Module):
       return None
     w1, w2 = n1.__dict__["_parameters"]["weight"], n2.__dict__["_parameters"]["weight"]
     cos, sin = position_embeddings
-    if has_torch_function((x, residual, cos, sin, w1, w2, *ws)):
+    if overridden(x, residual, cos, sin, w1, w2, *ws):
       return None
     return _native.llama_layer(
       x, residual, [w1, *ws[:4], w2, *ws[4:]], cos, sin, attn.num_heads, attn.num_key_value_heads, n1.variance_epsilon,
@@ -369,7 +369,7 @@ class LlamaForCausalLM(nn.Module):
       return project(model(input_ids=input_ids, attention_mask=attention_mask), self.lm_head)[0].float()
     x, residual = model.deferred(input_ids, attention_mask)
     norm = model.norm
-    if residual is not None and not has_torch_function((x, residual, norm.weight, head)):
+    if residual is not None and not overridden(x, residual, norm.weight, head):
       # norm of the sum, lm_head and .float() in one native call where the projection is small
       logits = _native.llama_head(x, residual, norm.weight, norm.variance_epsilon, head)
       if logits is not None:

@@ -9,7 +9,7 @@ import torch
 from torch import nn
 from torch.compiler import is_compiling
 from torch.nn.modules import module as _module
-from torch.overrides import has_torch_function
+from torch.overrides import has_torch_function_variadic as overridden
 
 from .ops import _native
 
@@ -43,7 +43,7 @@ def project(x: torch.Tensor, *modules: nn.Module) -> list[torch.Tensor]:
   if not is_compiling() and not global_hooks():
     ws = [weight_of(m) for m in modules]
     # (nor may the call be overridden: fx proxies, tensor subclasses and function modes see the modules' own calls)
-    if all(w is not None for w in ws) and not has_torch_function((x, *ws)):
+    if all(w is not None for w in ws) and not overridden(x, *ws):
       return _native.linears(x, ws)
   return [m(x) for m in modules]
 
@@ -53,6 +53,6 @@ def embed(module: nn.Module, ids: torch.Tensor) -> torch.Tensor:
   if not is_compiling() and plain(module, nn.Embedding) and not global_hooks():
     d = module.__dict__
     w = d["_parameters"]["weight"]
-    if d["padding_idx"] is None and d["max_norm"] is None and not d["scale_grad_by_freq"] and not d["sparse"] and not has_torch_function((ids, w)):
+    if d["padding_idx"] is None and d["max_norm"] is None and not d["scale_grad_by_freq"] and not d["sparse"] and not overridden(ids, w):
       return _native.embedding(ids, w)
   return module(ids)

@@ -17,7 +17,7 @@ import math
 import torch
 from torch import Tensor
 from torch.compiler import is_compiling
-from torch.overrides import has_torch_function
+from torch.overrides import has_torch_function_variadic as overridden
 
 try:
   from . import _tprime_ops as _native
@@ -177,27 +177,23 @@ def _(dloss, logits, labels, lse, loss_and_count, ignore_index):
 # ------------------------------------------------------------------------------------------------
 # what users call
 # ------------------------------------------------------------------------------------------------
-def _by_name(*tensors: Tensor | None) -> bool:
-  """The operator is to be called as a ``torch.ops`` function: a compiler traces, or calls on these tensors are overridden
-  (``__torch_function__``: fx proxies, tensor subclasses, an active function mode).  None of them sees into ``_native``."""
-  return is_compiling() or has_torch_function(tensors)
-
-
+# (A compiler that traces does not see into _native, nor does what overrides calls on these tensors, __torch_function__: fx
+# proxies, tensor subclasses, an active function mode.  For them the operators are called by name, as torch.ops functions.)
 def rmsnorm(x: Tensor, weight: Tensor, eps: float) -> Tensor:
   """``weight * (x.float() * rsqrt(mean(x.float()**2, -1) + eps)).to(x.dtype)`` in one pass."""
-  return rmsnorm_fwd(x, weight, eps)[0] if _by_name(x, weight) else _native.rmsnorm(x, weight, eps)
+  return rmsnorm_fwd(x, weight, eps)[0] if is_compiling() or overridden(x, weight) else _native.rmsnorm(x, weight, eps)
 
 
 def add_rmsnorm(x: Tensor, residual: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
   """``h = residual + x; y = rms_norm(h, weight, eps)`` in one pass; returns ``(y, h)``."""
-  if _by_name(x, residual, weight):
+  if is_compiling() or overridden(x, residual, weight):
     return add_rmsnorm_fwd(x, residual, weight, eps)[:2]
   return _native.add_rmsnorm(x, residual, weight, eps)
 
 
 def rope_table_like(inv_freq: Tensor, position_ids: Tensor, attention_scaling: float, x: Tensor) -> tuple[Tensor, Tensor]:
   """cos/sin tables ``(Bp, S, 2*half)`` in ``x``'s dtype from ``inv_freq (half)`` and float ``position_ids (Bp, S)``."""
-  if _by_name(inv_freq, position_ids, x):
+  if is_compiling() or overridden(inv_freq, position_ids, x):
     return rope_table(inv_freq, position_ids, attention_scaling, x.dtype)
   return _native.rope_table(inv_freq, position_ids, attention_scaling, x)
 
@@ -206,7 +202,7 @@ def rope_apply(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor, pos: Tensor | Non
   """``(q*cos + rotate_half(q)*sin, k*cos + rotate_half(k)*sin)`` for (B,H,S,D) q and k in one launch.
 
   ``interleaved``: 0 rotate-half, 1 DeepSeek ([evens | odds] output), 2 adjacent pairs in place (Llama-4)."""
-  if _by_name(q, k, cos, sin, pos):
+  if is_compiling() or overridden(q, k, cos, sin, pos):
     return rope_apply_op(q, k, cos, sin, pos, int(interleaved), False)
   return _native.rope_apply(q, k, cos, sin, pos, int(interleaved))
 
@@ -234,13 +230,13 @@ def attention(
     sm_scale = 1.0 / math.sqrt(v.shape[-1])
   wl, wr = (-1, -1) if window is None else tuple(-1 if w is None else int(w) for w in window)
   if bias is None and q_positions is None and wl < 0 and wr < 0 and soft_cap is None and (causal_offset == 0 or not causal):
-    if _by_name(q, k, v, segment_ids):
+    if is_compiling() or overridden(q, k, v, segment_ids):
       return attn_fwd(q, k, v, segment_ids, sm_scale, causal)[0]
     return _native.attention(q, k, v, segment_ids, sm_scale, causal)
   if bias is not None:
     bias = bias.detach()
   args = (q, k, v, segment_ids, q_positions, sm_scale, causal, causal_offset, wl, wr, float(soft_cap or 0.0), bias)
-  return attn_fwd_masked(*args)[0] if _by_name(q, k, v, segment_ids, q_positions, bias) else _native.attention_masked(*args)
+  return attn_fwd_masked(*args)[0] if is_compiling() or overridden(q, k, v, segment_ids, q_positions, bias) else _native.attention_masked(*args)
 
 
 # kinds of additive masks (mask_kind)
@@ -263,23 +259,23 @@ def attention_pairs_fit(q: Tensor, k: Tensor, v: Tensor, mask: Tensor) -> bool:
 def attention_pairs(q: Tensor, k: Tensor, v: Tensor, mask: Tensor, sm_scale: float) -> Tensor:
   """Attention under an additive mask of kind ``MASK_PAIRS`` (1|B, 1, Sq, Skv): as ``attention(bias=mask)``, with the
   mask as one bit per pair, tiles without a pair left out and tiles with every pair unmasked.  bfloat16 and float16."""
-  if _by_name(q, k, v, mask):
+  if is_compiling() or overridden(q, k, v, mask):
     return attn_fwd_pairs(q, k, v, mask, sm_scale)[0]
   return _native.attention_pairs(q, k, v, mask, sm_scale)
 
 
 def l2norm(x: Tensor, eps: float) -> Tensor:
   """``(x.float() * rsqrt(mean(x.float()**2, -1) + eps)).type_as(x)`` over the last dim."""
-  return l2norm_fwd(x, eps)[0] if _by_name(x) else _native.l2norm(x, eps)
+  return l2norm_fwd(x, eps)[0] if is_compiling() or overridden(x) else _native.l2norm(x, eps)
 
 
 def swiglu(gate: Tensor, up: Tensor) -> Tensor:
   """``silu(gate) * up`` with the eager roundings, one pass."""
-  return swiglu_fwd(gate, up) if _by_name(gate, up) else _native.swiglu(gate, up)
+  return swiglu_fwd(gate, up) if is_compiling() or overridden(gate, up) else _native.swiglu(gate, up)
 
 
 def cross_entropy(logits: Tensor, labels: Tensor, ignore_index: int) -> Tensor:
   """Mean of ``logsumexp(logits[b, s]) - logits[b, s, labels[b, s+1]]`` over the labels that are not ``ignore_index``."""
-  if _by_name(logits, labels):
+  if is_compiling() or overridden(logits, labels):
     return cross_entropy_fwd(logits, labels, ignore_index, True)[0]
   return _native.cross_entropy(logits, labels, ignore_index)
