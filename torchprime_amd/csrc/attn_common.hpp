@@ -268,11 +268,16 @@ __device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, 
   return group < n_groups;
 }
 // How many groups: all where an XCD gets fewer than four rounds of workgroups (per_cu of them share a CU), else the last
-// ones that make up two rounds; 0 where one group has that many by itself.  More of them in turns balances better still
-// and loses more in the L2 than that gains.  us, none | two rounds | four | all in turns, bf16, causal:
-//   forward, 128 heads of (192,128): B1 S4096 684 | 657 | 671 | 677;  B2 S2048 405 | 362 | 391 | 437
-//   forward + backward: B8 8 heads of 64 S4096 718 | 629 | 621 | 634;  B8 32q/8kv of 128 S2048 1321 | 1261 | 1252 | 1267
-//   packed documents: B4 32q/8kv of 128 S4096 1085 | 1039 | 1084 | 1090;  S8192 (one group is two rounds) 3556 | - | 3628 | 3812
+// ones that make up two rounds; 0 where one group has that many by itself.  That is never slower than group after group
+// beyond the runs' differences (0.6 %) and up to a tenth faster.  It counts workgroups only and knows nothing of what a group
+// keeps in an L2, so it is not the best number everywhere: with documents, or heads of 64, more groups in turns are up to
+// 6 % faster still, with long rows of plain heads slower.  Forward + backward, us, medians of 7, bf16, causal;
+// none | the rule | four rounds | eight | all (p: packed documents):
+//   (192,128), 128 heads    B1 S4096 3162 | 3180 | 3208 | 3194 | 3259;  B2 S2048 1922 | 1874 | 1901 | 1980 | 2023;  p B1 S4096 1573 | 1552 | 1514 | 1512 | 1531
+//   64, 8 heads             B8 S4096 734 | 656 | 654 | 644 | 647;  p B4 S8192 595 | 563 | 544 | 545 | 548
+//   128, 32q/8kv            B8 S2048 1372 | 1307 | 1276 | 1306 | 1301;  p B4 S4096 1122 | 1100 | 1107 | 1109 | 1123;  window 1000, B4 S4096 1207 | 1204 | 1217 | 1214 | 1214
+//   (one group is two rounds: none and the rule are the same)  B4 S8192 8862 | 8823 | 8760 | 8816 | 8908;  p 3752 | 3741 | 3759 | 3838 | 3883
+//   128, 64q/8kv            B4 S3001 2779 | 2669 | 2677 | 2673 | 2681;  p 1272 | 1268 | 1273 | 1271 | 1269 (two rounds: 1220)
 inline int groups_in_turns(int n_tiles, int n_inner, int n_groups, int per_cu) {
   const int64_t n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, per_group = (int64_t)n_tiles * n_inner, round = CUS_PER_XCD * per_cu;
   const int64_t n = n_gl * per_group < 4 * round ? n_gl : std::min(n_gl, (2 * round + per_group - 1) / per_group);
