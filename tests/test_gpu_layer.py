@@ -215,6 +215,33 @@ def test_norm_backward_of_few_rows(rows, hidden):
     assert ((a - b).norm() / b.norm()).item() <= 1e-2
 
 
+@pytest.mark.parametrize("unpack", ["as it was", "other strides"])
+def test_saved_tensor_hooks(unpack):
+  """Everything the nodes keep goes through the host and comes back, once in other strides than it went in."""
+  cfg = tpa.Config(vocab_size=136, num_hidden_layers=2, max_position_embeddings=512, hidden_size=128, intermediate_size=64,
+                   num_attention_heads=2, num_key_value_heads=2, hidden_act="silu", initializer_range=0.02, rms_norm_eps=1e-5,
+                   attention_dropout=False, attention_bias=False, rope_theta=500000.0, attention_kernel="splash_attention")  # fmt: skip
+  model = tpa.LlamaForCausalLM(cfg).to(DEV).to(torch.bfloat16)
+  ids = torch.randint(136, (2, 37), generator=torch.Generator().manual_seed(1)).to(DEV)
+  params = list(model.parameters())
+  want = torch.autograd.grad(model(ids, labels=ids)[1], params)
+
+  def back(t):
+    t = t.to(DEV)
+    return t if unpack == "as it was" or t.dim() < 2 else t.transpose(0, 1).contiguous().transpose(0, 1)
+
+  with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), back):
+    logits, loss = model(ids, labels=ids)
+    mlp = model.model.layers[0].mlp(logits.detach()[..., :128].to(torch.bfloat16))
+  assert logits.grad_fn.name() == "TprimeLlamaHeadBackward"
+  got = torch.autograd.grad(loss, params)
+  assert all(torch.equal(a, b) for a, b in zip(got, want))
+  w = list(model.model.layers[0].mlp.parameters())
+  again = model.model.layers[0].mlp(logits.detach()[..., :128].to(torch.bfloat16))
+  for a, b in zip(torch.autograd.grad(mlp.float().sum(), w), torch.autograd.grad(again.float().sum(), w)):
+    assert torch.equal(a, b)
+
+
 def test_a_function_mode_sees_the_modules():
   """Under an active function mode the model runs module by module, so that the mode sees every projection and lookup; the
   logits are the same but for the order of fp32 sums."""
