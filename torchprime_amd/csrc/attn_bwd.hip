@@ -920,26 +920,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
     }
     return;
   }
-  if (row < Skv) {
-    T* dkp = (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row * a.dks[2];
-    T* dvp = (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row * a.dvs[2];
-    const float sc = a.sm_scale;
-#pragma unroll
-    for (int d = 0; d < DKB; d++)
-#pragma unroll
-      for (int vq = 0; vq < 4; vq++) {
-        const f32x16& o = dkacc[d];
-        *(u32x2*)(dkp + d * 32 + 8 * vq + 4 * g) =
-            pack4<T>(o[4 * vq] * sc, o[4 * vq + 1] * sc, o[4 * vq + 2] * sc, o[4 * vq + 3] * sc);
-      }
-#pragma unroll
-    for (int d = 0; d < DVB; d++)
-#pragma unroll
-      for (int vq = 0; vq < 4; vq++) {
-        const f32x16& o = dvacc[d];
-        *(u32x2*)(dvp + d * 32 + 8 * vq + 4 * g) = pack4<T>(o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]);
-      }
-  }
+  __syncthreads();  // every wave is done with the tiles: the sums go out through their LDS
+  const unsigned lds = (unsigned)(size_t)smem + (unsigned)(wave * 4096);
+  store_rows<T, DKB>(dkacc, a.sm_scale, (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + wkv0 * a.dks[2], a.dks[2], Skv - wkv0, lds, lane);
+  store_rows<T, DVB>(dvacc, 1.f, (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + wkv0 * a.dvs[2], a.dvs[2], Skv - wkv0, lds, lane);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1971,18 +1955,9 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
     for (int d = 0; d < DB; d++) asm volatile("s_nop 15\n\ts_nop 3" : "+a"(dqacc[d]) :: "memory");
   }
 
-  if (qrow < Sq) {
-    T* dqp = (T*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qrow * a.dqs[2];
-    const float sc = a.sm_scale;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int vq = 0; vq < 4; vq++) {
-        const f32x16& o = dqacc[d];
-        *(u32x2*)(dqp + d * 32 + 8 * vq + 4 * g) =
-            pack4<T>(o[4 * vq] * sc, o[4 * vq + 1] * sc, o[4 * vq + 2] * sc, o[4 * vq + 3] * sc);
-      }
-  }
+  // (every wave is past the last tile's barrier and every tile load has landed: the K tiles' LDS is free)
+  store_rows<T, DB>(dqacc, a.sm_scale, (T*)a.dq + b * a.dqs[0] + h * a.dqs[1] + wq0_s * a.dqs[2], a.dqs[2], Sq - wq0_s,
+                    lds_base + (unsigned)(K_AT + wave_s * 4096), lane);
 }
 
 // ------------------------------------------------------------------------------------------------

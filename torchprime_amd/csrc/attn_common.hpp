@@ -476,6 +476,39 @@ __device__ __forceinline__ u32x4 make_rsrc_words(const void* base, unsigned byte
   return r;
 }
 
+// 32 rows x 32 DB values that a wave holds one row per lane (C layout of a transposed product: lane ln + 32 g has columns
+// 32 d + 8 (v / 4) + 4 g + v % 4 of row ln), times `scale` (the lane's row's), to memory as T.  Stored straight from the
+// registers, an instruction writes 8 bytes to each of 64 places, and the address path takes them one a cycle: 40 such stores
+// a wave were 6 us of every dK/dV workgroup.  Through 4 KB of LDS of the wave's own, 64 columns at a time, an instruction
+// writes eight whole 128-byte lines.  Rows at `rows` and past it are not written; rows need 8-byte alignment only.
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
+template <typename T, int DB>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[DB], float scale, T* p, int64_t stride, int rows, unsigned lds, int lane) {
+  static_assert(DB % 2 == 0, "64 columns at a time");
+  const int g = lane >> 5, ln = lane & 31;
+  // chunks of 16 bytes swizzled by the row: 8-byte writes by lanes in consecutive rows and 16-byte reads along a row are both
+  // conflict free
+  const unsigned wr = lds + (unsigned)(ln * 128 + 8 * g), ws = (unsigned)((ln >> 1) & 7);
+  const int r0 = lane >> 3, ch = lane & 7;
+#pragma unroll
+  for (int d2 = 0; d2 < DB; d2 += 2) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const f32x16& o = acc[d2 + j / 4];
+      const int v = 4 * (j % 4);
+      *(__attribute__((address_space(3))) u32x2*)(wr + (((unsigned)j ^ ws) << 4)) = pack4<T>(o[v] * scale, o[v + 1] * scale, o[v + 2] * scale, o[v + 3] * scale);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int r = 8 * i + r0;
+      const u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(lds + (unsigned)(r * 128 + ((ch ^ ((r >> 1) & 7)) << 4)));
+      if (r < rows) *(u32x4_a8*)(p + r * stride + d2 * 32 + ch * 8) = x;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
 // ---- fp32 kernels ----------------------------------------------------------------------------------
 // Sum of the four waves' accumulators, in wave 0: (w0 + w2) + (w1 + w3).  red: 2 x N x 16 x 64 floats of LDS, free to use
 // again after the next barrier.

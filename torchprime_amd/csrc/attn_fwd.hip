@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   vdma.init(a.vs[2], wave, lane);
   const u32x4 krw = make_rsrc_words(kb, span_bytes(Skv, a.ks[2], DQK));
   const u32x4 vrw = make_rsrc_words(vb, span_bytes(Skv, a.vs[2], DV));
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
+  const int wave_s = __builtin_amdgcn_readfirstlane(wave), wq0_s = q0 + wave_s * 32;
   const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
   // this wave's first LDS destinations in buffer 0 (scalar byte addresses)
   const unsigned kdst0 = lds_base + (unsigned)K_AT + (unsigned)(wave_s * K_ITEMS * 1024);
@@ -596,18 +596,12 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   {
     const float l = half_sum(l_run);
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    if (qrow < Sq) {
-      if (g == 0) lb[qrow] = l > 0.f ? (m_run + log2f(l)) * LN2 : -INFINITY;
-      T* op = ob + qrow * a.os[2];
-#pragma unroll
-      for (int d = 0; d < DVB; d++)
-#pragma unroll
-        for (int vq = 0; vq < 4; vq++) {
-          const f32x16& o = oacc[d];
-          *(u32x2*)(op + d * 32 + 8 * vq + 4 * g) =
-              pack4<T>(o[4 * vq] * inv, o[4 * vq + 1] * inv, o[4 * vq + 2] * inv, o[4 * vq + 3] * inv);
-        }
-    }
+    if (qrow < Sq && g == 0) lb[qrow] = l > 0.f ? (m_run + log2f(l)) * LN2 : -INFINITY;
+    // (the buffer of the last tile is free; loads that nobody waits for any more may still write the other one)
+    const int buf = (nact - 1) & 1;
+    const unsigned ko = (unsigned)(K_AT + buf * K_STEP), vo = (unsigned)(V_AT + buf * V_STEP);
+    store_rows<T, DVB>(oacc, inv, ob + wq0_s * a.os[2], a.os[2], Sq - wq0_s,
+                       lds_base + (K_BYTES >= 4 * 4096 ? ko + (unsigned)(wave_s * 4096) : (wave_s < 2 ? ko : vo) + (unsigned)((wave_s & 1) * 4096)), lane);
   }
 }
 
