@@ -346,7 +346,8 @@ int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float*
  *   pairs, mask_batches   see tp_mask_pairs; goes with no other mask
  *   parts, parts_bytes    tp_attn_bwd_parts_bytes() bytes, 16-byte aligned, or NULL / 0.  With it the walk of a
  *                         key tile over its queries is split over several workgroups where one each would
- *                         leave CUs idle; 0 bytes are asked for where it would not pay
+ *                         leave CUs idle, or a large problem's key tiles are handed out by counters that lie
+ *                         there; 0 bytes are asked for where neither pays.  Nothing has to be cleared
  * ---------------------------------------------------------------------------------------------- */
 typedef struct tp_attn_bwd_problem {
   const void *dout, *q, *k, *v, *out;

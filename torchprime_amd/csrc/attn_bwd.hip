@@ -9,7 +9,7 @@
 // Kernels:
 //   attn_delta_kernel     -delta[b,h,i] = -sum_d dO*O, and the LSE in log2 units      (HBM-bound; only where the
 //                         general dQ kernel runs: the lean dQ kernel computes both itself and runs first)
-//   attn_bwd_dkdv_kernel  one workgroup = 128 KV rows of one (batch, kv head); K and V fragments stay
+//   attn_bwd_dkdv_kernel  one workgroup = 128 KV rows of one (batch, kv head), or one after the other from a queue; K and V fragments stay
 //                         in registers, row-major Q / dO tiles of every query head of the group stream through
 //                         three LDS buffers (fragment reads for S = QK^T and dP = dO V^T, transposing reads
 //                         for dV^T += dO^T P and dK^T += Q^T dS).  S is computed un-transposed here so
@@ -51,6 +51,13 @@ __host__ __device__ constexpr AbSlot ab_slot(int j, int n0, int n1) {
   return AbSlot{0, 0};
 }
 
+// workgroups of the dK/dV kernel that share a CU (registers)
+constexpr int dkdv_per_cu(int Dqk) { return Dqk <= 64 ? 2 : 1; }
+
+// A work queue: one counter per XCD, each in a 128-byte line of its own.
+constexpr int QUEUE_STRIDE = 32;
+constexpr size_t QUEUE_BYTES = NUM_XCD * QUEUE_STRIDE * sizeof(unsigned);
+
 struct BwdArgs {
   const void* q;
   const void* k;
@@ -76,6 +83,7 @@ struct BwdArgs {
   // dK/dV: partial results of the splits of a kv tile's work (split_plan), NULL: no tile is split
   float* parts;
   size_t parts_bytes;
+  unsigned* queue;                // next item of each XCD, QUEUE_STRIDE apart (NULL: a workgroup does one item)
   int split;                      // the plan below is in use
   unsigned short split_first[65]; // per XCD: number of workgroups before kv tile t
 };
@@ -152,8 +160,14 @@ static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk,
 // ------------------------------------------------------------------------------------------------
 // delta = rowsum(dO o O)
 // ------------------------------------------------------------------------------------------------
+// the counters of the dK/dV kernel's queues, cleared by the kernel that runs before it
+__device__ __forceinline__ void clear_queue(const BwdArgs& a) {
+  if (a.queue && blockIdx.x == 0 && threadIdx.x < NUM_XCD) a.queue[threadIdx.x * QUEUE_STRIDE] = 0u;
+}
+
 template <typename T, int DV>
 __global__ __launch_bounds__(256) void attn_delta_kernel(const BwdArgs a) {
+  clear_queue(a);
   constexpr int TPR = DV / 8;  // threads per row, one 16-byte chunk each
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t total = (int64_t)a.B * a.Hq * a.Sq;
@@ -272,7 +286,7 @@ struct Stage64 {
 // dK / dV
 // ------------------------------------------------------------------------------------------------
 template <typename T, int DQK, int DV, int NBUF, bool CAUSAL, int SEG>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
   typedef typename MT<T>::v8 v8;
   constexpr int BMQ = 64;   // query rows per streamed tile
   constexpr int BNK = 128;  // kv rows per workgroup, 32 per wave
@@ -295,635 +309,662 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs a) {
 
   extern __shared__ __align__(16) unsigned char smem[];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
-  int tile, inner, group, n_split = 1, split = 0;
-  if (a.split) {
-    // tile after tile, groups inside, pieces inside those; a lane per tile finds the workgroup's tile
-    const int n_tiles = (a.Skv + BNK - 1) / BNK, r = blockIdx.x / NUM_XCD;
-    const bool before = lane < n_tiles && r >= (int)a.split_first[lane + 1];
-    tile = (int)__popcll(__ballot(before));
-    const int n_gl = (a.B * a.Hkv + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
-    n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
-    const int gl = (r - f) / n_split;
-    split = (r - f) - gl * n_split;
-    group = gl * NUM_XCD + blockIdx.x % NUM_XCD;
-    if (group >= a.B * a.Hkv) return;
-  } else if (!xcd_map((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.turns)) return;
-  const int b = group / a.Hkv, hk = group - b * a.Hkv;
-  const int kv0 = tile * BNK;  // low kv tiles see the most queries: they start first
-  const int wkv0 = kv0 + wave * 32;
-  const int Sq = a.Sq, Skv = a.Skv;
-  // GEN: the instantiation that also evaluates the mask extensions (and then may run without segment ids)
-  constexpr bool GEN = !CAUSAL && SEG == SEG_IDS;
-  const bool has_seg = SEG == SEG_IDS && (!GEN || a.seg != nullptr);
-  const bool ext = GEN && a.mx.on;
-  const bool capped = GEN && a.mx.cap_in != 0.f;
-  const bool biased = GEN && a.mx.bias != nullptr;
-  const bool has_pos = ext && a.mx.qpos != nullptr;
-  const int32_t* segb = has_seg ? a.seg + (int64_t)b * Skv : nullptr;
-
-  // ---- K, V fragments of this wave's 32 kv rows (B operands: lane = kv column)
-  v8 kf[KS_QK], vf[KS_DV];
-  const int kvrow = min(wkv0 + ln, Skv - 1);
-  {
-    const T* kp = (const T*)a.k + b * a.ks[0] + hk * a.ks[1] + kvrow * a.ks[2] + 8 * g;
-    const T* vp = (const T*)a.v + b * a.vs[0] + hk * a.vs[1] + kvrow * a.vs[2] + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < KS_QK; ks++) kf[ks] = *(const v8*)(kp + 16 * ks);
-#pragma unroll
-    for (int ks = 0; ks < KS_DV; ks++) vf[ks] = *(const v8*)(vp + 16 * ks);
-  }
-  const int segk = has_seg ? segb[kvrow] : 0;
-
-  // ---- query tiles to visit: causal => tiles that reach the first kv row; segments => id ranges overlap
-  // (band: row i sees keys i - band_lo .. i + band_hi, so key j is seen by rows j - band_hi .. j + band_lo)
-  const int band_lo = CAUSAL ? a.band_lo : BAND_INF, band_hi = CAUSAL ? a.band_hi : BAND_INF;
-  const int nqt_tot = (Sq + BMQ - 1) / BMQ;
-  const int nqt_all = CAUSAL ? min((kv0 + BNK - 1 + band_lo) / BMQ + 1, nqt_tot) : nqt_tot;  // one past the last tile in reach
-  const int qt_first = CAUSAL ? min(max(kv0 - band_hi, 0) / BMQ, nqt_all) : 0;
-  const int nqt = nqt_all - qt_first;
-  // id ranges of all query tiles and the list of those to visit: only needed until the control entries below are
-  // built, so they borrow the tile buffers, which nothing has been loaded into yet
-  int* qmin = (int*)smem;
-  int* qmax = qmin + nqt;
-  int* active = qmax + nqt;
-  int* bk = (int*)(smem + NBUF * BUF_BYTES + 3 * ROW_BYTES);  // 8 ints: per-wave (min,max) of kv ids
-  int* pmin = bk + 8;      // per query tile: (min,max) of the rows' positions in the key order (mask extensions)
-  int* pmax = pmin + nqt;
-  // per visited tile, in visiting order: (query tile, min id, max id, index into the position ranges), 16 bytes that
-  // one LDS read fetches a whole tile ahead of their use (the tile loop would otherwise start every tile by waiting
-  // out a chain of dependent LDS reads: list entry -> its ranges -> which body to run)
-  // (its address is formed as an offset from the LDS array: rounded through an integer the pointer loses its address
-  // space, every read of an entry becomes a flat load, and waiting for a flat load waits, the vector-memory counter
-  // being in-order, for the tile loads issued before it)
-  const unsigned ctl_off = ((unsigned)((const unsigned char*)(pmax + nqt) - smem) + 15u) & ~15u;
-  int* ctl = (int*)(smem + ctl_off);
-  int nact = nqt;
-  int wkmin = 0, wkmax = 0;
-  if (SEG) {
-    wkmin = segk; wkmax = segk;
-    if (!PAIRS) {
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) {
-      wkmin = min(wkmin, __shfl_xor(wkmin, o, 64));
-      wkmax = max(wkmax, __shfl_xor(wkmax, o, 64));
-    }
-    wkmin = __builtin_amdgcn_readfirstlane(wkmin);
-    wkmax = __builtin_amdgcn_readfirstlane(wkmax);
-    if (lane == 0) { bk[2 * wave] = wkmin; bk[2 * wave + 1] = wkmax; }
-    }
-    if (has_seg) {
-      seg_tile_ranges(segb, Sq, qt_first, nqt_all, qmin, qmax, tid, 256);
-    } else if (PAIRS) {  // (the tile's four classes take the place of the id range)
-      const int* cls = a.pm.kcls + ((int64_t)(a.pm.per_batch ? b : 0) * ((Skv + BNK - 1) / BNK) + tile) * nqt_tot;
-      for (int t = tid; t < nqt; t += 256) { qmin[t] = cls[t]; qmax[t] = 0; }
-    } else {
-      for (int t = tid; t < nqt; t += 256) { qmin[t] = 0; qmax[t] = 0; }
-    }
-    if (ext) {
-      if (has_pos) {
-        seg_tile_ranges(a.mx.qpos, Sq, qt_first, nqt_all, pmin, pmax, tid, 256);
-      } else {
-        for (int t = tid; t < nqt; t += 256) { pmin[t] = (qt_first + t) * BMQ; pmax[t] = min((qt_first + t) * BMQ + BMQ - 1, Sq - 1); }
-      }
-    }
-    __syncthreads();
-    const int bkmin = min(min(bk[0], bk[2]), min(bk[4], bk[6]));
-    const int bkmax = max(max(bk[1], bk[3]), max(bk[5], bk[7]));
-    int cnt = 0;
-    for (int base = 0; base < nqt; base += 64) {
-      const int t = base + lane;
-      bool act = t < nqt && (PAIRS ? qmin[t] != 0 : !(qmax[t] < bkmin || qmin[t] > bkmax));
-      // (band: some row of the tile must reach into this workgroup's 128 kv rows)
-      if (ext && act) act = kv0 <= pmax[t] + a.mx.hi_off && kv0 + BNK - 1 >= pmin[t] - a.mx.lo_off;
-      const unsigned long long m = __ballot(act);
-      if (act && wave == 0) active[cnt + __popcll(m & ((1ull << lane) - 1ull))] = t;
-      cnt += __popcll(m);
-    }
-    nact = cnt;
-    __syncthreads();
-    for (int i = tid; i < nact; i += 256) {
-      const int t = active[nact - 1 - i];  // visiting order: last query tile first (see qtile_of)
-      *(i32x4*)(ctl + 4 * i) = i32x4{qt_first + t, qmin[t], qmax[t], t};
-    }
-    __syncthreads();
-  }
-  // this workgroup's piece of the walk: iterations it_first .. it_first + n_iter - 1
-  const int n_walk = nact * a.n_rep;
-  const int it_first = n_split > 1 ? split * n_walk / n_split : 0;
-  const int n_iter = n_split > 1 ? (split + 1) * n_walk / n_split - it_first : n_walk;
-
-  // ---- staging: every piece of a query tile (Q, dO row-major; log2-scaled LSE, delta, segment ids of its
-  // rows) is written into LDS by the loads themselves; the transposed copies are made LDS-to-LDS
-  QT qdma;
-  OT dodma;
-  qdma.init(a.qs[2], wave, lane);
-  dodma.init(a.dos[2], wave, lane);
-  const unsigned q_span = span_bytes(Sq, a.qs[2], DQK), do_span = span_bytes(Sq, a.dos[2], DV);
-  const unsigned q_tile_bytes = (unsigned)(BMQ * a.qs[2] * 2), do_tile_bytes = (unsigned)(BMQ * a.dos[2] * 2);
-  const float* lse2 = a.delta + (int64_t)a.B * a.Hq * Sq;  // second half of the workspace (written by the kernel before this one)
-  unsigned char* const rows_base = smem + NBUF * BUF_BYTES;
-  // Query tiles are visited from the last one down.  The workgroups of a (batch, kv head) run side by side on one XCD
-  // and all stream the same Q / dO tiles; each needs the tiles from its own kv rows on, so counting up they would start
-  // at different tiles and never meet in the L2 (every tile fetched from memory once per workgroup); counting down
-  // they start together at the last tile and stay within an L2's reach of each other.
-  // pair masks: this wave's 32 kv rows' words of a query tile, 256 bytes
-  const int skp = (Skv + BNK - 1) / BNK * BNK;
-  const u32x4 brw = make_rsrc_words(PAIRS ? (const void*)(a.pm.kbits + (int64_t)(a.pm.per_batch ? b : 0) * nqt_tot * skp) : a.k,
-                                    PAIRS ? (unsigned)nqt_tot * (unsigned)skp * 8u : 0u);
-  auto qtile_of = [&](int idx) { return SEG ? ctl[4 * idx] : nqt_all - 1 - idx; };
-  auto issue_tile = [&](int hl, int idx, int buf, int rslot) {
-    const int hq = hk * a.n_rep + hl;
-    const int qt = qtile_of(idx);
-    qdma.issue(make_rsrc_words((const T*)a.q + b * a.qs[0] + hq * a.qs[1], q_span), (unsigned)qt * q_tile_bytes,
-               smem + Q_AT + buf * Q_BYTES, wave);
-    dodma.issue(make_rsrc_words((const T*)a.dout + b * a.dos[0] + hq * a.dos[1], do_span), (unsigned)qt * do_tile_bytes,
-                smem + DO_AT + buf * DO_BYTES, wave);
-    // waves 0..2 fetch one 64-entry row vector each: 4 bytes per lane, rows past Sq arrive as zeros
-    const int64_t ro = ((int64_t)b * a.Hq + hq) * Sq;
-    const void* src = wave == 0 ? (const void*)(lse2 + ro) : wave == 1 ? (const void*)(a.delta + ro)
-                    : wave == 2 ? (const void*)segb : (const void*)a.mx.qpos;
-    if (wave < 2 || (wave == 2 && has_seg) || (wave == 3 && has_pos))
-      dma_dword(make_rsrc_words(src, (unsigned)Sq * 4u), (unsigned)(qt * BMQ) * 4u, rows_base + rslot * ROW_BYTES + wave * BMQ * 4, lane);
-    if constexpr (PAIRS)
-      dma_dword(brw, ((unsigned)qt * (unsigned)skp + (unsigned)wkv0) * 8u, rows_base + rslot * ROW_BYTES + VEC_BYTES + wave * 256, lane);
-  };
-
-  // per-lane byte offsets of the MFMA fragments inside a tile (the swizzles are resolved once, here)
-  unsigned faq[KS_QK], fao[KS_DV];
-#pragma unroll
-  for (int ks = 0; ks < KS_QK; ks++) faq[ks] = (unsigned)QT::off(ln, 2 * ks + g);
-#pragma unroll
-  for (int ks = 0; ks < KS_DV; ks++) fao[ks] = (unsigned)OT::off(ln, 2 * ks + g);
-
+  // With a queue a workgroup does one item (kv tile of a group) after the other; see dkdv_queued.  (The general
+  // instantiation spills as it is: one item per workgroup.)
+  constexpr bool PERSIST = (CAUSAL || SEG == SEG_NONE) && dkdv_per_cu(DQK) == 1;
+  int* const next_at = (int*)(smem + NBUF * BUF_BYTES + 3 * ROW_BYTES);  // the slot of the workgroup's next item
   f32x16 dkacc[DKB], dvacc[DVB];
-  {
-    // whole-vector values from the start: element-wise initialisation makes the compiler track 16 scalars per
-    // accumulator across the loop and reassemble the tuple around every accumulating MFMA
-    f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int d = 0; d < DKB; d++) {
-      asm volatile("" : "+a"(zero16));
-      dkacc[d] = zero16;
-    }
-#pragma unroll
-    for (int d = 0; d < DVB; d++) {
-      asm volatile("" : "+a"(zero16));
-      dvacc[d] = zero16;
-    }
-  }
-  const float c = a.scale_log2;
+  int slot = blockIdx.x / NUM_XCD;
+  for (;;) {
+    // (the arguments and the lane, read anew for every item: what is derived from them would otherwise be kept across items
+    // in registers that the tile loop needs)
+    const BwdArgs& a = kernel_args<BwdArgs>();
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
+    int tile, inner, group, n_split = 1, split = 0;
+    if (a.split) {
+      // tile after tile, groups inside, pieces inside those; a lane per tile finds the workgroup's tile
+      const int n_tiles = (a.Skv + BNK - 1) / BNK, r = blockIdx.x / NUM_XCD;
+      const bool before = lane < n_tiles && r >= (int)a.split_first[lane + 1];
+      tile = (int)__popcll(__ballot(before));
+      const int n_gl = (a.B * a.Hkv + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
+      n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
+      const int gl = (r - f) / n_split;
+      split = (r - f) - gl * n_split;
+      group = gl * NUM_XCD + blockIdx.x % NUM_XCD;
+      if (group >= a.B * a.Hkv) return;
+    } else if (!xcd_item(slot, blockIdx.x % NUM_XCD, (a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.turns)) return;
+    const int b = group / a.Hkv, hk = group - b * a.Hkv;
+    const int kv0 = tile * BNK;  // low kv tiles see the most queries: they start first
+    const int wkv0 = kv0 + wave * 32;
+    const int Sq = a.Sq, Skv = a.Skv;
+    // GEN: the instantiation that also evaluates the mask extensions (and then may run without segment ids)
+    constexpr bool GEN = !CAUSAL && SEG == SEG_IDS;
+    const bool has_seg = SEG == SEG_IDS && (!GEN || a.seg != nullptr);
+    const bool ext = GEN && a.mx.on;
+    const bool capped = GEN && a.mx.cap_in != 0.f;
+    const bool biased = GEN && a.mx.bias != nullptr;
+    const bool has_pos = ext && a.mx.qpos != nullptr;
+    const int32_t* segb = has_seg ? a.seg + (int64_t)b * Skv : nullptr;
 
-  // wave-level decisions for a query tile (uniform): skip if every query row precedes every kv row
-  // (lo, hi: id range of the query tile; t: its index into the position ranges)
-  // (The decisions are taken on the wave's first kv row as it arrives, in a vector register.  With a scalar copy the
-  // compiler turns the choice of the tile body into scalar branches and copies the pinned accumulators between them,
-  // right behind the MFMAs that write them: the build's hazard check rejects that code.  The same change in the
-  // forward and the lean dQ kernel passed the check and ran 45 % and 64 % slower.)
-  auto tile_mode_of = [&](int lo, int hi, int t, int qi0) {  // 0 = nothing to compute, 1 = no masking needed, 2 = masked
-    bool skip = (CAUSAL && (qi0 + BMQ - 1 + band_hi < wkv0 || qi0 - band_lo > wkv0 + 31)) || wkv0 >= Skv;
-    bool need_mask = (qi0 + BMQ > Sq) || (wkv0 + 32 > Skv) ||
-                     (CAUSAL && (qi0 + band_hi < wkv0 + 31 || qi0 + BMQ - 1 - band_lo > wkv0));
+    // ---- K, V fragments of this wave's 32 kv rows (B operands: lane = kv column)
+    v8 kf[KS_QK], vf[KS_DV];
+    const int kvrow = min(wkv0 + ln, Skv - 1);
+    {
+      const T* kp = (const T*)a.k + b * a.ks[0] + hk * a.ks[1] + kvrow * a.ks[2] + 8 * g;
+      const T* vp = (const T*)a.v + b * a.vs[0] + hk * a.vs[1] + kvrow * a.vs[2] + 8 * g;
+#pragma unroll
+      for (int ks = 0; ks < KS_QK; ks++) kf[ks] = *(const v8*)(kp + 16 * ks);
+#pragma unroll
+      for (int ks = 0; ks < KS_DV; ks++) vf[ks] = *(const v8*)(vp + 16 * ks);
+    }
+    const int segk = has_seg ? segb[kvrow] : 0;
+
+    // ---- query tiles to visit: causal => tiles that reach the first kv row; segments => id ranges overlap
+    // (band: row i sees keys i - band_lo .. i + band_hi, so key j is seen by rows j - band_hi .. j + band_lo)
+    const int band_lo = CAUSAL ? a.band_lo : BAND_INF, band_hi = CAUSAL ? a.band_hi : BAND_INF;
+    const int nqt_tot = (Sq + BMQ - 1) / BMQ;
+    const int nqt_all = CAUSAL ? min((kv0 + BNK - 1 + band_lo) / BMQ + 1, nqt_tot) : nqt_tot;  // one past the last tile in reach
+    const int qt_first = CAUSAL ? min(max(kv0 - band_hi, 0) / BMQ, nqt_all) : 0;
+    const int nqt = nqt_all - qt_first;
+    // id ranges of all query tiles and the list of those to visit: only needed until the control entries below are
+    // built, so they borrow the tile buffers, which nothing has been loaded into yet
+    int* qmin = (int*)smem;
+    int* qmax = qmin + nqt;
+    int* active = qmax + nqt;
+    int* bk = next_at + 4;   // 8 ints: per-wave (min,max) of kv ids
+    int* pmin = bk + 8;      // per query tile: (min,max) of the rows' positions in the key order (mask extensions)
+    int* pmax = pmin + nqt;
+    // per visited tile, in visiting order: (query tile, min id, max id, index into the position ranges), 16 bytes that
+    // one LDS read fetches a whole tile ahead of their use (the tile loop would otherwise start every tile by waiting
+    // out a chain of dependent LDS reads: list entry -> its ranges -> which body to run)
+    // (its address is formed as an offset from the LDS array: rounded through an integer the pointer loses its address
+    // space, every read of an entry becomes a flat load, and waiting for a flat load waits, the vector-memory counter
+    // being in-order, for the tile loads issued before it)
+    const unsigned ctl_off = ((unsigned)((const unsigned char*)(pmax + nqt) - smem) + 15u) & ~15u;
+    int* ctl = (int*)(smem + ctl_off);
+    int nact = nqt;
+    int wkmin = 0, wkmax = 0;
     if (SEG) {
-      if (PAIRS) {
-        const int cls = (lo >> (8 * wave)) & 255;
-        skip = skip || cls == 0;
-        need_mask = need_mask || cls != 2;
+      wkmin = segk; wkmax = segk;
+      if (!PAIRS) {
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) {
+        wkmin = min(wkmin, __shfl_xor(wkmin, o, 64));
+        wkmax = max(wkmax, __shfl_xor(wkmax, o, 64));
+      }
+      wkmin = __builtin_amdgcn_readfirstlane(wkmin);
+      wkmax = __builtin_amdgcn_readfirstlane(wkmax);
+      if (lane == 0) { bk[2 * wave] = wkmin; bk[2 * wave + 1] = wkmax; }
+      }
+      if (has_seg) {
+        seg_tile_ranges(segb, Sq, qt_first, nqt_all, qmin, qmax, tid, 256);
+      } else if (PAIRS) {  // (the tile's four classes take the place of the id range)
+        const int* cls = a.pm.kcls + ((int64_t)(a.pm.per_batch ? b : 0) * ((Skv + BNK - 1) / BNK) + tile) * nqt_tot;
+        for (int t = tid; t < nqt; t += 256) { qmin[t] = cls[t]; qmax[t] = 0; }
       } else {
-        skip = skip || hi < wkmin || lo > wkmax;
-        need_mask = need_mask || !(lo == hi && wkmin == wkmax && lo == wkmin);
+        for (int t = tid; t < nqt; t += 256) { qmin[t] = 0; qmax[t] = 0; }
       }
-    }
-    if (ext) {
-      const int plo = pmin[t], phi = pmax[t];
-      skip = skip || wkv0 > phi + a.mx.hi_off || wkv0 + 31 < plo - a.mx.lo_off;
-      need_mask = need_mask || capped || biased || !(wkv0 >= phi - a.mx.lo_off && wkv0 + 31 <= plo + a.mx.hi_off);
-    }
-    return skip ? 0 : (need_mask ? 2 : 1);
-  };
-  auto tile_mode = [&](int idx, int qi0) {
-    const int* e = ctl + 4 * idx;
-    return tile_mode_of(SEG ? e[1] : 0, SEG ? e[2] : 0, SEG ? e[3] : 0, qi0);
-  };
-  // iteration -> (query head of the group, query tile): heads outer, tiles inner, no division in the loop.  (Tiles
-  // outer would keep the group's workgroups on the same tile for the whole launch and cut the fetches from memory to
-  // 1.8 GB at the benchmark's shape, against 6.5 GB this way - and ran 4 % slower: 32 CUs asking one L2 for the same
-  // lines at the same time, and the descriptors rebuilt every tile.)
-  auto advance = [&](int& hl, int& idx) {
-    if (++idx == nact) { idx = 0; hl++; }
-  };
-
-  {
-    // Software pipeline over query tiles t, three row-major buffers and three row-vector slots (tile t lives in
-    // buffer and slot t % 3), one barrier per tile:
-    //   part 1 (S, dP: fragment reads of buffer t % 3)
-    //   wait for this wave's share of tile t+1 (issued a whole tile earlier), barrier
-    //                                  -> tile t+1 has landed for everybody, everybody is done with tile t-1
-    //   part 2 (dV, dK: transposing reads of buffer t % 3), with the loads of tile t+2 issued between its MFMAs
-    //   into the buffer tile t-1 used
-    const int hl_first = n_split > 1 ? it_first / max(nact, 1) : 0, idx_first = it_first - hl_first * nact;
-    int c_hl = hl_first, c_idx = idx_first, n_hl = hl_first, n_idx = idx_first;  // tile being computed, tile whose loads are issued next
-    // Per-lane LDS byte addresses of the operands inside a tile (base of the workgroup's LDS included), each an
-    // opaque register: every read below is such a register plus an immediate.  (Formed from the `smem` symbol, the
-    // same addresses cost an add per read whenever the constant part happens to be zero, and the compiler
-    // recomputes what it could have kept.)  Addresses into the dO tiles carry O_BIAS: constants there would
-    // otherwise exceed the reach of an instruction offset.
-    //   aq / ao   fragment reads of the row-major tiles (S, dP): row ln, chunk 2 ks + g
-    //   trq / tro transposing reads (dK, dV): head-dim block d (32 columns), half h2 (rows +8); the query block and
-    //             the k-step are immediates (multiples of 16 rows leave the swizzle alone)
-    constexpr int O_BIAS = DO_AT;
-    const unsigned lb = (unsigned)(size_t)smem;
-    unsigned aq[KS_QK], ao[KS_DV], trq[DKB][2], tro[DVB][2];
-#pragma unroll
-    for (int ks = 0; ks < KS_QK; ks++) { aq[ks] = faq[ks] + lb; asm volatile("" : "+v"(aq[ks])); }
-#pragma unroll
-    for (int ks = 0; ks < KS_DV; ks++) { ao[ks] = fao[ks] + lb + (unsigned)O_BIAS; asm volatile("" : "+v"(ao[ks])); }
-#pragma unroll
-    for (int d = 0; d < DKB; d++)
-#pragma unroll
-      for (int h2 = 0; h2 < 2; h2++) {
-        trq[d][h2] = (unsigned)QT::tr_off(8 * h2 + 4 * g, 2 * d + ((lane >> 4) & 1), lane & 15) + lb;
-        asm volatile("" : "+v"(trq[d][h2]));
-      }
-#pragma unroll
-    for (int d = 0; d < DVB; d++)
-#pragma unroll
-      for (int h2 = 0; h2 < 2; h2++) {
-        tro[d][h2] = (unsigned)OT::tr_off(8 * h2 + 4 * g, 2 * d + ((lane >> 4) & 1), lane & 15) + lb + (unsigned)O_BIAS;
-        asm volatile("" : "+v"(tro[d][h2]));
-      }
-    auto ld16 = [](unsigned addr) { return *(const __attribute__((address_space(3))) v8*)addr; };
-    auto ldtr = [](unsigned a0, unsigned a1) {
-      return tr_read8<v8>((const __attribute__((address_space(3))) unsigned char*)a0, (const __attribute__((address_space(3))) unsigned char*)a1);
-    };
-    if (n_iter > 0) { issue_tile(n_hl, n_idx, 0, 0); advance(n_hl, n_idx); }
-    if (n_iter > 1) { issue_tile(n_hl, n_idx, 1, 1); advance(n_hl, n_idx); }
-    // the control entry of the tile being computed and the query tile whose loads are issued next, as scalars; their
-    // successors are read at the top of a tile and taken over at its end
-    auto entry = [&](int idx) {
-      if constexpr (SEG) return *(const i32x4*)(ctl + 4 * min(idx, max(nact - 1, 0)));
-      else return i32x4{nqt_all - 1 - idx, 0, 0, 0};
-    };
-    auto scalar4 = [&](i32x4 v) {
-      return i32x4{__builtin_amdgcn_readfirstlane(v[0]), __builtin_amdgcn_readfirstlane(v[1]),
-                   __builtin_amdgcn_readfirstlane(v[2]), __builtin_amdgcn_readfirstlane(v[3])};
-    };
-    i32x4 cur = scalar4(entry(c_idx));
-    int nq_cur = __builtin_amdgcn_readfirstlane(entry(n_idx)[0]);
-    // all earlier loads (the K/V fragments, the first tiles) have landed
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    // fragment ring: slot i's LDS fragment is requested AHEAD slots earlier and kept in fr[i % NF]; the
-    // first AHEAD fragments of a tile are requested at the end of the tile before it (its row-major
-    // tiles are complete by then), so that the LDS round trip and the scalar bookkeeping at the top of
-    // the loop overlap
-    constexpr int AHEAD = KS_QK >= 8 ? 5 : 3, NF = AHEAD + 1;
-    v8 fr[NF];
-    static_for<0, AHEAD>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      static_assert(AHEAD <= KS_QK, "the carried fragments all belong to S of the first query block");
-      fr[i % NF] = ld16(aq[i] + Q_AT);
-    });
-    struct { u32x4 rq, ro, rr; unsigned offq, offo, offr, offb; } nx;
-    const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
-    const unsigned wave_q = __builtin_amdgcn_readfirstlane((unsigned)(wave * QT::PER_WAVE * 1024));
-    const unsigned wave_o = __builtin_amdgcn_readfirstlane((unsigned)(wave * OT::PER_WAVE * 1024));
-    const unsigned wave_r = __builtin_amdgcn_readfirstlane((unsigned)(wave * BMQ * 4));
-    // one query tile; the buffer index is a constant (the loop below rotates three copies of this)
-    auto iteration = [&](auto BUFc, const int it) {
-      constexpr int buf = decltype(BUFc)::value;
-      const int qi0 = cur[0] * BMQ;
-      const int mode = tile_mode_of(cur[1], cur[2], cur[3], qi0);
-      const bool issue_next = it + 2 < n_iter;
-      // successors of the two cursors (read now, used when this tile is done)
-      int c_hl2 = c_hl, c_idx2 = c_idx, n_hl2 = n_hl, n_idx2 = n_idx;
-      advance(c_hl2, c_idx2);
-      if (issue_next) advance(n_hl2, n_idx2);
-      const i32x4 cur_next = entry(c_idx2);
-      const int nq_next = entry(n_idx2)[0];
-      constexpr int buf1 = (buf + 1) % 3, buf2 = (buf + 2) % 3;  // tile t+1 (read first in the next iteration), tile t+2
-      constexpr unsigned ql = Q_AT + buf * Q_BYTES;                // + aq[] / trq[]
-      constexpr unsigned dol = DO_AT + buf * DO_BYTES - O_BIAS;    // + ao[] / tro[]
-      constexpr unsigned nxq = Q_AT + buf1 * Q_BYTES;
-      const float* lsel = (const float*)(rows_base + buf * ROW_BYTES);
-      const float* deltal = lsel + BMQ;
-      const int* segl = (const int*)(deltal + BMQ);
-      const int* posl = segl + BMQ;  // query positions of the tile's rows (mask extensions)
-      const float* bias_head = biased ? a.mx.bias + b * a.mx.bias_s[0] + (hk * a.n_rep + c_hl) * a.mx.bias_s[1] : nullptr;
-      // LDS destinations of this wave's loads of tile t+2 (scalar byte addresses)
-      const unsigned dma_q = lds_base + (unsigned)(Q_AT + buf2 * Q_BYTES) + wave_q;
-      const unsigned dma_o = lds_base + (unsigned)(DO_AT + buf2 * DO_BYTES) + wave_o;
-      const unsigned dma_b = lds_base + (unsigned)(NBUF * BUF_BYTES + buf2 * ROW_BYTES + VEC_BYTES) + wave_r;  // (wave_r: 256 bytes a wave)
-      const unsigned dma_r = lds_base + (unsigned)(NBUF * BUF_BYTES + buf2 * ROW_BYTES) + wave_r;
-      // descriptors of tile t+2's loads (wave-uniform), issued piecewise in part 2.  The bases change with
-      // the query head only; they are rebuilt when a new head starts (and when the tiles run out: size 0).
-      if (it == 0 || n_idx == 0 || !issue_next) {
-        const int hq = hk * a.n_rep + (issue_next ? n_hl : 0);
-        nx.rq = make_rsrc_words((const T*)a.q + b * a.qs[0] + hq * a.qs[1], issue_next ? q_span : 0u);
-        nx.ro = make_rsrc_words((const T*)a.dout + b * a.dos[0] + hq * a.dos[1], issue_next ? do_span : 0u);
-        const int64_t ro = ((int64_t)b * a.Hq + hq) * Sq;
-        const void* src = wave == 0 ? (const void*)(lse2 + ro) : wave == 1 ? (const void*)(a.delta + ro)
-                        : wave == 2 ? (const void*)segb : (const void*)a.mx.qpos;
-        // a wave with no row vector to fetch (wave 2 without segment ids, wave 3 without query positions): size 0
-        nx.rr = make_rsrc_words(src, (issue_next && (wave < 2 || (wave == 2 && has_seg) || (wave == 3 && has_pos))) ? (unsigned)Sq * 4u : 0u);
-      }
-      {
-        const int qt = issue_next ? nq_cur : 0;
-        nx.offq = __builtin_amdgcn_readfirstlane((unsigned)qt * q_tile_bytes);
-        nx.offo = __builtin_amdgcn_readfirstlane((unsigned)qt * do_tile_bytes);
-        nx.offr = __builtin_amdgcn_readfirstlane((unsigned)(qt * BMQ) * 4u);
-        nx.offb = PAIRS ? __builtin_amdgcn_readfirstlane(((unsigned)qt * (unsigned)skp + (unsigned)wkv0) * 8u) : 0u;
-      }
-
-      // The tile body is laid out by hand as a sequence of slots, one MFMA each, with a scheduling barrier
-      // after every slot: the LDS fragment a slot needs was requested AHEAD slots earlier, and the
-      // exponentials / products that turn S, dP into the 16-bit operands P, dS are spread over the slots
-      // under the MFMAs of the other query block.  (Left to itself the compiler reads each fragment right
-      // before its MFMA and the matrix unit waits out every LDS round trip.)
-      //   slots   part 1: S0 = Q0 K^T, S1 = Q1 K^T, dP0 = dO0 V^T, dP1 = dO1 V^T
-      //           part 2: dV^T += dO0^T P0, dK^T += Q0^T dS0, dV^T += dO1^T P1, dK^T += Q1^T dS1
-      //   VALU    P0 from S1 on, P1 from dP0 on, dS0 from dP1 on, dS1 from part 2 on
-      auto body = [&](auto mode_c) {
-        constexpr int MODE = decltype(mode_c)::value;
-        constexpr bool COMPUTE = MODE != 0, MASKED = MODE == 2;
-        // part 1: S0, S1, dP0, dP1 (the exponentials can start as soon as S0 is complete and are over
-        // before part 2, which carries the transposition of the next tile);
-        // part 2: dV0, dK0, dV1, dK1 (four accumulators each, used round robin)
-        // (K1 / K2 k-steps per S / dP product; CLV / CLK slots per query block of dV / dK)
-        constexpr int K1 = KS_QK, K2 = KS_DV, CLV = 2 * DVB, CLK = 2 * DKB;
-        constexpr int S1_AT = K1, D0_AT = 2 * K1, D1_AT = 2 * K1 + K2, C0 = 2 * (K1 + K2);
-        constexpr int V0_AT = C0, K0_AT = V0_AT + CLV, V1_AT = K0_AT + CLK, K1_AT = V1_AT + CLV, NS = K1_AT + CLK;
-        // VALU groups of VL slots each: P of a block starts when its S is complete, dS when its dP is; each
-        // group is over before the MFMAs that consume its packed operand
-        constexpr int EPS = K2 >= 8 ? 1 : 2, VL = 16 / EPS;
-        constexpr int VP0 = S1_AT, VP1 = D0_AT, VS0 = D1_AT, VS1 = C0;
-        static_assert(VP0 + VL <= V0_AT && VS0 + VL <= K0_AT && VP1 + VL <= V1_AT && VS1 + VL <= K1_AT, "operands not ready");
-        constexpr int N_DMA = QT::PER_WAVE + OT::PER_WAVE + 1 + (PAIRS ? 1 : 0), DMA_EVERY = (NS - C0) / N_DMA;
-        static_assert(DMA_EVERY >= 1, "second half too short for the loads");
-        const int kvcol = wkv0 + ln;
-        f32x16 s[2], dp[2];
-        v8 pf[2][2], df[2][2];
-        // -LSE (log2 units) and -delta of the 16 rows a lane holds of either query block.  LDS reads return in
-        // order, so each group is requested a ring depth or more before its first use: waiting for it then waits
-        // for no fragment that is not due anyway
-        f32x4 nl0[4], nl1[4], nd0[4], nd1[4];
-        float fc[2][16];  // soft cap: 1 - tanh^2 of every score, kept from P to dS
-        // Masked tiles without the mask extensions: which of the tile's 64 query rows this lane's kv column may see,
-        // as one bit per row, built once per tile (bounds and causality are a bit range; the rows of each id present
-        // among the wave's columns come from a ballot over the tile's id vector).  An element then costs a bit-field
-        // extract and an AND instead of four compares.  rowbits[qb] is shifted so that value v of the lane's 16 is
-        // bit 8 (v / 4) + v % 4.
-        unsigned rowbits[2] = {0u, 0u};
-        const bool by_bits = MASKED && !(GEN && ext);
-        if (MASKED && PAIRS) {
-          const u32x2 w = *(const u32x2*)(rows_base + buf * ROW_BYTES + VEC_BYTES + wave * 256 + ln * 8);
-          rowbits[0] = w[0] >> (4 * g);
-          rowbits[1] = w[1] >> (4 * g);
-        } else if (MASKED && by_bits) {
-          const int lo_r = CAUSAL ? max(kvcol - band_hi - qi0, 0) : 0;
-          int hi_r = kvcol < Skv ? min(Sq - qi0, BMQ) : 0;
-          if (CAUSAL) hi_r = min(hi_r, kvcol + band_lo - qi0 + 1);
-          unsigned long long m = 0ull;
-          if (hi_r > lo_r) m = (~0ull << lo_r) & (~0ull >> (64 - hi_r));
-          if (SEG == SEG_IDS && has_seg) {
-            const int rowseg = segl[lane];  // lane l: id of the tile's query row l
-            unsigned long long ms = 0ull, todo = ~0ull;
-            while (todo) {
-              const int x = __builtin_amdgcn_readlane(segk, (int)__builtin_ctzll(todo));
-              const unsigned long long rows = __ballot(rowseg == x);
-              const bool mine = segk == x;
-              ms = mine ? rows : ms;
-              todo &= ~__ballot(mine);
-            }
-            m &= ms;
-          }
-          rowbits[0] = (unsigned)m >> (4 * g);
-          rowbits[1] = (unsigned)(m >> 32) >> (4 * g);
+      if (ext) {
+        if (has_pos) {
+          seg_tile_ranges(a.mx.qpos, Sq, qt_first, nqt_all, pmin, pmax, tid, 256);
+        } else {
+          for (int t = tid; t < nqt; t += 256) { pmin[t] = (qt_first + t) * BMQ; pmax[t] = min((qt_first + t) * BMQ + BMQ - 1, Sq - 1); }
         }
-
-        auto frag = [&](auto I) -> v8 {
-          constexpr int i = decltype(I)::value;
-          if constexpr (i < D0_AT) {
-            constexpr int qb = i / K1, ks = i % K1;
-            return ld16(aq[ks] + (ql + qb * 32 * QT::ROWB));
-          } else if constexpr (i < C0) {
-            constexpr int qb = (i - D0_AT) / K2, ks = (i - D0_AT) % K2;
-            return ld16(ao[ks] + (dol + qb * 32 * OT::ROWB));
-          } else {
-            // operand of an accumulating product: rows = head-dim block d, contraction over query rows
-            // 32 qb + 16 hh + {4g..4g+3, 8+4g..8+4g+3} (the order in which P / dS hold them), read transposed
-            constexpr int qb = i >= V1_AT ? 1 : 0, base = qb ? V1_AT : V0_AT;
-            if constexpr (i - base < CLV) {
-              constexpr int j = i - base, hh = j / DVB, d = j % DVB;
-              constexpr int rows = (32 * qb + 16 * hh) * OT::ROWB;
-              return ldtr(tro[d][0] + (dol + rows), tro[d][1] + (dol + rows));
-            } else {
-              constexpr int j = i - base - CLV, hh = j / DKB, d = j % DKB;
-              constexpr int rows = (32 * qb + 16 * hh) * QT::ROWB;
-              return ldtr(trq[d][0] + (ql + rows), trq[d][1] + (ql + rows));
-            }
-          }
-        };
-        auto mma = [&](auto I, const v8& f) {
-          constexpr int i = decltype(I)::value;
-          const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-          if constexpr (i < D0_AT) {
-            constexpr int qb = i / K1, ks = i % K1;
-            s[qb] = MT<T>::mfma32(f, kf[ks], ks == 0 ? zero : s[qb]);
-          } else if constexpr (i < C0) {
-            constexpr int qb = (i - D0_AT) / K2, ks = (i - D0_AT) % K2;
-            if constexpr (ks == 0) {
-              // dP starts from -delta of its rows (C layout: value v belongs to row 8 (v/4) + 4 g + v%4), so
-              // that dS = P o dP needs no subtraction
-              const f32x4 (&nd)[4] = qb == 0 ? nd0 : nd1;
-              const f32x16 init = {nd[0][0], nd[0][1], nd[0][2], nd[0][3], nd[1][0], nd[1][1], nd[1][2], nd[1][3],
-                                   nd[2][0], nd[2][1], nd[2][2], nd[2][3], nd[3][0], nd[3][1], nd[3][2], nd[3][3]};
-              dp[qb] = MT<T>::mfma32(f, vf[ks], init);
-            } else {
-              dp[qb] = MT<T>::mfma32(f, vf[ks], dp[qb]);
-            }
-          } else {
-            constexpr int qb = i >= V1_AT ? 1 : 0, base = qb ? V1_AT : V0_AT;
-            if constexpr (i - base < CLV) {
-              constexpr int j = i - base, hh = j / DVB, d = j % DVB;
-              MT<T>::mfma32_acc(dvacc[d], f, pf[qb][hh]);
-            } else {
-              constexpr int j = i - base - CLV, hh = j / DKB, d = j % DKB;
-              MT<T>::mfma32_acc(dkacc[d], f, df[qb][hh]);
-            }
-          }
-        };
-        // VALU group of query block QB starting at slot START: EPS elements per slot for VL slots.
-        // IS_P: s <- exp2(s c - lse) (masked), else dp <- s (dp - delta); the 16-bit operands are packed as
-        // soon as the eight values of a half are done.
-        auto valu = [&](auto I, auto START, auto QBc, auto IS_Pc) {
-          constexpr int i = decltype(I)::value, st = decltype(START)::value, qb = decltype(QBc)::value;
-          constexpr bool IS_P = decltype(IS_Pc)::value;
-          constexpr int QS = 4 / EPS;  // slots per quad of rows
-          if constexpr (i >= st && i < st + VL) {
-            constexpr int k = i - st, vq = k / QS;
-#pragma unroll
-            for (int e2 = 0; e2 < EPS; e2++) {
-              const int e = EPS * (k % QS) + e2, v = 4 * vq + e;
-              if constexpr (IS_P) {
-                const f32x4 (&nl)[4] = qb == 0 ? nl0 : nl1;
-                float sval = s[qb][v];
-                if (GEN && MASKED) {
-                  if (capped) {
-                    const float th = fast_tanh(sval * a.mx.cap_in);
-                    fc[qb][v] = 1.f - th * th;
-                    sval = a.mx.cap_out * th;
-                  }
-                  if (biased) {  // additive mask, in units of the raw score (-inf stays -inf)
-                    const int qrow_b = min(qi0 + qb * 32 + 8 * vq + 4 * g + e, Sq - 1);
-                    sval += a.mx.bias_mul * bias_head[(int64_t)qrow_b * a.mx.bias_s[2] + min(kvcol, Skv - 1)];
-                  }
-                }
-                float pv = fast_exp2(__builtin_fmaf(sval, c, nl[vq][e]));
-                if (MASKED) {
-                  if (by_bits) {
-                    pv = __builtin_bit_cast(float, __builtin_bit_cast(int, pv) & __builtin_amdgcn_sbfe((int)rowbits[qb], 8 * vq + e, 1));
-                  } else {
-                    const int r = qb * 32 + 8 * vq + 4 * g + e;
-                    const int qrow = qi0 + r;
-                    bool ok = qrow < Sq && kvcol < Skv && (!CAUSAL || kvcol <= qrow) && (!SEG || !has_seg || segl[r] == segk);
-                    if (GEN) {
-                      if (ext) {
-                        const int qp = has_pos ? posl[r] : qrow;
-                        ok = ok && kvcol >= qp - a.mx.lo_off && kvcol <= qp + a.mx.hi_off;
-                      }
-                    }
-                    pv = ok ? pv : 0.f;
-                  }
-                }
-                asm volatile("" : "+v"(pv));  // anchors the computation in this slot (it would sink past the barrier)
-                s[qb][v] = pv;
-              } else {
-                float dsv = s[qb][v] * dp[qb][v];
-                if (GEN && MASKED) {
-                  if (capped) dsv *= fc[qb][v];  // derivative of the capped score with respect to the raw one
-                }
-                asm volatile("" : "+v"(dsv));
-                dp[qb][v] = dsv;
-              }
-            }
-            if constexpr (((k + 1) * EPS) % 8 == 0) {
-              constexpr int hh = (k + 1) * EPS / 8 - 1;
-              const f32x16& x = IS_P ? s[qb] : dp[qb];
-              const v8 packed = pack8<T>(x[8 * hh + 0], x[8 * hh + 1], x[8 * hh + 2], x[8 * hh + 3], x[8 * hh + 4],
-                                         x[8 * hh + 5], x[8 * hh + 6], x[8 * hh + 7]);
-              if constexpr (IS_P) pf[qb][hh] = packed;
-              else df[qb][hh] = packed;
-            }
-          }
-        };
-        typedef std::integral_constant<int, 0> I0;
-        typedef std::integral_constant<int, 1> I1;
-        static_for<0, NS>([&](auto I) {
-          constexpr int i = decltype(I)::value;
-          if constexpr (i == C0) {
-            // this wave's loads of tile t+1 were issued a tile ago (vmcnt only: fragment reads stay in flight)
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-            __syncthreads();
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          // the loads of tile t+2, one instruction every few slots: the texture path takes a kilobyte in
-          // some 25 cycles for the whole CU, and a wave that issues them back to back sits out the queue
-          if constexpr (i >= C0 && (i - C0) % DMA_EVERY == 0 && (i - C0) / DMA_EVERY < N_DMA) {
-            constexpr int m = (i - C0) / DMA_EVERY;
-            // (no branch here: past the last tile the descriptors have size 0 and the loads deliver zeros
-            // into buffers nobody reads any more)
-            if constexpr (m < QT::PER_WAVE) qdma.template issue_one_at<m>(nx.rq, nx.offq, dma_q);
-            else if constexpr (m < QT::PER_WAVE + OT::PER_WAVE) dodma.template issue_one_at<m - QT::PER_WAVE>(nx.ro, nx.offo, dma_o);
-            else if constexpr (m == QT::PER_WAVE + OT::PER_WAVE) dma_dword_at(nx.rr, nx.offr, dma_r, lane);
-            else dma_dword_at(brw, nx.offb, dma_b, lane);
-          }
-          if constexpr (COMPUTE) {
-            // row vectors, a quad of rows at a time: -LSE of query block qb LEAD slots before the exponentials of that
-            // quad (VP0 / VP1 + QS vq), -delta two slots before the first dP MFMA of the block (2K, 3K)
-            constexpr int QS = 4 / EPS, LEAD = 3;
-            static_for<0, 4>([&](auto VQ) {
-              constexpr int vq = decltype(VQ)::value;
-              constexpr int r0 = VP0 + QS * vq - LEAD, r1 = VP1 + QS * vq - LEAD;
-              if constexpr (i == (r0 < 0 ? 0 : r0)) nl0[vq] = *(const f32x4*)(lsel + 8 * vq + 4 * g);
-              if constexpr (i == (r1 < 0 ? 0 : r1)) nl1[vq] = *(const f32x4*)(lsel + 32 + 8 * vq + 4 * g);
-            });
-            if constexpr (i == D0_AT - 2) {
-#pragma unroll
-              for (int vq = 0; vq < 4; vq++) nd0[vq] = *(const f32x4*)(deltal + 8 * vq + 4 * g);
-            }
-            if constexpr (i == D1_AT - 2) {
-#pragma unroll
-              for (int vq = 0; vq < 4; vq++) nd1[vq] = *(const f32x4*)(deltal + 32 + 8 * vq + 4 * g);
-            }
-            if constexpr (i + AHEAD < NS) fr[(i + AHEAD) % NF] = frag(std::integral_constant<int, i + AHEAD>{});
-            mma(I, fr[i % NF]);
-            valu(I, std::integral_constant<int, VP0>{}, I0{}, std::true_type{});
-            valu(I, std::integral_constant<int, VP1>{}, I1{}, std::true_type{});
-            valu(I, std::integral_constant<int, VS0>{}, I0{}, std::false_type{});
-            valu(I, std::integral_constant<int, VS1>{}, I1{}, std::false_type{});
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        });
-        static_for<0, AHEAD>([&](auto I) {
-          constexpr int i = decltype(I)::value;
-          fr[i % NF] = ld16(aq[i] + nxq);
-        });
-      };
-      if (mode == 1) body(std::integral_constant<int, 1>{});
-      else if (mode == 2) body(std::integral_constant<int, 2>{});
-      else body(std::integral_constant<int, 0>{});
-      n_hl = n_hl2; n_idx = n_idx2;
-      c_hl = c_hl2; c_idx = c_idx2;
-      cur = scalar4(cur_next);
-      nq_cur = __builtin_amdgcn_readfirstlane(nq_next);
-    };
-    for (int it = 0; it < n_iter; it += 3) {
-      iteration(std::integral_constant<int, 0>{}, it);
-      if (it + 1 < n_iter) iteration(std::integral_constant<int, 1>{}, it + 1);
-      if (it + 2 < n_iter) iteration(std::integral_constant<int, 2>{}, it + 2);
+      }
+      __syncthreads();
+      const int bkmin = min(min(bk[0], bk[2]), min(bk[4], bk[6]));
+      const int bkmax = max(max(bk[1], bk[3]), max(bk[5], bk[7]));
+      int cnt = 0;
+      for (int base = 0; base < nqt; base += 64) {
+        const int t = base + lane;
+        bool act = t < nqt && (PAIRS ? qmin[t] != 0 : !(qmax[t] < bkmin || qmin[t] > bkmax));
+        // (band: some row of the tile must reach into this workgroup's 128 kv rows)
+        if (ext && act) act = kv0 <= pmax[t] + a.mx.hi_off && kv0 + BNK - 1 >= pmin[t] - a.mx.lo_off;
+        const unsigned long long m = __ballot(act);
+        if (act && wave == 0) active[cnt + __popcll(m & ((1ull << lane) - 1ull))] = t;
+        cnt += __popcll(m);
+      }
+      nact = cnt;
+      __syncthreads();
+      for (int i = tid; i < nact; i += 256) {
+        const int t = active[nact - 1 - i];  // visiting order: last query tile first (see qtile_of)
+        *(i32x4*)(ctl + 4 * i) = i32x4{qt_first + t, qmin[t], qmax[t], t};
+      }
+      __syncthreads();
     }
-  }
+    // this workgroup's piece of the walk: iterations it_first .. it_first + n_iter - 1
+    const int n_walk = nact * a.n_rep;
+    const int it_first = n_split > 1 ? split * n_walk / n_split : 0;
+    const int n_iter = n_split > 1 ? (split + 1) * n_walk / n_split - it_first : n_walk;
 
-  // every LDS-writing load of this wave has landed before it leaves (the last ones write zeros nobody reads,
-  // but they must not outlive the workgroup's LDS allocation)
-  __builtin_amdgcn_s_waitcnt(0);
-  // The accumulating MFMAs are opaque assembly (mfma32_acc): the compiler does not know that dkacc / dvacc come
-  // out of a 16-pass matrix instruction and inserts no wait states before reading them.  Make the distance
-  // explicit (the longest MFMA-write -> VALU-read hazard is 18 wait states).
-  // (the accumulators are operands of the statement, so that no read of them can be scheduled ahead of it)
-  static_assert(DKB <= 6 && DVB <= 4, "operand lists below");
-  asm volatile("s_nop 15\n\ts_nop 3" : "+a"(dkacc[0]), "+a"(dkacc[1]), "+a"(dvacc[0]), "+a"(dvacc[1]) :: "memory");
-  if constexpr (DKB > 2) asm volatile("" : "+a"(dkacc[2]), "+a"(dkacc[3]));
-  if constexpr (DKB > 4) asm volatile("" : "+a"(dkacc[4]), "+a"(dkacc[5]));
-  if constexpr (DVB > 2) asm volatile("" : "+a"(dvacc[2]), "+a"(dvacc[3]));
-  // ---- epilogue: lane = kv row, 4 consecutive head-dim values per store
-  const int row = wkv0 + ln;
-  if (n_split > 1) {
-    // a piece: its sums as they are, [row][dk | dv], for attn_bwd_parts_kernel
-    if (row < Skv) {
-      float* pp = a.parts + ((int64_t)blockIdx.x * BNK + wave * 32 + ln) * (DQK + DV) + 4 * g;
+    // ---- staging: every piece of a query tile (Q, dO row-major; log2-scaled LSE, delta, segment ids of its
+    // rows) is written into LDS by the loads themselves; the transposed copies are made LDS-to-LDS
+    QT qdma;
+    OT dodma;
+    qdma.init(a.qs[2], wave, lane);
+    dodma.init(a.dos[2], wave, lane);
+    const unsigned q_span = span_bytes(Sq, a.qs[2], DQK), do_span = span_bytes(Sq, a.dos[2], DV);
+    const unsigned q_tile_bytes = (unsigned)(BMQ * a.qs[2] * 2), do_tile_bytes = (unsigned)(BMQ * a.dos[2] * 2);
+    const float* lse2 = a.delta + (int64_t)a.B * a.Hq * Sq;  // second half of the workspace (written by the kernel before this one)
+    unsigned char* const rows_base = smem + NBUF * BUF_BYTES;
+    // Query tiles are visited from the last one down.  The workgroups of a (batch, kv head) run side by side on one XCD
+    // and all stream the same Q / dO tiles; each needs the tiles from its own kv rows on, so counting up they would start
+    // at different tiles and never meet in the L2 (every tile fetched from memory once per workgroup); counting down
+    // they start together at the last tile and stay within an L2's reach of each other.
+    // pair masks: this wave's 32 kv rows' words of a query tile, 256 bytes
+    const int skp = (Skv + BNK - 1) / BNK * BNK;
+    const u32x4 brw = make_rsrc_words(PAIRS ? (const void*)(a.pm.kbits + (int64_t)(a.pm.per_batch ? b : 0) * nqt_tot * skp) : a.k,
+                                      PAIRS ? (unsigned)nqt_tot * (unsigned)skp * 8u : 0u);
+    auto qtile_of = [&](int idx) { return SEG ? ctl[4 * idx] : nqt_all - 1 - idx; };
+    // The sources of a query head's tiles: those of the group's first head, and the step from head to head.  (Put together
+    // from the arguments whenever a head starts, the descriptors waited for scalar loads: 4 % of the loop where the walks are
+    // short, heads of 64.)  Row vectors: waves 0..2 fetch one of 64 entries each, 4 bytes per lane, rows past Sq as zeros;
+    // a wave with none to fetch (wave 2 without segment ids, wave 3 without query positions) has size 0.
+    const T* const q_first = (const T*)a.q + b * a.qs[0] + (int64_t)hk * a.n_rep * a.qs[1];
+    const T* const do_first = (const T*)a.dout + b * a.dos[0] + (int64_t)hk * a.n_rep * a.dos[1];
+    const int64_t q_step = a.qs[1], do_step = a.dos[1], rv_at = ((int64_t)b * a.Hq + hk * a.n_rep) * Sq;
+    const float* const rv_first = wave == 0 ? lse2 + rv_at : wave == 1 ? a.delta + rv_at : wave == 2 ? (const float*)segb : (const float*)a.mx.qpos;
+    const int rv_step = wave < 2 ? Sq : 0;
+    const unsigned rv_span = (wave < 2 || (wave == 2 && has_seg) || (wave == 3 && has_pos)) ? (unsigned)Sq * 4u : 0u;
+    auto issue_tile = [&](int hl, int idx, int buf, int rslot) {
+      const int qt = qtile_of(idx);
+      qdma.issue(make_rsrc_words(q_first + hl * q_step, q_span), (unsigned)qt * q_tile_bytes, smem + Q_AT + buf * Q_BYTES, wave);
+      dodma.issue(make_rsrc_words(do_first + hl * do_step, do_span), (unsigned)qt * do_tile_bytes, smem + DO_AT + buf * DO_BYTES, wave);
+      dma_dword(make_rsrc_words(rv_first + (int64_t)hl * rv_step, rv_span), (unsigned)(qt * BMQ) * 4u, rows_base + rslot * ROW_BYTES + wave * BMQ * 4, lane);
+      if constexpr (PAIRS)
+        dma_dword(brw, ((unsigned)qt * (unsigned)skp + (unsigned)wkv0) * 8u, rows_base + rslot * ROW_BYTES + VEC_BYTES + wave * 256, lane);
+    };
+
+    // per-lane byte offsets of the MFMA fragments inside a tile (the swizzles are resolved once, here)
+    unsigned faq[KS_QK], fao[KS_DV];
+#pragma unroll
+    for (int ks = 0; ks < KS_QK; ks++) faq[ks] = (unsigned)QT::off(ln, 2 * ks + g);
+#pragma unroll
+    for (int ks = 0; ks < KS_DV; ks++) fao[ks] = (unsigned)OT::off(ln, 2 * ks + g);
+
+    const float c = a.scale_log2;
+
+    // wave-level decisions for a query tile (uniform): skip if every query row precedes every kv row
+    // (lo, hi: id range of the query tile; t: its index into the position ranges)
+    // (The decisions are taken on the wave's first kv row as it arrives, in a vector register.  With a scalar copy the
+    // compiler turns the choice of the tile body into scalar branches and copies the pinned accumulators between them,
+    // right behind the MFMAs that write them: the build's hazard check rejects that code.  The same change in the
+    // forward and the lean dQ kernel passed the check and ran 45 % and 64 % slower.)
+    auto tile_mode_of = [&](int lo, int hi, int t, int qi0) {  // 0 = nothing to compute, 1 = no masking needed, 2 = masked
+      bool skip = (CAUSAL && (qi0 + BMQ - 1 + band_hi < wkv0 || qi0 - band_lo > wkv0 + 31)) || wkv0 >= Skv;
+      bool need_mask = (qi0 + BMQ > Sq) || (wkv0 + 32 > Skv) ||
+                       (CAUSAL && (qi0 + band_hi < wkv0 + 31 || qi0 + BMQ - 1 - band_lo > wkv0));
+      if (SEG) {
+        if (PAIRS) {
+          const int cls = (lo >> (8 * wave)) & 255;
+          skip = skip || cls == 0;
+          need_mask = need_mask || cls != 2;
+        } else {
+          skip = skip || hi < wkmin || lo > wkmax;
+          need_mask = need_mask || !(lo == hi && wkmin == wkmax && lo == wkmin);
+        }
+      }
+      if (ext) {
+        const int plo = pmin[t], phi = pmax[t];
+        skip = skip || wkv0 > phi + a.mx.hi_off || wkv0 + 31 < plo - a.mx.lo_off;
+        need_mask = need_mask || capped || biased || !(wkv0 >= phi - a.mx.lo_off && wkv0 + 31 <= plo + a.mx.hi_off);
+      }
+      return skip ? 0 : (need_mask ? 2 : 1);
+    };
+    auto tile_mode = [&](int idx, int qi0) {
+      const int* e = ctl + 4 * idx;
+      return tile_mode_of(SEG ? e[1] : 0, SEG ? e[2] : 0, SEG ? e[3] : 0, qi0);
+    };
+    // iteration -> (query head of the group, query tile): heads outer, tiles inner, no division in the loop.  (Tiles
+    // outer would keep the group's workgroups on the same tile for the whole launch and cut the fetches from memory to
+    // 1.8 GB at the benchmark's shape, against 6.5 GB this way - and ran 4 % slower: 32 CUs asking one L2 for the same
+    // lines at the same time, and the descriptors rebuilt every tile.)
+    auto advance = [&](int& hl, int& idx) {
+      if (++idx == nact) { idx = 0; hl++; }
+    };
+
+    {
+      // Software pipeline over query tiles t, three row-major buffers and three row-vector slots (tile t lives in
+      // buffer and slot t % 3), one barrier per tile:
+      //   part 1 (S, dP: fragment reads of buffer t % 3)
+      //   wait for this wave's share of tile t+1 (issued a whole tile earlier), barrier
+      //                                  -> tile t+1 has landed for everybody, everybody is done with tile t-1
+      //   part 2 (dV, dK: transposing reads of buffer t % 3), with the loads of tile t+2 issued between its MFMAs
+      //   into the buffer tile t-1 used
+      const int hl_first = n_split > 1 ? it_first / max(nact, 1) : 0, idx_first = it_first - hl_first * nact;
+      int c_hl = hl_first, c_idx = idx_first, n_hl = hl_first, n_idx = idx_first;  // tile being computed, tile whose loads are issued next
+      // Per-lane LDS byte addresses of the operands inside a tile (base of the workgroup's LDS included), each an
+      // opaque register: every read below is such a register plus an immediate.  (Formed from the `smem` symbol, the
+      // same addresses cost an add per read whenever the constant part happens to be zero, and the compiler
+      // recomputes what it could have kept.)  Addresses into the dO tiles carry O_BIAS: constants there would
+      // otherwise exceed the reach of an instruction offset.
+      //   aq / ao   fragment reads of the row-major tiles (S, dP): row ln, chunk 2 ks + g
+      //   trq / tro transposing reads (dK, dV): head-dim block d (32 columns), half h2 (rows +8); the query block and
+      //             the k-step are immediates (multiples of 16 rows leave the swizzle alone)
+      constexpr int O_BIAS = DO_AT;
+      const unsigned lb = (unsigned)(size_t)smem;
+      unsigned aq[KS_QK], ao[KS_DV], trq[DKB][2], tro[DVB][2];
+#pragma unroll
+      for (int ks = 0; ks < KS_QK; ks++) { aq[ks] = faq[ks] + lb; asm volatile("" : "+v"(aq[ks])); }
+#pragma unroll
+      for (int ks = 0; ks < KS_DV; ks++) { ao[ks] = fao[ks] + lb + (unsigned)O_BIAS; asm volatile("" : "+v"(ao[ks])); }
 #pragma unroll
       for (int d = 0; d < DKB; d++)
 #pragma unroll
-        for (int vq = 0; vq < 4; vq++) {
-          const f32x16& o = dkacc[d];
-          *(f32x4*)(pp + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+        for (int h2 = 0; h2 < 2; h2++) {
+          trq[d][h2] = (unsigned)QT::tr_off(8 * h2 + 4 * g, 2 * d + ((lane >> 4) & 1), lane & 15) + lb;
+          asm volatile("" : "+v"(trq[d][h2]));
         }
 #pragma unroll
       for (int d = 0; d < DVB; d++)
 #pragma unroll
-        for (int vq = 0; vq < 4; vq++) {
-          const f32x16& o = dvacc[d];
-          *(f32x4*)(pp + DQK + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+        for (int h2 = 0; h2 < 2; h2++) {
+          tro[d][h2] = (unsigned)OT::tr_off(8 * h2 + 4 * g, 2 * d + ((lane >> 4) & 1), lane & 15) + lb + (unsigned)O_BIAS;
+          asm volatile("" : "+v"(tro[d][h2]));
         }
+      auto ld16 = [](unsigned addr) { return *(const __attribute__((address_space(3))) v8*)addr; };
+      auto ldtr = [](unsigned a0, unsigned a1) {
+        return tr_read8<v8>((const __attribute__((address_space(3))) unsigned char*)a0, (const __attribute__((address_space(3))) unsigned char*)a1);
+      };
+      if (n_iter > 0) { issue_tile(n_hl, n_idx, 0, 0); advance(n_hl, n_idx); }
+      if (n_iter > 1) { issue_tile(n_hl, n_idx, 1, 1); advance(n_hl, n_idx); }
+      {
+        // whole-vector values from the start: element-wise initialisation makes the compiler track 16 scalars per
+        // accumulator across the loop and reassemble the tuple around every accumulating MFMA
+        f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < DKB; d++) {
+          asm volatile("" : "+a"(zero16));
+          dkacc[d] = zero16;
+        }
+#pragma unroll
+        for (int d = 0; d < DVB; d++) {
+          asm volatile("" : "+a"(zero16));
+          dvacc[d] = zero16;
+        }
+      }
+      // the control entry of the tile being computed and the query tile whose loads are issued next, as scalars; their
+      // successors are read at the top of a tile and taken over at its end
+      auto entry = [&](int idx) {
+        if constexpr (SEG) return *(const i32x4*)(ctl + 4 * min(idx, max(nact - 1, 0)));
+        else return i32x4{nqt_all - 1 - idx, 0, 0, 0};
+      };
+      auto scalar4 = [&](i32x4 v) {
+        return i32x4{__builtin_amdgcn_readfirstlane(v[0]), __builtin_amdgcn_readfirstlane(v[1]),
+                     __builtin_amdgcn_readfirstlane(v[2]), __builtin_amdgcn_readfirstlane(v[3])};
+      };
+      i32x4 cur = scalar4(entry(c_idx));
+      int nq_cur = __builtin_amdgcn_readfirstlane(entry(n_idx)[0]);
+      // all earlier loads (the K/V fragments, the first tiles) have landed
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      // (too few tiles to ask on the way; behind the barrier, where nobody reads the last answer any more)
+      auto ask_queue = [&]() {
+        return __hip_atomic_fetch_add(a.queue + (blockIdx.x % NUM_XCD) * QUEUE_STRIDE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      unsigned ticket = 0;
+      if (PERSIST && a.queue != nullptr && n_iter < 2 && tid == 0) *next_at = (int)(ask_queue() + gridDim.x / NUM_XCD);
+      // fragment ring: slot i's LDS fragment is requested AHEAD slots earlier and kept in fr[i % NF]; the
+      // first AHEAD fragments of a tile are requested at the end of the tile before it (its row-major
+      // tiles are complete by then), so that the LDS round trip and the scalar bookkeeping at the top of
+      // the loop overlap
+      constexpr int AHEAD = KS_QK >= 8 ? 5 : 3, NF = AHEAD + 1;
+      v8 fr[NF];
+      static_for<0, AHEAD>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        static_assert(AHEAD <= KS_QK, "the carried fragments all belong to S of the first query block");
+        fr[i % NF] = ld16(aq[i] + Q_AT);
+      });
+      struct { u32x4 rq, ro, rr; unsigned offq, offo, offr, offb; } nx;
+      const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
+      const unsigned wave_q = __builtin_amdgcn_readfirstlane((unsigned)(wave * QT::PER_WAVE * 1024));
+      const unsigned wave_o = __builtin_amdgcn_readfirstlane((unsigned)(wave * OT::PER_WAVE * 1024));
+      const unsigned wave_r = __builtin_amdgcn_readfirstlane((unsigned)(wave * BMQ * 4));
+      // one query tile; the buffer index is a constant (the loop below rotates three copies of this)
+      auto iteration = [&](auto BUFc, const int it) {
+        constexpr int buf = decltype(BUFc)::value;
+        const int qi0 = cur[0] * BMQ;
+        const int mode = tile_mode_of(cur[1], cur[2], cur[3], qi0);
+        const bool issue_next = it + 2 < n_iter;
+        // successors of the two cursors (read now, used when this tile is done)
+        int c_hl2 = c_hl, c_idx2 = c_idx, n_hl2 = n_hl, n_idx2 = n_idx;
+        advance(c_hl2, c_idx2);
+        if (issue_next) advance(n_hl2, n_idx2);
+        const i32x4 cur_next = entry(c_idx2);
+        const int nq_next = entry(n_idx2)[0];
+        constexpr int buf1 = (buf + 1) % 3, buf2 = (buf + 2) % 3;  // tile t+1 (read first in the next iteration), tile t+2
+        constexpr unsigned ql = Q_AT + buf * Q_BYTES;                // + aq[] / trq[]
+        constexpr unsigned dol = DO_AT + buf * DO_BYTES - O_BIAS;    // + ao[] / tro[]
+        constexpr unsigned nxq = Q_AT + buf1 * Q_BYTES;
+        const float* lsel = (const float*)(rows_base + buf * ROW_BYTES);
+        const float* deltal = lsel + BMQ;
+        const int* segl = (const int*)(deltal + BMQ);
+        const int* posl = segl + BMQ;  // query positions of the tile's rows (mask extensions)
+        const float* bias_head = biased ? a.mx.bias + b * a.mx.bias_s[0] + (hk * a.n_rep + c_hl) * a.mx.bias_s[1] : nullptr;
+        // LDS destinations of this wave's loads of tile t+2 (scalar byte addresses)
+        const unsigned dma_q = lds_base + (unsigned)(Q_AT + buf2 * Q_BYTES) + wave_q;
+        const unsigned dma_o = lds_base + (unsigned)(DO_AT + buf2 * DO_BYTES) + wave_o;
+        const unsigned dma_b = lds_base + (unsigned)(NBUF * BUF_BYTES + buf2 * ROW_BYTES + VEC_BYTES) + wave_r;  // (wave_r: 256 bytes a wave)
+        const unsigned dma_r = lds_base + (unsigned)(NBUF * BUF_BYTES + buf2 * ROW_BYTES) + wave_r;
+        // descriptors of tile t+2's loads (wave-uniform), issued piecewise in part 2.  The bases change with
+        // the query head only; they are rebuilt when a new head starts (and when the tiles run out: size 0).
+        if (it == 0 || n_idx == 0 || !issue_next) {
+          const int hl = issue_next ? n_hl : 0;
+          nx.rq = make_rsrc_words(q_first + hl * q_step, issue_next ? q_span : 0u);
+          nx.ro = make_rsrc_words(do_first + hl * do_step, issue_next ? do_span : 0u);
+          nx.rr = make_rsrc_words(rv_first + (int64_t)hl * rv_step, issue_next ? rv_span : 0u);
+          // the last tile but one asks for the workgroup's next item, the last one puts the answer down (both pass here; a
+          // test of its own in every tile cost 2 % of the loop)
+          if (PERSIST && a.queue != nullptr && n_iter > 1 && it + 2 >= n_iter && tid == 0) {
+            if (it + 2 == n_iter) ticket = ask_queue();
+            else *next_at = (int)(ticket + gridDim.x / NUM_XCD);
+          }
+        }
+        {
+          const int qt = issue_next ? nq_cur : 0;
+          nx.offq = __builtin_amdgcn_readfirstlane((unsigned)qt * q_tile_bytes);
+          nx.offo = __builtin_amdgcn_readfirstlane((unsigned)qt * do_tile_bytes);
+          nx.offr = __builtin_amdgcn_readfirstlane((unsigned)(qt * BMQ) * 4u);
+          nx.offb = PAIRS ? __builtin_amdgcn_readfirstlane(((unsigned)qt * (unsigned)skp + (unsigned)wkv0) * 8u) : 0u;
+        }
+
+        // The tile body is laid out by hand as a sequence of slots, one MFMA each, with a scheduling barrier
+        // after every slot: the LDS fragment a slot needs was requested AHEAD slots earlier, and the
+        // exponentials / products that turn S, dP into the 16-bit operands P, dS are spread over the slots
+        // under the MFMAs of the other query block.  (Left to itself the compiler reads each fragment right
+        // before its MFMA and the matrix unit waits out every LDS round trip.)
+        //   slots   part 1: S0 = Q0 K^T, S1 = Q1 K^T, dP0 = dO0 V^T, dP1 = dO1 V^T
+        //           part 2: dV^T += dO0^T P0, dK^T += Q0^T dS0, dV^T += dO1^T P1, dK^T += Q1^T dS1
+        //   VALU    P0 from S1 on, P1 from dP0 on, dS0 from dP1 on, dS1 from part 2 on
+        auto body = [&](auto mode_c) {
+          constexpr int MODE = decltype(mode_c)::value;
+          constexpr bool COMPUTE = MODE != 0, MASKED = MODE == 2;
+          // part 1: S0, S1, dP0, dP1 (the exponentials can start as soon as S0 is complete and are over
+          // before part 2, which carries the transposition of the next tile);
+          // part 2: dV0, dK0, dV1, dK1 (four accumulators each, used round robin)
+          // (K1 / K2 k-steps per S / dP product; CLV / CLK slots per query block of dV / dK)
+          constexpr int K1 = KS_QK, K2 = KS_DV, CLV = 2 * DVB, CLK = 2 * DKB;
+          constexpr int S1_AT = K1, D0_AT = 2 * K1, D1_AT = 2 * K1 + K2, C0 = 2 * (K1 + K2);
+          constexpr int V0_AT = C0, K0_AT = V0_AT + CLV, V1_AT = K0_AT + CLK, K1_AT = V1_AT + CLV, NS = K1_AT + CLK;
+          // VALU groups of VL slots each: P of a block starts when its S is complete, dS when its dP is; each
+          // group is over before the MFMAs that consume its packed operand
+          constexpr int EPS = K2 >= 8 ? 1 : 2, VL = 16 / EPS;
+          constexpr int VP0 = S1_AT, VP1 = D0_AT, VS0 = D1_AT, VS1 = C0;
+          static_assert(VP0 + VL <= V0_AT && VS0 + VL <= K0_AT && VP1 + VL <= V1_AT && VS1 + VL <= K1_AT, "operands not ready");
+          constexpr int N_DMA = QT::PER_WAVE + OT::PER_WAVE + 1 + (PAIRS ? 1 : 0), DMA_EVERY = (NS - C0) / N_DMA;
+          static_assert(DMA_EVERY >= 1, "second half too short for the loads");
+          const int kvcol = wkv0 + ln;
+          f32x16 s[2], dp[2];
+          v8 pf[2][2], df[2][2];
+          // -LSE (log2 units) and -delta of the 16 rows a lane holds of either query block.  LDS reads return in
+          // order, so each group is requested a ring depth or more before its first use: waiting for it then waits
+          // for no fragment that is not due anyway
+          f32x4 nl0[4], nl1[4], nd0[4], nd1[4];
+          float fc[2][16];  // soft cap: 1 - tanh^2 of every score, kept from P to dS
+          // Masked tiles without the mask extensions: which of the tile's 64 query rows this lane's kv column may see,
+          // as one bit per row, built once per tile (bounds and causality are a bit range; the rows of each id present
+          // among the wave's columns come from a ballot over the tile's id vector).  An element then costs a bit-field
+          // extract and an AND instead of four compares.  rowbits[qb] is shifted so that value v of the lane's 16 is
+          // bit 8 (v / 4) + v % 4.
+          unsigned rowbits[2] = {0u, 0u};
+          const bool by_bits = MASKED && !(GEN && ext);
+          if (MASKED && PAIRS) {
+            const u32x2 w = *(const u32x2*)(rows_base + buf * ROW_BYTES + VEC_BYTES + wave * 256 + ln * 8);
+            rowbits[0] = w[0] >> (4 * g);
+            rowbits[1] = w[1] >> (4 * g);
+          } else if (MASKED && by_bits) {
+            const int lo_r = CAUSAL ? max(kvcol - band_hi - qi0, 0) : 0;
+            int hi_r = kvcol < Skv ? min(Sq - qi0, BMQ) : 0;
+            if (CAUSAL) hi_r = min(hi_r, kvcol + band_lo - qi0 + 1);
+            unsigned long long m = 0ull;
+            if (hi_r > lo_r) m = (~0ull << lo_r) & (~0ull >> (64 - hi_r));
+            if (SEG == SEG_IDS && has_seg) {
+              const int rowseg = segl[lane];  // lane l: id of the tile's query row l
+              unsigned long long ms = 0ull, todo = ~0ull;
+              while (todo) {
+                const int x = __builtin_amdgcn_readlane(segk, (int)__builtin_ctzll(todo));
+                const unsigned long long rows = __ballot(rowseg == x);
+                const bool mine = segk == x;
+                ms = mine ? rows : ms;
+                todo &= ~__ballot(mine);
+              }
+              m &= ms;
+            }
+            rowbits[0] = (unsigned)m >> (4 * g);
+            rowbits[1] = (unsigned)(m >> 32) >> (4 * g);
+          }
+
+          auto frag = [&](auto I) -> v8 {
+            constexpr int i = decltype(I)::value;
+            if constexpr (i < D0_AT) {
+              constexpr int qb = i / K1, ks = i % K1;
+              return ld16(aq[ks] + (ql + qb * 32 * QT::ROWB));
+            } else if constexpr (i < C0) {
+              constexpr int qb = (i - D0_AT) / K2, ks = (i - D0_AT) % K2;
+              return ld16(ao[ks] + (dol + qb * 32 * OT::ROWB));
+            } else {
+              // operand of an accumulating product: rows = head-dim block d, contraction over query rows
+              // 32 qb + 16 hh + {4g..4g+3, 8+4g..8+4g+3} (the order in which P / dS hold them), read transposed
+              constexpr int qb = i >= V1_AT ? 1 : 0, base = qb ? V1_AT : V0_AT;
+              if constexpr (i - base < CLV) {
+                constexpr int j = i - base, hh = j / DVB, d = j % DVB;
+                constexpr int rows = (32 * qb + 16 * hh) * OT::ROWB;
+                return ldtr(tro[d][0] + (dol + rows), tro[d][1] + (dol + rows));
+              } else {
+                constexpr int j = i - base - CLV, hh = j / DKB, d = j % DKB;
+                constexpr int rows = (32 * qb + 16 * hh) * QT::ROWB;
+                return ldtr(trq[d][0] + (ql + rows), trq[d][1] + (ql + rows));
+              }
+            }
+          };
+          auto mma = [&](auto I, const v8& f) {
+            constexpr int i = decltype(I)::value;
+            const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if constexpr (i < D0_AT) {
+              constexpr int qb = i / K1, ks = i % K1;
+              s[qb] = MT<T>::mfma32(f, kf[ks], ks == 0 ? zero : s[qb]);
+            } else if constexpr (i < C0) {
+              constexpr int qb = (i - D0_AT) / K2, ks = (i - D0_AT) % K2;
+              if constexpr (ks == 0) {
+                // dP starts from -delta of its rows (C layout: value v belongs to row 8 (v/4) + 4 g + v%4), so
+                // that dS = P o dP needs no subtraction
+                const f32x4 (&nd)[4] = qb == 0 ? nd0 : nd1;
+                const f32x16 init = {nd[0][0], nd[0][1], nd[0][2], nd[0][3], nd[1][0], nd[1][1], nd[1][2], nd[1][3],
+                                     nd[2][0], nd[2][1], nd[2][2], nd[2][3], nd[3][0], nd[3][1], nd[3][2], nd[3][3]};
+                dp[qb] = MT<T>::mfma32(f, vf[ks], init);
+              } else {
+                dp[qb] = MT<T>::mfma32(f, vf[ks], dp[qb]);
+              }
+            } else {
+              constexpr int qb = i >= V1_AT ? 1 : 0, base = qb ? V1_AT : V0_AT;
+              if constexpr (i - base < CLV) {
+                constexpr int j = i - base, hh = j / DVB, d = j % DVB;
+                MT<T>::mfma32_acc(dvacc[d], f, pf[qb][hh]);
+              } else {
+                constexpr int j = i - base - CLV, hh = j / DKB, d = j % DKB;
+                MT<T>::mfma32_acc(dkacc[d], f, df[qb][hh]);
+              }
+            }
+          };
+          // VALU group of query block QB starting at slot START: EPS elements per slot for VL slots.
+          // IS_P: s <- exp2(s c - lse) (masked), else dp <- s (dp - delta); the 16-bit operands are packed as
+          // soon as the eight values of a half are done.
+          auto valu = [&](auto I, auto START, auto QBc, auto IS_Pc) {
+            constexpr int i = decltype(I)::value, st = decltype(START)::value, qb = decltype(QBc)::value;
+            constexpr bool IS_P = decltype(IS_Pc)::value;
+            constexpr int QS = 4 / EPS;  // slots per quad of rows
+            if constexpr (i >= st && i < st + VL) {
+              constexpr int k = i - st, vq = k / QS;
+#pragma unroll
+              for (int e2 = 0; e2 < EPS; e2++) {
+                const int e = EPS * (k % QS) + e2, v = 4 * vq + e;
+                if constexpr (IS_P) {
+                  const f32x4 (&nl)[4] = qb == 0 ? nl0 : nl1;
+                  float sval = s[qb][v];
+                  if (GEN && MASKED) {
+                    if (capped) {
+                      const float th = fast_tanh(sval * a.mx.cap_in);
+                      fc[qb][v] = 1.f - th * th;
+                      sval = a.mx.cap_out * th;
+                    }
+                    if (biased) {  // additive mask, in units of the raw score (-inf stays -inf)
+                      const int qrow_b = min(qi0 + qb * 32 + 8 * vq + 4 * g + e, Sq - 1);
+                      sval += a.mx.bias_mul * bias_head[(int64_t)qrow_b * a.mx.bias_s[2] + min(kvcol, Skv - 1)];
+                    }
+                  }
+                  float pv = fast_exp2(__builtin_fmaf(sval, c, nl[vq][e]));
+                  if (MASKED) {
+                    if (by_bits) {
+                      pv = __builtin_bit_cast(float, __builtin_bit_cast(int, pv) & __builtin_amdgcn_sbfe((int)rowbits[qb], 8 * vq + e, 1));
+                    } else {
+                      const int r = qb * 32 + 8 * vq + 4 * g + e;
+                      const int qrow = qi0 + r;
+                      bool ok = qrow < Sq && kvcol < Skv && (!CAUSAL || kvcol <= qrow) && (!SEG || !has_seg || segl[r] == segk);
+                      if (GEN) {
+                        if (ext) {
+                          const int qp = has_pos ? posl[r] : qrow;
+                          ok = ok && kvcol >= qp - a.mx.lo_off && kvcol <= qp + a.mx.hi_off;
+                        }
+                      }
+                      pv = ok ? pv : 0.f;
+                    }
+                  }
+                  asm volatile("" : "+v"(pv));  // anchors the computation in this slot (it would sink past the barrier)
+                  s[qb][v] = pv;
+                } else {
+                  float dsv = s[qb][v] * dp[qb][v];
+                  if (GEN && MASKED) {
+                    if (capped) dsv *= fc[qb][v];  // derivative of the capped score with respect to the raw one
+                  }
+                  asm volatile("" : "+v"(dsv));
+                  dp[qb][v] = dsv;
+                }
+              }
+              if constexpr (((k + 1) * EPS) % 8 == 0) {
+                constexpr int hh = (k + 1) * EPS / 8 - 1;
+                const f32x16& x = IS_P ? s[qb] : dp[qb];
+                const v8 packed = pack8<T>(x[8 * hh + 0], x[8 * hh + 1], x[8 * hh + 2], x[8 * hh + 3], x[8 * hh + 4],
+                                           x[8 * hh + 5], x[8 * hh + 6], x[8 * hh + 7]);
+                if constexpr (IS_P) pf[qb][hh] = packed;
+                else df[qb][hh] = packed;
+              }
+            }
+          };
+          typedef std::integral_constant<int, 0> I0;
+          typedef std::integral_constant<int, 1> I1;
+          static_for<0, NS>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            if constexpr (i == C0) {
+              // this wave's loads of tile t+1 were issued a tile ago (vmcnt only: fragment reads stay in flight)
+              __builtin_amdgcn_s_waitcnt(0x0F70);
+              __syncthreads();
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            // the loads of tile t+2, one instruction every few slots: the texture path takes a kilobyte in
+            // some 25 cycles for the whole CU, and a wave that issues them back to back sits out the queue
+            if constexpr (i >= C0 && (i - C0) % DMA_EVERY == 0 && (i - C0) / DMA_EVERY < N_DMA) {
+              constexpr int m = (i - C0) / DMA_EVERY;
+              // (no branch here: past the last tile the descriptors have size 0 and the loads deliver zeros
+              // into buffers nobody reads any more)
+              if constexpr (m < QT::PER_WAVE) qdma.template issue_one_at<m>(nx.rq, nx.offq, dma_q);
+              else if constexpr (m < QT::PER_WAVE + OT::PER_WAVE) dodma.template issue_one_at<m - QT::PER_WAVE>(nx.ro, nx.offo, dma_o);
+              else if constexpr (m == QT::PER_WAVE + OT::PER_WAVE) dma_dword_at(nx.rr, nx.offr, dma_r, lane);
+              else dma_dword_at(brw, nx.offb, dma_b, lane);
+            }
+            if constexpr (COMPUTE) {
+              // row vectors, a quad of rows at a time: -LSE of query block qb LEAD slots before the exponentials of that
+              // quad (VP0 / VP1 + QS vq), -delta two slots before the first dP MFMA of the block (2K, 3K)
+              constexpr int QS = 4 / EPS, LEAD = 3;
+              static_for<0, 4>([&](auto VQ) {
+                constexpr int vq = decltype(VQ)::value;
+                constexpr int r0 = VP0 + QS * vq - LEAD, r1 = VP1 + QS * vq - LEAD;
+                if constexpr (i == (r0 < 0 ? 0 : r0)) nl0[vq] = *(const f32x4*)(lsel + 8 * vq + 4 * g);
+                if constexpr (i == (r1 < 0 ? 0 : r1)) nl1[vq] = *(const f32x4*)(lsel + 32 + 8 * vq + 4 * g);
+              });
+              if constexpr (i == D0_AT - 2) {
+#pragma unroll
+                for (int vq = 0; vq < 4; vq++) nd0[vq] = *(const f32x4*)(deltal + 8 * vq + 4 * g);
+              }
+              if constexpr (i == D1_AT - 2) {
+#pragma unroll
+                for (int vq = 0; vq < 4; vq++) nd1[vq] = *(const f32x4*)(deltal + 32 + 8 * vq + 4 * g);
+              }
+              if constexpr (i + AHEAD < NS) fr[(i + AHEAD) % NF] = frag(std::integral_constant<int, i + AHEAD>{});
+              mma(I, fr[i % NF]);
+              valu(I, std::integral_constant<int, VP0>{}, I0{}, std::true_type{});
+              valu(I, std::integral_constant<int, VP1>{}, I1{}, std::true_type{});
+              valu(I, std::integral_constant<int, VS0>{}, I0{}, std::false_type{});
+              valu(I, std::integral_constant<int, VS1>{}, I1{}, std::false_type{});
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+          static_for<0, AHEAD>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            fr[i % NF] = ld16(aq[i] + nxq);
+          });
+        };
+        if (mode == 1) body(std::integral_constant<int, 1>{});
+        else if (mode == 2) body(std::integral_constant<int, 2>{});
+        else body(std::integral_constant<int, 0>{});
+        n_hl = n_hl2; n_idx = n_idx2;
+        c_hl = c_hl2; c_idx = c_idx2;
+        cur = scalar4(cur_next);
+        nq_cur = __builtin_amdgcn_readfirstlane(nq_next);
+      };
+      for (int it = 0; it < n_iter; it += 3) {
+        iteration(std::integral_constant<int, 0>{}, it);
+        if (it + 1 < n_iter) iteration(std::integral_constant<int, 1>{}, it + 1);
+        if (it + 2 < n_iter) iteration(std::integral_constant<int, 2>{}, it + 2);
+      }
     }
-    return;
+
+    // every LDS-writing load of this wave has landed before it leaves (the last ones write zeros nobody reads,
+    // but they must not outlive the workgroup's LDS allocation)
+    __builtin_amdgcn_s_waitcnt(0);
+    // The accumulating MFMAs are opaque assembly (mfma32_acc): the compiler does not know that dkacc / dvacc come
+    // out of a 16-pass matrix instruction and inserts no wait states before reading them.  Make the distance
+    // explicit (the longest MFMA-write -> VALU-read hazard is 18 wait states).
+    // (the accumulators are operands of the statement, so that no read of them can be scheduled ahead of it)
+    static_assert(DKB <= 6 && DVB <= 4, "operand lists below");
+    asm volatile("s_nop 15\n\ts_nop 3" : "+a"(dkacc[0]), "+a"(dkacc[1]), "+a"(dvacc[0]), "+a"(dvacc[1]) :: "memory");
+    if constexpr (DKB > 2) asm volatile("" : "+a"(dkacc[2]), "+a"(dkacc[3]));
+    if constexpr (DKB > 4) asm volatile("" : "+a"(dkacc[4]), "+a"(dkacc[5]));
+    if constexpr (DVB > 2) asm volatile("" : "+a"(dvacc[2]), "+a"(dvacc[3]));
+    // ---- epilogue: lane = kv row, 4 consecutive head-dim values per store
+    const int row = wkv0 + ln;
+    if (n_split > 1) {
+      // a piece: its sums as they are, [row][dk | dv], for attn_bwd_parts_kernel
+      if (row < Skv) {
+        float* pp = a.parts + ((int64_t)blockIdx.x * BNK + wave * 32 + ln) * (DQK + DV) + 4 * g;
+#pragma unroll
+        for (int d = 0; d < DKB; d++)
+#pragma unroll
+          for (int vq = 0; vq < 4; vq++) {
+            const f32x16& o = dkacc[d];
+            *(f32x4*)(pp + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+          }
+#pragma unroll
+        for (int d = 0; d < DVB; d++)
+#pragma unroll
+          for (int vq = 0; vq < 4; vq++) {
+            const f32x16& o = dvacc[d];
+            *(f32x4*)(pp + DQK + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+          }
+      }
+      return;
+    }
+    __syncthreads();  // every wave is done with the tiles: the sums go out through their LDS, the next item's may land there
+    {
+      const unsigned lds = (unsigned)(size_t)smem + (unsigned)(wave * 4096);
+      store_rows<T, DKB>(dkacc, a.sm_scale, (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + wkv0 * a.dks[2], a.dks[2], Skv - wkv0, lds, lane);
+      store_rows<T, DVB>(dvacc, 1.f, (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + wkv0 * a.dvs[2], a.dvs[2], Skv - wkv0, lds, lane);
+    }
+    if (!PERSIST || a.queue == nullptr) return;
+    slot = __builtin_amdgcn_readfirstlane(*next_at);
+    __syncthreads();
   }
-  __syncthreads();  // every wave is done with the tiles: the sums go out through their LDS
-  const unsigned lds = (unsigned)(size_t)smem + (unsigned)(wave * 4096);
-  store_rows<T, DKB>(dkacc, a.sm_scale, (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + wkv0 * a.dks[2], a.dks[2], Skv - wkv0, lds, lane);
-  store_rows<T, DVB>(dvacc, 1.f, (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + wkv0 * a.dvs[2], a.dvs[2], Skv - wkv0, lds, lane);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1452,7 +1493,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
                         st = decltype(STARTc)::value, len = decltype(LENc)::value;
           if constexpr (i >= st && i < st + len) {
             constexpr int k = i - st, lo = e0 + (k * n + len - 1) / len, hi = e0 + ((k + 1) * n + len - 1) / len;
-  #pragma unroll
+#pragma unroll
             for (int v = lo; v < hi; v++) {
               float sval = s[nb][v], dcap = 1.f;
               if (GEN && MASKED) {
@@ -1581,6 +1622,7 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
+  clear_queue(a);
   int tile, inner, group;
   if (!xcd_map(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;  // the longest rows first
@@ -1997,9 +2039,21 @@ struct DkdvLds {
   static constexpr size_t BUF = DmaTile<DQK>::BYTES + DmaTile<DV>::BYTES;
   static_assert(NBUF * BUF <= 144 * 1024, "the three buffers must leave room for the row vectors and the tile list");
   static size_t tiles(int Sq) { return (size_t)((Sq + BMQ - 1) / BMQ); }
-  static size_t bytes(int Sq) { return NBUF * BUF + 3 * (BMQ * 16 + (SEG == SEG_PAIRS ? BNK * 8 : 0)) + (SEG ? (6 * tiles(Sq) + 8 + 4) * 4 : 0); }
+  static size_t bytes(int Sq) { return NBUF * BUF + 3 * (BMQ * 16 + (SEG == SEG_PAIRS ? BNK * 8 : 0)) + 16 + (SEG ? (6 * tiles(Sq) + 8 + 4) * 4 : 0); }
   static bool fits(int Sq) { return bytes(Sq) <= 160 * 1024 && 3 * tiles(Sq) * 4 <= NBUF * BUF; }
 };
+
+// Whether a problem's key tiles go through a queue: 256 workgroups that each take the next tile of their XCD when they are
+// done with one.  The workgroups of a plain grid are dealt to an XCD's four shader engines in turn and in order: one waits
+// for a CU of its engine while CUs of the others are free, 6 us of every 96 where neighbours differ in length (causal, 128
+// heads of (192,128)), 15 of 164 with packed documents.  Measured in one binary, dK/dV, us, grid : queue: 128 heads of
+// (192,128) B1 S4096 1350 : 1309, B4 S1024 with a window of 163 keys 349 : 320; 32q/8kv heads of 128, B4 S8192 3896 : 3800,
+// packed documents 1455 : 1425.  Where two workgroups share a CU one fills the other's gaps and the queue only costs the
+// neighbourhood in the L2: heads of 64, 8q/8kv B8 S4096 263 : 266, packed 32q/8kv B4 S4096 206 : 210, window of 512 keys
+// 300 : 314.
+static bool dkdv_queued(int groups, int Skv, int Dqk) {
+  return dkdv_per_cu(Dqk) == 1 && (int64_t)((groups + NUM_XCD - 1) / NUM_XCD) * ((Skv + 127) / 128) > CUS_PER_XCD;
+}
 
 // the plan of a problem as the dK/dV kernel sees it: its band (all keys where the mask is something else)
 static SplitPlan bwd_split_plan(const BwdArgs& a, bool causal) {
@@ -2018,6 +2072,13 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
   constexpr int DKDV_NBUF = Dkdv::NBUF, DKDV_BNK = Dkdv::BNK;
   const size_t dkdv_smem = Dkdv::bytes(a.Sq);  // (checked before anything is launched)
   TP_REQUIRE(Dkdv::fits(a.Sq), TP_ERR_UNSUPPORTED, "tp_attn_bwd: Sq=%d needs %zu bytes of LDS (max 163840)", a.Sq, dkdv_smem);
+  constexpr int DKDV_PER_CU = dkdv_per_cu(DQK);
+  SplitPlan plan;
+  plan.on = false;
+  if (a.parts) plan = bwd_split_plan(a, CAUSAL);
+  a.split = plan.on && plan.bytes <= a.parts_bytes;
+  constexpr bool GENERAL = !CAUSAL && SEG == SEG_IDS;
+  a.queue = !GENERAL && !a.split && a.parts && a.parts_bytes >= QUEUE_BYTES && dkdv_queued(groups, a.Skv, DQK) ? (unsigned*)a.parts : nullptr;
   mark(ev, 0, st);
   if (!lean) {
     // delta
@@ -2055,13 +2116,10 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
       attr_set = true;
     }
     const int n_tiles = (a.Skv + DKDV_BNK - 1) / DKDV_BNK;
-    SplitPlan plan;
-    plan.on = false;
-    if (a.parts) plan = bwd_split_plan(a, CAUSAL);
-    a.split = plan.on && plan.bytes <= a.parts_bytes;
     if (a.split) memcpy(a.split_first, plan.first, sizeof(a.split_first));
-    a.turns = groups_in_turns(n_tiles, 1, groups, DQK <= 64 ? 2 : 1);
-    kern<<<dim3(a.split ? NUM_XCD * plan.first[n_tiles] : xcd_grid(n_tiles, 1, groups)), dim3(256), dkdv_smem, st>>>(a);
+    a.turns = groups_in_turns(n_tiles, 1, groups, DKDV_PER_CU);
+    const unsigned grid = a.split ? NUM_XCD * plan.first[n_tiles] : a.queue ? (unsigned)(NUM_XCD * CUS_PER_XCD * DKDV_PER_CU) : xcd_grid(n_tiles, 1, groups);
+    kern<<<dim3(grid), dim3(256), dkdv_smem, st>>>(a);
     int rc = check_launch("tp_attn_bwd(dkdv)");
     if (rc) return rc;
     if (a.split) {
@@ -2236,7 +2294,7 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   a.q = q; a.k = k; a.v = v; a.out = out; a.dout = dout; a.lse = lse; a.seg = seg;
   a.dq = dq; a.dk = dk; a.dv = dv; a.delta = ws;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv; a.n_rep = Hq / Hkv; a.dqk = Dqk; a.dv_dim = Dv;
-  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.turns = 0;
+  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.queue = nullptr; a.turns = 0;
   bool ok = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(dout) && aligned16(dq) &&
             aligned16(dk) && aligned16(dv);
   for (int i = 0; i < 3; i++) {
@@ -2346,7 +2404,7 @@ extern "C" size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* p) {
     hi = 0;
   }
   const SplitPlan plan = split_plan(p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi);
-  return plan.on ? plan.bytes : 0;
+  return plan.on ? plan.bytes : dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk) ? QUEUE_BYTES : 0;
 }
 
 extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {

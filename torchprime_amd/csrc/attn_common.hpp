@@ -234,6 +234,15 @@ __device__ __forceinline__ unsigned span_bytes(int rows, int64_t stride, int row
   return (unsigned)(((int64_t)(rows - 1) * stride + row_elems) * 2);
 }
 
+// The kernel's (single) argument, read through a pointer the compiler cannot see through: a value that is loaded through it
+// is loaded again after the next call, not kept in a register until then.
+template <typename A>
+__device__ __forceinline__ const A& kernel_args() {
+  unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const A*)(const __attribute__((address_space(4))) A*)p;
+}
+
 // ---- workgroup -> work mapping ---------------------------------------------------------------------
 // The 256 CUs sit in 8 XCDs with one L2 each, and workgroups of a 1-D grid are handed to the XCDs round
 // robin by linear id.  Work is therefore numbered so that every workgroup that streams the same K/V (or
@@ -243,13 +252,15 @@ __device__ __forceinline__ unsigned span_bytes(int rows, int64_t stride, int row
 // With group after group the last group's heaviest tile starts when nearly everything else is done.  The last groups of
 // an XCD therefore take turns tile by tile (`turns` of them; the host's rule is groups_in_turns), heaviest tiles of all
 // of them first; the ones before run group after group, which shares an L2 best.
-// Returns false for the padding ids of a group count that is not a multiple of 8.
+// (Ids past an XCD's last item, where the group count is not a multiple of 8, do nothing.)
 constexpr int NUM_XCD = 8, CUS_PER_XCD = 32;
-__device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns = 0) {
-  const int n = blockIdx.x;
-  const int xcd = n % NUM_XCD;
-  int slot = n / NUM_XCD, gl, r;
-  const int per_group = n_tiles * n_inner, first = (n_groups + NUM_XCD - 1) / NUM_XCD - turns;
+// Item `slot` of XCD `xcd`; false past its last one.
+__device__ __forceinline__ bool xcd_item(int slot, int xcd, int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns) {
+  const int n_gl = (n_groups - xcd + NUM_XCD - 1) / NUM_XCD, per_group = n_tiles * n_inner;
+  if (slot >= n_gl * per_group) return false;
+  int gl, r;
+  turns = min(turns, n_gl);
+  const int first = n_gl - turns;
   if (turns && slot >= first * per_group) {
     const int per_tile = turns * n_inner;
     slot -= first * per_group;
@@ -265,7 +276,10 @@ __device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, 
     inner = r - tile * n_inner;
   }
   group = gl * NUM_XCD + xcd;
-  return group < n_groups;
+  return true;
+}
+__device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns = 0) {
+  return xcd_item(blockIdx.x / NUM_XCD, blockIdx.x % NUM_XCD, n_tiles, n_inner, n_groups, tile, inner, group, turns);
 }
 // How many groups: all where an XCD gets fewer than four rounds of workgroups (per_cu of them share a CU), else the last
 // ones that make up two rounds; 0 where one group has that many by itself.  That is never slower than group after group
