@@ -348,17 +348,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
     const bool has_pos = ext && a.mx.qpos != nullptr;
     const int32_t* segb = has_seg ? a.seg + (int64_t)b * Skv : nullptr;
 
-    // ---- K, V fragments of this wave's 32 kv rows (B operands: lane = kv column)
-    v8 kf[KS_QK], vf[KS_DV];
     const int kvrow = min(wkv0 + ln, Skv - 1);
-    {
-      const T* kp = (const T*)a.k + b * a.ks[0] + hk * a.ks[1] + kvrow * a.ks[2] + 8 * g;
-      const T* vp = (const T*)a.v + b * a.vs[0] + hk * a.vs[1] + kvrow * a.vs[2] + 8 * g;
-#pragma unroll
-      for (int ks = 0; ks < KS_QK; ks++) kf[ks] = *(const v8*)(kp + 16 * ks);
-#pragma unroll
-      for (int ks = 0; ks < KS_DV; ks++) vf[ks] = *(const v8*)(vp + 16 * ks);
-    }
     const int segk = has_seg ? segb[kvrow] : 0;
 
     // ---- query tiles to visit: causal => tiles that reach the first kv row; segments => id ranges overlap
@@ -438,6 +428,18 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
     const int n_walk = nact * a.n_rep;
     const int it_first = n_split > 1 ? split * n_walk / n_split : 0;
     const int n_iter = n_split > 1 ? (split + 1) * n_walk / n_split - it_first : n_walk;
+
+    // ---- K, V fragments of this wave's 32 kv rows (B operands: lane = kv column); behind the ids of
+    // the list, which are waited for first
+    v8 kf[KS_QK], vf[KS_DV];
+    {
+      const T* kp = (const T*)a.k + b * a.ks[0] + hk * a.ks[1] + kvrow * a.ks[2] + 8 * g;
+      const T* vp = (const T*)a.v + b * a.vs[0] + hk * a.vs[1] + kvrow * a.vs[2] + 8 * g;
+#pragma unroll
+      for (int ks = 0; ks < KS_QK; ks++) kf[ks] = *(const v8*)(kp + 16 * ks);
+#pragma unroll
+      for (int ks = 0; ks < KS_DV; ks++) vf[ks] = *(const v8*)(vp + 16 * ks);
+    }
 
     // ---- staging: every piece of a query tile (Q, dO row-major; log2-scaled LSE, delta, segment ids of its
     // rows) is written into LDS by the loads themselves; the transposed copies are made LDS-to-LDS
@@ -1634,53 +1636,8 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   const int ntiles = (kv_end + BN - 1) / BN;
   const int t_first = CAUSAL ? min(max(q0 - band_lo, 0) / BN, ntiles) : 0;  // (tiles before it lie left of every row's band)
 
-  // ---- Q, dO fragments (B operands: lane = query column), per-lane LSE / -delta
   const int qrow = wq0 + ln, qrow_c = min(qrow, Sq - 1);
   const int wq0_s = __builtin_amdgcn_readfirstlane(wq0);  // (for the masked tiles, which form the row again)
-  v8 qf[KS], dof[KSV];
-  {
-    const T* qp = (const T*)a.q + b * a.qs[0] + h * a.qs[1] + qrow_c * a.qs[2] + 8 * g;
-    const T* dp = (const T*)a.dout + b * a.dos[0] + h * a.dos[1] + qrow_c * a.dos[2] + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[ks] = *(const v8*)(qp + 16 * ks);
-#pragma unroll
-    for (int ks = 0; ks < KSV; ks++) dof[ks] = *(const v8*)(dp + 16 * ks);
-  }
-  const int64_t ro = ((int64_t)b * a.Hq + h) * Sq + qrow_c;
-  const float lraw = a.lse[ro];
-  const float nlse = (lraw == -INFINITY) ? -INFINITY : -lraw * LOG2E;  // (a row without keys: P = exp2(-inf) = 0)
-  // -delta = -rowsum(dO o O) of this lane's row, computed here from the dO fragments and the matching pieces of O
-  // (the two lanes that share a row hold the two halves of the head dim), and left in the workspace together with
-  // -LSE in log2 units for the dK/dV kernel, which runs after this one: no separate pass over dO and O
-  float ndelta;
-  {
-    const T* op = (const T*)a.out + b * a.os[0] + h * a.os[1] + qrow_c * a.os[2] + 8 * g;
-    float acc = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KSV; ks++) {
-      const v8 of = *(const v8*)(op + 16 * ks);
-#pragma unroll
-      for (int e = 0; e < 8; e++) acc = __builtin_fmaf((float)of[e], (float)dof[ks][e], acc);
-    }
-    acc += __shfl_xor(acc, 32, 64);
-    ndelta = -acc;
-    if (g == 0 && qrow < Sq) {
-      a.delta[ro] = ndelta;
-      a.delta[(int64_t)a.B * a.Hq * Sq + ro] = nlse;
-    }
-  }
-  v8 ones_a, ndelta_b;
-  {
-    const float hi = (float)(T)ndelta, lo = ndelta - hi;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      ones_a[e] = (T)((g == 0 && e < 2) ? 1.0f : 0.0f);
-      ndelta_b[e] = (T)0.0f;
-    }
-    if (g == 0) { ndelta_b[0] = (T)hi; ndelta_b[1] = (T)lo; }
-    asm volatile("" : "+v"(ones_a), "+v"(ndelta_b));
-  }
-
   // ---- segment ids: the list of kv tiles to visit (tile, min id, max id), this wave's own id range
   const int32_t* segb = SEG == SEG_IDS ? a.seg + (int64_t)b * Skv : nullptr;
   const int segq = SEG == SEG_IDS ? segb[qrow_c] : 0;
@@ -1762,6 +1719,65 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
       if (wave == 0) dma_dword_at(srw, __builtin_amdgcn_readfirstlane((unsigned)(t * BN) * 4u), lds_base + (unsigned)(SEG_AT + buf * VEC), lane);
     }
   };
+
+  // the list entries of the tile being computed and of the next one, as scalars, read a tile ahead of their use
+  i32x4 cur = entry(0), nxt = entry(1);
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    cur[j] = __builtin_amdgcn_readfirstlane(cur[j]);
+    nxt[j] = __builtin_amdgcn_readfirstlane(nxt[j]);
+  }
+  if (nact > 0) {
+    static_for<0, NLOAD2>([&](auto P) { load_piece(P, cur[0], 0); });
+  }
+  // ---- Q, dO fragments (B operands: lane = query column) and O for delta, beside the first tile: all on their way before
+  // anything is waited for, and behind the id loads of the list, which would otherwise queue behind the fragments'
+  v8 qf[KS], dof[KSV];
+  {
+    const T* qp = (const T*)a.q + b * a.qs[0] + h * a.qs[1] + qrow_c * a.qs[2] + 8 * g;
+    const T* dp = (const T*)a.dout + b * a.dos[0] + h * a.dos[1] + qrow_c * a.dos[2] + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qf[ks] = *(const v8*)(qp + 16 * ks);
+#pragma unroll
+    for (int ks = 0; ks < KSV; ks++) dof[ks] = *(const v8*)(dp + 16 * ks);
+  }
+  v8 of[KSV];
+  {
+    const T* op = (const T*)a.out + b * a.os[0] + h * a.os[1] + qrow_c * a.os[2] + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < KSV; ks++) of[ks] = *(const v8*)(op + 16 * ks);
+  }
+  const int64_t ro = ((int64_t)b * a.Hq + h) * Sq + qrow_c;
+  const float lraw = a.lse[ro];
+  const float nlse = (lraw == -INFINITY) ? -INFINITY : -lraw * LOG2E;  // (a row without keys: P = exp2(-inf) = 0)
+  // -delta = -rowsum(dO o O) of this lane's row, computed here from the dO fragments and the matching pieces of O
+  // (the two lanes that share a row hold the two halves of the head dim), and left in the workspace together with
+  // -LSE in log2 units for the dK/dV kernel, which runs after this one: no separate pass over dO and O
+  float ndelta;
+  {
+    float acc = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KSV; ks++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) acc = __builtin_fmaf((float)of[ks][e], (float)dof[ks][e], acc);
+    acc += __shfl_xor(acc, 32, 64);
+    ndelta = -acc;
+    if (g == 0 && qrow < Sq) {
+      a.delta[ro] = ndelta;
+      a.delta[(int64_t)a.B * a.Hq * Sq + ro] = nlse;
+    }
+  }
+  v8 ones_a, ndelta_b;
+  {
+    const float hi = (float)(T)ndelta, lo = ndelta - hi;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      ones_a[e] = (T)((g == 0 && e < 2) ? 1.0f : 0.0f);
+      ndelta_b[e] = (T)0.0f;
+    }
+    if (g == 0) { ndelta_b[0] = (T)hi; ndelta_b[1] = (T)lo; }
+    asm volatile("" : "+v"(ones_a), "+v"(ndelta_b));
+  }
 
   // ---- per-lane LDS addresses in buffer 0 (opaque registers; reads add immediates)
   const unsigned lds0 = (unsigned)(size_t)smem;
@@ -1941,16 +1957,6 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of the next tile has landed
   };
 
-  // the list entries of the tile being computed and of the next one, as scalars, read a tile ahead of their use
-  i32x4 cur = entry(0), nxt = entry(1);
-#pragma unroll
-  for (int j = 0; j < 3; j++) {
-    cur[j] = __builtin_amdgcn_readfirstlane(cur[j]);
-    nxt[j] = __builtin_amdgcn_readfirstlane(nxt[j]);
-  }
-  if (nact > 0) {
-    static_for<0, NLOAD2>([&](auto P) { load_piece(P, cur[0], 0); });
-  }
   __builtin_amdgcn_s_waitcnt(0);  // the fragments above and the first tile have landed (see the forward kernel)
   __syncthreads();
   auto iteration = [&](auto BUFc, int it) {
