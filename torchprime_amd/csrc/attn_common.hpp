@@ -253,7 +253,7 @@ __device__ __forceinline__ const A& kernel_args() {
 // an XCD therefore take turns tile by tile (`turns` of them; the host's rule is groups_in_turns), heaviest tiles of all
 // of them first; the ones before run group after group, which shares an L2 best.
 // (Ids past an XCD's last item, where the group count is not a multiple of 8, do nothing.)
-constexpr int NUM_XCD = 8, CUS_PER_XCD = 32;
+constexpr int NUM_XCD = 8, CUS_PER_XCD = 32;  // (four shader engines of eight CUs)
 // Item `slot` of XCD `xcd`; false past its last one.
 __device__ __forceinline__ bool xcd_item(int slot, int xcd, int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns) {
   const int n_gl = (n_groups - xcd + NUM_XCD - 1) / NUM_XCD, per_group = n_tiles * n_inner;
@@ -278,8 +278,24 @@ __device__ __forceinline__ bool xcd_item(int slot, int xcd, int n_tiles, int n_i
   group = gl * NUM_XCD + xcd;
   return true;
 }
+// The item of a workgroup of a plain grid.  An XCD deals its workgroups to its four shader engines in turn, and a workgroup
+// waits for a CU of its own engine.  Numbered by falling length, the first engine gets the longest of every four and the others
+// wait for it; every second four therefore come in reverse (SNAKE: dQ of 128 causal heads of (192,128), S4096 1133 -> 1089 us).
+// Documents have no such order, and there it costs what neighbours share (the same heads, S1898: 341 : 354), so they go without.
+// Where two workgroups share a CU and all of them run at once, number k + 32 joins number k: the second 32 are numbered from the
+// shortest up, so that the longest shares its CU with the shortest (32q/8kv causal heads of 128, S1728: forward 41.4 -> 39.2, dQ
+// 55.8 -> 52.4).  (Both were read from the hardware ids of running workgroups; only speed depends on them.)
+template <int PER_CU, bool SNAKE>
 __device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns = 0) {
-  return xcd_item(blockIdx.x / NUM_XCD, blockIdx.x % NUM_XCD, n_tiles, n_inner, n_groups, tile, inner, group, turns);
+  const int xcd = blockIdx.x % NUM_XCD, n = (n_groups - xcd + NUM_XCD - 1) / NUM_XCD * n_tiles * n_inner;
+  int slot = blockIdx.x / NUM_XCD;
+  if (slot >= n) return false;
+  if (PER_CU == 2 && n <= 2 * CUS_PER_XCD) {
+    if (slot >= CUS_PER_XCD) slot = CUS_PER_XCD + n - 1 - slot;
+  } else if (SNAKE && (slot & 4) && (slot | 3) < n) {
+    slot ^= 3;
+  }
+  return xcd_item(slot, xcd, n_tiles, n_inner, n_groups, tile, inner, group, turns);
 }
 // How many groups: all where an XCD gets fewer than four rounds of workgroups (per_cu of them share a CU), else the last
 // ones that make up two rounds; 0 where one group has that many by itself.  That is never slower than group after group
