@@ -92,3 +92,26 @@ def test_more_masks_than_one_launch_takes():
   assert_close(m(q, q, q, mask)[-1:], ref, "out")
   mask[-1, :, 3, 1] = 0.5
   assert tpa.ops.mask_kind(mask) == tpa.ops.MASK_GENERAL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("Skv", [1, 3, 4, 5, 7, 8, 9, 63, 64, 65, 67, 68, 71, 72, 73, 100, 127, 128, 129])
+def test_bits_at_the_rows_ends(Skv, dtype):
+  """Every bit of a random mask whose rows end inside a tile; the entries behind a row's end (0: kept) must not show."""
+  B, Sq = 2, 70
+  g = torch.Generator().manual_seed(Skv)
+  keep = torch.rand((B, Sq, Skv), generator=g) < 0.5
+  memory = torch.zeros((B, 1, Sq, Skv + 5), dtype=dtype)
+  memory[..., :Skv].masked_fill_(~keep[:, None], float("-inf"))
+  q, k = (torch.zeros((B, 1, n, 64), dtype=torch.bfloat16, device=DEV) for n in (Sq, Skv))
+  nkt, nqt, nqb, nkb = (Skv + 63) // 64, (Sq + 63) // 64, (Sq + 127) // 128, (Skv + 127) // 128
+  for mask in (memory.to(DEV)[..., :Skv], memory[..., :Skv].contiguous().to(DEV)):
+    pairs = torch.ops.tprime.attn_fwd_pairs(q, k, k, mask, 0.125)[2].cpu().numpy().tobytes()
+    words = torch.frombuffer(bytearray(pairs[64:]), dtype=torch.int64)
+    n = B * nkt * nqb * 128
+    qbits, kbits = words[:n].view(B, nkt, nqb * 128), words[n : n + B * nqt * nkb * 128].view(B, nqt, nkb * 128)
+    bit = torch.arange(64)
+    got = ((qbits[..., None] >> bit) & 1).bool().permute(0, 2, 1, 3).reshape(B, nqb * 128, nkt * 64)
+    assert torch.equal(got[:, :Sq, :Skv], keep) and not got[:, Sq:].any() and not got[:, :, Skv:].any()
+    got = ((kbits[..., None] >> bit) & 1).bool().permute(0, 1, 3, 2).reshape(B, nqt * 64, nkb * 128)
+    assert torch.equal(got[:, :Sq, :Skv], keep) and not got[:, Sq:].any() and not got[:, :, Skv:].any()
