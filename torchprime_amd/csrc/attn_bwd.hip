@@ -936,27 +936,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
     if constexpr (DKB > 2) asm volatile("" : "+a"(dkacc[2]), "+a"(dkacc[3]));
     if constexpr (DKB > 4) asm volatile("" : "+a"(dkacc[4]), "+a"(dkacc[5]));
     if constexpr (DVB > 2) asm volatile("" : "+a"(dvacc[2]), "+a"(dvacc[3]));
-    // ---- epilogue: lane = kv row, 4 consecutive head-dim values per store
-    const int row = wkv0 + ln;
+    // ---- epilogue
     if (n_split > 1) {
-      // a piece: its sums as they are, [row][dk | dv], for attn_bwd_parts_kernel
-      if (row < Skv) {
-        float* pp = a.parts + ((int64_t)blockIdx.x * BNK + wave * 32 + ln) * (DQK + DV) + 4 * g;
+      // a piece: its sums as they are, for attn_bwd_parts_kernel: four values of a lane side by side with the other lanes' (in
+      // rows, 16 bytes to each of 64 places, an instruction took as long as four of these)
+      float* pp = a.parts + ((int64_t)blockIdx.x * BNK + wave * 32) * (DQK + DV) + lane * 4;
+      auto put = [&](const f32x16& o, int d) {
 #pragma unroll
-        for (int d = 0; d < DKB; d++)
+        for (int vq = 0; vq < 4; vq++) *(f32x4*)(pp + (4 * d + vq) * 256) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
+      };
 #pragma unroll
-          for (int vq = 0; vq < 4; vq++) {
-            const f32x16& o = dkacc[d];
-            *(f32x4*)(pp + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
-          }
+      for (int d = 0; d < DKB; d++) put(dkacc[d], d);
 #pragma unroll
-        for (int d = 0; d < DVB; d++)
-#pragma unroll
-          for (int vq = 0; vq < 4; vq++) {
-            const f32x16& o = dvacc[d];
-            *(f32x4*)(pp + DQK + d * 32 + 8 * vq) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
-          }
-      }
+      for (int d = 0; d < DVB; d++) put(dvacc[d], DKB + d);
       return;
     }
     __syncthreads();  // every wave is done with the tiles: the sums go out through their LDS, the next item's may land there
@@ -978,30 +970,35 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
 // issues at most one instruction every four cycles, and at ~600 instructions for 48 MFMAs per tile a single
 // wave per SIMD leaves the matrix unit idle most of the time, whatever the order of its instructions.
 
-// sums of the pieces of the split kv tiles: one thread per four values of a row, pieces in order
+// Sums of the pieces of the split kv tiles, pieces in order: a workgroup per tile and 64 columns of dK or dV, a wave per 32 rows.
+// Bound by latency: 32q/8kv heads of 128, window of 1024 keys over 2047 rows 6.8 us (7.3 when a thread took four values of a row of
+// row-major sums); heads of 64, packed B2 S4288 16.4 (15.5), with the dK/dV kernel, whose stores the order is for, 169 -> 161.
 template <typename T, int DQK, int DV>
 __global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
-  constexpr int BNK = 128, W = (DQK + DV) / 4, PER_TILE = BNK * W / 256;  // workgroups per (tile, group)
-  static_assert(BNK * W % 256 == 0, "whole workgroups");
-  const int n_groups = a.B * a.Hkv;
-  const int item = blockIdx.x % PER_TILE * 256 + threadIdx.x, tg = blockIdx.x / PER_TILE;
+  constexpr int BNK = 128, PER_TILE = (DQK + DV) / 64;
+  __shared__ __align__(16) unsigned char smem[4 * 4096];
+  const int n_groups = a.B * a.Hkv, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int part = blockIdx.x % PER_TILE, tg = blockIdx.x / PER_TILE;
   const int tile = tg / n_groups, group = tg - tile * n_groups;
   const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
   const int n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
-  const int r = item / W, d = (item - r * W) * 4, row = tile * BNK + r;
-  if (n_split == 1 || row >= a.Skv) return;
-  const float* p = a.parts + (((int64_t)(f + group / NUM_XCD * n_split) * NUM_XCD + group % NUM_XCD) * BNK + r) * (DQK + DV) + d;
-  f32x4 acc = *(const f32x4*)p;
-  for (int s = 1; s < n_split; s++) {
+  if (n_split == 1) return;
+  const float* p = a.parts + (((int64_t)(f + group / NUM_XCD * n_split) * NUM_XCD + group % NUM_XCD) * BNK + wave * 32) * (DQK + DV) + part * 2048 + lane * 4;
+  f32x16 acc[2];
+  for (int s = 0; s < n_split; s++) {
+    f32x4 x[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) x[i] = *(const f32x4*)(p + i * 256);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] = s ? acc[i / 4][4 * (i % 4) + e] + x[i][e] : x[i][e];
     p += (int64_t)NUM_XCD * BNK * (DQK + DV);
-    const f32x4 x = *(const f32x4*)p;
-    acc[0] += x[0]; acc[1] += x[1]; acc[2] += x[2]; acc[3] += x[3];
   }
-  const int b = group / a.Hkv, hk = group - b * a.Hkv;
-  const float sc = d < DQK ? a.sm_scale : 1.f;
-  T* o = d < DQK ? (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row * a.dks[2] + d
-                 : (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row * a.dvs[2] + (d - DQK);
-  *(u32x2*)o = pack4<T>(acc[0] * sc, acc[1] * sc, acc[2] * sc, acc[3] * sc);
+  const int b = group / a.Hkv, hk = group - b * a.Hkv, row0 = tile * BNK + wave * 32;
+  const bool is_k = part < DQK / 64;
+  T* o = is_k ? (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row0 * a.dks[2] + part * 64 : (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row0 * a.dvs[2] + (part * 64 - DQK);
+  store_rows<T, 2>(acc, is_k ? a.sm_scale : 1.f, o, is_k ? a.dks[2] : a.dvs[2], a.Skv - row0, (unsigned)(size_t)smem + (unsigned)(wave * 4096), lane);
 }
 
 template <typename T, int DQK, int DV, int NW, bool CAUSAL, int SEG>
@@ -2131,7 +2128,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
     int rc = check_launch("tp_attn_bwd(dkdv)");
     if (rc) return rc;
     if (a.split) {
-      constexpr int PER_TILE = DKDV_BNK * (DQK + DV) / 4 / 256;
+      constexpr int PER_TILE = (DQK + DV) / 64;
       attn_bwd_parts_kernel<T, DQK, DV><<<dim3((unsigned)(n_tiles * groups * PER_TILE)), dim3(256), 0, st>>>(a);
       rc = check_launch("tp_attn_bwd(parts)");
       if (rc) return rc;
