@@ -29,8 +29,8 @@ class _Problem(ctypes.Structure):  # tp_attn_bwd_problem
   _fields_ += [("soft_cap", ctypes.c_float), ("dtype", ctypes.c_int)]
 
 
-def _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=False, pairs=False, soft_cap=0.0):
-  p = _Problem(B=B, Hq=Hq, Hkv=Hkv, Sq=S, Skv=S, Dqk=Dqk, Dv=Dv, causal=int(causal), window_left=-1, window_right=-1, sm_scale=0.1,
+def _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=False, pairs=False, soft_cap=0.0, ids=False):
+  p = _Problem(seg=16 if ids else None, B=B, Hq=Hq, Hkv=Hkv, Sq=S, Skv=S, Dqk=Dqk, Dv=Dv, causal=int(causal), window_left=-1, window_right=-1, sm_scale=0.1,
                soft_cap=soft_cap, pairs=16 if pairs else None, mask_batches=int(pairs))  # fmt: skip
   assert _lib.load().tp_attn_bwd_parts_bytes(ctypes.byref(p)) > 0
 
@@ -44,8 +44,8 @@ def _documents(S, lengths):
   return torch.tensor([ids[:S]], dtype=torch.int32)
 
 
-def _leaves(Hq, Hkv, S, Dqk, Dv):
-  q, k, v, do = (heads_view(1, h, S, d, i, torch.bfloat16) for i, (h, d) in enumerate(((Hq, Dqk), (Hkv, Dqk), (Hkv, Dv), (Hq, Dv))))
+def _leaves(Hq, Hkv, S, Dqk, Dv, B=1):
+  q, k, v, do = (heads_view(B, h, S, d, i, torch.bfloat16) for i, (h, d) in enumerate(((Hq, Dqk), (Hkv, Dqk), (Hkv, Dv), (Hq, Dv))))
   return (q, k, v, do), [t.to(DEV).requires_grad_(True) for t in (q, k, v)], do.to(DEV)
 
 
@@ -54,7 +54,7 @@ def _leaves(Hq, Hkv, S, Dqk, Dv):
 @pytest.mark.parametrize("kw", [{"causal": True}, {"causal": False}, {"causal": True, "soft_cap": 4.0}])
 def test_segment_ids(Dqk, Dv, S, lengths, kw):
   Hq, Hkv, scale = 4, 2, 1 / math.sqrt(Dv)
-  _assert_split(1, Hq, Hkv, S, Dqk, Dv, **kw)
+  _assert_split(1, Hq, Hkv, S, Dqk, Dv, ids=True, **kw)
   (q, k, v, do), leaves, dod = _leaves(Hq, Hkv, S, Dqk, Dv)
   seg = _documents(S, lengths)
   ext = {k: x for k, x in kw.items() if k != "causal"}
@@ -86,3 +86,27 @@ def test_pair_masks(Dqk, Dv, S, lengths, unseen):
     assert_close(a, b, name, scale_abs=name != "out")
   if unseen:
     assert not got[1][:, :, S - unseen :].any() and not got[2][:, :, S - unseen :].any()
+
+
+@pytest.mark.parametrize("Dqk,Dv", [(128, 128), (64, 64)])
+@pytest.mark.parametrize("what", ["causal", "padding", "ids"])
+def test_more_groups_than_engines(Dqk, Dv, what):
+  """Three groups of heads on some XCDs and two on the others, pieces that start by falling length; walks that padding or a
+  short document ends before the plan's last piece, in some sequences only."""
+  B, Hq, Hkv, S, scale = 5, 16, 4, 600, 1 / math.sqrt(Dv)
+  _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=what != "padding", pairs=what == "padding", ids=what == "ids")
+  (q, k, v, do), leaves, dod = _leaves(Hq, Hkv, S, Dqk, Dv, B)
+  if what == "padding":
+    seen = torch.tensor([600, 1, 129, 64, 383])
+    keep = (torch.arange(S) < seen[:, None])[:, None] & torch.ones(S, S, dtype=torch.bool).tril()
+    mask = torch.zeros((B, 1, S, S)).masked_fill_(~keep[:, None], float("-inf"))
+    m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=Hq, num_key_value_heads=Hkv))
+    out = m(*leaves, mask.to(DEV, torch.bfloat16))
+    refs = _eager_grads(q, k, v, do, mask)
+  else:
+    seg = torch.cat([_documents(S, n) for n in ((600,), (5, 200), (300,), (16, 70, 33), (599, 1))]) if what == "ids" else None
+    out = tpa.ops.attention(*leaves, seg.to(DEV) if what == "ids" else None, scale, True)
+    refs = orc.attention_grads_ref(q, k, v, do, seg, True, scale, torch.float32)
+  got = torch.autograd.grad(out, leaves, dod)
+  for name, a, b in zip(("out", "dq", "dk", "dv"), (out, *got), refs):
+    assert_close(a, b, name, scale_abs=name != "out")

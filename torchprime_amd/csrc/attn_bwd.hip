@@ -80,42 +80,49 @@ struct BwdArgs {
   MaskExt mx;
   PairMask pm;
   int turns;       // order of the workgroups (xcd_map)
-  // dK/dV: partial results of the splits of a kv tile's work (split_plan), NULL: no tile is split
+  // dK/dV: scratch for the queue's counters, or for the sums of the pieces of a kv tile's walk and the pieces' numbers
+  // (split_plan); NULL: neither
   float* parts;
   size_t parts_bytes;
   unsigned* queue;                // next item of each XCD, QUEUE_STRIDE apart (NULL: a workgroup does one item)
-  int split;                      // the plan below is in use
-  unsigned short split_first[65]; // per XCD: number of workgroups before kv tile t
+  int split;                      // most tiles of a piece's walk, 0: no tile is split
+  int split_sums;                 // where the sums start in parts (floats), behind the number of pieces of every tile and group
+  unsigned short split_first[65]; // per XCD: number of workgroups before the j-th kv tile of the plan
+  unsigned char split_tile[64];   // which tile that is
 };
 
 // ------------------------------------------------------------------------------------------------
 // splitting a kv tile's work
 // ------------------------------------------------------------------------------------------------
-// A dK/dV workgroup walks every query tile of every query head of its group: with few kv tiles (one sequence of a few
-// thousand tokens and eight kv heads) that is one workgroup for every second CU or fewer, each with the longest chain
-// there can be.  Such a tile's walk is cut into pieces of at most `cap` iterations, one workgroup each, which leave
-// their sums as fp32 in a workspace for a short kernel to add up in order (deterministic).  The cap is the one for which
-// the estimate below is least; pieces cost their start-up and 2 x 128 x (dqk + dv) x 4 bytes of traffic each.
-// Measured (bf16, 32q/8kv heads of 128, B1): dK/dV of a 1024-key window over 2047 rows 116 -> 71 us and 7 us for the sums.
+// A dK/dV workgroup walks every query tile of every query head of its group.  Where there are few rounds of workgroups the longest
+// walk is what the kernel takes, and the first kv tiles of a causal problem keep their CUs busy when the others have long been
+// free.  Such a tile's walk is cut into pieces of at most `cap` tiles, one workgroup each, which start by falling length and
+// leave their sums as fp32 in a workspace for a short kernel to add up in order (deterministic).  Ids or a pair mask may leave
+// less to do than the plan knows: the pieces of a tile are then fewer, and the first one tells the short kernel how many.
+// The cap is the one for which the estimate below is least; each finer one has to be worth another 8 %.
+// Measured (bf16, 32q/8kv heads), dK/dV and the sums, us, whole walks : pieces.  Heads of 128: window of 1024 keys over 2047 rows
+// 114 : 70 + 7; causal 2 x 2048 200 : 160 + 9; causal and padded 4 x 1000 114 : 95 + 9, 4 x 664 76 : 47 + 7; packed 2047 123 :
+// 59 + 7.  Heads of 64: causal 4096 278 : 140 + 8, 4 x 246 24 : 15 + 6.  16 heads of (192,128), padded 1472: 52 : 41 + 8.
+// Twice as fine as chosen: 80 + 11 (window), 105 + 14 (4 x 1000), 50 + 10 (4 x 664).  Three rounds of workgroups or more: none
+// was faster in pieces (heads of 64, causal 8 x 3044: 622 : 656 + 41).
 struct SplitPlan {
   bool on;
-  int n_tiles, n_gl;
+  int n_tiles, n_gl, cap, sums_at;
   unsigned short first[65];
+  unsigned char tile[64];
   size_t bytes;
 };
-static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk, int Dv, int band_lo, int band_hi) {
+static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk, int Dv, int band_lo, int band_hi, bool ids) {
   SplitPlan p;
   p.on = false;
   p.bytes = 0;
+  p.cap = p.sums_at = 0;
   p.n_tiles = (Skv + 127) / 128;
   const int groups = B * Hkv;
   p.n_gl = (groups + NUM_XCD - 1) / NUM_XCD;
-  const bool two = Dqk <= 64;  // workgroups per CU
-  const int slots = CUS_PER_XCD * (two ? 2 : 1);
+  const int slots = CUS_PER_XCD * dkdv_per_cu(Dqk);
   // (four rounds and more balance themselves)
   if (p.n_tiles > 64 || (int64_t)p.n_tiles * p.n_gl >= 4 * slots) return p;
-  // time of an iteration and of a workgroup's start, us (measured: a chain of iterations on an otherwise idle chip)
-  const float ti = Dqk <= 64 ? 1.0f : Dqk <= 128 ? 1.4f : 2.0f, start = 4.f;
   const int nqt = (Sq + 63) / 64;
   int per[64], longest = 0;
   int64_t total = 0;
@@ -126,34 +133,72 @@ static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk,
     longest = per[t] > longest ? per[t] : longest;
     total += per[t];
   }
-  const float wg_mb = 128.f * (Dqk + Dv) * 4.f * 2.f * 1e-6f;  // a partial tile, written and read
+  // us, measured inside the kernel: start and end of a workgroup, leaving a piece's sums, the kernel that adds them up (at 8 TB/s
+  // out of the caches), a tile of a walk in a CU's only workgroup, beside another one at times, and always beside one
+  const float ends = Dqk <= 64 ? 4.f : 7.f, leave = 4.f, sums = 6.5f, piece_mb = 128.f * (Dqk + Dv) * 4.f * 1e-6f;
+  const float alone = Dqk <= 64 ? 1.25f : Dqk <= 128 ? 1.7f : 2.2f, beside = Dqk <= 64 ? 1.4f : alone, shared = Dqk <= 64 ? 1.8f : alone;
   float best = 0.f;
-  int best_cap = 0;
-  for (int s = 1; s <= 16 && s <= longest; s++) {
-    const int cap = (longest + s - 1) / s;
-    int64_t wgs = 0, parts = 0;
+  int best_cap = 0, last_cap = 0, order[64], n_of[64];
+  for (int n = 1; n <= 16 && n <= longest; n++) {
+    const int cap = (longest + n - 1) / n;
+    if (cap == last_cap) continue;
+    last_cap = cap;
+    // the tiles by falling length of a piece
+    int wgs = 0, pieces = 0, of[64], k[64];
     for (int t = 0; t < p.n_tiles; t++) {
-      const int n = per[t] > cap ? (per[t] + cap - 1) / cap : 1;
-      wgs += n;
-      parts += n > 1 ? n : 0;
+      k[t] = per[t] > cap ? (per[t] + cap - 1) / cap : 1;
+      wgs += k[t] * p.n_gl;
+      pieces += k[t] > 1 ? k[t] * p.n_gl : 0;
+      int j = t;
+      for (; j > 0 && per[of[j - 1]] * k[t] < per[t] * k[of[j - 1]]; j--) of[j] = of[j - 1];
+      of[j] = t;
     }
-    wgs *= p.n_gl;
-    const float rounds = (float)((wgs + slots - 1) / slots), share = (float)total * p.n_gl / slots;
-    const float chain = wgs <= slots ? (float)cap : (share + 0.5f * cap > cap ? share + 0.5f * cap : (float)cap);
-    const float est = start * rounds + ti * chain + (parts ? 5.f + parts * p.n_gl * NUM_XCD * wg_mb / 4.f : 0.f);
-    if (s == 1 || est < best * (best_cap == longest ? 0.9f : 1.f)) { best = est; best_cap = cap; }
+    // at least: the longest piece; what an XCD has to do, spread over its slots; where the pieces are more than r rounds, r + 1
+    // of the shortest of those that start one after the other
+    float est = (wgs <= CUS_PER_XCD ? alone : beside) * per[of[0]] / k[of[0]] + ends;
+    const float share = (shared * total * p.n_gl + ends * wgs + leave * pieces) / slots;
+    est = est < share ? share : est;
+    int seen = 0;
+    float before = 0.f;
+    for (int j = 0, r = 1; j < p.n_tiles && r < 4; j++) {
+      const float len = (float)per[of[j]] / k[of[j]];
+      for (seen += k[of[j]] * p.n_gl; r < 4 && seen > r * slots; r++) {
+        const float rounds = shared * (r * (seen - k[of[j]] * p.n_gl == r * slots ? before : len) + len) + (r + 1) * ends;
+        est = est < rounds ? rounds : est;
+      }
+      before = len;
+    }
+    if (pieces) est += leave + sums + pieces * NUM_XCD * piece_mb / 8.f;
+    if (ids) {
+      // documents end the walks somewhere, and the pieces that are left start in any order: what fits then is a share of the work
+      // and half of a piece at most, at the rate of a chip that is not full.  (With the estimate above, packed 2 x 4288 with heads
+      // of 64 takes 184 + 6 instead of 159 + 11, 4 x 1000 with heads of 128 89 + 5 instead of 80, whole.)
+      const float ti = Dqk <= 64 ? 1.f : Dqk <= 128 ? 1.4f : 2.f, even = (float)total * p.n_gl / slots;
+      const float chain = wgs <= slots ? (float)cap : (float)fmax(even + 0.5f * cap, cap);
+      est = 4.f * ((wgs + slots - 1) / slots) + ti * chain + (pieces ? 5.f + pieces * NUM_XCD * piece_mb / 2.f : 0.f);
+    }
+    if (n == 1 || est < (best_cap == longest ? 0.9f : ids ? 1.f : 0.92f) * best) {
+      best = est;
+      best_cap = cap;
+      memcpy(order, of, sizeof(order));
+      memcpy(n_of, k, sizeof(n_of));
+    }
   }
   if (best_cap == longest) return p;
   int at = 0, last = 0;
-  for (int t = 0; t < p.n_tiles; t++) {
-    p.first[t] = (unsigned short)at;
-    const int n = per[t] > best_cap ? (per[t] + best_cap - 1) / best_cap : 1;
-    at += n * p.n_gl;
-    if (n > 1) last = at;
+  for (int j = 0; j < p.n_tiles; j++) {
+    p.first[j] = (unsigned short)at;
+    p.tile[j] = (unsigned char)order[j];
+    at += n_of[order[j]] * p.n_gl;
+    if (n_of[order[j]] > 1) last = at;
   }
   p.first[p.n_tiles] = (unsigned short)at;
   p.on = true;
-  p.bytes = (size_t)last * NUM_XCD * 128 * (Dqk + Dv) * 4;  // one slot per workgroup up to the last split tile
+  // (with ids, pieces of half the cap where walks are shorter: whole ones 165 + 7 instead of 159 + 11 (packed 2 x 4288), 66 + 5
+  // instead of 59 + 7 (2047))
+  p.cap = ids ? (best_cap + 1) / 2 : best_cap;
+  p.sums_at = (groups * p.n_tiles + 63) / 64 * 64;
+  p.bytes = (size_t)p.sums_at * 4 + (size_t)last * NUM_XCD * 128 * (Dqk + Dv) * 4;  // one slot per workgroup up to the last split tile
   return p;
 }
 
@@ -324,12 +369,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
     const int lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
     int tile, inner, group, n_split = 1, split = 0;
     if (a.split) {
-      // tile after tile, groups inside, pieces inside those; a lane per tile finds the workgroup's tile
+      // tile after tile in the plan's order, groups inside, pieces inside those; a lane per tile finds the workgroup's place
       const int n_tiles = (a.Skv + BNK - 1) / BNK, r = blockIdx.x / NUM_XCD;
       const bool before = lane < n_tiles && r >= (int)a.split_first[lane + 1];
-      tile = (int)__popcll(__ballot(before));
-      const int n_gl = (a.B * a.Hkv + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
-      n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
+      const int at = (int)__popcll(__ballot(before));
+      tile = a.split_tile[at];
+      const int n_gl = (a.B * a.Hkv + NUM_XCD - 1) / NUM_XCD, f = a.split_first[at];
+      n_split = ((int)a.split_first[at + 1] - f) / n_gl;
       const int gl = (r - f) / n_split;
       split = (r - f) - gl * n_split;
       group = gl * NUM_XCD + blockIdx.x % NUM_XCD;
@@ -428,6 +474,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
     }
     // this workgroup's piece of the walk: iterations it_first .. it_first + n_iter - 1
     const int n_walk = nact * a.n_rep;
+    if (n_split > 1) {
+      n_split = min(n_split, max((n_walk + a.split - 1) / a.split, 1));
+      if (split >= n_split) return;
+      if (split == 0 && tid == 0) ((int*)a.parts)[tile * a.B * a.Hkv + group] = n_split;
+    }
     const int it_first = n_split > 1 ? split * n_walk / n_split : 0;
     const int n_iter = n_split > 1 ? (split + 1) * n_walk / n_split - it_first : n_walk;
 
@@ -940,7 +991,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
     if (n_split > 1) {
       // a piece: its sums as they are, for attn_bwd_parts_kernel: four values of a lane side by side with the other lanes' (in
       // rows, 16 bytes to each of 64 places, an instruction took as long as four of these)
-      float* pp = a.parts + ((int64_t)blockIdx.x * BNK + wave * 32) * (DQK + DV) + lane * 4;
+      float* pp = a.parts + a.split_sums + ((int64_t)blockIdx.x * BNK + wave * 32) * (DQK + DV) + lane * 4;
       auto put = [&](const f32x16& o, int d) {
 #pragma unroll
         for (int vq = 0; vq < 4; vq++) *(f32x4*)(pp + (4 * d + vq) * 256) = f32x4{o[4 * vq], o[4 * vq + 1], o[4 * vq + 2], o[4 * vq + 3]};
@@ -971,29 +1022,45 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
 // wave per SIMD leaves the matrix unit idle most of the time, whatever the order of its instructions.
 
 // Sums of the pieces of the split kv tiles, pieces in order: a workgroup per tile and 64 columns of dK or dV, a wave per 32 rows.
-// Bound by latency: 32q/8kv heads of 128, window of 1024 keys over 2047 rows 6.8 us (7.3 when a thread took four values of a row of
-// row-major sums); heads of 64, packed B2 S4288 16.4 (15.5), with the dK/dV kernel, whose stores the order is for, 169 -> 161.
+// Bound by latency: 32q/8kv heads of 128, window of 1024 keys over 2047 rows 7.1 us (7.2 when a thread took four values of a row of
+// row-major sums); heads of 64, causal 900 rows in eight pieces 6.6 (4.6), with the dK/dV kernel, whose stores the order is for,
+// packed 2 x 4288 154 (168).  Four pieces' loads at once instead of two: 7.0, 7.2 and 160 + 15, for places no piece was left in.
 template <typename T, int DQK, int DV>
 __global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
   constexpr int BNK = 128, PER_TILE = (DQK + DV) / 64;
   __shared__ __align__(16) unsigned char smem[4 * 4096];
   const int n_groups = a.B * a.Hkv, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int part = blockIdx.x % PER_TILE, tg = blockIdx.x / PER_TILE;
-  const int tile = tg / n_groups, group = tg - tile * n_groups;
-  const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, f = a.split_first[tile];
-  const int n_split = ((int)a.split_first[tile + 1] - f) / n_gl;
-  if (n_split == 1) return;
-  const float* p = a.parts + (((int64_t)(f + group / NUM_XCD * n_split) * NUM_XCD + group % NUM_XCD) * BNK + wave * 32) * (DQK + DV) + part * 2048 + lane * 4;
-  f32x16 acc[2];
-  for (int s = 0; s < n_split; s++) {
-    f32x4 x[8];
+  const int at = tg / n_groups, group = tg - at * n_groups, tile = a.split_tile[at];
+  const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, f = a.split_first[at];
+  const int planned = ((int)a.split_first[at + 1] - f) / n_gl;
+  if (planned == 1) return;
+  const float* p = a.parts + a.split_sums + (((int64_t)(f + group / NUM_XCD * planned) * NUM_XCD + group % NUM_XCD) * BNK + wave * 32) * (DQK + DV) + part * 2048 + lane * 4;
+  f32x4 x[8], y[8];
+  auto load = [&](f32x4 (&t)[8]) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) x[i] = *(const f32x4*)(p + i * 256);
+    for (int i = 0; i < 8; i++) t[i] = *(const f32x4*)(p + i * 256);
+    p += (int64_t)NUM_XCD * BNK * (DQK + DV);
+  };
+  // (two pieces' places are there in any case: their loads go out beside the one of the pieces' number)
+  load(x);
+  load(y);
+  const int n_split = ((const int*)a.parts)[tile * n_groups + group];
+  if (n_split == 1) return;
+  f32x16 acc[2];
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] = x[i][e];
+  for (int s = 1;;) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) x[i] = y[i];
+    if (s + 1 < n_split) load(y);
 #pragma unroll
     for (int i = 0; i < 8; i++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] = s ? acc[i / 4][4 * (i % 4) + e] + x[i][e] : x[i][e];
-    p += (int64_t)NUM_XCD * BNK * (DQK + DV);
+      for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] += x[i][e];
+    if (++s == n_split) break;
   }
   const int b = group / a.Hkv, hk = group - b * a.Hkv, row0 = tile * BNK + wave * 32;
   const bool is_k = part < DQK / 64;
@@ -2060,11 +2127,14 @@ static bool dkdv_queued(int groups, int Skv, int Dqk) {
   return dkdv_per_cu(Dqk) == 1 && (int64_t)((groups + NUM_XCD - 1) / NUM_XCD) * ((Skv + 127) / 128) > CUS_PER_XCD;
 }
 
+// A pair mask is on the device; what models hand over as one is causal, with or without padding: square ones are planned as such.
+static int pairs_band_hi(int Sq, int Skv) { return Sq == Skv ? 0 : BAND_INF; }
+
 // the plan of a problem as the dK/dV kernel sees it: its band (all keys where the mask is something else)
 static SplitPlan bwd_split_plan(const BwdArgs& a, bool causal) {
   const int lo = causal ? a.band_lo : a.mx.on && !a.mx.qpos ? a.mx.lo_off : BAND_INF;
-  const int hi = causal ? a.band_hi : a.mx.on && !a.mx.qpos ? a.mx.hi_off : BAND_INF;
-  return split_plan(a.B, a.Hkv, a.n_rep, a.Sq, a.Skv, a.dqk, a.dv_dim, lo, hi);
+  const int hi = a.pm.qbits ? pairs_band_hi(a.Sq, a.Skv) : causal ? a.band_hi : a.mx.on && !a.mx.qpos ? a.mx.hi_off : BAND_INF;
+  return split_plan(a.B, a.Hkv, a.n_rep, a.Sq, a.Skv, a.dqk, a.dv_dim, lo, hi, a.seg != nullptr);
 }
 
 template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
@@ -2080,8 +2150,10 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
   constexpr int DKDV_PER_CU = dkdv_per_cu(DQK);
   SplitPlan plan;
   plan.on = false;
+  plan.sums_at = 0;
   if (a.parts) plan = bwd_split_plan(a, CAUSAL);
-  a.split = plan.on && plan.bytes <= a.parts_bytes;
+  a.split = plan.on && plan.bytes <= a.parts_bytes ? plan.cap : 0;
+  a.split_sums = plan.sums_at;
   constexpr bool GENERAL = !CAUSAL && SEG == SEG_IDS;
   a.queue = !GENERAL && !a.split && a.parts && a.parts_bytes >= QUEUE_BYTES && dkdv_queued(groups, a.Skv, DQK) ? (unsigned*)a.parts : nullptr;
   mark(ev, 0, st);
@@ -2121,7 +2193,10 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
       attr_set = true;
     }
     const int n_tiles = (a.Skv + DKDV_BNK - 1) / DKDV_BNK;
-    if (a.split) memcpy(a.split_first, plan.first, sizeof(a.split_first));
+    if (a.split) {
+      memcpy(a.split_first, plan.first, sizeof(a.split_first));
+      memcpy(a.split_tile, plan.tile, sizeof(a.split_tile));
+    }
     a.turns = groups_in_turns(n_tiles, 1, groups, DKDV_PER_CU);
     const unsigned grid = a.split ? NUM_XCD * plan.first[n_tiles] : a.queue ? (unsigned)(NUM_XCD * CUS_PER_XCD * DKDV_PER_CU) : xcd_grid(n_tiles, 1, groups);
     kern<<<dim3(grid), dim3(256), dkdv_smem, st>>>(a);
@@ -2299,7 +2374,7 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   a.q = q; a.k = k; a.v = v; a.out = out; a.dout = dout; a.lse = lse; a.seg = seg;
   a.dq = dq; a.dk = dk; a.dv = dv; a.delta = ws;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv; a.n_rep = Hq / Hkv; a.dqk = Dqk; a.dv_dim = Dv;
-  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.queue = nullptr; a.turns = 0;
+  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.split_sums = 0; a.queue = nullptr; a.turns = 0;
   bool ok = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(dout) && aligned16(dq) &&
             aligned16(dk) && aligned16(dv);
   for (int i = 0; i < 3; i++) {
@@ -2405,10 +2480,12 @@ extern "C" size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* p) {
   int lo = BAND_INF, hi = BAND_INF;
   if (mx.on) {
     if (!mx.qpos) { lo = mx.lo_off; hi = mx.hi_off; }
-  } else if (p->causal && !p->pairs) {
+  } else if (p->pairs) {
+    hi = pairs_band_hi(p->Sq, p->Skv);
+  } else if (p->causal) {
     hi = 0;
   }
-  const SplitPlan plan = split_plan(p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi);
+  const SplitPlan plan = split_plan(p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi, p->seg != nullptr);
   return plan.on ? plan.bytes : dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk) ? QUEUE_BYTES : 0;
 }
 
