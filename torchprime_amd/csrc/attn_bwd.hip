@@ -1021,16 +1021,17 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
 // issues at most one instruction every four cycles, and at ~600 instructions for 48 MFMAs per tile a single
 // wave per SIMD leaves the matrix unit idle most of the time, whatever the order of its instructions.
 
-// Sums of the pieces of the split kv tiles, pieces in order: a workgroup per tile and 64 columns of dK or dV, a wave per 32 rows.
+// Sums of the pieces of the split kv tiles, pieces in order: a wave per 32 rows and 64 columns of dK or dV, a workgroup each (small
+// problems have few: four in one workgroup leave half of the CUs out, heads of 64, causal 900 rows 6.6 us instead of 6.1).
 // Bound by latency: 32q/8kv heads of 128, window of 1024 keys over 2047 rows 7.1 us (7.2 when a thread took four values of a row of
-// row-major sums); heads of 64, causal 900 rows in eight pieces 6.6 (4.6), with the dK/dV kernel, whose stores the order is for,
+// row-major sums); heads of 64, causal 900 rows in eight pieces 6.1 (4.6), with the dK/dV kernel, whose stores the order is for,
 // packed 2 x 4288 154 (168).  Four pieces' loads at once instead of two: 7.0, 7.2 and 160 + 15, for places no piece was left in.
 template <typename T, int DQK, int DV>
-__global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(64) void attn_bwd_parts_kernel(const BwdArgs a) {
   constexpr int BNK = 128, PER_TILE = (DQK + DV) / 64;
-  __shared__ __align__(16) unsigned char smem[4 * 4096];
-  const int n_groups = a.B * a.Hkv, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int part = blockIdx.x % PER_TILE, tg = blockIdx.x / PER_TILE;
+  __shared__ __align__(16) unsigned char smem[4096];
+  const int n_groups = a.B * a.Hkv, lane = threadIdx.x, wave = blockIdx.x & 3;
+  const int part = blockIdx.x / 4 % PER_TILE, tg = blockIdx.x / (4 * PER_TILE);
   const int at = tg / n_groups, group = tg - at * n_groups, tile = a.split_tile[at];
   const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, f = a.split_first[at];
   const int planned = ((int)a.split_first[at + 1] - f) / n_gl;
@@ -1065,7 +1066,7 @@ __global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
   const int b = group / a.Hkv, hk = group - b * a.Hkv, row0 = tile * BNK + wave * 32;
   const bool is_k = part < DQK / 64;
   T* o = is_k ? (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row0 * a.dks[2] + part * 64 : (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row0 * a.dvs[2] + (part * 64 - DQK);
-  store_rows<T, 2>(acc, is_k ? a.sm_scale : 1.f, o, is_k ? a.dks[2] : a.dvs[2], a.Skv - row0, (unsigned)(size_t)smem + (unsigned)(wave * 4096), lane);
+  store_rows<T, 2>(acc, is_k ? a.sm_scale : 1.f, o, is_k ? a.dks[2] : a.dvs[2], a.Skv - row0, (unsigned)(size_t)smem, lane);
 }
 
 template <typename T, int DQK, int DV, int NW, bool CAUSAL, int SEG>
@@ -2204,7 +2205,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
     if (rc) return rc;
     if (a.split) {
       constexpr int PER_TILE = (DQK + DV) / 64;
-      attn_bwd_parts_kernel<T, DQK, DV><<<dim3((unsigned)(n_tiles * groups * PER_TILE)), dim3(256), 0, st>>>(a);
+      attn_bwd_parts_kernel<T, DQK, DV><<<dim3((unsigned)(n_tiles * groups * PER_TILE * 4)), dim3(64), 0, st>>>(a);
       rc = check_launch("tp_attn_bwd(parts)");
       if (rc) return rc;
     }
