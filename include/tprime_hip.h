@@ -369,7 +369,22 @@ typedef struct tp_attn_bwd_problem {
   float soft_cap;
   int dtype;
 } tp_attn_bwd_problem;
+/* How the key tiles of a problem are handed to workgroups.  Made on the host from the problem's sizes, mask arguments and
+ * which of its pointers are NULL; a caller that keeps it between asking for `parts` and running saves making it twice, and may
+ * keep it for as long as it runs such problems.  Everything behind parts_bytes is the library's. */
+typedef struct tp_attn_bwd_plan {
+  size_t parts_bytes; /* what tp_attn_bwd_parts_bytes() says */
+  int32_t sizes[8], queue, cap, sums_at;
+  uint16_t first[65];
+  uint8_t tile[64];
+} tp_attn_bwd_plan;
+/* returns plan->parts_bytes */
+size_t tp_attn_bwd_make_plan(const tp_attn_bwd_problem* problem, tp_attn_bwd_plan* plan);
 size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* problem);
+/* plan: NULL (as without parts), or made for a problem of the same sizes.
+ * events: NULL, or 4 hipEvent_t recorded as by tp_attn_bwd_ex. */
+int tp_attn_bwd_run_planned(const tp_attn_bwd_problem* problem, const tp_attn_bwd_plan* plan, void* stream, void* const* events);
+/* the same with a plan of its own */
 int tp_attn_bwd_run(const tp_attn_bwd_problem* problem, void* stream);
 
 /* ------------------------------------------------------------------------------------------------

@@ -91,7 +91,9 @@ SIGNATURES = {
   "tp_mask_pairs": (c_int, [c_void_p, c_int64 * 2] + [c_int] * 4 + [c_void_p, c_int, c_void_p]),
   "tp_attn_fwd_pairs": (c_int, [c_void_p] * 4 + [c_int] + [c_void_p] * 2 + [c_int] * 7 + [_I64x3] * 4 + [c_float, c_int, c_void_p]),
   "tp_attn_bwd_parts_bytes": (c_size_t, [c_void_p]),
+  "tp_attn_bwd_make_plan": (c_size_t, [c_void_p, c_void_p]),
   "tp_attn_bwd_run": (c_int, [c_void_p, c_void_p]),
+  "tp_attn_bwd_run_planned": (c_int, [c_void_p] * 4),
   "tp_attn_bwd_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
   "tp_attn_bwd_dq_first": (c_int, [c_int] * 7),
   "tp_attn_bwd": (

@@ -83,7 +83,6 @@ struct BwdArgs {
   // dK/dV: scratch for the queue's counters, or for the sums of the pieces of a kv tile's walk and the pieces' numbers
   // (split_plan); NULL: neither
   float* parts;
-  size_t parts_bytes;
   unsigned* queue;                // next item of each XCD, QUEUE_STRIDE apart (NULL: a workgroup does one item)
   int split;                      // most tiles of a piece's walk, 0: no tile is split
   int split_sums;                 // where the sums start in parts (floats), behind the number of pieces of every tile and group
@@ -105,31 +104,22 @@ struct BwdArgs {
 // 59 + 7.  Heads of 64: causal 4096 278 : 140 + 8, 4 x 246 24 : 15 + 6.  16 heads of (192,128), padded 1472: 52 : 41 + 8.
 // Twice as fine as chosen: 80 + 11 (window), 105 + 14 (4 x 1000), 50 + 10 (4 x 664).  Three rounds of workgroups or more: none
 // was faster in pieces (heads of 64, causal 8 x 3044: 622 : 656 + 41).
-struct SplitPlan {
-  bool on;
-  int n_tiles, n_gl, cap, sums_at;
-  unsigned short first[65];
-  unsigned char tile[64];
-  size_t bytes;
-};
-static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk, int Dv, int band_lo, int band_hi, bool ids) {
-  SplitPlan p;
-  p.on = false;
-  p.bytes = 0;
-  p.cap = p.sums_at = 0;
-  p.n_tiles = (Skv + 127) / 128;
-  const int groups = B * Hkv;
-  p.n_gl = (groups + NUM_XCD - 1) / NUM_XCD;
+// (host: the plan is made by the C entry points, tp_attn_bwd_make_plan)
+#ifndef TP_BWD_UNIT
+static_assert(sizeof(tp_attn_bwd_plan::first) == sizeof(BwdArgs::split_first) && sizeof(tp_attn_bwd_plan::tile) == sizeof(BwdArgs::split_tile), "the plan's tables");
+// Whether walks are split, and if so the plan's cap, sums_at, first, tile and parts_bytes.
+static bool split_plan(tp_attn_bwd_plan& p, int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk, int Dv, int band_lo, int band_hi, bool ids) {
+  const int n_tiles = (Skv + 127) / 128, groups = B * Hkv, n_gl = (groups + NUM_XCD - 1) / NUM_XCD;
   const int slots = CUS_PER_XCD * dkdv_per_cu(Dqk);
   // (four rounds and more balance themselves)
-  if (p.n_tiles > 64 || (int64_t)p.n_tiles * p.n_gl >= 4 * slots) return p;
+  if (n_tiles > 64 || (int64_t)n_tiles * n_gl >= 4 * slots) return false;
   const int nqt = (Sq + 63) / 64;
   int per[64], longest = 0;
   int64_t total = 0;
-  for (int t = 0; t < p.n_tiles; t++) {
-    const int64_t lo = (int64_t)t * 128 - band_hi, hi = (int64_t)t * 128 + 127 + band_lo;
-    const int q0 = (int)((lo > 0 ? lo : 0) / 64), q1 = hi < 0 ? 0 : (int)(hi / 64 + 1 < nqt ? hi / 64 + 1 : nqt);
-    per[t] = (q1 > q0 ? q1 - q0 : 0) * n_rep;
+  for (int t = 0; t < n_tiles; t++) {
+    const int last = (int)std::min<int64_t>(((int64_t)t * 128 + 127 + band_lo) / 64 + 1, nqt);
+    const int64_t lo = (int64_t)t * 128 - band_hi;
+    per[t] = std::max(last - (int)((lo > 0 ? lo : 0) / 64), 0) * n_rep;
     longest = per[t] > longest ? per[t] : longest;
     total += per[t];
   }
@@ -138,69 +128,80 @@ static SplitPlan split_plan(int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk,
   const float ends = Dqk <= 64 ? 4.f : 7.f, leave = 4.f, sums = 6.5f, piece_mb = 128.f * (Dqk + Dv) * 4.f * 1e-6f;
   const float alone = Dqk <= 64 ? 1.25f : Dqk <= 128 ? 1.7f : 2.2f, beside = Dqk <= 64 ? 1.4f : alone, shared = Dqk <= 64 ? 1.8f : alone;
   float best = 0.f;
-  int best_cap = 0, last_cap = 0, order[64], n_of[64];
-  for (int n = 1; n <= 16 && n <= longest; n++) {
-    const int cap = (longest + n - 1) / n;
-    if (cap == last_cap) continue;
-    last_cap = cap;
-    // the tiles by falling length of a piece
-    int wgs = 0, pieces = 0, of[64], k[64];
-    for (int t = 0; t < p.n_tiles; t++) {
-      k[t] = per[t] > cap ? (per[t] + cap - 1) / cap : 1;
-      wgs += k[t] * p.n_gl;
-      pieces += k[t] > 1 ? k[t] * p.n_gl : 0;
+  int best_cap = 0, last_cap = 0, k[64], n_of[64], of[64];
+  // the tiles by falling length of a piece
+  auto sort = [&](const int* k) {
+    for (int t = 0; t < n_tiles; t++) {
       int j = t;
       for (; j > 0 && per[of[j - 1]] * k[t] < per[t] * k[of[j - 1]]; j--) of[j] = of[j - 1];
       of[j] = t;
     }
-    // at least: the longest piece; what an XCD has to do, spread over its slots; where the pieces are more than r rounds, r + 1
-    // of the shortest of those that start one after the other
-    float est = (wgs <= CUS_PER_XCD ? alone : beside) * per[of[0]] / k[of[0]] + ends;
-    const float share = (shared * total * p.n_gl + ends * wgs + leave * pieces) / slots;
-    est = est < share ? share : est;
-    int seen = 0;
-    float before = 0.f;
-    for (int j = 0, r = 1; j < p.n_tiles && r < 4; j++) {
-      const float len = (float)per[of[j]] / k[of[j]];
-      for (seen += k[of[j]] * p.n_gl; r < 4 && seen > r * slots; r++) {
-        const float rounds = shared * (r * (seen - k[of[j]] * p.n_gl == r * slots ? before : len) + len) + (r + 1) * ends;
-        est = est < rounds ? rounds : est;
-      }
-      before = len;
+  };
+  for (int n = 1; n <= 16 && n <= longest; n++) {
+    const int cap = (longest + n - 1) / n;
+    if (cap == last_cap) continue;
+    last_cap = cap;
+    int wgs = 0, pieces = 0;
+    float piece = 0.f;  // the longest
+    for (int t = 0; t < n_tiles; t++) {
+      k[t] = per[t] > cap ? (per[t] + cap - 1) / cap : 1;
+      wgs += k[t] * n_gl;
+      pieces += k[t] > 1 ? k[t] * n_gl : 0;
+      piece = fmaxf(piece, (float)per[t] / k[t]);
     }
-    if (pieces) est += leave + sums + pieces * NUM_XCD * piece_mb / 8.f;
+    const float enough = n == 1 ? INFINITY : (best_cap == longest ? 0.9f : ids ? 1.f : 0.92f) * best;
+    float est;
     if (ids) {
       // documents end the walks somewhere, and the pieces that are left start in any order: what fits then is a share of the work
       // and half of a piece at most, at the rate of a chip that is not full.  (With the estimate above, packed 2 x 4288 with heads
       // of 64 takes 184 + 6 instead of 159 + 11, 4 x 1000 with heads of 128 89 + 5 instead of 80, whole.)
-      const float ti = Dqk <= 64 ? 1.f : Dqk <= 128 ? 1.4f : 2.f, even = (float)total * p.n_gl / slots;
+      const float ti = Dqk <= 64 ? 1.f : Dqk <= 128 ? 1.4f : 2.f, even = (float)total * n_gl / slots;
       const float chain = wgs <= slots ? (float)cap : (float)fmax(even + 0.5f * cap, cap);
       est = 4.f * ((wgs + slots - 1) / slots) + ti * chain + (pieces ? 5.f + pieces * NUM_XCD * piece_mb / 2.f : 0.f);
+    } else {
+      // at least: the longest piece; what an XCD has to do, spread over its slots; where the pieces are more than r rounds, r + 1
+      // of the shortest of those that start one after the other (looked at only where the rest leaves a chance: the order of
+      // the pieces is what a plan costs the host; 8192 rows with 8kv heads, all candidates put in order 8.8 us, so 3.9)
+      const float with_pieces = pieces ? leave + sums + pieces * NUM_XCD * piece_mb / 8.f : 0.f;
+      est = fmaxf((wgs <= CUS_PER_XCD ? alone : beside) * piece + ends, (shared * total * n_gl + ends * wgs + leave * pieces) / slots);
+      if (est + with_pieces >= enough) continue;
+      if (wgs > slots) {
+        sort(k);
+        int seen = 0;
+        float before = 0.f;
+        for (int j = 0, r = 1; j < n_tiles && r < 4; j++) {
+          const float len = (float)per[of[j]] / k[of[j]];
+          for (seen += k[of[j]] * n_gl; r < 4 && seen > r * slots; r++)
+            est = fmaxf(est, shared * (r * (seen - k[of[j]] * n_gl == r * slots ? before : len) + len) + (r + 1) * ends);
+          before = len;
+        }
+      }
+      est += with_pieces;
     }
-    if (n == 1 || est < (best_cap == longest ? 0.9f : ids ? 1.f : 0.92f) * best) {
+    if (est < enough) {
       best = est;
       best_cap = cap;
-      memcpy(order, of, sizeof(order));
       memcpy(n_of, k, sizeof(n_of));
     }
   }
-  if (best_cap == longest) return p;
+  if (best_cap == longest) return false;
   int at = 0, last = 0;
-  for (int j = 0; j < p.n_tiles; j++) {
-    p.first[j] = (unsigned short)at;
-    p.tile[j] = (unsigned char)order[j];
-    at += n_of[order[j]] * p.n_gl;
-    if (n_of[order[j]] > 1) last = at;
+  sort(n_of);
+  for (int j = 0; j < n_tiles; j++) {
+    p.first[j] = (uint16_t)at;
+    p.tile[j] = (uint8_t)of[j];
+    at += n_of[of[j]] * n_gl;
+    if (n_of[of[j]] > 1) last = at;
   }
-  p.first[p.n_tiles] = (unsigned short)at;
-  p.on = true;
+  p.first[n_tiles] = (uint16_t)at;
   // (with ids, pieces of half the cap where walks are shorter: whole ones 165 + 7 instead of 159 + 11 (packed 2 x 4288), 66 + 5
   // instead of 59 + 7 (2047))
   p.cap = ids ? (best_cap + 1) / 2 : best_cap;
-  p.sums_at = (groups * p.n_tiles + 63) / 64 * 64;
-  p.bytes = (size_t)p.sums_at * 4 + (size_t)last * NUM_XCD * 128 * (Dqk + Dv) * 4;  // one slot per workgroup up to the last split tile
-  return p;
+  p.sums_at = (groups * n_tiles + 63) / 64 * 64;
+  p.parts_bytes = (size_t)p.sums_at * 4 + (size_t)last * NUM_XCD * 128 * (Dqk + Dv) * 4;  // one slot per workgroup up to the last split tile
+  return true;
 }
+#endif
 
 // ------------------------------------------------------------------------------------------------
 // delta = rowsum(dO o O)
@@ -2128,16 +2129,6 @@ static bool dkdv_queued(int groups, int Skv, int Dqk) {
   return dkdv_per_cu(Dqk) == 1 && (int64_t)((groups + NUM_XCD - 1) / NUM_XCD) * ((Skv + 127) / 128) > CUS_PER_XCD;
 }
 
-// A pair mask is on the device; what models hand over as one is causal, with or without padding: square ones are planned as such.
-static int pairs_band_hi(int Sq, int Skv) { return Sq == Skv ? 0 : BAND_INF; }
-
-// the plan of a problem as the dK/dV kernel sees it: its band (all keys where the mask is something else)
-static SplitPlan bwd_split_plan(const BwdArgs& a, bool causal) {
-  const int lo = causal ? a.band_lo : a.mx.on && !a.mx.qpos ? a.mx.lo_off : BAND_INF;
-  const int hi = a.pm.qbits ? pairs_band_hi(a.Sq, a.Skv) : causal ? a.band_hi : a.mx.on && !a.mx.qpos ? a.mx.hi_off : BAND_INF;
-  return split_plan(a.B, a.Hkv, a.n_rep, a.Sq, a.Skv, a.dqk, a.dv_dim, lo, hi, a.seg != nullptr);
-}
-
 template <typename T, int DQK, int DV, bool CAUSAL, int SEG>
 static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
   BwdArgs a = args;
@@ -2149,14 +2140,8 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
   const size_t dkdv_smem = Dkdv::bytes(a.Sq);  // (checked before anything is launched)
   TP_REQUIRE(Dkdv::fits(a.Sq), TP_ERR_UNSUPPORTED, "tp_attn_bwd: Sq=%d needs %zu bytes of LDS (max 163840)", a.Sq, dkdv_smem);
   constexpr int DKDV_PER_CU = dkdv_per_cu(DQK);
-  SplitPlan plan;
-  plan.on = false;
-  plan.sums_at = 0;
-  if (a.parts) plan = bwd_split_plan(a, CAUSAL);
-  a.split = plan.on && plan.bytes <= a.parts_bytes ? plan.cap : 0;
-  a.split_sums = plan.sums_at;
   constexpr bool GENERAL = !CAUSAL && SEG == SEG_IDS;
-  a.queue = !GENERAL && !a.split && a.parts && a.parts_bytes >= QUEUE_BYTES && dkdv_queued(groups, a.Skv, DQK) ? (unsigned*)a.parts : nullptr;
+  if (GENERAL) a.queue = nullptr;
   mark(ev, 0, st);
   if (!lean) {
     // delta
@@ -2194,12 +2179,8 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
       attr_set = true;
     }
     const int n_tiles = (a.Skv + DKDV_BNK - 1) / DKDV_BNK;
-    if (a.split) {
-      memcpy(a.split_first, plan.first, sizeof(a.split_first));
-      memcpy(a.split_tile, plan.tile, sizeof(a.split_tile));
-    }
     a.turns = groups_in_turns(n_tiles, 1, groups, DKDV_PER_CU);
-    const unsigned grid = a.split ? NUM_XCD * plan.first[n_tiles] : a.queue ? (unsigned)(NUM_XCD * CUS_PER_XCD * DKDV_PER_CU) : xcd_grid(n_tiles, 1, groups);
+    const unsigned grid = a.split ? (unsigned)NUM_XCD * a.split_first[n_tiles] : a.queue ? (unsigned)(NUM_XCD * CUS_PER_XCD * DKDV_PER_CU) : xcd_grid(n_tiles, 1, groups);
     kern<<<dim3(grid), dim3(256), dkdv_smem, st>>>(a);
     int rc = check_launch("tp_attn_bwd(dkdv)");
     if (rc) return rc;
@@ -2354,7 +2335,7 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
                          const int64_t o_strides[3], const int64_t dq_strides[3], const int64_t dk_strides[3],
                          const int64_t dv_strides[3], float sm_scale, int causal, int dtype, void* stream,
                          void* const* events, const MaskExt& mx, const PairMask& pm = no_pair_mask(),
-                         void* parts = nullptr, size_t parts_bytes = 0) {
+                         const tp_attn_bwd_plan* plan = nullptr, void* parts = nullptr, size_t parts_bytes = 0) {
   TP_REQUIRE(dout && q && k && v && out && lse && dq && dk && dv && ws, TP_ERR_BAD_ARG, "tp_attn_bwd: null pointer");
   TP_REQUIRE(do_strides && q_strides && k_strides && v_strides && o_strides && dq_strides && dk_strides && dv_strides,
              TP_ERR_BAD_ARG, "tp_attn_bwd: null stride array");
@@ -2375,7 +2356,16 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   a.q = q; a.k = k; a.v = v; a.out = out; a.dout = dout; a.lse = lse; a.seg = seg;
   a.dq = dq; a.dk = dk; a.dv = dv; a.delta = ws;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv; a.n_rep = Hq / Hkv; a.dqk = Dqk; a.dv_dim = Dv;
-  a.parts = (float*)parts; a.parts_bytes = parts_bytes; a.split = 0; a.split_sums = 0; a.queue = nullptr; a.turns = 0;
+  a.parts = (float*)parts; a.split = 0; a.split_sums = 0; a.queue = nullptr; a.turns = 0;
+  // (shorter `parts` than the plan asks for: the counters, or nothing)
+  if (plan && plan->cap && plan->parts_bytes <= parts_bytes) {
+    a.split = plan->cap;
+    a.split_sums = plan->sums_at;
+    memcpy(a.split_first, plan->first, sizeof(a.split_first));
+    memcpy(a.split_tile, plan->tile, sizeof(a.split_tile));
+  } else if (plan && plan->queue && QUEUE_BYTES <= parts_bytes) {
+    a.queue = (unsigned*)parts;
+  }
   bool ok = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(dout) && aligned16(dq) &&
             aligned16(dk) && aligned16(dv);
   for (int i = 0; i < 3; i++) {
@@ -2475,22 +2465,41 @@ static MaskExt problem_mask(const tp_attn_bwd_problem& p) {
   return make_mask_ext(p.q_positions, p.causal, p.causal_offset, p.window_left, p.window_right, p.soft_cap, p.sm_scale, p.bias, p.bias_strides);
 }
 
-extern "C" size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* p) {
-  if (!p || (p->dtype != TP_BF16 && p->dtype != TP_F16) || p->B <= 0 || p->Hkv <= 0 || p->Hq <= 0 || p->Sq <= 0 || p->Skv <= 0) return 0;
+// the sizes a plan is good for: what its workgroups touch follows from them
+static void plan_sizes(const tp_attn_bwd_problem& p, int32_t (&s)[8]) {
+  const int32_t of[8] = {p.B, p.Hq, p.Hkv, p.Sq, p.Skv, p.Dqk, p.Dv, p.dtype};
+  memcpy(s, of, sizeof(of));
+}
+
+extern "C" size_t tp_attn_bwd_make_plan(const tp_attn_bwd_problem* p, tp_attn_bwd_plan* plan) {
+  if (!plan) return 0;
+  memset(plan, 0, sizeof(*plan));
+  if (!p) return 0;
+  plan_sizes(*p, plan->sizes);
+  if ((p->dtype != TP_BF16 && p->dtype != TP_F16) || p->B <= 0 || p->Hkv <= 0 || p->Hq <= 0 || p->Sq <= 0 || p->Skv <= 0) return 0;
+  // the band as the dK/dV kernel sees it (all keys where the mask is something else)
   const MaskExt mx = problem_mask(*p);
   int lo = BAND_INF, hi = BAND_INF;
   if (mx.on) {
     if (!mx.qpos) { lo = mx.lo_off; hi = mx.hi_off; }
   } else if (p->pairs) {
-    hi = pairs_band_hi(p->Sq, p->Skv);
+    // A pair mask is on the device; what models hand over as one is causal, with or without padding: square ones are planned as such.
+    hi = p->Sq == p->Skv ? 0 : BAND_INF;
   } else if (p->causal) {
     hi = 0;
   }
-  const SplitPlan plan = split_plan(p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi, p->seg != nullptr);
-  return plan.on ? plan.bytes : dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk) ? QUEUE_BYTES : 0;
+  plan->queue = dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk);
+  if (plan->queue) plan->parts_bytes = QUEUE_BYTES;
+  split_plan(*plan, p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi, p->seg != nullptr);
+  return plan->parts_bytes;
 }
 
-extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {
+extern "C" size_t tp_attn_bwd_parts_bytes(const tp_attn_bwd_problem* p) {
+  tp_attn_bwd_plan plan;
+  return tp_attn_bwd_make_plan(p, &plan);
+}
+
+extern "C" int tp_attn_bwd_run_planned(const tp_attn_bwd_problem* p, const tp_attn_bwd_plan* plan, void* stream, void* const* events) {
   TP_REQUIRE(p, TP_ERR_BAD_ARG, "tp_attn_bwd_run: null problem");
   TP_REQUIRE(p->sm_scale > 0.f, TP_ERR_BAD_ARG, "tp_attn_bwd_run: sm_scale must be positive");
   TP_REQUIRE(p->window_left < BAND_INF && p->window_right < BAND_INF && p->causal_offset > -BAND_INF && p->causal_offset < BAND_INF, TP_ERR_BAD_ARG,
@@ -2498,6 +2507,11 @@ extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {
   TP_REQUIRE(!p->bias || (p->bias_strides[0] >= 0 && p->bias_strides[1] >= 0 && p->bias_strides[2] >= 0), TP_ERR_BAD_ARG,
              "tp_attn_bwd_run: negative bias stride");
   TP_REQUIRE((p->parts != nullptr) == (p->parts_bytes != 0) && aligned16(p->parts), TP_ERR_BAD_ARG, "tp_attn_bwd_run: parts and parts_bytes disagree");
+  if (plan) {
+    int32_t sizes[8];
+    plan_sizes(*p, sizes);
+    TP_REQUIRE(memcmp(sizes, plan->sizes, sizeof(sizes)) == 0, TP_ERR_BAD_ARG, "tp_attn_bwd_run: the plan was made for other sizes");
+  }
   PairMask pm = no_pair_mask();
   if (p->pairs) {
     TP_REQUIRE(!p->seg && !p->bias && !p->q_positions && !p->causal && p->window_left < 0 && p->window_right < 0 && !(p->soft_cap > 0.f), TP_ERR_BAD_ARG,
@@ -2511,6 +2525,12 @@ extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {
   const MaskExt mx = problem_mask(*p);
   return attn_bwd_impl(p->dout, p->q, p->k, p->v, p->out, p->lse, p->seg, p->dq, p->dk, p->dv, p->ws, p->B, p->Hq, p->Hkv, p->Sq, p->Skv, p->Dqk,
                        p->Dv, p->do_strides, p->q_strides, p->k_strides, p->v_strides, p->o_strides, p->dq_strides, p->dk_strides, p->dv_strides,
-                       p->sm_scale, p->causal, p->dtype, stream, nullptr, mx, pm, p->parts, p->parts_bytes);
+                       p->sm_scale, p->causal, p->dtype, stream, events, mx, pm, plan, p->parts, p->parts_bytes);
+}
+
+extern "C" int tp_attn_bwd_run(const tp_attn_bwd_problem* p, void* stream) {
+  tp_attn_bwd_plan plan;
+  if (p && p->parts) tp_attn_bwd_make_plan(p, &plan);
+  return tp_attn_bwd_run_planned(p, p && p->parts ? &plan : nullptr, stream, nullptr);
 }
 #endif  // !TP_BWD_UNIT

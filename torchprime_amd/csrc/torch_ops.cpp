@@ -511,11 +511,12 @@ struct BwdCall {
     if (dq.numel() == 0 || dk.numel() == 0) return {dq.zero_(), dk.zero_(), dv.zero_()};
     // one workspace: the row vectors, then the pieces of split key tiles (none for most problems)
     const size_t rows = tp_attn_bwd_workspace_bytes(s.B, s.Hq, s.Sq), at = (rows + 255) / 256 * 256;
-    p.parts_bytes = tp_attn_bwd_parts_bytes(&p);
+    tp_attn_bwd_plan plan;
+    p.parts_bytes = tp_attn_bwd_make_plan(&p, &plan);
     const Tensor ws = empty_f32({(int64_t)((p.parts_bytes ? at + p.parts_bytes : rows) / 4)}, q);
     p.ws = (float*)ws.data_ptr();
     p.parts = p.parts_bytes ? (char*)ws.data_ptr() + at : nullptr;
-    check(tp_attn_bwd_run(&p, stream_of(dev)), "tp_attn_bwd_run");
+    check(tp_attn_bwd_run_planned(&p, &plan, stream_of(dev), nullptr), "tp_attn_bwd_run");
     return {dq, dk, dv};
   }
 };
@@ -1161,7 +1162,8 @@ variable_list LayerNode::apply(variable_list&& g) {
   tp_attn_bwd_problem ab{};
   ab.B = (int)s.B; ab.Hq = (int)s.Hq; ab.Hkv = (int)s.Hkv; ab.Sq = ab.Skv = (int)s.S; ab.Dqk = ab.Dv = (int)s.D;
   ab.causal = s.causal; ab.window_left = ab.window_right = -1; ab.dtype = s.dtype; ab.sm_scale = (float)(1.0 / std::sqrt((double)s.D));
-  ab.parts_bytes = want.attn ? tp_attn_bwd_parts_bytes(&ab) : 0;
+  tp_attn_bwd_plan plan;
+  ab.parts_bytes = want.attn ? tp_attn_bwd_make_plan(&ab, &plan) : 0;
   size_t at = 0;
   const auto take = [&](bool used, size_t n) { const size_t o = at; at += used ? (n + 255) / 256 * 256 : 0; return o; };
   const size_t o_act = take(want.mlp, R * s.I * e), o_dg = take(want.mlp, R * s.I * e), o_du = take(want.mlp, R * s.I * e);
@@ -1214,7 +1216,7 @@ variable_list LayerNode::apply(variable_list&& g) {
       ab.do_strides[i] = ab.q_strides[i] = ab.o_strides[i] = ab.dq_strides[i] = qs[i];
       ab.k_strides[i] = ab.v_strides[i] = ab.dk_strides[i] = ab.dv_strides[i] = ks[i];
     }
-    check(tp_attn_bwd_run(&ab, st), "tp_attn_bwd_run");
+    check(tp_attn_bwd_run_planned(&ab, &plan, st, nullptr), "tp_attn_bwd_run");
     layer_rope(s, t + o_dq, t + o_dk, C, Sn, true, st);
   }
   // q, k, v
