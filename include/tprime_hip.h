@@ -149,8 +149,10 @@ int tp_attn_fwd(const void* q, const void* k, const void* v, const int32_t* seg,
  *   pairs         tp_mask_pairs_bytes() bytes, 16-byte aligned
  *   verdict       non-zero: also set the int32 flags at the start of `pairs`, which the caller has cleared:
  *                 [0] some entry is neither 0 nor drops its pair, [1] the mask is not the exact causal mask
- *                 (0 / -inf), [2] a row without a pair has entries other than -inf.  The attention entry
- *                 points give the eager formula's results if [0] and [2] are 0.
+ *                 (0 / -inf), [2] a row without a pair has entries other than -inf, [3] the pairs
+ *                 are not causality and padding: one lies above the diagonal, or of two neighbouring rows with
+ *                 pairs only one has some key that both come after.  The attention entry points give the eager
+ *                 formula's results if [0] and [2] are 0.
  * tp_attn_fwd_pairs   tp_attn_fwd (no segment ids, no causality of its own) over the pairs of `pairs`, made for
  *   mask_batches (1 or B) masks.  bf16 and fp16.  Backward: tp_attn_bwd_run with `pairs`.
  * tp_attn_pairs_fit   non-zero where all three take masks and heads of these sizes (for head dims (128,128) up to
@@ -344,6 +346,8 @@ int tp_cross_entropy_bwd(const void* logits, const int64_t* labels, const float*
  * The attention backward as one struct: everything tp_attn_bwd / _masked / _biased take (fields that do not
  * apply: NULL, windows -1, soft_cap 0), a pair mask, and workspace for problems with few key tiles.
  *   pairs, mask_batches   see tp_mask_pairs; goes with no other mask
+ *   pairs_causal           with pairs: non-zero if they are known to be causality and padding (the verdict's [3] is 0).
+ *                         Key tiles are handed out by it; the results are the same either way
  *   parts, parts_bytes    tp_attn_bwd_parts_bytes() bytes, 16-byte aligned, or NULL / 0.  With it the walk of a
  *                         key tile over its queries is split over several workgroups where one each would
  *                         leave CUs idle, or a large problem's key tiles are handed out by counters that lie
@@ -368,6 +372,7 @@ typedef struct tp_attn_bwd_problem {
   int causal, causal_offset, window_left, window_right;
   float soft_cap;
   int dtype;
+  int pairs_causal;
 } tp_attn_bwd_problem;
 /* How the key tiles of a problem are handed to workgroups.  Made on the host from the problem's sizes, mask arguments and
  * which of its pointers are NULL; a caller that keeps it between asking for `parts` and running saves making it twice, and may

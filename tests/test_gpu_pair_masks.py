@@ -115,3 +115,56 @@ def test_bits_at_the_rows_ends(Skv, dtype):
     assert torch.equal(got[:, :Sq, :Skv], keep) and not got[:, Sq:].any() and not got[:, :, Skv:].any()
     got = ((kbits[..., None] >> bit) & 1).bool().permute(0, 1, 3, 2).reshape(B, nqt * 64, nkb * 128)
     assert torch.equal(got[:, :Sq, :Skv], keep) and not got[:, Sq:].any() and not got[:, :, Skv:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("Sq,Skv", [(3, 3), (5, 5), (64, 64), (65, 65), (129, 129), (200, 200), (4200, 4200), (70, 131), (131, 70)])
+def test_causality_and_padding_are_told_from_other_pairs(Sq, Skv, dtype):
+  """Causal masks less whole rows and keys; one pair more above the diagonal or one less below it, anywhere, makes the difference."""
+  keep = torch.ones((2, 1, Sq, Skv), dtype=torch.bool, device=DEV).tril()
+  keep[0, :, :, Skv // 2 + 1 :] = False  # padding on the right ...
+  keep[1, :, :, : Skv // 3] = False  # ... and on the left, whose rows have no pair
+  fill = lambda keep: torch.zeros(keep.shape, dtype=dtype, device=DEV).masked_fill_(~keep, float("-inf"))  # noqa: E731
+  verdict = lambda keep: tpa.ops.mask_verdict(fill(keep))  # noqa: E731
+  assert verdict(keep) == tpa.ops.MASK_PAIRS_CAUSAL and tpa.ops.mask_kind(fill(keep)) == tpa.ops.MASK_PAIRS
+  m = min(Sq, Skv)
+  for i, j in {(0, 1), (0, Skv - 1), (62, 63), (63, 64), (64, 65), (127, 128), (m - 2, m - 1), (Sq - 1, Sq), (4100, 4101)}:
+    if 0 <= i < Sq and i < j < Skv:
+      one = keep.clone()
+      one[1, 0, i, j] = True
+      assert verdict(one) == tpa.ops.MASK_PAIRS, ("above", i, j)
+  for i, j in {(m - 1, m // 2), (Sq - 1, m // 2), (Sq // 2, Skv // 3), (64, 63), (63, 62), (64, 40), (128, 64), (128, 127), (4100, 4000)}:
+    if i < Sq and j < min(i, Skv) and keep[0, 0, i, j] and int(keep[0, 0, i].sum()) > 1:
+      one = keep.clone()
+      one[0, 0, i, j] = False
+      assert verdict(one) == tpa.ops.MASK_PAIRS, ("below", i, j)
+
+
+def test_documents_and_windows_are_not_padding():
+  S = 300
+  i, j = torch.arange(S)[:, None], torch.arange(S)[None]
+  for keep in (i // 100 == j // 100, (i // 100 == j // 100) & (j <= i), (j <= i) & (j > i - 50), (j <= i) | (j < 20), torch.ones((S, S), dtype=torch.bool),
+               (j < 200) & (i >= 0)):  # fmt: skip
+    mask = torch.zeros((1, 1, S, S)).masked_fill_(~keep, float("-inf")).to(DEV, torch.bfloat16)
+    assert tpa.ops.mask_verdict(mask) == tpa.ops.mask_kind(mask) == tpa.ops.MASK_PAIRS
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_the_backward_knows_the_kind(causal):
+  """What the module's check says of the mask reaches the operator that plans the backward."""
+  from torch.utils._python_dispatch import TorchDispatchMode
+
+  seen = []
+
+  class Calls(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+      if func is torch.ops.tprime.attn_bwd_pairs.default:
+        seen.append(len(args) > 9 and args[9])
+      return func(*args, **(kwargs or {}))
+
+  q = torch.randn((2, 4, 300, 64), device=DEV, dtype=torch.bfloat16, requires_grad=True)
+  mask = _padding_mask(2, 300, 300, [300, 100], causal=causal, dtype=torch.bfloat16, fill=LOWEST[torch.bfloat16]).to(DEV)
+  m = tpa.AttentionModule(tpa.Config(attention_kernel=None, num_attention_heads=4, num_key_value_heads=4))
+  with Calls():
+    m(q, q, q, mask).sum().backward()
+  assert seen == [causal]

@@ -26,12 +26,12 @@ class _Problem(ctypes.Structure):  # tp_attn_bwd_problem
   _fields_ += [(n, ctypes.c_int) for n in ("B", "Hq", "Hkv", "Sq", "Skv", "Dqk", "Dv")]
   _fields_ += [(n, I3) for n in ("do_s", "q_s", "k_s", "v_s", "o_s", "dq_s", "dk_s", "dv_s")]
   _fields_ += [("sm_scale", ctypes.c_float)] + [(n, ctypes.c_int) for n in ("causal", "causal_offset", "window_left", "window_right")]
-  _fields_ += [("soft_cap", ctypes.c_float), ("dtype", ctypes.c_int)]
+  _fields_ += [("soft_cap", ctypes.c_float), ("dtype", ctypes.c_int), ("pairs_causal", ctypes.c_int)]
 
 
-def _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=False, pairs=False, soft_cap=0.0, ids=False):
+def _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=False, pairs=False, soft_cap=0.0, ids=False, padded=False):
   p = _Problem(seg=16 if ids else None, B=B, Hq=Hq, Hkv=Hkv, Sq=S, Skv=S, Dqk=Dqk, Dv=Dv, causal=int(causal), window_left=-1, window_right=-1, sm_scale=0.1,
-               soft_cap=soft_cap, pairs=16 if pairs else None, mask_batches=int(pairs))  # fmt: skip
+               soft_cap=soft_cap, pairs=16 if pairs else None, mask_batches=int(pairs), pairs_causal=int(padded))  # fmt: skip
   assert _lib.load().tp_attn_bwd_parts_bytes(ctypes.byref(p)) > 0
 
 
@@ -94,7 +94,7 @@ def test_more_groups_than_engines(Dqk, Dv, what):
   """Three groups of heads on some XCDs and two on the others, pieces that start by falling length; walks that padding or a
   short document ends before the plan's last piece, in some sequences only."""
   B, Hq, Hkv, S, scale = 5, 16, 4, 600, 1 / math.sqrt(Dv)
-  _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=what != "padding", pairs=what == "padding", ids=what == "ids")
+  _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=what != "padding", pairs=what == "padding", ids=what == "ids", padded=True)
   (q, k, v, do), leaves, dod = _leaves(Hq, Hkv, S, Dqk, Dv, B)
   if what == "padding":
     seen = torch.tensor([600, 1, 129, 64, 383])

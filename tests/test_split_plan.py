@@ -14,9 +14,9 @@ class _Plan(ctypes.Structure):  # tp_attn_bwd_plan
   _fields_ += [(n, ctypes.c_int32) for n in ("queue", "cap", "sums_at")] + [("first", ctypes.c_uint16 * 65), ("tile", ctypes.c_uint8 * 64)]
 
 
-def _problem(B=1, Hq=32, Hkv=8, S=1024, Dqk=128, Dv=128, causal=True, ids=False, pairs=False):
+def _problem(B=1, Hq=32, Hkv=8, S=1024, Dqk=128, Dv=128, causal=True, ids=False, pairs=False, padded=False):
   return _Problem(B=B, Hq=Hq, Hkv=Hkv, Sq=S, Skv=S, Dqk=Dqk, Dv=Dv, causal=int(causal), window_left=-1, window_right=-1, sm_scale=0.1,
-                  seg=16 if ids else None, pairs=16 if pairs else None, mask_batches=int(pairs))  # fmt: skip
+                  seg=16 if ids else None, pairs=16 if pairs else None, mask_batches=int(pairs), pairs_causal=int(padded))  # fmt: skip
 
 
 def _plan(p):
@@ -54,3 +54,25 @@ def test_a_plan_is_for_its_sizes():
     assert lib.tp_attn_bwd_run_planned(ctypes.byref(o), ctypes.byref(plan), None, None) != 0 and b"other sizes" in lib.tp_last_error()
   assert lib.tp_attn_bwd_make_plan(None, ctypes.byref(plan)) == 0 and plan.parts_bytes == 0
   assert lib.tp_attn_bwd_make_plan(ctypes.byref(p), None) == 0
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,Dqk", [(4, 32, 8, 1000, 128), (1, 32, 8, 1024, 128), (1, 32, 8, 2047, 128), (2, 32, 8, 2048, 128), (1, 16, 16, 1472, 192),
+                                            (1, 32, 8, 900, 64), (4, 8, 8, 333, 64)])  # fmt: skip
+def test_pair_masks_are_planned_by_what_is_known_of_them(B, Hq, Hkv, S, Dqk):
+  """Nothing known: every key tile may be seen by every query or by few, as under segment ids without causality.  Causality and
+  padding: the causal plan."""
+  sizes = dict(B=B, Hq=Hq, Hkv=Hkv, S=S, Dqk=Dqk, Dv=min(Dqk, 128))
+  assert bytes(_plan(_problem(causal=False, pairs=True, **sizes))) == bytes(_plan(_problem(causal=False, ids=True, **sizes)))
+  assert bytes(_plan(_problem(causal=False, pairs=True, padded=True, **sizes))) == bytes(_plan(_problem(causal=True, **sizes)))
+
+
+@pytest.mark.parametrize("Dqk", [64, 128, 192])
+def test_equal_walks_are_cut_alike(Dqk):
+  """Under a pair mask of which nothing is known no key tile's workgroups walk more than the longest that one XCD's share allows:
+  the tiles are cut into the same number of pieces, or none is."""
+  for B in (1, 2, 4):
+    for S in range(256, 2304, 128):
+      plan = _plan(_problem(B=B, S=S, Dqk=Dqk, Dv=min(Dqk, 128), causal=False, pairs=True))
+      if plan.cap:
+        n = S // 128
+        assert len({plan.first[t + 1] - plan.first[t] for t in range(n)}) == 1, (B, S)

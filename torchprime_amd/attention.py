@@ -31,7 +31,7 @@ def repeat_kv(hidden_states: torch.Tensor, n_rep: int) -> torch.Tensor:
   return hidden_states.unsqueeze(2).expand(b, h, n_rep, s, d).reshape(b, h * n_rep, s, d)
 
 
-# Kinds of the masks handed to the eager branch (ops.mask_kind), kept per mask tensor object (a weak reference and the
+# Kinds of the masks handed to the eager branch (ops.mask_verdict), kept per mask tensor object (a weak reference and the
 # tensor's version counter).  A model builds its mask once per forward and hands the same tensor to every layer, so the
 # pass over the mask and its host sync run once per mask rather than once per layer.  The key is the object, never its
 # address: a mask built for the next forward is a new tensor that the caching allocator may well place where the last
@@ -50,7 +50,7 @@ def _mask_verdict(mask: torch.Tensor, q_len: int, kv_len: int) -> int:
   if mask.dim() == 4 and mask.shape[1] == 1 and mask.shape[2] == q_len and mask.shape[3] >= kv_len:
     m = mask[:, :, :, :kv_len]
     if m.is_cuda and m.dtype in (torch.bfloat16, torch.float16, torch.float32):
-      kind = ops.mask_kind(m)
+      kind = ops.mask_verdict(m)
     else:  # (a causal mask is not read any further: it may be of any type and on the host)
       keep = torch.ones((q_len, kv_len), dtype=torch.bool, device=m.device).tril()
       if bool((((m == 0) == keep) & ((m == float("-inf")) == ~keep)).all()):
@@ -143,11 +143,11 @@ class AttentionModule(nn.Module):
       if bias is not None:
         scale = 1.0 / math.sqrt(head_dim)
         # (a float16 mask's lowest value drops a pair for float16 logits only; fp32 has no kernels for pair bits)
-        by_bits = kind == ops.MASK_PAIRS and bias.shape[0] in (1, bsz) and (
+        by_bits = kind in (ops.MASK_PAIRS, ops.MASK_PAIRS_CAUSAL) and bias.shape[0] in (1, bsz) and (
           query_states.dtype == torch.bfloat16 and bias.dtype != torch.float16 or query_states.dtype == torch.float16
         ) and ops.attention_pairs_fit(query_states, key_states, value_states, bias)
         if by_bits:
-          attn_output = ops.attention_pairs(query_states, key_states, value_states, bias.detach(), scale)
+          attn_output = ops.attention_pairs(query_states, key_states, value_states, bias.detach(), scale, kind == ops.MASK_PAIRS_CAUSAL)
         else:
           attn_output = ops.attention(query_states, key_states, value_states, None, scale, False, bias=bias)
         if attn_output.size() != (bsz, num_heads, q_len, head_dim):

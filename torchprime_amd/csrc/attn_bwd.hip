@@ -107,7 +107,8 @@ struct BwdArgs {
 // (host: the plan is made by the C entry points, tp_attn_bwd_make_plan)
 #ifndef TP_BWD_UNIT
 static_assert(sizeof(tp_attn_bwd_plan::first) == sizeof(BwdArgs::split_first) && sizeof(tp_attn_bwd_plan::tile) == sizeof(BwdArgs::split_tile), "the plan's tables");
-// Whether walks are split, and if so the plan's cap, sums_at, first, tile and parts_bytes.
+// Whether walks are split, and if so the plan's cap, sums_at, first, tile and parts_bytes.  ids: segment ids, or a mask of which
+// nothing else is known.
 static bool split_plan(tp_attn_bwd_plan& p, int B, int Hkv, int n_rep, int Sq, int Skv, int Dqk, int Dv, int band_lo, int band_hi, bool ids) {
   const int n_tiles = (Skv + 127) / 128, groups = B * Hkv, n_gl = (groups + NUM_XCD - 1) / NUM_XCD;
   const int slots = CUS_PER_XCD * dkdv_per_cu(Dqk);
@@ -2483,14 +2484,18 @@ extern "C" size_t tp_attn_bwd_make_plan(const tp_attn_bwd_problem* p, tp_attn_bw
   if (mx.on) {
     if (!mx.qpos) { lo = mx.lo_off; hi = mx.hi_off; }
   } else if (p->pairs) {
-    // A pair mask is on the device; what models hand over as one is causal, with or without padding: square ones are planned as such.
-    hi = p->Sq == p->Skv ? 0 : BAND_INF;
+    // A pair mask is on the device, and what it drops is not known here but for the caller's word.  dK/dV and dQ, us, heads of
+    // 128, 32q/8kv, planned over all pairs : as causal.  Causality and padding: 4 x 1000 163 : 157, 1 x 2047 178 : 151.  Not causal:
+    // the last key tiles are left whole and start last, 242 : 293 and 237 : 397, with padding 213 : 276 and 239 : 397.  Causal
+    // documents: the little that is left to a tile starts in two rounds, 96 : 124 and 64 : 79.
+    hi = p->pairs_causal && p->Sq == p->Skv ? 0 : BAND_INF;
   } else if (p->causal) {
     hi = 0;
   }
   plan->queue = dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk);
   if (plan->queue) plan->parts_bytes = QUEUE_BYTES;
-  split_plan(*plan, p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi, p->seg != nullptr);
+  const bool unknown = p->seg || (p->pairs && !p->pairs_causal);
+  split_plan(*plan, p->B, p->Hkv, p->Hq / p->Hkv, p->Sq, p->Skv, p->Dqk, p->Dv, lo, hi, unknown);
   return plan->parts_bytes;
 }
 

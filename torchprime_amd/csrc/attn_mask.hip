@@ -19,8 +19,8 @@ namespace tp {
 template <typename T> constexpr float Dropped = -1e30f;
 template <> constexpr float Dropped<f16_t> = -65504.f;
 // flags[]: entries that are neither 0 nor dropped; entries that differ from the exact causal mask (0 / -inf); rows
-// without a pair whose entries are not all -inf
-constexpr int F_OTHER = 0, F_NOT_CAUSAL = 1, F_EMPTY_FINITE = 2;
+// without a pair whose entries are not all -inf; pairs that are not the causal ones less rows and keys as a whole (padding)
+constexpr int F_OTHER = 0, F_NOT_CAUSAL = 1, F_EMPTY_FINITE = 2, F_NOT_PADDED = 3;
 
 // One wave per 64 x 64 block.  Lane r reads its row's 64 entries, 128 or 256 contiguous bytes, in 16-byte loads that are
 // all in flight together, and builds the row's word; the columns' words are 64 ballots over the rows' words.  (A lane
@@ -106,15 +106,29 @@ __global__ __launch_bounds__(256) void mask_bits_kernel(const T* __restrict__ ma
   }
 }
 
-// one wave per row: a row without a pair must be -inf throughout
+// One wave per row: a row without a pair must be -inf throughout; the others of a padded causal mask have no pair above the
+// diagonal and, up to the row before, that row's keys (where it has any).
 template <typename T>
 __global__ __launch_bounds__(256) void mask_rows_kernel(const T* __restrict__ mask, int64_t bs, int64_t rs, int Sq, int Skv, int nkt, int nqb,
                                                         const unsigned long long* __restrict__ qbits, int* __restrict__ flags) {
   const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), b = blockIdx.y;
   if (row >= Sq) return;
-  bool any = false;
-  for (int t = lane; t < nkt; t += 64) any = any || qbits[((int64_t)b * nkt + t) * (nqb * 128) + row] != 0ull;
-  if (__ballot(any)) return;
+  bool any = false, before = false, above = false, uneven = false;
+  for (int t = lane; t < nkt; t += 64) {
+    const unsigned long long* at = qbits + ((int64_t)b * nkt + t) * (nqb * 128) + row;
+    const unsigned long long w = at[0], p = row > 0 ? at[-1] : 0ull;
+    // the first n keys of the tile
+    auto first = [](int n) { return n <= 0 ? 0ull : n >= 64 ? ~0ull : (1ull << n) - 1ull; };
+    any = any || w != 0ull;
+    before = before || p != 0ull;
+    above = above || (w & ~first(row + 1 - 64 * t)) != 0ull;
+    uneven = uneven || (w & first(row - 64 * t)) != p;
+  }
+  if (__ballot(any)) {
+    const bool other = __ballot(above) || (__ballot(before) && __ballot(uneven));
+    if (other && lane == 0) flags[F_NOT_PADDED] = 1;
+    return;
+  }
   bool finite = false;
   for (int j = lane; j < Skv; j += 64) finite = finite || (float)mask[b * bs + row * rs + j] != -INFINITY;
   if (__ballot(finite) && lane == 0) flags[F_EMPTY_FINITE] = 1;

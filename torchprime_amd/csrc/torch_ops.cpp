@@ -162,8 +162,8 @@ TP_OP(attn_fwd_masked, T2(const Tensor&, const Tensor&, const Tensor&, OptTensor
                           double, OptTensor))
 TP_OP(attn_bwd_masked, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, OptTensor, OptTensor,
                           double, bool, int64_t, int64_t, int64_t, double, OptTensor))
-TP_OP(attn_fwd_pairs, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, double))
-TP_OP(attn_bwd_pairs, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, int64_t, double))
+TP_OP(attn_fwd_pairs, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, double, bool))
+TP_OP(attn_bwd_pairs, T3(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, int64_t, double, bool))
 TP_OP(l2norm_fwd, T2(const Tensor&, double))
 TP_OP(l2norm_bwd, Tensor(const Tensor&, const Tensor&, const Tensor&))
 TP_OP(scale_rows, Tensor(const Tensor&, const Tensor&))
@@ -647,7 +647,7 @@ Tensor make_pairs(const PairsIn& m, int64_t Sq, int64_t Skv, bool verdict, void*
   return pairs;
 }
 // (out, lse, pairs): the bits are made once per forward and kept for the backward
-T3 attn_fwd_pairs_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& mask, double sm_scale) {
+T3 attn_fwd_pairs_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& mask, double sm_scale, bool /*causal_padded*/) {
   const c10::Device dev = require_gpu(q_, k_, v_, mask);
   const AttnShape s = check_attn(q_, k_, v_, undef());
   TORCH_CHECK_VALUE(mask.size(0) == 1 || mask.size(0) == s.B, "mask batch ", mask.size(0), " does not broadcast to ", s.B);
@@ -663,32 +663,35 @@ T3 attn_fwd_pairs_cuda(const Tensor& q_, const Tensor& k_, const Tensor& v_, con
   return {out, lse, pairs};
 }
 T3 attn_bwd_pairs_cuda(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
-                       const Tensor& pairs, int64_t mask_batches, double sm_scale) {
+                       const Tensor& pairs, int64_t mask_batches, double sm_scale, bool causal_padded) {
   BwdCall c(require_gpu(dout, q, k, v, out, lse, pairs), dout, q, k, v, out, lse, undef(), sm_scale);
   TORCH_CHECK_VALUE(pairs.is_contiguous() && pairs.scalar_type() == at::kInt && mask_batches > 0 &&
                     pairs.numel() == (int64_t)tp_mask_pairs_bytes((int)mask_batches, c.s.Sq, c.s.Skv) / 4, "pairs were not made for this problem");
   c.p.pairs = pairs.data_ptr();
   c.p.mask_batches = (int)mask_batches;
+  c.p.pairs_causal = causal_padded;
   return c.run();
 }
 struct AttnPairsNode : OpNode {
   int64_t mask_batches;
   double sm_scale;
+  bool causal_padded;
   std::string name() const override { return "TprimeAttnPairsBackward"; }
   variable_list bwd(variable_list&& g) override {
     if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
-    T3 r = op_attn_bwd_pairs()(g[0], get(0), get(1), get(2), get(3), get(4), get(5), mask_batches, sm_scale);
+    T3 r = op_attn_bwd_pairs()(g[0], get(0), get(1), get(2), get(3), get(4), get(5), mask_batches, sm_scale, causal_padded);
     return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
   }
 };
-T3 attn_fwd_pairs_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+T3 attn_fwd_pairs_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale, bool causal_padded) {
   auto node = make_node<AttnPairsNode>(q, k, v);
-  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_attn_fwd_pairs()(q, k, v, mask, sm_scale); }();
+  T3 r = [&] { at::AutoDispatchBelowADInplaceOrView below; return op_attn_fwd_pairs()(q, k, v, mask, sm_scale, causal_padded); }();
   if (node) {
     torch::autograd::set_history(std::get<0>(r), node);
     node->keep(q); node->keep(k); node->keep(v); node->keep(std::get<0>(r), true); node->keep(std::get<1>(r)); node->keep(std::get<2>(r));
     node->mask_batches = mask.size(0);
     node->sm_scale = sm_scale;
+    node->causal_padded = causal_padded;
   }
   return r;
 }
@@ -1509,13 +1512,13 @@ Tensor py_attention_masked(const Tensor& q, const Tensor& k, const Tensor& v, Op
   require_gpu(q, k, v, seg, qpos, bias);
   return std::get<0>(op_attn_fwd_masked()(q, k, v, seg, qpos, sm_scale, causal, causal_offset, window_left, window_right, soft_cap, bias));
 }
-Tensor py_attention_pairs(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+Tensor py_attention_pairs(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale, bool causal_padded) {
   require_gpu(q, k, v, mask);
-  return std::get<0>(op_attn_fwd_pairs()(q, k, v, mask, sm_scale));
+  return std::get<0>(op_attn_fwd_pairs()(q, k, v, mask, sm_scale, causal_padded));
 }
-// What a (1|B, 1, Sq, Skv) mask is: 1 the exact causal mask, 2 one that only drops pairs, 0 anything else.  Two short
-// kernels and one synchronisation (for each 65535 masks, as many as their grid takes).
-int64_t py_mask_kind(const Tensor& mask) {
+// What a (1|B, 1, Sq, Skv) mask is: 1 the exact causal mask, 2 one that only drops pairs, 3 one that is causality and
+// padding, 0 anything else.  Two short kernels and one synchronisation (for each 65535 masks, as many as their grid takes).
+int64_t py_mask_verdict(const Tensor& mask) {
   const c10::Device dev = require_gpu(mask);
   TORCH_CHECK_VALUE(mask.dim() == 4, "expected a 4-D mask");
   if (mask.numel() == 0) return 0;
@@ -1523,14 +1526,14 @@ int64_t py_mask_kind(const Tensor& mask) {
   at::AutoDispatchBelowADInplaceOrView below;
   constexpr int64_t MOST = 65535;
   const int64_t Sq = mask.size(2), Skv = mask.size(3);
-  int other = 0, not_causal = 0, empty_finite = 0;
+  int other = 0, not_causal = 0, empty_finite = 0, not_padded = 0;
   for (int64_t b = 0; b < mask.size(0); b += MOST) {
     const PairsIn m = prep_pairs(mask.size(0) <= MOST ? mask : mask.slice(0, b, b + MOST), Sq, Skv);
     const Tensor flags = make_pairs(m, Sq, Skv, true, stream_of(dev)).slice(0, 0, 16).cpu();
     const int* f = flags.const_data_ptr<int>();
-    other |= f[0]; not_causal |= f[1]; empty_finite |= f[2];
+    other |= f[0]; not_causal |= f[1]; empty_finite |= f[2]; not_padded |= f[3];
   }
-  return !not_causal ? 1 : (!other && !empty_finite) ? 2 : 0;
+  return !not_causal ? 1 : other || empty_finite ? 0 : not_padded ? 2 : 3;
 }
 Tensor py_l2norm(const Tensor& x, double eps) { return std::get<0>(op_l2norm_fwd()(x, eps)); }
 Tensor py_swiglu(const Tensor& g, const Tensor& u) { return op_swiglu_fwd()(g, u); }
@@ -1552,8 +1555,8 @@ TORCH_LIBRARY(tprime, m) {
         "int window_left, int window_right, float soft_cap, Tensor? bias=None) -> (Tensor, Tensor)");
   m.def("attn_bwd_masked(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor? seg, Tensor? qpos, float sm_scale, "
         "bool causal, int causal_offset, int window_left, int window_right, float soft_cap, Tensor? bias=None) -> (Tensor, Tensor, Tensor)");
-  m.def("attn_fwd_pairs(Tensor q, Tensor k, Tensor v, Tensor mask, float sm_scale) -> (Tensor, Tensor, Tensor)");
-  m.def("attn_bwd_pairs(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor pairs, int mask_batches, float sm_scale) "
+  m.def("attn_fwd_pairs(Tensor q, Tensor k, Tensor v, Tensor mask, float sm_scale, bool causal_padded=False) -> (Tensor, Tensor, Tensor)");
+  m.def("attn_bwd_pairs(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, Tensor pairs, int mask_batches, float sm_scale, bool causal_padded=False) "
         "-> (Tensor, Tensor, Tensor)");
   m.def("l2norm_fwd(Tensor x, float eps) -> (Tensor, Tensor)");
   m.def("l2norm_bwd(Tensor dy, Tensor x, Tensor rstd) -> Tensor");
@@ -1603,7 +1606,7 @@ TORCH_LIBRARY_IMPL(tprime, Autograd, m) {
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  // Other Python threads run meanwhile: some of these wait for the device (mask_kind, rope_apply with positions), and any
+  // Other Python threads run meanwhile: some of these wait for the device (mask_verdict, rope_apply with positions), and any
   // launch or allocation may.
   const py::call_guard<py::gil_scoped_release> no_gil;
   m.def("rmsnorm", &py_rmsnorm, no_gil);
@@ -1613,7 +1616,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention", &py_attention, no_gil);
   m.def("attention_masked", &py_attention_masked, no_gil);
   m.def("attention_pairs", &py_attention_pairs, no_gil);
-  m.def("mask_kind", &py_mask_kind, no_gil);
+  m.def("mask_verdict", &py_mask_verdict, no_gil);
   m.def("mask_pairs_words", [](int64_t Bm, int64_t Sq, int64_t Skv) { return (int64_t)tp_mask_pairs_bytes((int)Bm, (int)Sq, (int)Skv) / 4; });
   m.def("attention_pairs_fit", [](int64_t Bm, int64_t Sq, int64_t Skv, int64_t Dqk, int64_t Dv) {
     const auto is_int = [](int64_t v) { return v >= 0 && v < (1ll << 31); };

@@ -127,14 +127,14 @@ def _(dout, q, k, v, out, lse, seg, qpos, sm_scale, causal, causal_offset, windo
 
 
 @torch.library.register_fake("tprime::attn_fwd_pairs")
-def _(q, k, v, mask, sm_scale):
+def _(q, k, v, mask, sm_scale, causal_padded=False):
   B, Hq, Sq, _ = q.shape
   words = _native.mask_pairs_words(mask.shape[0], Sq, k.shape[2])
   return _empty_like_heads(q, v.shape[-1]), q.new_empty((B, Hq, Sq), dtype=torch.float32), q.new_empty((words,), dtype=torch.int32)
 
 
 @torch.library.register_fake("tprime::attn_bwd_pairs")
-def _(dout, q, k, v, out, lse, pairs, mask_batches, sm_scale):
+def _(dout, q, k, v, out, lse, pairs, mask_batches, sm_scale, causal_padded=False):
   return _empty_like_heads(q), _empty_like_heads(k), _empty_like_heads(v)
 
 
@@ -239,15 +239,21 @@ def attention(
   return attn_fwd_masked(*args)[0] if is_compiling() or overridden(q, k, v, segment_ids, q_positions, bias) else _native.attention_masked(*args)
 
 
-# kinds of additive masks (mask_kind)
-MASK_GENERAL, MASK_CAUSAL, MASK_PAIRS = 0, 1, 2
+# kinds of additive masks (mask_kind; the last one of mask_verdict only)
+MASK_GENERAL, MASK_CAUSAL, MASK_PAIRS, MASK_PAIRS_CAUSAL = 0, 1, 2, 3
+
+
+def mask_verdict(mask: Tensor) -> int:
+  """``mask_kind``, or ``MASK_PAIRS_CAUSAL`` for a mask of kind ``MASK_PAIRS`` that is causality and padding: the pairs on
+  and below the diagonal less rows and keys as a whole."""
+  return _native.mask_verdict(mask)
 
 
 def mask_kind(mask: Tensor) -> int:
   """What a (1|B, 1, Sq, Skv) additive mask is: ``MASK_CAUSAL`` (exactly 0 on and below the diagonal, -inf above),
   ``MASK_PAIRS`` (every entry 0 or one that lets its pair drop out of the softmax, and no row of finite such entries
   only: causality + padding) or ``MASK_GENERAL``.  Waits for the device."""
-  return _native.mask_kind(mask)
+  return min(mask_verdict(mask), MASK_PAIRS)
 
 
 def attention_pairs_fit(q: Tensor, k: Tensor, v: Tensor, mask: Tensor) -> bool:
@@ -256,12 +262,14 @@ def attention_pairs_fit(q: Tensor, k: Tensor, v: Tensor, mask: Tensor) -> bool:
   return _native.attention_pairs_fit(mask.shape[0], q.shape[2], k.shape[2], q.shape[3], v.shape[3])
 
 
-def attention_pairs(q: Tensor, k: Tensor, v: Tensor, mask: Tensor, sm_scale: float) -> Tensor:
+def attention_pairs(q: Tensor, k: Tensor, v: Tensor, mask: Tensor, sm_scale: float, causal_padded: bool = False) -> Tensor:
   """Attention under an additive mask of kind ``MASK_PAIRS`` (1|B, 1, Sq, Skv): as ``attention(bias=mask)``, with the
-  mask as one bit per pair, tiles without a pair left out and tiles with every pair unmasked.  bfloat16 and float16."""
+  mask as one bit per pair, tiles without a pair left out and tiles with every pair unmasked.  bfloat16 and float16.
+  ``causal_padded``: the mask is known to be causality and padding (``MASK_PAIRS_CAUSAL``); the backward shares out its
+  work by that, the results are the same either way."""
   if is_compiling() or overridden(q, k, v, mask):
-    return attn_fwd_pairs(q, k, v, mask, sm_scale)[0]
-  return _native.attention_pairs(q, k, v, mask, sm_scale)
+    return attn_fwd_pairs(q, k, v, mask, sm_scale, causal_padded)[0]
+  return _native.attention_pairs(q, k, v, mask, sm_scale, causal_padded)
 
 
 def l2norm(x: Tensor, eps: float) -> Tensor:
