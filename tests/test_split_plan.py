@@ -76,3 +76,13 @@ def test_equal_walks_are_cut_alike(Dqk):
       if plan.cap:
         n = S // 128
         assert len({plan.first[t + 1] - plan.first[t] for t in range(n)}) == 1, (B, S)
+
+
+@pytest.mark.parametrize("what", ["ids", "pairs"])
+def test_all_pieces_of_tiles_that_are_planned_alike(what):
+  """Without causality a tile's pieces are as many as planned however short documents or a mask leave its walk (a cap of one tile);
+  under causality the walks' lengths say how many."""
+  sizes = dict(Hq=32, Hkv=8, S=2047)
+  plan = _plan(_problem(causal=False, **{what: True}, **sizes))
+  assert plan.cap == 1 and plan.first[1] > 1
+  assert _plan(_problem(causal=True, ids=True, **sizes)).cap > 1 and _plan(_problem(causal=False, pairs=True, padded=True, **sizes)).cap > 1
