@@ -1023,52 +1023,64 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
 // issues at most one instruction every four cycles, and at ~600 instructions for 48 MFMAs per tile a single
 // wave per SIMD leaves the matrix unit idle most of the time, whatever the order of its instructions.
 
-// Sums of the pieces of the split kv tiles, pieces in order: a wave per 32 rows and 64 columns of dK or dV, a workgroup each (small
-// problems have few: four in one workgroup leave half of the CUs out, heads of 64, causal 900 rows 6.6 us instead of 6.1).
-// Bound by latency: 32q/8kv heads of 128, window of 1024 keys over 2047 rows 7.1 us (7.2 when a thread took four values of a row of
-// row-major sums); heads of 64, causal 900 rows in eight pieces 6.1 (4.6), with the dK/dV kernel, whose stores the order is for,
-// packed 2 x 4288 154 (168).  Four pieces' loads at once instead of two: 7.0, 7.2 and 160 + 15, for places no piece was left in.
+// Sums of the pieces of the split kv tiles, pieces in order: a workgroup per 32 rows and 64 columns of dK or dV, a wave of it per
+// 16 of the columns.  Bound by latency: what counts is how many loads are on their way, so all pieces' loads go out together.
+// 32q/8kv, us, this : a wave per 64 columns and one piece's loads beside the one that is added : a thread per four values of rows
+// that the pieces leave row by row.  Heads of 128, 900 rows without a mask in four pieces 7.8 : 10.5 : 6.9, 600 rows 6.6 : 7.3 : 6.0;
+// heads of 64, causal 900 rows in seven 5.3 : 6.3 : 5.0 (dK/dV, whose stores the order is for, 21.1 : 21.1 : 21.6), 600 rows
+// without a mask 4.6 : 5.4 : 4.3 (19.8 : 19.9 : 20.1).
 template <typename T, int DQK, int DV>
-__global__ __launch_bounds__(64) void attn_bwd_parts_kernel(const BwdArgs a) {
-  constexpr int BNK = 128, PER_TILE = (DQK + DV) / 64;
+__global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
+  constexpr int BNK = 128, PER_TILE = (DQK + DV) / 64, RING = 8;
   __shared__ __align__(16) unsigned char smem[4096];
-  const int n_groups = a.B * a.Hkv, lane = threadIdx.x, wave = blockIdx.x & 3;
-  const int part = blockIdx.x / 4 % PER_TILE, tg = blockIdx.x / (4 * PER_TILE);
+  const int n_groups = a.B * a.Hkv, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
+  const int rows32 = blockIdx.x & 3, part = blockIdx.x / 4 % PER_TILE, tg = blockIdx.x / (4 * PER_TILE);
   const int at = tg / n_groups, group = tg - at * n_groups, tile = a.split_tile[at];
   const int n_gl = (n_groups + NUM_XCD - 1) / NUM_XCD, f = a.split_first[at];
   const int planned = ((int)a.split_first[at + 1] - f) / n_gl;
   if (planned == 1) return;
-  const float* p = a.parts + a.split_sums + (((int64_t)(f + group / NUM_XCD * planned) * NUM_XCD + group % NUM_XCD) * BNK + wave * 32) * (DQK + DV) + part * 2048 + lane * 4;
-  f32x4 x[8], y[8];
-  auto load = [&](f32x4 (&t)[8]) {
-#pragma unroll
-    for (int i = 0; i < 8; i++) t[i] = *(const f32x4*)(p + i * 256);
+  const float* p = a.parts + a.split_sums + (((int64_t)(f + group / NUM_XCD * planned) * NUM_XCD + group % NUM_XCD) * BNK + rows32 * 32) * (DQK + DV) + part * 2048 +
+                   wave * 512 + lane * 4;
+  f32x4 x[RING][2];
+  auto load = [&](f32x4 (&t)[2]) {
+    t[0] = *(const f32x4*)p;
+    t[1] = *(const f32x4*)(p + 256);
     p += (int64_t)NUM_XCD * BNK * (DQK + DV);
   };
-  // (two pieces' places are there in any case: their loads go out beside the one of the pieces' number)
-  load(x);
-  load(y);
+  // (where ids or a mask may have left fewer pieces than planned, the third and on wait for the number)
+  const int ahead = a.seg || a.pm.qbits ? 2 : planned;
+#pragma unroll
+  for (int s = 0; s < RING; s++)
+    if (s < 2 || s < ahead) load(x[s]);
   const int n_split = ((const int*)a.parts)[tile * n_groups + group];
   if (n_split == 1) return;
-  f32x16 acc[2];
 #pragma unroll
-  for (int i = 0; i < 8; i++)
+  for (int s = 2; s < RING; s++)
+    if (s >= ahead && s < n_split) load(x[s]);
+  f32x4 acc[2] = {};
+  for (int s0 = 0; s0 < n_split; s0 += RING) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] = x[i][e];
-  for (int s = 1;;) {
+    for (int j = 0; j < RING; j++) {
+      if (s0 + j < n_split) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) x[i] = y[i];
-    if (s + 1 < n_split) load(y);
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int i = 0; i < 8; i++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) acc[i / 4][4 * (i % 4) + e] += x[i][e];
-    if (++s == n_split) break;
+          for (int e = 0; e < 4; e++) acc[i][e] += x[j][i][e];
+        if (s0 + j + RING < n_split) load(x[j]);
+      }
+    }
   }
-  const int b = group / a.Hkv, hk = group - b * a.Hkv, row0 = tile * BNK + wave * 32;
+  const int b = group / a.Hkv, hk = group - b * a.Hkv, row0 = tile * BNK + rows32 * 32;
   const bool is_k = part < DQK / 64;
+  const float sc = is_k ? a.sm_scale : 1.f;
+  // (through LDS to whole lines, as store_rows)
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    *(u32x2*)(smem + ln * 128 + 8 * g + (((2 * wave + i) ^ ((ln >> 1) & 7)) << 4)) = pack4<T>(acc[i][0] * sc, acc[i][1] * sc, acc[i][2] * sc, acc[i][3] * sc);
+  __syncthreads();
+  const int r = tid >> 3, ch = tid & 7;
   T* o = is_k ? (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + row0 * a.dks[2] + part * 64 : (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + row0 * a.dvs[2] + (part * 64 - DQK);
-  store_rows<T, 2>(acc, is_k ? a.sm_scale : 1.f, o, is_k ? a.dks[2] : a.dvs[2], a.Skv - row0, (unsigned)(size_t)smem, lane);
+  if (row0 + r < a.Skv) *(u32x4_a8*)(o + r * (is_k ? a.dks[2] : a.dvs[2]) + ch * 8) = *(const u32x4*)(smem + r * 128 + ((ch ^ ((r >> 1) & 7)) << 4));
 }
 
 template <typename T, int DQK, int DV, int NW, bool CAUSAL, int SEG>
@@ -2187,7 +2199,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
     if (rc) return rc;
     if (a.split) {
       constexpr int PER_TILE = (DQK + DV) / 64;
-      attn_bwd_parts_kernel<T, DQK, DV><<<dim3((unsigned)(n_tiles * groups * PER_TILE * 4)), dim3(64), 0, st>>>(a);
+      attn_bwd_parts_kernel<T, DQK, DV><<<dim3((unsigned)(n_tiles * groups * PER_TILE * 4)), dim3(256), 0, st>>>(a);
       rc = check_launch("tp_attn_bwd(parts)");
       if (rc) return rc;
     }
