@@ -98,7 +98,7 @@ struct BwdArgs {
 // free.  Such a tile's walk is cut into pieces of at most `cap` tiles, one workgroup each, which start by falling length and
 // leave their sums as fp32 in a workspace for a short kernel to add up in order (deterministic).  Ids or a pair mask may leave
 // less to do than the plan knows: the pieces of a tile are then fewer, and the first one tells the short kernel how many.
-// The cap is the one for which the estimate below is least; each finer one has to be worth another 8 %.
+// The cap is the one for which the estimate below is least; each finer one has to be worth another 7 %.
 // Measured (bf16, 32q/8kv heads), dK/dV and the sums, us, whole walks : pieces.  Heads of 128: window of 1024 keys over 2047 rows
 // 114 : 70 + 7; causal 2 x 2048 200 : 160 + 9; causal and padded 4 x 1000 114 : 95 + 9, 4 x 664 76 : 47 + 7; packed 2047 123 :
 // 59 + 7.  Heads of 64: causal 4096 278 : 140 + 8, 4 x 246 24 : 15 + 6.  16 heads of (192,128), padded 1472: 52 : 41 + 8.
@@ -124,9 +124,11 @@ static bool split_plan(tp_attn_bwd_plan& p, int B, int Hkv, int n_rep, int Sq, i
     longest = per[t] > longest ? per[t] : longest;
     total += per[t];
   }
-  // us, measured inside the kernel: start and end of a workgroup, leaving a piece's sums, the kernel that adds them up (at 8 TB/s
-  // out of the caches), a tile of a walk in a CU's only workgroup, beside another one at times, and always beside one
-  const float ends = Dqk <= 64 ? 4.f : 7.f, leave = 4.f, sums = 6.5f, piece_mb = 128.f * (Dqk + Dv) * 4.f * 1e-6f;
+  // us, measured inside the kernel: start and end of a workgroup, leaving a piece's sums, a tile of a walk in a CU's only workgroup,
+  // beside another one at times, and always beside one.  The kernel that adds the sums up (with `chain` for each piece of a tile,
+  // at 5 TB/s), what leaving costs heads of 64 and what a finer cap has to be worth are those whose plans come closest to the
+  // best caps of 500 random problems of 128 to 6600 rows: 1.1 % from them, twice as close as without the last three.
+  const float ends = Dqk <= 64 ? 4.f : 7.f, leave = Dqk <= 64 ? 3.f : 4.f, sums = 3.f, chain = 0.1f, piece_mb = 128.f * (Dqk + Dv) * 4.f * 1e-6f;
   const float alone = Dqk <= 64 ? 1.25f : Dqk <= 128 ? 1.7f : 2.2f, beside = Dqk <= 64 ? 1.4f : alone, shared = Dqk <= 64 ? 1.8f : alone;
   float best = 0.f;
   int best_cap = 0, last_cap = 0, k[64], n_of[64], of[64];
@@ -142,29 +144,30 @@ static bool split_plan(tp_attn_bwd_plan& p, int B, int Hkv, int n_rep, int Sq, i
     const int cap = (longest + n - 1) / n;
     if (cap == last_cap) continue;
     last_cap = cap;
-    int wgs = 0, pieces = 0;
+    int wgs = 0, pieces = 0, most = 1;
     float piece = 0.f;  // the longest
     for (int t = 0; t < n_tiles; t++) {
       k[t] = per[t] > cap ? (per[t] + cap - 1) / cap : 1;
       wgs += k[t] * n_gl;
       pieces += k[t] > 1 ? k[t] * n_gl : 0;
+      most = std::max(most, k[t]);
       piece = fmaxf(piece, (float)per[t] / k[t]);
     }
-    const float enough = n == 1 ? INFINITY : (best_cap == longest ? 0.9f : ids ? 1.f : 0.92f) * best;
+    const float enough = n == 1 ? INFINITY : (ids ? (best_cap == longest ? 0.9f : 1.f) : best_cap == longest ? 0.92f : 0.93f) * best;
     float est;
     if (ids) {
       // documents end the walks somewhere, and the pieces that are left start in any order: what fits then is a share of the work
       // and half of a piece at most, at the rate of a chip that is not full.  (With the estimate above, packed 2 x 4288 with heads
       // of 64 takes 184 + 6 instead of 159 + 11, 4 x 1000 with heads of 128 89 + 5 instead of 80, whole.)
       const float ti = Dqk <= 64 ? 1.f : Dqk <= 128 ? 1.4f : 2.f, even = (float)total * n_gl / slots;
-      const float chain = wgs <= slots ? (float)cap : (float)fmax(even + 0.5f * cap, cap);
-      est = 4.f * ((wgs + slots - 1) / slots) + ti * chain + (pieces ? 5.f + pieces * NUM_XCD * piece_mb / 2.f : 0.f);
+      const float steps = wgs <= slots ? (float)cap : (float)fmax(even + 0.5f * cap, cap);
+      est = 4.f * ((wgs + slots - 1) / slots) + ti * steps + (pieces ? 5.f + pieces * NUM_XCD * piece_mb / 2.f : 0.f);
     } else {
       // at least: the longest piece; what an XCD has to do, spread over its slots; where the pieces are more than r rounds, r + 1
       // of the shortest of those that start one after the other (looked at only where the rest leaves a chance: the order of
       // the pieces is what a plan costs the host; 8192 rows with 8kv heads, all candidates put in order 8.8 us, so 3.9)
-      const float with_pieces = pieces ? leave + sums + pieces * NUM_XCD * piece_mb / 8.f : 0.f;
-      est = fmaxf((wgs <= CUS_PER_XCD ? alone : beside) * piece + ends, (shared * total * n_gl + ends * wgs + leave * pieces) / slots);
+      const float with_pieces = pieces ? sums + chain * most + pieces * NUM_XCD * piece_mb / 5.f : 0.f, left = pieces ? leave : 0.f;
+      est = fmaxf((wgs <= CUS_PER_XCD ? alone : beside) * piece + ends + left, (shared * total * n_gl + ends * wgs + leave * pieces) / slots);
       if (est + with_pieces >= enough) continue;
       if (wgs > slots) {
         sort(k);
@@ -173,7 +176,7 @@ static bool split_plan(tp_attn_bwd_plan& p, int B, int Hkv, int n_rep, int Sq, i
         for (int j = 0, r = 1; j < n_tiles && r < 4; j++) {
           const float len = (float)per[of[j]] / k[of[j]];
           for (seen += k[of[j]] * n_gl; r < 4 && seen > r * slots; r++)
-            est = fmaxf(est, shared * (r * (seen - k[of[j]] * n_gl == r * slots ? before : len) + len) + (r + 1) * ends);
+            est = fmaxf(est, shared * (r * (seen - k[of[j]] * n_gl == r * slots ? before : len) + len) + (r + 1) * ends + left);
           before = len;
         }
       }
