@@ -16,20 +16,22 @@ HOST = """
 #define __device__
 #define __forceinline__ inline
 using std::min;
+constexpr int SEG_NONE = 0, SEG_IDS = 1, SEG_PAIRS = 2;
 static struct { int x; } blockIdx;
 %s
-template <int PER_CU, bool SNAKE> static int grid(int nt, int ni, int ng, int turns, int* seen) {
+template <int PER_CU, int SEG> static int grid(int nt, int ni, int ng, int turns, int* seen) {
   for (unsigned n = 0; n < xcd_grid(nt, ni, ng); n++) {
     blockIdx.x = (int)n;
     int t, i, g;
-    if (!xcd_map<PER_CU, SNAKE>(nt, ni, ng, t, i, g, turns)) continue;
+    if (!xcd_map<PER_CU, SEG>(nt, ni, ng, t, i, g, turns)) continue;
     if (t < 0 || t >= nt || i < 0 || i >= ni || g < 0 || g >= ng || g %% NUM_XCD != (int)(n %% NUM_XCD)) return 1;
     seen[(g * nt + t) * ni + i]++;
   }
   return 0;
 }
-extern "C" int plain(int per_cu, int snake, int nt, int ni, int ng, int turns, int* seen) {
-  return per_cu == 1 ? (snake ? grid<1, true> : grid<1, false>)(nt, ni, ng, turns, seen) : (snake ? grid<2, true> : grid<2, false>)(nt, ni, ng, turns, seen);
+extern "C" int plain(int per_cu, int seg, int nt, int ni, int ng, int turns, int* seen) {
+  auto of = [&](auto f, auto g, auto h) { return (seg == SEG_NONE ? f : seg == SEG_IDS ? g : h)(nt, ni, ng, turns, seen); };
+  return per_cu == 1 ? of(grid<1, SEG_NONE>, grid<1, SEG_IDS>, grid<1, SEG_PAIRS>) : of(grid<2, SEG_NONE>, grid<2, SEG_IDS>, grid<2, SEG_PAIRS>);
 }
 extern "C" int queued(int nt, int ni, int ng, int turns, int* seen) {
   for (int x = 0; x < NUM_XCD; x++) {
@@ -60,13 +62,13 @@ SIZES = [*itertools.product((1, 2, 3, 5, 8, 13, 31, 64, 67), (1, 2, 4, 7), (1, 3
 
 
 @pytest.mark.parametrize("per_cu", [1, 2])
-@pytest.mark.parametrize("snake", [False, True])
-def test_a_grid_does_everything_once(lib, per_cu, snake):
+@pytest.mark.parametrize("seg", [0, 1, 2])
+def test_a_grid_does_everything_once(lib, per_cu, seg):
   for nt, ni, ng in SIZES:
     for turns in {0, 1, 2, (ng + 7) // 8, lib.turns_of(nt, ni, ng, per_cu)}:
       if turns <= (ng + 7) // 8:
         seen = (ctypes.c_int * (nt * ni * ng))()
-        assert lib.plain(per_cu, int(snake), nt, ni, ng, turns, seen) == 0 and set(seen) == {1}, (nt, ni, ng, turns)
+        assert lib.plain(per_cu, seg, nt, ni, ng, turns, seen) == 0 and set(seen) == {1}, (nt, ni, ng, turns)
 
 
 def test_a_queue_does_everything_once(lib):

@@ -387,7 +387,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
       if (group >= a.B * a.Hkv) return;
     } else if (PERSIST && a.queue != nullptr) {
       if (!xcd_item(slot, blockIdx.x % NUM_XCD, (a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.turns)) return;
-    } else if (!xcd_map<dkdv_per_cu(DQK), SEG == SEG_NONE>((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.turns)) return;
+    } else if (!xcd_map<dkdv_per_cu(DQK), SEG>((a.Skv + BNK - 1) / BNK, 1, a.B * a.Hkv, tile, inner, group, a.turns)) return;
     const int b = group / a.Hkv, hk = group - b * a.Hkv;
     const int kv0 = tile * BNK;  // low kv tiles see the most queries: they start first
     const int wkv0 = kv0 + wave * 32;
@@ -1106,7 +1106,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(const BwdArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map<1, false>(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
+  if (!xcd_map<1, SEG_IDS>(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM, wq0 = q0 + wave * 32;
@@ -1710,7 +1710,7 @@ __global__ __launch_bounds__(256, DQK == DV ? 2 : 1) void attn_bwd_dq_plain_kern
   const int n_qt = (a.Sq + BM - 1) / BM;
   clear_queue(a);
   int tile, inner, group;
-  if (!xcd_map<WIDE ? 1 : 2, SEG == SEG_NONE>(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
+  if (!xcd_map<WIDE ? 1 : 2, SEG>(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;  // the longest rows first
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM, wq0 = q0 + wave * 32;

@@ -280,19 +280,21 @@ __device__ __forceinline__ bool xcd_item(int slot, int xcd, int n_tiles, int n_i
 }
 // The item of a workgroup of a plain grid.  An XCD deals its workgroups to its four shader engines in turn, and a workgroup
 // waits for a CU of its own engine.  Numbered by falling length, the first engine gets the longest of every four and the others
-// wait for it; every second four therefore come in reverse (SNAKE: dQ of 128 causal heads of (192,128), S4096 1133 -> 1089 us).
-// Documents have no such order, and there it costs what neighbours share (the same heads, S1898: 341 : 354), so they go without.
+// wait for it; every second four therefore come in reverse (dQ of 128 causal heads of (192,128), S4096 1133 -> 1089 us).
 // Where two workgroups share a CU and all of them run at once, number k + 32 joins number k: the second 32 are numbered from the
 // shortest up, so that the longest shares its CU with the shortest (32q/8kv causal heads of 128, S1728: forward 41.4 -> 39.2, dQ
 // 55.8 -> 52.4).  (Both were read from the hardware ids of running workgroups; only speed depends on them.)
-template <int PER_CU, bool SNAKE>
+// Documents have no such order, and there it costs what neighbours share (the fours: dQ of the same heads, S1898 341 : 354; the
+// second 32: forward of documents of 420 rows without causality, heads of 64, S2000 26.0 : 28.4, heads of 128, 2 x 900 29.2 : 31.5,
+// of 1100 causal rows 27.0 : 28.0), so they go without.  Pair masks, padded causal ones above all, take the second only.
+template <int PER_CU, int SEG>
 __device__ __forceinline__ bool xcd_map(int n_tiles, int n_inner, int n_groups, int& tile, int& inner, int& group, int turns = 0) {
   const int xcd = blockIdx.x % NUM_XCD, n = (n_groups - xcd + NUM_XCD - 1) / NUM_XCD * n_tiles * n_inner;
   int slot = blockIdx.x / NUM_XCD;
   if (slot >= n) return false;
-  if (PER_CU == 2 && n <= 2 * CUS_PER_XCD) {
+  if (PER_CU == 2 && SEG != SEG_IDS && n <= 2 * CUS_PER_XCD) {
     if (slot >= CUS_PER_XCD) slot = CUS_PER_XCD + n - 1 - slot;
-  } else if (SNAKE && (slot & 4) && (slot | 3) < n) {
+  } else if (SEG == SEG_NONE && (slot & 4) && (slot | 3) < n) {
     slot ^= 3;
   }
   return xcd_item(slot, xcd, n_tiles, n_inner, n_groups, tile, inner, group, turns);

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256, (fwd_blocks_per_cu<DQK, CAUSAL, SEG>())) void 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, ln = lane & 31;
   const int n_qt = (a.Sq + BM - 1) / BM;
   int tile, inner, group;
-  if (!xcd_map<fwd_blocks_per_cu<DQK, CAUSAL, SEG>(), SEG == SEG_NONE>(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
+  if (!xcd_map<fwd_blocks_per_cu<DQK, CAUSAL, SEG>(), SEG>(n_qt, a.n_rep, a.B * a.Hkv, tile, inner, group, a.turns)) return;
   const int qt = n_qt - 1 - tile;  // longest (latest) query tiles are scheduled first
   const int b = group / a.Hkv, hk = group - b * a.Hkv, h = hk * a.n_rep + inner;
   const int q0 = qt * BM;
