@@ -86,3 +86,13 @@ def test_all_pieces_of_tiles_that_are_planned_alike(what):
   plan = _plan(_problem(causal=False, **{what: True}, **sizes))
   assert plan.cap == 1 and plan.first[1] > 1
   assert _plan(_problem(causal=True, ids=True, **sizes)).cap > 1 and _plan(_problem(causal=False, pairs=True, padded=True, **sizes)).cap > 1
+
+
+def test_no_counters_where_no_workgroup_loops():
+  """Mask extensions other than a band run on the general instantiation, which takes one key tile per workgroup."""
+  for more, queue in ((dict(), 1), (dict(window_left=500), 1), (dict(soft_cap=4.0), 0), (dict(bias=16), 0), (dict(q_positions=16), 0)):
+    p = _problem(B=8, S=4096)
+    for name, x in more.items():
+      setattr(p, name, x)
+    plan = _plan(p)
+    assert (plan.queue, plan.cap, plan.parts_bytes) == (queue, 0, 1024 * queue), more

@@ -54,6 +54,10 @@ __host__ __device__ constexpr AbSlot ab_slot(int j, int n0, int n1) {
 // workgroups of the dK/dV kernel that share a CU (registers)
 constexpr int dkdv_per_cu(int Dqk) { return Dqk <= 64 ? 2 : 1; }
 
+// Whether a workgroup of an instantiation takes one item after the other when there is a queue; see dkdv_queued.  (The general
+// instantiation spills as it is: one item per workgroup.)
+template <int DQK, bool CAUSAL, int SEG> constexpr bool dkdv_loops = (CAUSAL || SEG == SEG_NONE) && dkdv_per_cu(DQK) == 1;
+
 // A work queue: one counter per XCD, each in a 128-byte line of its own.
 constexpr int QUEUE_STRIDE = 32;
 constexpr size_t QUEUE_BYTES = NUM_XCD * QUEUE_STRIDE * sizeof(unsigned);
@@ -359,9 +363,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
 
   extern __shared__ __align__(16) unsigned char smem[];
 
-  // With a queue a workgroup does one item (kv tile of a group) after the other; see dkdv_queued.  (The general
-  // instantiation spills as it is: one item per workgroup.)
-  constexpr bool PERSIST = (CAUSAL || SEG == SEG_NONE) && dkdv_per_cu(DQK) == 1;
+  // With a queue a workgroup does one item (kv tile of a group) after the other
+  constexpr bool PERSIST = dkdv_loops<DQK, CAUSAL, SEG>;
   int* const next_at = (int*)(smem + NBUF * BUF_BYTES + 3 * ROW_BYTES);  // the slot of the workgroup's next item
   f32x16 dkacc[DKB], dvacc[DVB];
   int slot = blockIdx.x / NUM_XCD;
@@ -2156,8 +2159,7 @@ static int launch_bwd(const BwdArgs& args, hipStream_t st, void* const* ev) {
   const size_t dkdv_smem = Dkdv::bytes(a.Sq);  // (checked before anything is launched)
   TP_REQUIRE(Dkdv::fits(a.Sq), TP_ERR_UNSUPPORTED, "tp_attn_bwd: Sq=%d needs %zu bytes of LDS (max 163840)", a.Sq, dkdv_smem);
   constexpr int DKDV_PER_CU = dkdv_per_cu(DQK);
-  constexpr bool GENERAL = !CAUSAL && SEG == SEG_IDS;
-  if (GENERAL) a.queue = nullptr;
+  if (!dkdv_loops<DQK, CAUSAL, SEG>) a.queue = nullptr;
   mark(ev, 0, st);
   if (!lean) {
     // delta
@@ -2507,7 +2509,8 @@ extern "C" size_t tp_attn_bwd_make_plan(const tp_attn_bwd_problem* p, tp_attn_bw
   } else if (p->causal) {
     hi = 0;
   }
-  plan->queue = dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk);
+  // (mask extensions other than a band run on an instantiation without the loop)
+  plan->queue = dkdv_queued(p->B * p->Hkv, p->Skv, p->Dqk) && (!mx.on || band_only(mx));
   if (plan->queue) plan->parts_bytes = QUEUE_BYTES;
   // Where every tile is planned alike, all its pieces start in the same round: ids or a mask that leave less of them to walk
   // leave less to each.  (Fewer pieces, of at least half the planned length: documents of 230 rows without causality, 32q/8kv,
