@@ -32,7 +32,8 @@ class _Problem(ctypes.Structure):  # tp_attn_bwd_problem
 def _assert_split(B, Hq, Hkv, S, Dqk, Dv, causal=False, pairs=False, soft_cap=0.0, ids=False, padded=False):
   p = _Problem(seg=16 if ids else None, B=B, Hq=Hq, Hkv=Hkv, Sq=S, Skv=S, Dqk=Dqk, Dv=Dv, causal=int(causal), window_left=-1, window_right=-1, sm_scale=0.1,
                soft_cap=soft_cap, pairs=16 if pairs else None, mask_batches=int(pairs), pairs_causal=int(padded))  # fmt: skip
-  assert _lib.load().tp_attn_bwd_parts_bytes(ctypes.byref(p)) > 0
+  # (up to 1024 bytes: the counters of a queue, and no tile is split)
+  assert _lib.load().tp_attn_bwd_parts_bytes(ctypes.byref(p)) > 1024
 
 
 def _documents(S, lengths):
