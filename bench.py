@@ -9,7 +9,7 @@ resident in HBM.  Prints ONE JSON line:
                backward twice that; recomputation is not counted)
   roofline     the dominant kernel (dK/dV backward) against the 2.5 PFLOP/s dense bf16 MFMA peak;
                its launch time comes from HIP events recorded on the launch stream inside the timed
-               region (tp_attn_bwd_ex), `kernels` lists the same for every kernel of the step
+               region (tp_attn_bwd_run_planned), `kernels` lists the same for every kernel of the step
   cpu_baseline the oracle's eager attention (fwd+bwd by autograd) timed on this host's cores on a
                bounded sample of the same workload (one batch element, one kv-head group)
   extra        RMSNorm and RoPE at the same layer shape: GB/s against the 8 TB/s HBM3E peak
@@ -92,20 +92,47 @@ def make_inputs(B, Hq, Hkv, S, D, dev, seed=1235):
   return mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
 
 
+def attention_backward_fn(do, q, k, v, out, lse, seg, dq, dk, dv, sm_scale):
+  """Returns backward(stream, events=None): the causal backward as the operators run it, planned once, with caller-owned
+  buffers (``tp_attn_bwd_run_planned`` with the scratch that the plan asks for)."""
+  import torch
+
+  from torchprime_amd import _lib
+
+  lib = _lib.load()
+  B, Hq, S, Dqk = q.shape
+  p, plan = _lib.AttnBwdProblem(), _lib.AttnBwdPlan()
+  p.B, p.Hq, p.Hkv, p.Sq, p.Skv, p.Dqk, p.Dv = B, Hq, k.shape[1], S, S, Dqk, v.shape[-1]
+  tensors = dict(dout=do, q=q, k=k, v=v, out=out, lse=lse, seg=seg, dq=dq, dk=dk, dv=dv)
+  for name, t in tensors.items():
+    setattr(p, name, _lib.ptr(t))
+  for name, t in zip(("do", "q", "k", "v", "o", "dq", "dk", "dv"), (do, q, k, v, out, dq, dk, dv)):
+    setattr(p, name + "_strides", _lib.strides3(t))
+  p.sm_scale, p.causal, p.window_left, p.window_right, p.dtype = sm_scale, 1, -1, -1, _lib.dtype_code(q.dtype)
+  p.parts_bytes = lib.tp_attn_bwd_make_plan(ctypes.byref(p), ctypes.byref(plan))
+  ws = torch.empty((lib.tp_attn_bwd_workspace_bytes(B, Hq, S),), dtype=torch.uint8, device=q.device)
+  parts = torch.empty((p.parts_bytes,), dtype=torch.uint8, device=q.device)
+  p.ws, p.parts = ws.data_ptr(), parts.data_ptr() if p.parts_bytes else None
+
+  def backward(stream, events=None, keep=(tensors, ws, parts)):
+    _lib.call("tp_attn_bwd_run_planned", ctypes.byref(p), ctypes.byref(plan), stream, events)
+
+  return backward
+
+
 def attention_step_fn(q, k, v, do, sm_scale, hipev=None, ev=None):
   """Returns step(i): one fwd + bwd through the C ABI with caller-owned buffers, events optional."""
   import torch
 
   from torchprime_amd import _lib
 
-  lib = _lib.load()
   B, Hq, S, D = q.shape
   Hkv = k.shape[1]
   dev = q.device
   out = torch.empty((B, S, Hq, D), dtype=q.dtype, device=dev).transpose(1, 2)
   lse = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
   dq, dk, dv = (torch.empty_like(t.transpose(1, 2)).transpose(1, 2) for t in (q, k, v))
-  ws = torch.empty((lib.tp_attn_bwd_workspace_bytes(B, Hq, S) // 4,), dtype=torch.float32, device=dev)
+  backward = attention_backward_fn(do, q, k, v, out, lse, None, dq, dk, dv, sm_scale)
   st = _lib.stream_ptr(dev)
   s3 = _lib.strides3
   code = _lib.dtype_code(q.dtype)
@@ -117,9 +144,7 @@ def attention_step_fn(q, k, v, do, sm_scale, hipev=None, ev=None):
     _lib.call("tp_attn_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), None, out.data_ptr(), lse.data_ptr(),
               B, Hq, Hkv, S, S, D, D, s3(q), s3(k), s3(v), s3(out), sm_scale, 1, code, st)  # fmt: skip
     arr = EvArr(*[e.value for e in ev[i][1:5]]) if ev is not None else None
-    _lib.call("tp_attn_bwd_ex", do.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-              None, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), B, Hq, Hkv, S, S, D, D,
-              s3(do), s3(q), s3(k), s3(v), s3(out), s3(dq), s3(dk), s3(dv), sm_scale, 1, code, st, arr)  # fmt: skip
+    backward(st, arr)
 
   return step, (out, lse, dq, dk, dv)
 
@@ -370,7 +395,6 @@ def bench_other_configs(dev, iters=10, only=None):
 
   from torchprime_amd import _lib
 
-  lib = _lib.load()
   res = {}
   cases = [
     ("llama3_8b_packed_segments", 4, 32, 8, 8192, 128, 128, True),
@@ -398,17 +422,16 @@ def bench_other_configs(dev, iters=10, only=None):
     out = torch.empty((B, S, Hq, Dv), dtype=q.dtype, device=dev).transpose(1, 2)
     lse = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
     dq, dk, dv = (torch.empty_like(t.transpose(1, 2)).transpose(1, 2) for t in (q, k, v))
-    ws = torch.empty((lib.tp_attn_bwd_workspace_bytes(B, Hq, S) // 4,), dtype=torch.float32, device=dev)
     st, s3, code, sm = _lib.stream_ptr(dev), _lib.strides3, _lib.dtype_code(q.dtype), 1.0 / math.sqrt(Dv)
 
     def fwd():
       _lib.call("tp_attn_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.ptr(seg), out.data_ptr(), lse.data_ptr(),
                 B, Hq, Hkv, S, S, Dqk, Dv, s3(q), s3(k), s3(v), s3(out), sm, 1, code, st)  # fmt: skip
 
+    backward = attention_backward_fn(do, q, k, v, out, lse, seg, dq, dk, dv, sm)
+
     def bwd():
-      _lib.call("tp_attn_bwd", do.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                _lib.ptr(seg), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), B, Hq, Hkv, S, S, Dqk, Dv,
-                s3(do), s3(q), s3(k), s3(v), s3(out), s3(dq), s3(dk), s3(dv), sm, 1, code, st)  # fmt: skip
+      backward(st)
 
     for _ in range(3):  # warm-up steps, as for the headline workload
       fwd()
@@ -431,7 +454,7 @@ def bench_other_configs(dev, iters=10, only=None):
     res[name] = {"fwd_ms": round(tf, 4), "bwd_ms": round(tb, 4), "TFLOPs": round(tfl, 1),
                  "frac_of_bf16_mfma_peak": round(tfl / PEAK_BF16_TFLOPS, 4), "allowed_pairs": pairs,
                  "shape": dict(B=B, Hq=Hq, Hkv=Hkv, S=S, Dqk=Dqk, Dv=Dv)}  # fmt: skip
-    del q, k, v, do, out, lse, dq, dk, dv, ws
+    del q, k, v, do, out, lse, dq, dk, dv, backward
   return res
 
 

@@ -96,3 +96,12 @@ def test_no_counters_where_no_workgroup_loops():
       setattr(p, name, x)
     plan = _plan(p)
     assert (plan.queue, plan.cap, plan.parts_bytes) == (queue, 0, 1024 * queue), more
+
+
+def test_the_bindings_structs():
+  assert [(n, getattr(_Problem, n).offset) for n in ("pairs", "parts", "B", "sm_scale", "pairs_causal")] == [
+    (n, getattr(_lib.AttnBwdProblem, n).offset) for n in ("pairs", "parts", "B", "sm_scale", "pairs_causal")]  # fmt: skip
+  p, plan = _lib.AttnBwdProblem(), _lib.AttnBwdPlan()
+  ctypes.memmove(ctypes.byref(p), ctypes.byref(_problem()), ctypes.sizeof(p))
+  assert ctypes.sizeof(p) == ctypes.sizeof(_Problem) and _lib.load().tp_attn_bwd_make_plan(ctypes.byref(p), ctypes.byref(plan)) == plan.parts_bytes
+  assert bytes(plan) == bytes(_plan(_problem())) and list(plan.sizes) == [1, 32, 8, 1024, 1024, 128, 128, 0]

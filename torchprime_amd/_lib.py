@@ -20,6 +20,22 @@ _DTYPE_CODE = {torch.bfloat16: TP_BF16, torch.float16: TP_F16, torch.float32: TP
 
 _I64x3 = c_int64 * 3
 
+
+class AttnBwdProblem(ctypes.Structure):  # tp_attn_bwd_problem
+  _fields_ = [(n, c_void_p) for n in ("dout", "q", "k", "v", "out", "lse", "seg", "q_positions", "bias")]
+  _fields_ += [("bias_strides", _I64x3), ("pairs", c_void_p), ("mask_batches", c_int)]
+  _fields_ += [(n, c_void_p) for n in ("dq", "dk", "dv", "ws", "parts")] + [("parts_bytes", c_size_t)]
+  _fields_ += [(n, c_int) for n in ("B", "Hq", "Hkv", "Sq", "Skv", "Dqk", "Dv")]
+  _fields_ += [(n + "_strides", _I64x3) for n in ("do", "q", "k", "v", "o", "dq", "dk", "dv")]
+  _fields_ += [("sm_scale", c_float)] + [(n, c_int) for n in ("causal", "causal_offset", "window_left", "window_right")]
+  _fields_ += [("soft_cap", c_float), ("dtype", c_int), ("pairs_causal", c_int)]
+
+
+class AttnBwdPlan(ctypes.Structure):  # tp_attn_bwd_plan
+  _fields_ = [("parts_bytes", c_size_t), ("sizes", ctypes.c_int32 * 8)]
+  _fields_ += [(n, ctypes.c_int32) for n in ("queue", "cap", "sums_at")] + [("first", ctypes.c_uint16 * 65), ("tile", ctypes.c_uint8 * 64)]
+
+
 # name -> (restype, argtypes); every symbol the header declares
 SIGNATURES = {
   "tp_version": (c_int, []),
