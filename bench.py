@@ -887,7 +887,7 @@ def summarize_profiles(d, commit):
       o += ["", "Algorithmic bytes for comparison (each operand once): forward 640 MiB (q, k, v in; out, lse out), dK/dV kernel",
             "about 770 MiB (q, dO, k, v, row vectors in; dk, dv out), dQ kernel about 1160 MiB (q, dO, out, k, v, lse in; dq and",
             "the two row vectors for dK/dV out: it computes rowsum(dO o O) itself, there is no delta kernel).  The dK/dV kernel's workgroups",
-            "(one per 128 kv rows) each stream the Q and dO rows at or below their diagonal, 32 passes over Q and dO on",
+            "(256, which take key tiles of 128 rows from a queue) stream for each tile the Q and dO rows at or below its diagonal, 32 passes over Q and dO on",
             "average; what the table shows beyond the algorithmic bytes is the part of those passes that the L2 shared by a",
             "(batch, kv head) group's workgroups did not serve.  The kernels are MFMA-issue bound, not HBM-bound: at their",
             "launch times the read rates are a quarter of the 8 TB/s peak or less."]

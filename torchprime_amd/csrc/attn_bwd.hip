@@ -104,10 +104,9 @@ struct BwdArgs {
 // less to do than the plan knows: the pieces of a tile are then fewer, and the first one tells the short kernel how many.
 // The cap is the one for which the estimate below is least; each finer one has to be worth another 7 %.
 // Measured (bf16, 32q/8kv heads), dK/dV and the sums, us, whole walks : pieces.  Heads of 128: window of 1024 keys over 2047 rows
-// 114 : 70 + 7; causal 2 x 2048 200 : 160 + 9; causal and padded 4 x 1000 114 : 95 + 9, 4 x 664 76 : 47 + 7; packed 2047 123 :
-// 59 + 7.  Heads of 64: causal 4096 278 : 140 + 8, 4 x 246 24 : 15 + 6.  16 heads of (192,128), padded 1472: 52 : 41 + 8.
-// Twice as fine as chosen: 80 + 11 (window), 105 + 14 (4 x 1000), 50 + 10 (4 x 664).  Three rounds of workgroups or more: none
-// was faster in pieces (heads of 64, causal 8 x 3044: 622 : 656 + 41).
+// 114 : 70 + 7; causal 2 x 2048 204 : 157 + 13; causal and padded 4 x 1000 118 : 95 + 9.  Heads of 64: causal 4096 253 : 148 + 8,
+// 4 x 246 24 : 15 + 4.  16 heads of (192,128), causal 1472: 52 : 49 together.  Three rounds of workgroups or more: none was faster
+// in pieces (heads of 64, causal 8 x 3044: 622 : 656 + 41).
 // (host: the plan is made by the C entry points, tp_attn_bwd_make_plan)
 #ifndef TP_BWD_UNIT
 static_assert(sizeof(tp_attn_bwd_plan::first) == sizeof(BwdArgs::split_first) && sizeof(tp_attn_bwd_plan::tile) == sizeof(BwdArgs::split_tile), "the plan's tables");
