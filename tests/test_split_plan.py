@@ -27,8 +27,8 @@ def _plan(p):
 
 @pytest.mark.parametrize("ids", [False, True])
 def test_a_plan_costs_the_host_in_proportion_to_its_tiles(ids):
-  """32 and 64 key tiles (4096 and 8192 rows): at most twice the host's time.  (With every candidate's pieces put in order it
-  took 2.5 times as long; the bound lies between.)"""
+  """32 and 64 key tiles (4096 and 8192 rows): about twice the host's time at most (1.5 without ids, 1.9 with).  (With every
+  candidate's pieces put in order it took 2.5 times as long; the bound lies between.)"""
   def cost(S):
     p, plan = _problem(S=S, ids=ids), _Plan()
     at, to, make = ctypes.byref(p), ctypes.byref(plan), _lib.load().tp_attn_bwd_make_plan
