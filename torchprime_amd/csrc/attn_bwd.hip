@@ -1033,7 +1033,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdArgs) {
 // 32q/8kv, us, this : a wave per 64 columns and one piece's loads beside the one that is added : a thread per four values of rows
 // that the pieces leave row by row.  Heads of 128, 900 rows without a mask in four pieces 7.8 : 10.5 : 6.9, 600 rows 6.6 : 7.3 : 6.0;
 // heads of 64, causal 900 rows in seven 5.3 : 6.3 : 5.0 (dK/dV, whose stores the order is for, 21.1 : 21.1 : 21.6), 600 rows
-// without a mask 4.6 : 5.4 : 4.3 (19.8 : 19.9 : 20.1).
+// without a mask 4.6 : 5.4 : 4.3 (19.8 : 19.9 : 20.1).  Two pieces, which a wave per 64 columns had on their way as well, pay for
+// the waves: window of 1024 keys over 2047 rows 8.1 : 7.7.  (Two waves of 32 columns: 7.9 there, but four pieces 8.3, 900 rows of
+// heads of 64 5.2.)
 template <typename T, int DQK, int DV>
 __global__ __launch_bounds__(256) void attn_bwd_parts_kernel(const BwdArgs a) {
   constexpr int BNK = 128, PER_TILE = (DQK + DV) / 64, RING = 8;
